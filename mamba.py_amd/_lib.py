@@ -1,13 +1,17 @@
-"""ctypes binding of libmambapy_amd.so (declarations: include/mambapy_amd.h).
+"""Loading of the compiled parts: libmambapy_amd.so (the kernels; declarations in
+include/mambapy_amd.h, bound here through ctypes for the status, hash and workspace queries and for
+callers that pass raw pointers) and _mpa_host.so (the operators over PyTorch's C++ API).
 
-There is no fallback: if the library is missing or cannot be loaded, importing the ops
+There is no fallback: if one of them is missing or cannot be loaded, calling the ops
 raises ImportError with the build command; nothing here computes on the CPU.
 """
 import ctypes
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libmambapy_amd.so")
+HOST_PATH = os.path.join(_HERE, "csrc", "_mpa_host.so")
 
 MPA_F32, MPA_BF16 = 0, 1
 MPA_SSCAN_DELTA_SOFTPLUS = 1
@@ -105,6 +109,25 @@ def load():
         getattr(lib, name)
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The operator module, loaded once; ImportError (never a fallback) when it is not there."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise ImportError(f"{HOST_PATH} is missing: build it with `python mamba.py_amd/build.py`.  "
+                              "There is no CPU or PyTorch fallback.")
+        import torch  # noqa: F401  (its libraries have to be in the process first)
+        spec = importlib.util.spec_from_file_location("_mpa_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        _host = mod
+    return _host
 
 
 def check(status: int, what: str) -> None:

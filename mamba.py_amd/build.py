@@ -1,9 +1,9 @@
-"""Build recipe for libmambapy_amd.so (hand-written HIP kernels, gfx950 only).
+"""Build recipe for libmambapy_amd.so (hand-written HIP kernels, gfx950 only) and for
+_mpa_host.so (the operators over PyTorch's C++ API: host code only, compiled with g++).
 
-    python mamba.py_amd/build.py          # compile every csrc/*.hip and link the library
+    python mamba.py_amd/build.py          # compile every csrc/*.hip, link the library, compile csrc/host.cpp
 
-The library is built in-tree (csrc/libmambapy_amd.so) with hipcc; packed-FP32 code
-generation is switched off for the device pass.
+Both are built in-tree, in csrc/; packed-FP32 code generation is switched off for the device pass.
 """
 import hashlib
 import os
@@ -15,6 +15,8 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(CSRC, "libmambapy_amd.so")
 SOURCES = ["sscan_fwd.hip", "sscan_bwd.hip", "sscan_bwd_fast.hip", "pscan.hip", "step.hip", "conv1d.hip", "rmsnorm.hip"]
+HOST_SOURCE = "host.cpp"
+HOST_PATH = os.path.join(CSRC, "_mpa_host.so")
 ARCH = "gfx950"
 HIPCC_FLAGS = [f"--offload-arch={ARCH}", "-fPIC", "-std=c++17",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -64,14 +66,44 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _compile_host() -> str:
+    """csrc/host.cpp -> host.o: plain C++ against the headers of the installed torch."""
+    import sysconfig
+    import torch
+    inc = os.path.join(os.path.dirname(torch.__file__), "include")
+    obj = os.path.join(CSRC, "host.o")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I" + inc, "-I" + os.path.join(inc, "torch", "csrc", "api", "include"), "-I/opt/rocm/include",
+           "-I" + sysconfig.get_paths()["include"], "-c", os.path.join(CSRC, HOST_SOURCE), "-o", obj]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on {HOST_SOURCE}:\n{res.stderr}")
+    return obj
+
+
+def _link_host(obj: str) -> None:
+    import torch
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-shared", "-o", HOST_PATH, obj, "-L" + lib, "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip",
+           "-ltorch_python", "-L" + CSRC, "-lmambapy_amd", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"link failed:\n{res.stderr}")
+
+
 def build(verbose: bool = False) -> str:
-    """Compile all sources for gfx950 and link csrc/libmambapy_amd.so.  Always recompiles."""
-    with ThreadPoolExecutor(max_workers=min(4, len(SOURCES))) as pool:
+    """Compile all sources for gfx950, link csrc/libmambapy_amd.so and csrc/_mpa_host.so.  Always
+    recompiles."""
+    with ThreadPoolExecutor(max_workers=5) as pool:
+        host = pool.submit(_compile_host)
         objs = list(pool.map(_compile, SOURCES))
+        host_obj = host.result()
     cmd = [_hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", LIB_PATH, *objs]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
+    _link_host(host_obj)
     if verbose:
         print(LIB_PATH)
     return LIB_PATH
