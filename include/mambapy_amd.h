@@ -312,6 +312,45 @@ int mpa_ssm_step(const void* x, const void* delta, const float* A, const void* B
                  int64_t bc_stride, int64_t z_stride, int32_t io_dtype, int32_t delta_softplus,
                  void* stream);
 
+/* ---- decode step of a whole layer -----------------------------------------------------------
+ * Replaces, for one token of each of up to MPA_DECODE_MAX_BATCH sequences, the chain that
+ * ResidualBlock.step / MambaBlock.step run (mambapy/mamba.py:114-125, 351-414): RMSNorm, in_proj, the
+ * convolution over the rolling window with silu, x_proj, dt_proj, the state update with softplus, the
+ * gate, out_proj, residual add; four launches.
+ *   x, y : (batch, d_model) io_dtype contiguous.  norm = 1: y = x + block(rmsnorm(x)), the residual block;
+ *     norm = 0: y = block(x), the mixer alone.  y may not alias x.
+ *   x_scaled, x_ssq  optional (norm = 1): x times norm_weight in io_dtype, in the order in which the matrix
+ *     cores take it (mpa_decode_scaled_bytes() bytes), and ceil(d_model / 16) rows of `batch` partial
+ *     sums of squares of x, as the call of the layer before wrote them; NULL: formed here.
+ *   next_norm_weight, y_scaled, y_ssq  optional: the same two for the layer after, whose norm weight is given.
+ *   h_in (NULL: zeros), h_out : (batch, dim, dstate) float32;  window_in, window_out : (batch, dim,
+ *     d_conv-1) io_dtype.  The outputs may be the inputs (in-place update).
+ * Weights: in_weight (2*dim, d_model), x_weight (dt_rank + 2*dstate, dim), dt_weight (dim, dt_rank),
+ * out_weight (d_model, dim), biases of in_proj / out_proj in io_dtype or NULL; norm_weight (d_model),
+ * conv_weight (dim, d_conv), conv_bias, dt_bias (dim), A (dim, dstate), D (dim) float32 (norm_weight and the
+ * biases may be NULL).  d_model and dim are multiples of 4 (float32) / 8 (bfloat16), dstate of 4.
+ */
+#define MPA_DECODE_MAX_BATCH 128
+typedef struct mpa_decode_layer {
+    int64_t batch, d_model, dim, dstate, dt_rank;
+    int32_t d_conv, io_dtype;
+    int32_t norm;
+    float eps;
+    const float* norm_weight;
+    const void *in_weight, *in_bias;
+    const float *conv_weight, *conv_bias;
+    const void *x_weight, *dt_weight;
+    const float *dt_bias, *A, *D;
+    const void *out_weight, *out_bias;
+} mpa_decode_layer;
+
+size_t mpa_decode_layer_workspace_bytes(const mpa_decode_layer* s);
+size_t mpa_decode_scaled_bytes(const mpa_decode_layer* s);
+int mpa_decode_layer_step(const mpa_decode_layer* s, const void* x, const void* x_scaled, const float* x_ssq, void* y,
+                          const float* next_norm_weight, void* y_scaled, float* y_ssq, const float* h_in, float* h_out,
+                          const void* window_in, void* window_out, void* workspace, size_t workspace_bytes,
+                          void* stream);
+
 #ifdef __cplusplus
 }
 #endif

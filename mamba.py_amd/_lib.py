@@ -31,7 +31,8 @@ EXPORTS = ("mpa_version", "mpa_arch", "mpa_source_hash", "mpa_status_string", "m
            "mpa_sscan_ckpt_elems", "mpa_sscan_fwd_workspace_bytes", "mpa_sscan_bwd", "mpa_sscan_bwd_workspace_bytes",
            "mpa_pscan_fwd", "mpa_pscan_bwd", "mpa_pscan_workspace_bytes", "mpa_ssm_step",
            "mpa_conv1d_fwd", "mpa_conv1d_bwd", "mpa_conv1d_bwd_workspace_bytes",
-           "mpa_rmsnorm_fwd", "mpa_rmsnorm_bwd", "mpa_rmsnorm_bwd_workspace_bytes")
+           "mpa_rmsnorm_fwd", "mpa_rmsnorm_bwd", "mpa_rmsnorm_bwd_workspace_bytes",
+           "mpa_decode_layer_workspace_bytes", "mpa_decode_scaled_bytes", "mpa_decode_layer_step")
 
 
 class SscanShape(ctypes.Structure):
@@ -48,6 +49,14 @@ class ConvShape(ctypes.Structure):
                [(n, ctypes.c_int32) for n in ("kernel", "io_dtype", "flags", "reserved")] + \
                [(n, ctypes.c_int64) for n in (
                    "x_sb", "x_sl", "x_sd", "y_sb", "y_sl", "y_sd", "g_sb", "g_sl", "g_sd")]
+
+
+class DecodeLayer(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int64) for n in ("batch", "d_model", "dim", "dstate", "dt_rank")] + \
+               [(n, ctypes.c_int32) for n in ("d_conv", "io_dtype", "norm")] + [("eps", ctypes.c_float)] + \
+               [(n, ctypes.c_void_p) for n in (
+                   "norm_weight", "in_weight", "in_bias", "conv_weight", "conv_bias", "x_weight", "dt_weight",
+                   "dt_bias", "A", "D", "out_weight", "out_bias")]
 
 
 class PscanShape(ctypes.Structure):
@@ -105,6 +114,12 @@ def load():
     lib.mpa_rmsnorm_bwd.argtypes = [vp] * 6 + [i64, i64, f32, i32, vp, sz, vp]
     lib.mpa_rmsnorm_bwd_workspace_bytes.argtypes = [i64, i64]
     lib.mpa_rmsnorm_bwd_workspace_bytes.restype = sz
+    dp = ctypes.POINTER(DecodeLayer)
+    lib.mpa_decode_layer_workspace_bytes.argtypes = [dp]
+    lib.mpa_decode_layer_workspace_bytes.restype = sz
+    lib.mpa_decode_scaled_bytes.argtypes = [dp]
+    lib.mpa_decode_scaled_bytes.restype = sz
+    lib.mpa_decode_layer_step.argtypes = [dp] + [vp] * 12 + [sz, vp]
     for name in EXPORTS:
         getattr(lib, name)
     _lib = lib

@@ -1,7 +1,7 @@
 """Build recipe for libmambapy_amd.so (hand-written HIP kernels, gfx950 only) and for
 _mpa_host.so (the operators over PyTorch's C++ API: host code only, compiled with g++).
 
-    python mamba.py_amd/build.py          # compile every csrc/*.hip, link the library, compile csrc/host.cpp
+    python mamba.py_amd/build.py          # compile every csrc/*.hip, link the library, compile csrc/host*.cpp
 
 Both are built in-tree, in csrc/; packed-FP32 code generation is switched off for the device pass.
 """
@@ -14,8 +14,9 @@ from concurrent.futures import ThreadPoolExecutor
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(CSRC, "libmambapy_amd.so")
-SOURCES = ["sscan_fwd.hip", "sscan_bwd.hip", "sscan_bwd_fast.hip", "pscan.hip", "step.hip", "conv1d.hip", "rmsnorm.hip"]
-HOST_SOURCE = "host.cpp"
+SOURCES = ["sscan_fwd.hip", "sscan_bwd.hip", "sscan_bwd_fast.hip", "pscan.hip", "step.hip", "conv1d.hip", "rmsnorm.hip",
+           "decode.hip"]
+HOST_SOURCES = ["host.cpp", "host_model.cpp"]
 HOST_PATH = os.path.join(CSRC, "_mpa_host.so")
 ARCH = "gfx950"
 HIPCC_FLAGS = [f"--offload-arch={ARCH}", "-fPIC", "-std=c++17",
@@ -66,26 +67,26 @@ def _compile(src: str) -> str:
     return obj
 
 
-def _compile_host() -> str:
-    """csrc/host.cpp -> host.o: plain C++ against the headers of the installed torch."""
+def _compile_host(src: str) -> str:
+    """One of HOST_SOURCES: plain C++ against the headers of the installed torch."""
     import sysconfig
     import torch
     inc = os.path.join(os.path.dirname(torch.__file__), "include")
-    obj = os.path.join(CSRC, "host.o")
+    obj = os.path.join(CSRC, os.path.splitext(src)[0] + ".o")
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            "-I" + inc, "-I" + os.path.join(inc, "torch", "csrc", "api", "include"), "-I/opt/rocm/include",
-           "-I" + sysconfig.get_paths()["include"], "-c", os.path.join(CSRC, HOST_SOURCE), "-o", obj]
+           "-I" + sysconfig.get_paths()["include"], "-c", os.path.join(CSRC, src), "-o", obj]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError(f"g++ failed on {HOST_SOURCE}:\n{res.stderr}")
+        raise RuntimeError(f"g++ failed on {src}:\n{res.stderr}")
     return obj
 
 
-def _link_host(obj: str) -> None:
+def _link_host(objs) -> None:
     import torch
     lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    cmd = ["g++", "-shared", "-o", HOST_PATH, obj, "-L" + lib, "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip",
+    cmd = ["g++", "-shared", "-o", HOST_PATH, *objs, "-L" + lib, "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip",
            "-ltorch_python", "-L" + CSRC, "-lmambapy_amd", "-Wl,-rpath,$ORIGIN"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
@@ -95,15 +96,15 @@ def _link_host(obj: str) -> None:
 def build(verbose: bool = False) -> str:
     """Compile all sources for gfx950, link csrc/libmambapy_amd.so and csrc/_mpa_host.so.  Always
     recompiles."""
-    with ThreadPoolExecutor(max_workers=5) as pool:
-        host = pool.submit(_compile_host)
+    with ThreadPoolExecutor(max_workers=6) as pool:
+        host = [pool.submit(_compile_host, s) for s in HOST_SOURCES]
         objs = list(pool.map(_compile, SOURCES))
-        host_obj = host.result()
+        host_objs = [h.result() for h in host]
     cmd = [_hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", LIB_PATH, *objs]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
-    _link_host(host_obj)
+    _link_host(host_objs)
     if verbose:
         print(LIB_PATH)
     return LIB_PATH

@@ -1,0 +1,79 @@
+// Shared by the sources of the _mpa_host extension: argument conversion and the operators that the
+// layer code calls.
+#pragma once
+
+#include <torch/extension.h>
+
+#include <ATen/core/grad_mode.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+
+#include <array>
+#include <optional>
+
+#include "../../include/mambapy_amd.h"
+
+namespace py = pybind11;
+using at::Tensor;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+typedef std::optional<Tensor> Opt;
+
+namespace mpa_host {
+
+// launch-plan fields, in the order of scan.py: LaunchPlan.packed
+struct Plan {
+    int fwd_ns = 0, bwd_ns = 0, fwd_segments = 0, bwd_segments = 0, flags = 0, pscan_chunks = 0;
+};
+typedef std::array<int, 6> PackedPlan;
+inline Plan unpack(const PackedPlan& p) { return Plan{p[0], p[1], p[2], p[3], p[4], p[5]}; }
+
+inline Tensor val(const Opt& t) { return t.has_value() ? *t : Tensor(); }
+
+inline int io_dtype(at::ScalarType t) {
+    if (t == at::kFloat) return MPA_F32;
+    TORCH_CHECK_TYPE(t == at::kBFloat16, "unsupported dtype ", t,
+                     ": the kernels take float32 or bfloat16 tensors (state and accumulation are float32 in both cases)");
+    return MPA_BF16;
+}
+
+inline void require_gpu(std::initializer_list<const Tensor*> ts) {
+    for (const Tensor* t : ts)
+        TORCH_CHECK(!t->defined() || t->is_cuda(),
+                    "mambapy_amd ops need tensors on a ROCm device (there is no CPU implementation in this package)");
+}
+
+inline void check(int rc, const char* what) {
+    TORCH_CHECK(rc == MPA_OK, what, " failed with status ", rc, ": ", mpa_status_string(rc));
+}
+
+inline void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+inline float* fptr(const Tensor& t) { return static_cast<float*>(ptr(t)); }
+inline void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+inline Tensor cast(const Tensor& t, at::ScalarType dt) { return t.defined() && t.scalar_type() != dt ? t.to(dt) : t; }
+inline Tensor f32c(const Tensor& t) { return t.defined() ? cast(t, at::kFloat).contiguous() : t; }
+inline Tensor unit_rows(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
+inline Tensor empty(at::IntArrayRef shape, at::ScalarType dt, const Tensor& like) {
+    return at::empty(shape, at::TensorOptions().dtype(dt).device(like.device()));
+}
+inline Tensor scratch(size_t bytes, const Tensor& like) { return empty({(int64_t)bytes}, at::kByte, like); }
+
+inline bool tracked(std::initializer_list<const Tensor*> ts) {
+    if (!at::GradMode::is_enabled()) return false;
+    for (const Tensor* t : ts)
+        if (t->defined() && t->requires_grad()) return true;
+    return false;
+}
+
+inline SavedVariable keep(const Tensor& t) { return SavedVariable(t, false); }
+inline Tensor grad_as(const Tensor& g, at::ScalarType dt) { return g.defined() ? cast(g, dt) : g; }
+
+// host_model.cpp
+void bind_model(py::module_& m);
+
+}  // namespace mpa_host

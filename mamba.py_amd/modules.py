@@ -16,9 +16,10 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _lib
 from .conv import causal_conv1d_fn, causal_conv1d_update
 from .norm import add_rmsnorm_fn, rmsnorm_fn, rmsnorm_supported
-from .scan import selective_scan, selective_scan_fn, ssm_step
+from .scan import plan, selective_scan, selective_scan_fn, ssm_step
 
 
 @dataclass
@@ -66,6 +67,19 @@ class MambaConfig:
 # x_proj / dt_proj run on zero-padded copies of their weights where that gives the GEMM library better
 # tile shapes (see MambaBlock._padded_projections); False runs them on the parameters as they are
 PAD_PROJECTIONS = True
+
+
+_HOST = None
+
+
+def _host():
+    """The compiled layer code (csrc/host_model.cpp), told once which classes it stands in for."""
+    global _HOST
+    if _HOST is None:
+        host = _lib.host()
+        host.register_types(MambaBlock, RMSNorm)
+        _HOST = host
+    return _HOST
 
 
 def _frozen_f32(owner, key, p, fn=None):
@@ -297,6 +311,10 @@ class MambaBlock(nn.Module):
         """x : (B, D), cache = (h (B,ED,N) or None, inputs (B,ED,d_conv-1)) ->
         (y (B, D), new cache); mambapy/mamba.py:351-382.  The old cache tuple stays valid."""
         h, inputs = cache
+        if x.is_cuda and not torch.is_grad_enabled():
+            out = _host().block_step(self, x, h, inputs, False)
+            if out is not None:
+                return out[0], out[1:]
         xz = self.in_proj(x)
         xin, z = xz.chunk(2, dim=1)
         if 2 <= self.config.d_conv <= 4 and not torch.is_grad_enabled():
@@ -326,6 +344,10 @@ class MambaBlock(nn.Module):
         """In-place decode step for loops that must not allocate new cache tensors (HIP graph
         replay): x (B, D); h (B, ED, N) float32 and window (B, ED, d_conv-1) are updated in
         place.  Same arithmetic as step()."""
+        if x.is_cuda and not torch.is_grad_enabled():
+            out = _host().block_step(self, x, h, window, True)
+            if out is not None:
+                return out[0]
         xz = self.in_proj(x)
         xin, z = xz.chunk(2, dim=1)
         if 2 <= self.config.d_conv <= 4 and window.is_contiguous() and window.dtype == xin.dtype:
@@ -375,6 +397,11 @@ class Mamba(nn.Module):
         """x : (B, L, D) -> (B, L, D) [, caches].  `caches` (one (h, inputs) pair per layer, as
         returned by an earlier call with return_caches=True, by step() or by empty_caches()) makes
         the call continue that sequence."""
+        if x.is_cuda and not torch.is_grad_enabled():
+            # layers of the plain kind: the whole stack in one call
+            out = _host().stack_forward(list(self.layers), x, caches, bool(return_caches), plan.packed)
+            if out is not None:
+                return out if return_caches else out[0]
         # Same arithmetic as x = layer(x) for every layer, in another order of kernels: the add
         # that ends layer i is done by the norm kernel that starts layer i+1 (pre-norm
         # residual stream: `hidden` is the last mixer output, `residual` the running sum).
@@ -392,6 +419,10 @@ class Mamba(nn.Module):
         return (x, new_caches) if return_caches else x
 
     def step(self, x, caches):
+        if x.is_cuda and not torch.is_grad_enabled() and isinstance(caches, list):
+            y = _host().stack_step(list(self.layers), x, caches, False)
+            if y is not None:
+                return y, caches
         hidden, residual = x, None
         for i, layer in enumerate(self.layers):
             normed, residual = layer.norm.add_norm(hidden, residual)
@@ -401,6 +432,10 @@ class Mamba(nn.Module):
     def step_(self, x, caches):
         """In-place variant of step(): every (h, window) pair of `caches` is updated in place
         (h must be a float32 tensor, not None)."""
+        if x.is_cuda and not torch.is_grad_enabled():
+            y = _host().stack_step(list(self.layers), x, list(caches), True)
+            if y is not None:
+                return y
         hidden, residual = x, None
         for layer, (h, window) in zip(self.layers, caches):
             normed, residual = layer.norm.add_norm(hidden, residual)
