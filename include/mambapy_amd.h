@@ -351,6 +351,40 @@ int mpa_decode_layer_step(const mpa_decode_layer* s, const void* x, const void* 
                           const void* window_in, void* window_out, void* workspace, size_t workspace_bytes,
                           void* stream);
 
+/* ---- weight gradients --------------------------------------------------------------------------
+ * out = P^T . Q for up to MPA_WGRAD_MAX_JOBS pairs of matrices of T rows: what autograd forms for the
+ * projections of a layer (mambapy/mamba.py:210, 244, 247, 232), P the gradient of a projection's output
+ * (rows columns, row stride ldp), Q its input (cols columns, row stride ldq), io_dtype; sums in float32,
+ * added in a fixed order.  out is (rows - gap, keep_cols) contiguous, io_dtype: columns from keep_cols on
+ * and the `gap` rows from gap_at on (padding of P and Q) are left out.  rows, cols and the strides are
+ * multiples of 4, P and Q aligned to four elements.
+ */
+#define MPA_WGRAD_MAX_JOBS 4
+typedef struct mpa_wgrad_job {
+    const void *p, *q;
+    int64_t ldp, ldq;
+    int64_t rows, cols, keep_cols, gap_at, gap;
+    void* out;
+} mpa_wgrad_job;
+size_t mpa_wgrad_workspace_bytes(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_t io_dtype);
+int mpa_wgrad(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_t io_dtype, void* workspace,
+              size_t workspace_bytes, void* stream);
+
+/* ---- conversions of small matrices ----------------------------------------------------------------
+ * Up to MPA_CAST_MAX_JOBS copies of rows x cols elements between float32 and bfloat16 in one launch, each
+ * optionally through -exp(v) (A from A_log, mambapy/mamba.py:239) or v * factor (float32, contiguous).
+ */
+#define MPA_CAST_MAX_JOBS 10
+enum mpa_cast_op { MPA_CAST_COPY = 0, MPA_CAST_NEG_EXP = 1, MPA_CAST_TIMES = 2 };
+typedef struct mpa_cast_job {
+    const void* src;
+    void* dst;
+    const float* factor;
+    int64_t rows, cols, src_pitch, dst_pitch;
+    int32_t src_dtype, dst_dtype, op, reserved;
+} mpa_cast_job;
+int mpa_cast(const mpa_cast_job* jobs, int32_t n, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

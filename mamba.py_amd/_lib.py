@@ -32,7 +32,8 @@ EXPORTS = ("mpa_version", "mpa_arch", "mpa_source_hash", "mpa_status_string", "m
            "mpa_pscan_fwd", "mpa_pscan_bwd", "mpa_pscan_workspace_bytes", "mpa_ssm_step",
            "mpa_conv1d_fwd", "mpa_conv1d_bwd", "mpa_conv1d_bwd_workspace_bytes",
            "mpa_rmsnorm_fwd", "mpa_rmsnorm_bwd", "mpa_rmsnorm_bwd_workspace_bytes",
-           "mpa_decode_layer_workspace_bytes", "mpa_decode_scaled_bytes", "mpa_decode_layer_step")
+           "mpa_decode_layer_workspace_bytes", "mpa_decode_scaled_bytes", "mpa_decode_layer_step",
+           "mpa_wgrad_workspace_bytes", "mpa_wgrad", "mpa_cast")
 
 
 class SscanShape(ctypes.Structure):
@@ -57,6 +58,12 @@ class DecodeLayer(ctypes.Structure):
                [(n, ctypes.c_void_p) for n in (
                    "norm_weight", "in_weight", "in_bias", "conv_weight", "conv_bias", "x_weight", "dt_weight",
                    "dt_bias", "A", "D", "out_weight", "out_bias")]
+
+
+class WgradJob(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in ("p", "q")] + \
+               [(n, ctypes.c_int64) for n in ("ldp", "ldq", "rows", "cols", "keep_cols", "gap_at", "gap")] + \
+               [("out", ctypes.c_void_p)]
 
 
 class PscanShape(ctypes.Structure):
@@ -120,6 +127,11 @@ def load():
     lib.mpa_decode_scaled_bytes.argtypes = [dp]
     lib.mpa_decode_scaled_bytes.restype = sz
     lib.mpa_decode_layer_step.argtypes = [dp] + [vp] * 12 + [sz, vp]
+    wp = ctypes.POINTER(WgradJob)
+    lib.mpa_wgrad_workspace_bytes.argtypes = [wp, i32, i64, i32]
+    lib.mpa_wgrad_workspace_bytes.restype = sz
+    lib.mpa_wgrad.argtypes = [wp, i32, i64, i32, vp, sz, vp]
+    lib.mpa_cast.argtypes = [vp, i32, vp]
     for name in EXPORTS:
         getattr(lib, name)
     _lib = lib

@@ -15,8 +15,8 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(CSRC, "libmambapy_amd.so")
 SOURCES = ["sscan_fwd.hip", "sscan_bwd.hip", "sscan_bwd_fast.hip", "pscan.hip", "step.hip", "conv1d.hip", "rmsnorm.hip",
-           "decode.hip"]
-HOST_SOURCES = ["host.cpp", "host_model.cpp"]
+           "decode.hip", "layer.hip"]
+HOST_SOURCES = ["host.cpp", "host_model.cpp", "host_train.cpp"]
 HOST_PATH = os.path.join(CSRC, "_mpa_host.so")
 ARCH = "gfx950"
 HIPCC_FLAGS = [f"--offload-arch={ARCH}", "-fPIC", "-std=c++17",
@@ -96,7 +96,7 @@ def _link_host(objs) -> None:
 def build(verbose: bool = False) -> str:
     """Compile all sources for gfx950, link csrc/libmambapy_amd.so and csrc/_mpa_host.so.  Always
     recompiles."""
-    with ThreadPoolExecutor(max_workers=6) as pool:
+    with ThreadPoolExecutor(max_workers=7) as pool:
         host = [pool.submit(_compile_host, s) for s in HOST_SOURCES]
         objs = list(pool.map(_compile, SOURCES))
         host_objs = [h.result() for h in host]

@@ -10,16 +10,6 @@
 namespace mpa_host {
 namespace {
 
-template <typename N>
-std::shared_ptr<N> make_node(std::initializer_list<const Tensor*> inputs) {
-    std::shared_ptr<N> n(new N(), torch::autograd::deleteNode);
-    torch::autograd::edge_list edges;
-    edges.reserve(inputs.size());
-    for (const Tensor* t : inputs) edges.push_back(t->defined() ? torch::autograd::impl::gradient_edge(*t) : torch::autograd::Edge());
-    n->set_next_edges(std::move(edges));
-    return n;
-}
-
 // ---- fused selective scan -----------------------------------------------------------------------
 
 mpa_sscan_shape sscan_shape(const Tensor& x, const Tensor& delta, const Tensor& B, const Tensor& y, const Tensor& g,
@@ -435,4 +425,5 @@ PYBIND11_MODULE(_mpa_host, m) {
     m.def("rmsnorm", &rmsnorm, nogil());
     m.def("step", &step, nogil());
     bind_model(m);
+    bind_train(m);
 }

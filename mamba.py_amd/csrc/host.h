@@ -73,7 +73,17 @@ inline bool tracked(std::initializer_list<const Tensor*> ts) {
 inline SavedVariable keep(const Tensor& t) { return SavedVariable(t, false); }
 inline Tensor grad_as(const Tensor& g, at::ScalarType dt) { return g.defined() ? cast(g, dt) : g; }
 
-// host_model.cpp
-void bind_model(py::module_& m);
+template <typename N>
+std::shared_ptr<N> make_node(std::initializer_list<const Tensor*> inputs) {
+    std::shared_ptr<N> n(new N(), torch::autograd::deleteNode);
+    torch::autograd::edge_list edges;
+    edges.reserve(inputs.size());
+    for (const Tensor* t : inputs) edges.push_back(t->defined() ? torch::autograd::impl::gradient_edge(*t) : torch::autograd::Edge());
+    n->set_next_edges(std::move(edges));
+    return n;
+}
+
+void bind_model(py::module_& m);  // host_model.cpp
+void bind_train(py::module_& m);  // host_train.cpp
 
 }  // namespace mpa_host

@@ -1,0 +1,232 @@
+// One mixer (MambaBlock) with gradients as one graph node.
+//
+// Recorded operation by operation, the backward of a block spends a third of its time around the
+// kernels that do the work: concatenating the gradients of the two halves of in_proj's output, adding those
+// of x_proj's to the scan's, filling and copying slices for the padded projections, converting the
+// gradients of small parameters, and weight gradients as library GEMMs whose grids are too small.  Here the
+// kernels write where the next one reads: the scan leaves dz and the convolution dx as the two halves of
+// one matrix, dB and dC go into the columns of x_proj's output gradient, x_proj's input gradient is
+// added to the scan's by the GEMM itself, and the four weight gradients are one launch (mpa_wgrad).
+#include "host_layer.h"
+
+namespace mpa_host {
+namespace {
+
+enum { kIX, kIInW, kIInB, kIConvW, kIConvB, kIXW, kIDtW, kIDtB, kIALog, kID, kIOutW, kIOutB, kInputs };
+
+struct MixerBackward : public Node {
+    // inputs and activations; originals of the parameters whose derived forms are used (their
+    // version counters are checked when they are unpacked)
+    SavedVariable x, win, h0, params[kInputs];
+    Tensor xz, xs, dbc, delta, y, y_pre, ckpt;  // made here, seen by nobody else
+    Tensor A, D, dt_b, conv_w, conv_b, xp, dtp;
+    int64_t Bs = 0, L = 0, d = 0, ED = 0, N = 0, R = 0, Rp = 0, K = 0;
+    Plan plan;
+    std::string name() const override { return "MambaBlockBackward"; }
+    void release_variables() override {
+        x.reset_data(); win.reset_data(); h0.reset_data();
+        for (SavedVariable& v : params) v.reset_data();
+        for (Tensor* t : {&xz, &xs, &dbc, &delta, &y, &y_pre, &ckpt, &A, &D, &dt_b, &conv_w, &conv_b, &xp, &dtp}) t->reset();
+    }
+    variable_list apply(variable_list&& grads) override;
+};
+
+mpa_sscan_shape mixer_scan_shape(const MixerBackward& m, int io, bool backward) {
+    mpa_sscan_shape s{};
+    const int64_t L = m.L, ED = m.ED, P = m.dbc.size(1);
+    s.batch = m.Bs; s.seqlen = L; s.dim = ED; s.dstate = m.N;
+    s.io_dtype = io;
+    s.flags = MPA_SSCAN_DELTA_SOFTPLUS;
+    s.u_sb = s.d_sb = s.y_sb = L * ED; s.u_sl = s.d_sl = s.y_sl = ED;
+    s.u_sd = s.d_sd = s.y_sd = s.z_sd = s.g_sd = 1;
+    s.z_sb = L * 2 * ED; s.z_sl = 2 * ED;
+    // the gradients of x and delta are the halves of one (T, 2 ED) matrix, that of z the second half of another
+    s.g_sb = L * 2 * ED; s.g_sl = 2 * ED;
+    s.bc_sb = s.dbc_sb = L * P; s.bc_sl = s.dbc_sl = P;
+    s.plan_states_per_lane = backward ? m.plan.bwd_ns : m.plan.fwd_ns;
+    s.plan_segments = backward ? m.plan.bwd_segments : m.plan.fwd_segments;
+    s.plan_flags = m.plan.flags;
+    return s;
+}
+
+mpa_conv_shape mixer_conv_shape(const MixerBackward& m, int io, bool backward) {
+    mpa_conv_shape s{};
+    const int64_t L = m.L, ED = m.ED, out = backward ? 2 * ED : ED;
+    s.batch = m.Bs; s.seqlen = L; s.dim = ED;
+    s.kernel = (int)m.K;
+    s.io_dtype = io;
+    s.flags = MPA_CONV_SILU;
+    s.x_sb = s.g_sb = L * 2 * ED; s.x_sl = s.g_sl = 2 * ED;
+    s.y_sb = L * out; s.y_sl = out;
+    s.x_sd = s.y_sd = s.g_sd = 1;
+    return s;
+}
+
+// (y, h_last or None, window or None), or None: not a block that can run here
+py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h_in, const Opt& win_in, bool return_cache,
+                       const PackedPlan& packed) {
+    if (!at::GradMode::is_enabled() || autocast_on() || !x_in.is_cuda() || x_in.dim() != 3 || x_in.numel() == 0) return py::none();
+    LayerHandle* l = handle_of(block.ptr(), false);
+    const Tensor hc = val(h_in), wc = val(win_in);
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::DeviceGuard guard(x_in.device());
+        if (!l || !l->ready(x_in) || !l->forward_ok || l->N % 2) return py::none();
+        if (unpack(packed).flags & MPA_PLAN_BWD_GENERAL) return py::none();
+        const int64_t Bs = x_in.size(0);
+        if (hc.defined() && !fits(hc, {Bs, l->ED, l->N}, at::kFloat, l->device)) return py::none();
+        if (wc.defined() && !fits(wc, {Bs, l->ED, l->K - 1}, l->dt, l->device)) return py::none();
+        l->pad();
+    }
+    const std::array<int, kInputs> from = {-1, kInW, kInB, kConvW, kConvB, kXW, kDtW, kDtB, kALog, kD, kOutW, kOutB};
+    const Tensor none;
+    std::array<const Tensor*, kInputs> in;
+    in[kIX] = &x_in;
+    bool any = x_in.requires_grad();
+    for (int i = 1; i < kInputs; ++i) {
+        in[i] = &l->p[from[i]].t;
+        any |= in[i]->defined() && in[i]->requires_grad();
+    }
+    if (!any) return py::none();
+    auto node = make_node<MixerBackward>({in[0], in[1], in[2], in[3], in[4], in[5], in[6], in[7], in[8], in[9], in[10], in[11]});
+    Tensor out, h_last, window;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::DeviceGuard guard(x_in.device());
+        MixerBackward& m = *node;
+        const Tensor x = x_in.contiguous();
+        const auto dt = x.scalar_type();
+        const int io = io_dtype(dt);
+        const size_t es = x.element_size();
+        m.Bs = x.size(0); m.L = x.size(1); m.d = l->d; m.ED = l->ED; m.N = l->N; m.R = l->R; m.Rp = l->Rp; m.K = l->K;
+        m.plan = unpack(packed);
+        m.A = l->A; m.D = l->D.t; m.dt_b = l->dt_b.t; m.conv_w = l->conv_w.t; m.conv_b = l->conv_b.t; m.xp = l->xp; m.dtp = l->dtp;
+        const int64_t T = m.Bs * m.L, ED = m.ED, N = m.N;
+        const Tensor x2 = x.view({T, m.d});
+        void* stream = stream_of(x);
+        m.xz = l->p[kInB].t.defined() ? at::addmm(l->p[kInB].t, x2, l->in_wt) : at::mm(x2, l->in_wt);
+        m.xs = empty({T, ED}, dt, x);
+        if (return_cache) {
+            window = empty({m.Bs, ED, m.K - 1}, dt, x);
+            h_last = empty({m.Bs, ED, N}, at::kFloat, x);
+        }
+        const mpa_conv_shape cv = mixer_conv_shape(m, io, false);
+        check(mpa_conv1d_fwd(&cv, ptr(m.xz), fptr(m.conv_w), fptr(m.conv_b), ptr(wc), ptr(m.xs), ptr(window), stream), "mpa_conv1d_fwd");
+        m.dbc = at::mm(m.xs, l->xp_t);
+        m.delta = at::mm(m.dbc.narrow(1, 0, m.Rp), l->dtp_t);
+        m.y = empty({T, ED}, dt, x);
+        m.y_pre = empty({T, ED}, dt, x);
+        const mpa_sscan_shape sc = mixer_scan_shape(m, io, false);
+        m.ckpt = empty({mpa_sscan_ckpt_elems(&sc)}, at::kFloat, x);
+        const size_t nbytes = mpa_sscan_fwd_workspace_bytes(&sc, 1);
+        const Tensor ws = scratch(nbytes, x);
+        const char* bc = static_cast<const char*>(ptr(m.dbc)) + m.Rp * es;
+        check(mpa_sscan_fwd(&sc, ptr(m.xs), ptr(m.delta), fptr(m.A), bc, bc + N * es, fptr(m.D), static_cast<const char*>(ptr(m.xz)) + ED * es,
+                            fptr(m.dt_b), fptr(hc), ptr(m.y), ptr(m.y_pre), fptr(m.ckpt), fptr(h_last), ptr(ws), nbytes, stream),
+              "mpa_sscan_fwd");
+        out = (l->p[kOutB].t.defined() ? at::addmm(l->p[kOutB].t, m.y, l->out_wt) : at::mm(m.y, l->out_wt)).view({m.Bs, m.L, m.d});
+        m.x = keep(x);
+        m.win = keep(wc);
+        m.h0 = keep(hc);
+        for (int i = 1; i < kInputs; ++i) m.params[i] = keep(*in[i]);
+    }
+    torch::autograd::set_history(out, node);
+    return py::make_tuple(out, return_cache ? py::cast(h_last) : py::object(py::none()),
+                          return_cache ? py::cast(window) : py::object(py::none()));
+}
+
+variable_list MixerBackward::apply(variable_list&& grads) {
+    variable_list g(kInputs);
+    if (!grads[0].defined()) return g;
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor x_ = x.unpack(), win_ = win.unpack(), h0_ = h0.unpack();
+    TORCH_CHECK(xz.defined(), "Trying to backward through the graph a second time: the saved tensors have been freed "
+                              "(specify retain_graph=True)");
+    Tensor w[kInputs];
+    for (int i = 1; i < kInputs; ++i) w[i] = params[i].unpack();
+    const c10::DeviceGuard guard(x_.device());
+    const auto dt = x_.scalar_type();
+    const int io = io_dtype(dt);
+    const size_t es = x_.element_size();
+    const int64_t T = Bs * L, P = dbc.size(1), used = Rp + 2 * N;
+    void* stream = stream_of(x_);
+    auto at_col = [&](const Tensor& t, int64_t col) { return static_cast<char*>(ptr(t)) + col * es; };
+    const Tensor x2 = x_.view({T, d}), dout = cast(grads[0], dt).contiguous().view({T, d});
+
+    const Tensor dy = at::mm(dout, w[kIOutW]);
+    const Tensor dxz = empty({T, 2 * ED}, dt, x_), dxs_ddelta = empty({T, 2 * ED}, dt, x_), ddbc = empty({T, P}, dt, x_);
+    Tensor dxs = dxs_ddelta.narrow(1, 0, ED);
+    const Tensor ddelta = dxs_ddelta.narrow(1, ED, ED);
+    const Tensor dA = empty({ED, N}, at::kFloat, x_), dD = empty({ED}, at::kFloat, x_), ddt_b = empty({ED}, at::kFloat, x_);
+    {
+        const mpa_sscan_shape s = mixer_scan_shape(*this, io, true);
+        const size_t nbytes = mpa_sscan_bwd_workspace_bytes(&s);
+        const Tensor ws = scratch(nbytes, x_);
+        check(mpa_sscan_bwd(&s, ptr(xs), ptr(delta), fptr(A), at_col(dbc, Rp), at_col(dbc, Rp + N), fptr(D), at_col(xz, ED), fptr(dt_b),
+                            fptr(h0_), ptr(dy), ptr(y_pre), fptr(ckpt), ptr(dxs_ddelta), at_col(dxs_ddelta, ED), fptr(dA), at_col(ddbc, Rp),
+                            at_col(ddbc, Rp + N), fptr(dD), at_col(dxz, ED), fptr(ddt_b), ptr(ws), nbytes, stream),
+              "mpa_sscan_bwd");
+    }
+    Tensor ddlow = ddbc.narrow(1, 0, Rp);
+    at::mm_out(ddlow, ddelta, dtp);
+    // (the columns past `used` were never written)
+    at::addmm_out(dxs, dxs, ddbc.narrow(1, 0, used), xp.narrow(0, 0, used));
+    const Tensor dconv_w = empty({ED, K}, at::kFloat, x_), dconv_b = conv_b.defined() ? empty({ED}, at::kFloat, x_) : Tensor();
+    {
+        const mpa_conv_shape s = mixer_conv_shape(*this, io, true);
+        const size_t nbytes = mpa_conv1d_bwd_workspace_bytes(&s);
+        const Tensor ws = scratch(nbytes, x_);
+        check(mpa_conv1d_bwd(&s, ptr(xz), fptr(conv_w), fptr(conv_b), ptr(win_), ptr(dxs_ddelta), ptr(dxz), fptr(dconv_w), fptr(dconv_b),
+                             ptr(ws), nbytes, stream),
+              "mpa_conv1d_bwd");
+    }
+    if (task_should_compute_output(kIX)) g[kIX] = at::mm(dxz, w[kIInW]).view({Bs, L, d});
+
+    // weight gradients.  float32: the wide ones are compute bound and stay with the GEMM library
+    std::vector<mpa_wgrad_job> jobs;
+    auto want = [&](int i, const void* p, int64_t ldp, int64_t rows, const void* q, int64_t ldq, int64_t cols, int64_t keep_cols,
+                    int64_t gap_at, int64_t gap) {
+        if (!task_should_compute_output(i)) return;
+        g[i] = empty(w[i].sizes(), dt, x_);
+        jobs.push_back(mpa_wgrad_job{p, q, ldp, ldq, rows, cols, keep_cols, gap_at, gap, ptr(g[i])});
+    };
+    if (io == MPA_BF16) {
+        want(kIInW, ptr(dxz), 2 * ED, 2 * ED, ptr(x2), d, d, d, 0, 0);
+        want(kIOutW, ptr(dout), d, d, ptr(y), ED, ED, ED, 0, 0);
+    } else {
+        if (task_should_compute_output(kIInW)) g[kIInW] = at::mm(dxz.t(), x2);
+        if (task_should_compute_output(kIOutW)) g[kIOutW] = at::mm(dout.t(), y);
+    }
+    want(kIXW, ptr(ddbc), P, used, ptr(xs), ED, ED, ED, R, Rp - R);
+    want(kIDtW, at_col(dxs_ddelta, ED), 2 * ED, ED, ptr(dbc), P, Rp, R, 0, 0);
+    if (!jobs.empty()) {
+        const size_t nbytes = mpa_wgrad_workspace_bytes(jobs.data(), (int)jobs.size(), T, io);
+        const Tensor ws = scratch(nbytes, x_);
+        check(mpa_wgrad(jobs.data(), (int)jobs.size(), T, io, ptr(ws), nbytes, stream), "mpa_wgrad");
+    }
+    if (w[kIInB].defined() && task_should_compute_output(kIInB)) g[kIInB] = dxz.sum(0);
+    if (w[kIOutB].defined() && task_should_compute_output(kIOutB)) g[kIOutB] = dout.sum(0);
+
+    // small parameters: their own types; dA_log = dA * A, because A = -exp(A_log)
+    std::vector<mpa_cast_job> casts;
+    auto small = [&](int i, const Tensor& f32, int op, const float* factor) {
+        if (!w[i].defined() || !f32.defined() || !task_should_compute_output(i)) return;
+        if (op == MPA_CAST_COPY && w[i].scalar_type() == at::kFloat) { g[i] = f32.view(w[i].sizes()); return; }
+        g[i] = empty(w[i].sizes(), w[i].scalar_type(), x_);
+        casts.push_back(cast_job(f32, g[i], 1, f32.numel(), 0, 0, op, factor));
+        casts.back().src_pitch = casts.back().dst_pitch = f32.numel();
+    };
+    small(kIConvW, dconv_w, MPA_CAST_COPY, nullptr);
+    small(kIConvB, dconv_b, MPA_CAST_COPY, nullptr);
+    small(kIDtB, ddt_b, MPA_CAST_COPY, nullptr);
+    small(kIALog, dA, MPA_CAST_TIMES, fptr(A));
+    small(kID, dD, MPA_CAST_COPY, nullptr);
+    if (!casts.empty()) check(mpa_cast(casts.data(), (int)casts.size(), stream), "mpa_cast");
+    return g;
+}
+
+}  // namespace
+
+void bind_train(py::module_& m) { m.def("block_train", &block_train); }
+
+}  // namespace mpa_host

@@ -1,0 +1,357 @@
+// Kernels of a layer's training pass around the library GEMMs, for gfx950:
+//
+//   wgrad      weight gradients out = P^T . Q of several projections in one launch (P (T, M) the
+//              gradient of a projection's output, Q (T, N) its input, T = batch * length rows)
+//   prepare    the float32 and padded forms of a layer's parameters, in one launch
+//   finish     the float32 gradients of its small parameters in the parameters' own types, in one launch
+//
+// wgrad.  The sum runs over thousands of rows and gives a matrix of a few hundred rows and columns, so
+// a kernel that parallelises over the output alone leaves most of the chip idle: as library GEMMs
+// the four products of a layer at width 768 and 8000 rows (3072 x 768, 768 x 1536, 80 x 1536,
+// 1536 x 48) took 88 + 80 + 80 + 54 us.  Here the 128 x 128 output tiles of all of them are one grid,
+// cut over T into `splits` parts that a second kernel adds in a fixed order.
+#include "common.h"
+
+namespace mpa {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kWgTile = 128;
+
+struct WgradJob {
+    const void *p, *q;
+    int64_t ldp, ldq;
+    int M, N;
+    int tiles_n, first_tile;  // tiles of this job: first_tile + tm * tiles_n + tn (p_major) or tn * tiles_m + tm
+    int tiles_m, p_major;
+    int keep, gap_at, gap;  // output columns kept; output row r comes from row r (+ gap from gap_at on) of P^T Q
+    void* out;
+};
+struct WgradParams {
+    WgradJob job[MPA_WGRAD_MAX_JOBS];
+    int jobs, tiles, splits;
+    int64_t T;
+    float* part;  // [splits][tiles][128][128] in the order of the kernel's tiles
+};
+
+__device__ __forceinline__ int wgrad_find(const WgradParams& p, int tile) {
+    int j = 0;
+    while (j + 1 < p.jobs && tile >= p.job[j + 1].first_tile) ++j;
+    return j;
+}
+__device__ __forceinline__ void wgrad_tile_at(const WgradJob& j, int tile, int& tm, int& tn) {
+    const int local = tile - j.first_tile;
+    if (j.p_major) {
+        tm = local / j.tiles_n;
+        tn = local - tm * j.tiles_n;
+    } else {
+        tn = local / j.tiles_m;
+        tm = local - tn * j.tiles_m;
+    }
+}
+
+// Workgroup -> (tile, split).  The chip hands workgroups to its 8 XCDs in turn and each has its own L2:
+// an XCD works on one split of T and on a run of neighbouring tiles, which share their P or Q panel
+// (the wider of the two is the outer index of the run), so that an L2 fetches its part of the wide
+// operand once and of the narrow one once.
+__device__ __forceinline__ bool wgrad_work(const WgradParams& p, int& tile, int& split) {
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int groups = 8 / p.splits, per = (p.tiles + groups - 1) / groups;
+    split = xcd / groups;
+    tile = (xcd % groups) * per + slot;
+    return slot < per && tile < p.tiles;
+}
+
+// bfloat16.  Both operands have the summation index as their slow dimension, the matrix cores want it
+// fast: a lane loads four neighbouring columns of eight rows (8 bytes each), turns the 4 x 8 block with
+// v_perm and stores four 16-byte units (8 rows of one column), the operand of one lane, into LDS.
+// The units of a panel lie in the order column % 4, column / 4: neighbouring lanes write
+// neighbouring units, and a 16-row operand tile is 16 neighbouring units (its rows are then every
+// fourth column of the matrix, which only the order of the partial sums has to know).
+// 64 rows of T per step, four waves of 64 x 64 outputs, loads of the next step in registers meanwhile.
+constexpr int kWgStep = 64;
+__device__ __forceinline__ int wg_unit_to_col(int u) { return 4 * (u & 31) + (u >> 5); }
+
+__global__ void __launch_bounds__(256, 2) wgrad_bf16_kernel(const WgradParams p) {
+    __shared__ u32x4 lds[2][2][8][kWgTile];  // [buffer][P, Q][group of 8 rows][unit]
+    int tile, split;
+    if (!wgrad_work(p, tile, split)) return;
+    const WgradJob& job = p.job[wgrad_find(p, tile)];
+    int tm, tn;
+    wgrad_tile_at(job, tile, tm, tn);
+    const int lane = threadIdx.x & 63, wave = wave_id();
+    const int64_t steps = (p.T + kWgStep - 1) / kWgStep, per = (steps + p.splits - 1) / p.splits;
+    const int64_t t_begin = split * per * kWgStep, t_end = min(p.T, (split + 1) * per * kWgStep);
+    // this lane's columns and rows of a step: columns 4*(lane % 32) .., rows 16*wave + 8*(lane / 32) ..
+    const int cq = 4 * (lane & 31), r0 = 16 * wave + 8 * (lane >> 5), g = 2 * wave + (lane >> 5);
+    const uint16_t* src[2] = {static_cast<const uint16_t*>(job.p) + min(tm * kWgTile + cq, job.M - 4),
+                              static_cast<const uint16_t*>(job.q) + min(tn * kWgTile + cq, job.N - 4)};
+    const int64_t ld[2] = {job.ldp, job.ldq};
+    u32x2 raw[2][8];
+    auto request = [&](int64_t t) {
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                const int64_t row = t + r0 + r;
+                raw[o][r] = row < t_end ? *reinterpret_cast<const u32x2*>(src[o] + row * ld[o]) : u32x2{0, 0};
+            }
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                u32x4 unit;
+                // halves c % 2 of words c / 2 of two rows
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    unit[r] = __builtin_amdgcn_perm(raw[o][2 * r + 1][c >> 1], raw[o][2 * r][c >> 1], c & 1 ? 0x07060302u : 0x05040100u);
+                lds[buf][o][g][32 * c + (lane & 31)] = unit;
+            }
+    };
+    f32x4 acc[4][4] = {};
+    const int mu = 64 * (wave >> 1), nu = 64 * (wave & 1);  // the wave's units of P and Q
+    request(t_begin);
+    int buf = 0;
+    for (int64_t t = t_begin; t < t_end; t += kWgStep) {
+        stage(buf);
+        __syncthreads();
+        if (t + kWgStep < t_end) request(t + kWgStep);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            bf16x8 a[4], b[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                a[i] = __builtin_bit_cast(bf16x8, lds[buf][0][4 * k + (lane >> 4)][mu + 16 * i + (lane & 15)]);
+                b[i] = __builtin_bit_cast(bf16x8, lds[buf][1][4 * k + (lane >> 4)][nu + 16 * i + (lane & 15)]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+        buf ^= 1;  // (two buffers: the barrier of the next step separates these reads from the writes after it)
+    }
+    float* out = p.part + ((int64_t)split * p.tiles + tile) * kWgTile * kWgTile;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                out[(mu + 16 * i + 4 * (lane >> 4) + r) * kWgTile + nu + 16 * j + (lane & 15)] = acc[i][j][r];
+}
+
+// float32.  The matrix-core operand of four rows x 16 columns is what a row-major panel in LDS gives as
+// it is; rows are 16 floats longer than the tile so that the four rows of an operand fall on different banks.
+constexpr int kWgStepF = 16, kWgPitch = kWgTile + 16;
+__global__ void __launch_bounds__(256, 2) wgrad_f32_kernel(const WgradParams p) {
+    __shared__ float lds[2][2][kWgStepF][kWgPitch];
+    int tile, split;
+    if (!wgrad_work(p, tile, split)) return;
+    const WgradJob& job = p.job[wgrad_find(p, tile)];
+    int tm, tn;
+    wgrad_tile_at(job, tile, tm, tn);
+    const int lane = threadIdx.x & 63, wave = wave_id();
+    const int64_t steps = (p.T + kWgStepF - 1) / kWgStepF, per = (steps + p.splits - 1) / p.splits;
+    const int64_t t_begin = split * per * kWgStepF, t_end = min(p.T, (split + 1) * per * kWgStepF);
+    const int cq = 4 * (threadIdx.x & 31), r0 = threadIdx.x >> 5;  // four columns of rows r0 and r0 + 8
+    const float* src[2] = {static_cast<const float*>(job.p) + min(tm * kWgTile + cq, job.M - 4),
+                           static_cast<const float*>(job.q) + min(tn * kWgTile + cq, job.N - 4)};
+    const int64_t ld[2] = {job.ldp, job.ldq};
+    f32x4 raw[2][2];
+    auto request = [&](int64_t t) {
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const int64_t row = t + r0 + 8 * r;
+                raw[o][r] = row < t_end ? *reinterpret_cast<const f32x4*>(src[o] + row * ld[o]) : f32x4{0, 0, 0, 0};
+            }
+    };
+    f32x4 acc[4][4] = {};
+    const int mu = 64 * (wave >> 1), nu = 64 * (wave & 1);
+    request(t_begin);
+    int buf = 0;
+    for (int64_t t = t_begin; t < t_end; t += kWgStepF) {
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+#pragma unroll
+            for (int r = 0; r < 2; ++r) *reinterpret_cast<f32x4*>(&lds[buf][o][r0 + 8 * r][cq]) = raw[o][r];
+        __syncthreads();
+        if (t + kWgStepF < t_end) request(t + kWgStepF);
+#pragma unroll
+        for (int k = 0; k < kWgStepF / 4; ++k) {
+            float a[4], b[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                a[i] = lds[buf][0][4 * k + (lane >> 4)][mu + 16 * i + (lane & 15)];
+                b[i] = lds[buf][1][4 * k + (lane >> 4)][nu + 16 * i + (lane & 15)];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+        buf ^= 1;
+    }
+    float* out = p.part + ((int64_t)split * p.tiles + tile) * kWgTile * kWgTile;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                out[(mu + 16 * i + 4 * (lane >> 4) + r) * kWgTile + nu + 16 * j + (lane & 15)] = acc[i][j][r];
+}
+
+// Sum over the splits, in order; a thread takes four neighbouring output columns of one row of a tile.
+template <typename IO>
+__global__ void __launch_bounds__(256) wgrad_sum_kernel(const WgradParams p) {
+    const int tile = blockIdx.x >> 4, local = (blockIdx.x & 15) * 256 + threadIdx.x;  // 128 rows x 32 column groups
+    const WgradJob& job = p.job[wgrad_find(p, tile)];
+    int tm, tn;
+    wgrad_tile_at(job, tile, tm, tn);
+    constexpr bool UNITS = sizeof(IO) == 2;
+    const int u = local >> 5, q = local & 31;
+    const float* src = p.part + (int64_t)tile * kWgTile * kWgTile + u * kWgTile;
+    const int64_t pitch = (int64_t)p.tiles * kWgTile * kWgTile;
+    f32x4 s = {0, 0, 0, 0};
+    for (int k = 0; k < p.splits; ++k) {
+        const float* v = src + k * pitch;
+        if constexpr (UNITS) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) s[c] += v[32 * c + q];
+        } else {
+            s += *reinterpret_cast<const f32x4*>(v + 4 * q);
+        }
+    }
+    int row = tm * kWgTile + (UNITS ? wg_unit_to_col(u) : u);
+    const int col = tn * kWgTile + 4 * q;
+    if (row >= job.M || (row >= job.gap_at && row < job.gap_at + job.gap)) return;
+    if (row >= job.gap_at) row -= job.gap;
+    IO* out = static_cast<IO*>(job.out) + (int64_t)row * job.keep + col;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (col + c < job.keep) out[c] = from_float<IO>(s[c]);
+}
+
+static int wgrad_params(WgradParams& p, const mpa_wgrad_job* jobs, int n, int64_t T, int io_dtype) {
+    if (!jobs) return MPA_ERR_NULL_POINTER;
+    if (n <= 0 || n > MPA_WGRAD_MAX_JOBS || T <= 0) return MPA_ERR_BAD_SHAPE;
+    if (io_dtype != MPA_F32 && io_dtype != MPA_BF16) return MPA_ERR_BAD_DTYPE;
+    p.jobs = n;
+    p.T = T;
+    int64_t tiles = 0;
+    for (int i = 0; i < n; ++i) {
+        const mpa_wgrad_job& s = jobs[i];
+        WgradJob& j = p.job[i];
+        if (s.rows < 4 || s.cols < 4 || s.rows % 4 || s.cols % 4 || s.rows > 1 << 20 || s.cols > 1 << 20 || s.keep_cols < 1 ||
+            s.keep_cols > s.cols || s.gap < 0 || s.gap_at < 0 || s.gap_at + s.gap > s.rows)
+            return MPA_ERR_BAD_SHAPE;
+        if (s.ldp < s.rows || s.ldq < s.cols || s.ldp % 4 || s.ldq % 4) return MPA_ERR_BAD_STRIDE;
+        j.p = s.p; j.q = s.q; j.out = s.out;
+        j.ldp = s.ldp; j.ldq = s.ldq;
+        j.M = (int)s.rows; j.N = (int)s.cols;
+        j.keep = (int)s.keep_cols;
+        j.gap_at = s.gap ? (int)s.gap_at : j.M; j.gap = (int)s.gap;
+        j.tiles_m = (j.M + kWgTile - 1) / kWgTile;
+        j.tiles_n = (j.N + kWgTile - 1) / kWgTile;
+        j.p_major = j.tiles_m >= j.tiles_n;
+        j.first_tile = (int)tiles;
+        tiles += (int64_t)j.tiles_m * j.tiles_n;
+        if (tiles > 1 << 20) return MPA_ERR_BAD_SHAPE;
+    }
+    p.tiles = (int)tiles;
+    // parts of T: as few as give about two workgroups per CU (each part writes and reads back all partial
+    // tiles), none shorter than 256 rows
+    int s = 1;
+    while (s < 8 && tiles * s < 400 && T / (2 * s) >= 256) s *= 2;
+    p.splits = s;
+    return MPA_OK;
+}
+
+// ---- small parameters ---------------------------------------------------------------------------
+
+struct CastParams {
+    mpa_cast_job job[MPA_CAST_MAX_JOBS];
+    int jobs;
+};
+__device__ __forceinline__ float load_any(const void* p, int64_t i, int dt) {
+    return dt == MPA_F32 ? static_cast<const float*>(p)[i] : to_float(static_cast<const bf16_t*>(p)[i]);
+}
+// One job per blockIdx.y: rows x cols elements, row pitches of its own on either side.
+__global__ void __launch_bounds__(256) cast_kernel(const CastParams p) {
+    const mpa_cast_job& j = p.job[blockIdx.y];
+    const int64_t n = j.rows * j.cols;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const int64_t r = i / j.cols, c = i - r * j.cols;
+        float v = load_any(j.src, r * j.src_pitch + c, j.src_dtype);
+        if (j.op == MPA_CAST_NEG_EXP) v = -expf(v);
+        if (j.op == MPA_CAST_TIMES) v *= static_cast<const float*>(j.factor)[i];
+        const int64_t at = r * j.dst_pitch + c;
+        if (j.dst_dtype == MPA_F32) static_cast<float*>(j.dst)[at] = v;
+        else static_cast<bf16_t*>(j.dst)[at] = from_float<bf16_t>(v);
+    }
+}
+
+}  // namespace mpa
+
+using namespace mpa;
+
+extern "C" size_t mpa_wgrad_workspace_bytes(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_t io_dtype) {
+    WgradParams p{};
+    if (wgrad_params(p, jobs, n, T, io_dtype) != MPA_OK) return 0;
+    return (size_t)p.splits * p.tiles * kWgTile * kWgTile * sizeof(float);
+}
+
+extern "C" int mpa_wgrad(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_t io_dtype, void* workspace, size_t workspace_bytes,
+                         void* stream) {
+    WgradParams p{};
+    const int rc = wgrad_params(p, jobs, n, T, io_dtype);
+    if (rc != MPA_OK) return rc;
+    const size_t es = dtype_size(io_dtype);
+    for (int i = 0; i < n; ++i) {
+        if (!p.job[i].p || !p.job[i].q || !p.job[i].out) return MPA_ERR_NULL_POINTER;
+        if (!aligned_to(p.job[i].p, 4 * es) || !aligned_to(p.job[i].q, 4 * es) || !aligned_to(p.job[i].out, es)) return MPA_ERR_MISALIGNED;
+    }
+    if (!workspace) return MPA_ERR_NULL_POINTER;
+    if (!aligned_to(workspace, 256)) return MPA_ERR_MISALIGNED;
+    if (workspace_bytes < mpa_wgrad_workspace_bytes(jobs, n, T, io_dtype)) return MPA_ERR_WORKSPACE;
+    p.part = static_cast<float*>(workspace);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int groups = 8 / p.splits, per = (p.tiles + groups - 1) / groups;
+    const dim3 grid((unsigned)(8 * per)), sums((unsigned)(16 * p.tiles));
+    if (io_dtype == MPA_F32) {
+        hipLaunchKernelGGL(wgrad_f32_kernel, grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL(wgrad_sum_kernel<float>, sums, dim3(256), 0, st, p);
+    } else {
+        hipLaunchKernelGGL(wgrad_bf16_kernel, grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL(wgrad_sum_kernel<bf16_t>, sums, dim3(256), 0, st, p);
+    }
+    return check_launch();
+}
+
+extern "C" int mpa_cast(const mpa_cast_job* jobs, int32_t n, void* stream) {
+    if (!jobs) return MPA_ERR_NULL_POINTER;
+    if (n <= 0 || n > MPA_CAST_MAX_JOBS) return MPA_ERR_BAD_SHAPE;
+    CastParams p{};
+    p.jobs = n;
+    int64_t most = 0;
+    for (int i = 0; i < n; ++i) {
+        const mpa_cast_job& j = jobs[i];
+        if (!j.src || !j.dst || (j.op == MPA_CAST_TIMES && !j.factor)) return MPA_ERR_NULL_POINTER;
+        if (j.rows <= 0 || j.cols <= 0 || j.src_pitch < j.cols || j.dst_pitch < j.cols) return MPA_ERR_BAD_SHAPE;
+        for (int dt : {j.src_dtype, j.dst_dtype})
+            if (dt != MPA_F32 && dt != MPA_BF16) return MPA_ERR_BAD_DTYPE;
+        if (!aligned_to(j.src, dtype_size(j.src_dtype)) || !aligned_to(j.dst, dtype_size(j.dst_dtype))) return MPA_ERR_MISALIGNED;
+        p.job[i] = j;
+        most = j.rows * j.cols > most ? j.rows * j.cols : most;
+    }
+    const int64_t blocks = (most + 1023) / 1024;
+    hipLaunchKernelGGL(cast_kernel, dim3((unsigned)(blocks > 128 ? 128 : blocks), (unsigned)n), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), p);
+    return check_launch();
+}

@@ -239,6 +239,12 @@ class MambaBlock(nn.Module):
         continues from: the state before position 0 and the inputs before it.  No gradient
         flows into the cache."""
         L = x.shape[1]
+        if x.is_cuda and torch.is_grad_enabled():
+            # a block of the plain kind: one graph node
+            h_in, win_in = cache if cache is not None else (None, None)
+            out = _host().block_train(self, x, h_in, win_in, bool(return_cache), plan.packed)
+            if out is not None:
+                return (out[0], out[1:]) if return_cache else out[0]
         xz = self.in_proj(x)
         xin, z = xz.chunk(2, dim=-1)
         K = self.config.d_conv

@@ -1,0 +1,95 @@
+"""The one-node mixer (csrc/host_train.cpp) and its weight-gradient kernel (csrc/layer.hip)."""
+import ctypes
+
+import pytest
+import torch
+
+from test_modules_gpu import block_forward_ref
+from util import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 1e-2)])
+@pytest.mark.parametrize("T", [1, 63, 65, 1000, 4097])                 # step edges; one and several parts of T
+def test_weight_gradients_match_float64_products(pkg, dev, dtype, tol, T):
+    L = pkg._lib
+    g = torch.Generator().manual_seed(T)
+    # (columns of P, of Q, kept columns, first row of the gap, gap): tile edges, both tile orders, padding
+    sizes = [(4, 4, 4, 0, 0), (128, 132, 132, 0, 0), (260, 64, 17, 0, 0), (96, 388, 388, 17, 47)]
+    jobs, keep, want, outs = (L.WgradJob * 4)(), [], [], []
+    for j, (M, N, kept, at, gap) in zip(jobs, sizes):
+        P = torch.randn(T, M + 8, generator=g).to(dtype).to(dev)[:, 4:4 + M]      # strided, offset
+        Q = torch.randn(T, N, generator=g).to(dtype).to(dev)
+        out = torch.full((M - gap, kept), float("nan"), dtype=dtype, device=dev)
+        j.p, j.q, j.ldp, j.ldq, j.out = P.data_ptr(), Q.data_ptr(), P.stride(0), Q.stride(0), out.data_ptr()
+        j.rows, j.cols, j.keep_cols, j.gap_at, j.gap = M, N, kept, at, gap
+        ref = P.double().cpu().T @ Q.double().cpu()
+        want.append(torch.cat([ref[:at], ref[at + gap:]])[:, :kept])
+        keep += [P, Q]
+        outs.append(out)
+    lib, io = L.load(), pkg.scan._DTYPES[dtype]
+    n = lib.mpa_wgrad_workspace_bytes(jobs, 4, T, io)
+    ws = torch.empty(n, dtype=torch.uint8, device=dev)
+    L.check(lib.mpa_wgrad(jobs, 4, T, io, ctypes.c_void_p(ws.data_ptr()), n, pkg.scan._stream(dev)), "mpa_wgrad")
+    for got, ref in zip(outs, want):
+        assert rel_err(got, ref) <= tol
+    jobs[0].rows = 6
+    assert lib.mpa_wgrad(jobs, 4, T, io, ctypes.c_void_p(ws.data_ptr()), n, pkg.scan._stream(dev)) == 2
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-4), (torch.bfloat16, 5e-2)])
+@pytest.mark.parametrize("shape,width,kw", [
+    ((1, 3), 8, {}), ((2, 75), 48, {}), ((3, 130), 64, dict(d_state=8, d_conv=2)),
+    ((2, 40), 72, dict(dt_rank=64, bias=False)), ((1, 33), 40, dict(d_state=32, d_conv=3, expand_factor=1)),
+])
+def test_mixer_gradients_match_float64_layer(pkg, dev, dtype, tol, shape, width, kw):
+    torch.manual_seed(width)
+    blk = pkg.MambaBlock(pkg.MambaConfig(d_model=width, n_layers=1, **kw)).to(dev).to(dtype)
+    x = torch.randn(*shape, width).to(dtype)
+    g = torch.randn(*shape, width).to(dtype)
+    xr = x.double().requires_grad_()
+    yr, pr = block_forward_ref(blk, xr)
+    yr.backward(g.double())
+    xg = x.to(dev).requires_grad_()
+    y = blk(xg)
+    assert "MambaBlockBackward" in type(y.grad_fn).__name__ or y.grad_fn.name() == "MambaBlockBackward"
+    y.backward(g.to(dev), retain_graph=True)
+    first = {k: v.grad.clone() for k, v in blk.named_parameters()}
+    assert rel_err(y, yr) <= tol and rel_err(xg.grad, xr.grad) <= tol
+    for k, v in blk.named_parameters():
+        assert v.grad.dtype == v.dtype and rel_err(v.grad, pr[k].grad) <= 3 * tol, k
+    # a second backward over the kept graph adds the same again; frozen parameters get none
+    y.backward(g.to(dev))
+    for k, v in blk.named_parameters():
+        assert rel_err(v.grad, 2 * first[k].double()) <= 1e-2, k
+    with pytest.raises(RuntimeError):
+        y.backward(g.to(dev))
+    for p in blk.parameters():
+        p.grad = None
+    blk.in_proj.weight.requires_grad_(False)
+    blk(x.to(dev)).backward(g.to(dev))
+    assert blk.in_proj.weight.grad is None
+    assert all(rel_err(v.grad, first[k].double()) <= 1e-6 for k, v in blk.named_parameters() if v.grad is not None)
+    # parameters changed between forward and backward are refused, as autograd does
+    y = blk(x.to(dev))
+    with torch.no_grad():
+        blk.A_log.add_(1.0)
+    with pytest.raises(RuntimeError):
+        y.backward(g.to(dev))
+
+
+def test_mixer_leaves_autocast_and_backward_hooks_to_the_composed_path(pkg, dev):
+    torch.manual_seed(9)
+    blk = pkg.MambaBlock(pkg.MambaConfig(d_model=64, n_layers=1)).to(dev)
+    x = torch.randn(2, 50, 64, device=dev)
+    y = blk(x)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        ya = blk(x)
+    assert ya.dtype == torch.bfloat16 and rel_err(ya, y.double()) <= 3e-2
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        assert pkg.Mamba(pkg.MambaConfig(d_model=64, n_layers=1)).to(dev)(x).shape == x.shape
+    seen = []
+    blk.out_proj.register_full_backward_hook(lambda *_: seen.append(1))
+    blk(x.requires_grad_()).sum().backward()
+    assert seen == [1]
