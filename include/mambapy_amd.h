@@ -255,11 +255,13 @@ size_t mpa_conv1d_bwd_workspace_bytes(const mpa_conv_shape* s);
  * row; the backward then takes the sum as its `x` and `dsum`, the gradient that reaches the sum
  * from its other users, and returns dx = (gradient through the norm) + dsum, which is the gradient
  * of both x and residual.  residual, sum_out and dsum may be NULL (plain RMSNorm).
+ * io_dtype | MPA_NORM_WEIGHT_BF16: weight and dweight are bfloat16.
  */
-int mpa_rmsnorm_fwd(const void* x, const void* residual, const float* weight, void* y, void* sum_out,
+#define MPA_NORM_WEIGHT_BF16 256
+int mpa_rmsnorm_fwd(const void* x, const void* residual, const void* weight, void* y, void* sum_out,
                     float* rstd, int64_t rows, int64_t d, float eps, int32_t io_dtype, void* stream);
-int mpa_rmsnorm_bwd(const void* x, const float* weight, const void* dy, const void* dsum, void* dx,
-                    float* dweight, int64_t rows, int64_t d, float eps, int32_t io_dtype,
+int mpa_rmsnorm_bwd(const void* x, const void* weight, const void* dy, const void* dsum, void* dx,
+                    void* dweight, int64_t rows, int64_t d, float eps, int32_t io_dtype,
                     void* workspace, size_t workspace_bytes, void* stream);
 size_t mpa_rmsnorm_bwd_workspace_bytes(int64_t rows, int64_t d);
 
@@ -357,7 +359,7 @@ int mpa_decode_layer_step(const mpa_decode_layer* s, const void* x, const void* 
  * (rows columns, row stride ldp), Q its input (cols columns, row stride ldq), io_dtype; sums in float32,
  * added in a fixed order.  out is (rows - gap, keep_cols) contiguous, io_dtype: columns from keep_cols on
  * and the `gap` rows from gap_at on (padding of P and Q) are left out.  rows, cols and the strides are
- * multiples of 4, P and Q aligned to four elements.
+ * multiples of 4 (float32) / 8 (bfloat16), P and Q 16-byte aligned.
  */
 #define MPA_WGRAD_MAX_JOBS 4
 typedef struct mpa_wgrad_job {

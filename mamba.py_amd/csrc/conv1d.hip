@@ -214,9 +214,14 @@ __global__ void __launch_bounds__(kFinCols* kFinRows)
     const int col = threadIdx.x % kFinCols, rg = threadIdx.x / kFinCols;
     const int i = blockIdx.x * kFinCols + col;  // (k5, d), d fastest
     const int width = (kConvMaxK + 1) * ED;
-    float s = 0.0f;
+    // (four partial rows requested at a time: one after the other they cost a memory latency each)
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (i < width)
-        for (int q = rg; q < nparts; q += kFinRows) s += part[(int64_t)q * width + i];
+        for (int q = rg; q < nparts; q += 4 * kFinRows)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (q + j * kFinRows < nparts) v[j] += part[(int64_t)(q + j * kFinRows) * width + i];
+    float s = (v[0] + v[1]) + (v[2] + v[3]);
     acc[rg][col] = s;
     __syncthreads();
     if (rg != 0 || i >= width) return;

@@ -308,6 +308,8 @@ Tensor conv_update(const Tensor& x, const Tensor& window, const Tensor& w_in, co
 // ---- RMSNorm ------------------------------------------------------------------------------------
 
 // (x [, residual]) -> rmsnorm(x [+ residual]) [, x + residual]; inputs of the node: x, residual, weight
+int weight_flag(const Tensor& w) { return w.defined() && w.scalar_type() == at::kBFloat16 ? MPA_NORM_WEIGHT_BF16 : 0; }
+
 struct NormBackward : public Node {
     SavedVariable x, w;
     double eps = 0;
@@ -330,12 +332,12 @@ struct NormBackward : public Node {
         Tensor dw, ws;
         size_t nbytes = 0;
         if (w_.defined()) {
-            dw = empty({d}, at::kFloat, x_);
+            dw = empty({d}, w_.scalar_type(), x_);
             nbytes = mpa_rmsnorm_bwd_workspace_bytes(rows, d);
             ws = scratch(nbytes, x_);
         }
-        check(mpa_rmsnorm_bwd(ptr(x_), fptr(w_), ptr(dy), ptr(ds), ptr(dx), fptr(dw), rows, d, (float)eps, io_dtype(dt), ptr(ws), nbytes,
-                              stream_of(x_)),
+        check(mpa_rmsnorm_bwd(ptr(x_), ptr(w_), ptr(dy), ptr(ds), ptr(dx), ptr(dw), rows, d, (float)eps, io_dtype(dt) | weight_flag(w_),
+                              ptr(ws), nbytes, stream_of(x_)),
               "mpa_rmsnorm_bwd");
         out[0] = dx;
         if (with_sum) out[1] = dx;
@@ -358,11 +360,11 @@ std::tuple<Tensor, Opt> rmsnorm(const Tensor& x_in, const Opt& res_in, const Opt
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::DeviceGuard guard(x_in.device());
         x = x_in.contiguous();
-        w = f32c(wc);
+        w = wc.defined() && wc.scalar_type() == at::kBFloat16 ? wc.contiguous() : f32c(wc);
         const Tensor r = rc.defined() ? rc.contiguous() : rc;
         y = at::empty_like(x);
         if (r.defined()) sum = at::empty_like(x);
-        check(mpa_rmsnorm_fwd(ptr(x), ptr(r), fptr(w), ptr(y), ptr(sum), nullptr, rows, d, (float)eps, io, stream_of(x)),
+        check(mpa_rmsnorm_fwd(ptr(x), ptr(r), ptr(w), ptr(y), ptr(sum), nullptr, rows, d, (float)eps, io | weight_flag(w), stream_of(x)),
               "mpa_rmsnorm_fwd");
     }
     if (node) {

@@ -71,7 +71,7 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::DeviceGuard guard(x_in.device());
-        if (!l || !l->ready(x_in) || !l->forward_ok || l->N % 2) return py::none();
+        if (!l || !l->ready(x_in) || !l->forward_ok || l->N % 4) return py::none();
         if (unpack(packed).flags & MPA_PLAN_BWD_GENERAL) return py::none();
         const int64_t Bs = x_in.size(0);
         if (hc.defined() && !fits(hc, {Bs, l->ED, l->N}, at::kFloat, l->device)) return py::none();

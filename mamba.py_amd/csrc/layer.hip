@@ -64,14 +64,15 @@ __device__ __forceinline__ bool wgrad_work(const WgradParams& p, int& tile, int&
 }
 
 // bfloat16.  Both operands have the summation index as their slow dimension, the matrix cores want it
-// fast: a lane loads four neighbouring columns of eight rows (8 bytes each), turns the 4 x 8 block with
-// v_perm and stores four 16-byte units (8 rows of one column), the operand of one lane, into LDS.
-// The units of a panel lie in the order column % 4, column / 4: neighbouring lanes write
+// fast: a lane loads eight neighbouring columns of eight rows (16 bytes each), turns the 8 x 8 block with
+// v_perm and stores eight 16-byte units (8 rows of one column), each the operand of one lane, into LDS.
+// The units of a panel lie in the order column % 8, column / 8: neighbouring lanes write
 // neighbouring units, and a 16-row operand tile is 16 neighbouring units (its rows are then every
-// fourth column of the matrix, which only the order of the partial sums has to know).
-// 64 rows of T per step, four waves of 64 x 64 outputs, loads of the next step in registers meanwhile.
+// eighth column of the matrix, which only the order of the partial sums has to know).
+// 64 rows of T per step, loads of the next step in registers meanwhile: waves 0 and 1 bring the rows of P,
+// 2 and 3 those of Q; each wave computes 64 x 64 outputs.
 constexpr int kWgStep = 64;
-__device__ __forceinline__ int wg_unit_to_col(int u) { return 4 * (u & 31) + (u >> 5); }
+__device__ __forceinline__ int wg_unit_to_col(int u) { return 8 * (u & 15) + (u >> 4); }
 
 __global__ void __launch_bounds__(256, 2) wgrad_bf16_kernel(const WgradParams p) {
     __shared__ u32x4 lds[2][2][8][kWgTile];  // [buffer][P, Q][group of 8 rows][unit]
@@ -83,33 +84,27 @@ __global__ void __launch_bounds__(256, 2) wgrad_bf16_kernel(const WgradParams p)
     const int lane = threadIdx.x & 63, wave = wave_id();
     const int64_t steps = (p.T + kWgStep - 1) / kWgStep, per = (steps + p.splits - 1) / p.splits;
     const int64_t t_begin = split * per * kWgStep, t_end = min(p.T, (split + 1) * per * kWgStep);
-    // this lane's columns and rows of a step: columns 4*(lane % 32) .., rows 16*wave + 8*(lane / 32) ..
-    const int cq = 4 * (lane & 31), r0 = 16 * wave + 8 * (lane >> 5), g = 2 * wave + (lane >> 5);
-    const uint16_t* src[2] = {static_cast<const uint16_t*>(job.p) + min(tm * kWgTile + cq, job.M - 4),
-                              static_cast<const uint16_t*>(job.q) + min(tn * kWgTile + cq, job.N - 4)};
-    const int64_t ld[2] = {job.ldp, job.ldq};
-    u32x2 raw[2][8];
+    // this lane's columns and rows of a step
+    const int o = wave >> 1, g = 4 * (wave & 1) + (lane >> 4);
+    const int64_t ld = o ? job.ldq : job.ldp;
+    const uint16_t* src = static_cast<const uint16_t*>(o ? job.q : job.p) + (int64_t)(8 * g) * ld +
+                          min((o ? tn : tm) * kWgTile + 8 * (lane & 15), (o ? job.N : job.M) - 8);
+    u32x4 raw[8];
     auto request = [&](int64_t t) {
+        const int64_t left = t_end - t - 8 * g;
 #pragma unroll
-        for (int o = 0; o < 2; ++o)
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                const int64_t row = t + r0 + r;
-                raw[o][r] = row < t_end ? *reinterpret_cast<const u32x2*>(src[o] + row * ld[o]) : u32x2{0, 0};
-            }
+        for (int r = 0; r < 8; ++r) raw[r] = r < left ? *reinterpret_cast<const u32x4*>(src + (t + r) * ld) : u32x4{0, 0, 0, 0};
     };
     auto stage = [&](int buf) {
 #pragma unroll
-        for (int o = 0; o < 2; ++o)
+        for (int c = 0; c < 8; ++c) {
+            u32x4 unit;
+            // halves c % 2 of words c / 2 of two rows
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                u32x4 unit;
-                // halves c % 2 of words c / 2 of two rows
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    unit[r] = __builtin_amdgcn_perm(raw[o][2 * r + 1][c >> 1], raw[o][2 * r][c >> 1], c & 1 ? 0x07060302u : 0x05040100u);
-                lds[buf][o][g][32 * c + (lane & 31)] = unit;
-            }
+            for (int r = 0; r < 4; ++r)
+                unit[r] = __builtin_amdgcn_perm(raw[2 * r + 1][c >> 1], raw[2 * r][c >> 1], c & 1 ? 0x07060302u : 0x05040100u);
+            lds[buf][o][g][16 * c + (lane & 15)] = unit;
+        }
     };
     f32x4 acc[4][4] = {};
     const int mu = 64 * (wave >> 1), nu = 64 * (wave & 1);  // the wave's units of P and Q
@@ -145,9 +140,12 @@ __global__ void __launch_bounds__(256, 2) wgrad_bf16_kernel(const WgradParams p)
 }
 
 // float32.  The matrix-core operand of four rows x 16 columns is what a row-major panel in LDS gives as
-// it is; rows are 16 floats longer than the tile so that the four rows of an operand fall on different banks.
-constexpr int kWgStepF = 16, kWgPitch = kWgTile + 16;
-__global__ void __launch_bounds__(256, 2) wgrad_f32_kernel(const WgradParams p) {
+// it is; rows are 16 floats longer than the tile so that the four rows of an operand fall on different
+// banks.  The products that come here are narrow (the wide ones are left to the GEMM library), and a
+// float32 product keeps a wave busy 16 times as long as a bfloat16 one: 64 x 64 tiles, 32 x 32 per wave,
+// make enough waves (128 x 128 tiles: 54 us for 96 x 2048 and 2048 x 64 over 4096 rows).
+constexpr int kWgTileF = 64, kWgStepF = 32, kWgPitch = kWgTileF + 16;
+__global__ void __launch_bounds__(256) wgrad_f32_kernel(const WgradParams p) {
     __shared__ float lds[2][2][kWgStepF][kWgPitch];
     int tile, split;
     if (!wgrad_work(p, tile, split)) return;
@@ -157,9 +155,9 @@ __global__ void __launch_bounds__(256, 2) wgrad_f32_kernel(const WgradParams p) 
     const int lane = threadIdx.x & 63, wave = wave_id();
     const int64_t steps = (p.T + kWgStepF - 1) / kWgStepF, per = (steps + p.splits - 1) / p.splits;
     const int64_t t_begin = split * per * kWgStepF, t_end = min(p.T, (split + 1) * per * kWgStepF);
-    const int cq = 4 * (threadIdx.x & 31), r0 = threadIdx.x >> 5;  // four columns of rows r0 and r0 + 8
-    const float* src[2] = {static_cast<const float*>(job.p) + min(tm * kWgTile + cq, job.M - 4),
-                           static_cast<const float*>(job.q) + min(tn * kWgTile + cq, job.N - 4)};
+    const int cq = 4 * (threadIdx.x & 15), r0 = threadIdx.x >> 4;  // four columns of rows r0 and r0 + 16
+    const float* src[2] = {static_cast<const float*>(job.p) + min(tm * kWgTileF + cq, job.M - 4),
+                           static_cast<const float*>(job.q) + min(tn * kWgTileF + cq, job.N - 4)};
     const int64_t ld[2] = {job.ldp, job.ldq};
     f32x4 raw[2][2];
     auto request = [&](int64_t t) {
@@ -167,76 +165,75 @@ __global__ void __launch_bounds__(256, 2) wgrad_f32_kernel(const WgradParams p) 
         for (int o = 0; o < 2; ++o)
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
-                const int64_t row = t + r0 + 8 * r;
+                const int64_t row = t + r0 + 16 * r;
                 raw[o][r] = row < t_end ? *reinterpret_cast<const f32x4*>(src[o] + row * ld[o]) : f32x4{0, 0, 0, 0};
             }
     };
-    f32x4 acc[4][4] = {};
-    const int mu = 64 * (wave >> 1), nu = 64 * (wave & 1);
+    f32x4 acc[2][2] = {};
+    const int mu = 32 * (wave >> 1), nu = 32 * (wave & 1);
     request(t_begin);
     int buf = 0;
     for (int64_t t = t_begin; t < t_end; t += kWgStepF) {
 #pragma unroll
         for (int o = 0; o < 2; ++o)
 #pragma unroll
-            for (int r = 0; r < 2; ++r) *reinterpret_cast<f32x4*>(&lds[buf][o][r0 + 8 * r][cq]) = raw[o][r];
+            for (int r = 0; r < 2; ++r) *reinterpret_cast<f32x4*>(&lds[buf][o][r0 + 16 * r][cq]) = raw[o][r];
         __syncthreads();
         if (t + kWgStepF < t_end) request(t + kWgStepF);
 #pragma unroll
         for (int k = 0; k < kWgStepF / 4; ++k) {
-            float a[4], b[4];
+            float a[2], b[2];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < 2; ++i) {
                 a[i] = lds[buf][0][4 * k + (lane >> 4)][mu + 16 * i + (lane & 15)];
                 b[i] = lds[buf][1][4 * k + (lane >> 4)][nu + 16 * i + (lane & 15)];
             }
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
         }
         buf ^= 1;
     }
-    float* out = p.part + ((int64_t)split * p.tiles + tile) * kWgTile * kWgTile;
+    float* out = p.part + ((int64_t)split * p.tiles + tile) * kWgTileF * kWgTileF;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                out[(mu + 16 * i + 4 * (lane >> 4) + r) * kWgTile + nu + 16 * j + (lane & 15)] = acc[i][j][r];
+                out[(mu + 16 * i + 4 * (lane >> 4) + r) * kWgTileF + nu + 16 * j + (lane & 15)] = acc[i][j][r];
 }
 
-// Sum over the splits, in order; a thread takes four neighbouring output columns of one row of a tile.
+// Sum over the splits, in order; a thread takes kCols neighbouring output columns of one row of a tile.
 template <typename IO>
 __global__ void __launch_bounds__(256) wgrad_sum_kernel(const WgradParams p) {
-    const int tile = blockIdx.x >> 4, local = (blockIdx.x & 15) * 256 + threadIdx.x;  // 128 rows x 32 column groups
+    constexpr bool UNITS = sizeof(IO) == 2;
+    constexpr int kTileIO = UNITS ? kWgTile : kWgTileF, kCols = UNITS ? 8 : 4, kGroups = kTileIO / kCols;
+    const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int tile = (int)(id / (kTileIO * kGroups)), local = (int)(id % (kTileIO * kGroups));
     const WgradJob& job = p.job[wgrad_find(p, tile)];
     int tm, tn;
     wgrad_tile_at(job, tile, tm, tn);
-    constexpr bool UNITS = sizeof(IO) == 2;
-    const int u = local >> 5, q = local & 31;
-    const float* src = p.part + (int64_t)tile * kWgTile * kWgTile + u * kWgTile;
-    const int64_t pitch = (int64_t)p.tiles * kWgTile * kWgTile;
-    f32x4 s = {0, 0, 0, 0};
+    const int u = local / kGroups, q = local % kGroups;
+    const int row_in = tm * kTileIO + (UNITS ? wg_unit_to_col(u) : u), col = tn * kTileIO + kCols * q;
+    if (row_in >= job.M || (row_in >= job.gap_at && row_in < job.gap_at + job.gap) || col >= job.keep) return;
+    const float* src = p.part + (int64_t)tile * kTileIO * kTileIO + u * kTileIO;
+    const int64_t pitch = (int64_t)p.tiles * kTileIO * kTileIO;
+    float s[kCols] = {};
     for (int k = 0; k < p.splits; ++k) {
         const float* v = src + k * pitch;
-        if constexpr (UNITS) {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) s[c] += v[32 * c + q];
-        } else {
-            s += *reinterpret_cast<const f32x4*>(v + 4 * q);
-        }
+        for (int c = 0; c < kCols; ++c) s[c] += v[UNITS ? kGroups * c + q : kCols * q + c];
     }
-    int row = tm * kWgTile + (UNITS ? wg_unit_to_col(u) : u);
-    const int col = tn * kWgTile + 4 * q;
-    if (row >= job.M || (row >= job.gap_at && row < job.gap_at + job.gap)) return;
-    if (row >= job.gap_at) row -= job.gap;
+    const int row = row_in >= job.gap_at ? row_in - job.gap : row_in;
     IO* out = static_cast<IO*>(job.out) + (int64_t)row * job.keep + col;
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < kCols; ++c)
         if (col + c < job.keep) out[c] = from_float<IO>(s[c]);
 }
+
+static int wgrad_tile(int io_dtype) { return io_dtype == MPA_F32 ? kWgTileF : kWgTile; }
 
 static int wgrad_params(WgradParams& p, const mpa_wgrad_job* jobs, int n, int64_t T, int io_dtype) {
     if (!jobs) return MPA_ERR_NULL_POINTER;
@@ -245,20 +242,22 @@ static int wgrad_params(WgradParams& p, const mpa_wgrad_job* jobs, int n, int64_
     p.jobs = n;
     p.T = T;
     int64_t tiles = 0;
+    const int tile = wgrad_tile(io_dtype);
     for (int i = 0; i < n; ++i) {
         const mpa_wgrad_job& s = jobs[i];
         WgradJob& j = p.job[i];
-        if (s.rows < 4 || s.cols < 4 || s.rows % 4 || s.cols % 4 || s.rows > 1 << 20 || s.cols > 1 << 20 || s.keep_cols < 1 ||
+        const int64_t v = io_dtype == MPA_BF16 ? 8 : 4;  // elements of a 16-byte load
+        if (s.rows < v || s.cols < v || s.rows % v || s.cols % v || s.rows > 1 << 20 || s.cols > 1 << 20 || s.keep_cols < 1 ||
             s.keep_cols > s.cols || s.gap < 0 || s.gap_at < 0 || s.gap_at + s.gap > s.rows)
             return MPA_ERR_BAD_SHAPE;
-        if (s.ldp < s.rows || s.ldq < s.cols || s.ldp % 4 || s.ldq % 4) return MPA_ERR_BAD_STRIDE;
+        if (s.ldp < s.rows || s.ldq < s.cols || s.ldp % v || s.ldq % v) return MPA_ERR_BAD_STRIDE;
         j.p = s.p; j.q = s.q; j.out = s.out;
         j.ldp = s.ldp; j.ldq = s.ldq;
         j.M = (int)s.rows; j.N = (int)s.cols;
         j.keep = (int)s.keep_cols;
         j.gap_at = s.gap ? (int)s.gap_at : j.M; j.gap = (int)s.gap;
-        j.tiles_m = (j.M + kWgTile - 1) / kWgTile;
-        j.tiles_n = (j.N + kWgTile - 1) / kWgTile;
+        j.tiles_m = (j.M + tile - 1) / tile;
+        j.tiles_n = (j.N + tile - 1) / tile;
         j.p_major = j.tiles_m >= j.tiles_n;
         j.first_tile = (int)tiles;
         tiles += (int64_t)j.tiles_m * j.tiles_n;
@@ -266,9 +265,9 @@ static int wgrad_params(WgradParams& p, const mpa_wgrad_job* jobs, int n, int64_
     }
     p.tiles = (int)tiles;
     // parts of T: as few as give about two workgroups per CU (each part writes and reads back all partial
-    // tiles), none shorter than 256 rows
+    // tiles), none shorter than 128 rows
     int s = 1;
-    while (s < 8 && tiles * s < 400 && T / (2 * s) >= 256) s *= 2;
+    while (s < 8 && tiles * s < 400 && T / (2 * s) >= 128) s *= 2;
     p.splits = s;
     return MPA_OK;
 }
@@ -304,7 +303,7 @@ using namespace mpa;
 extern "C" size_t mpa_wgrad_workspace_bytes(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_t io_dtype) {
     WgradParams p{};
     if (wgrad_params(p, jobs, n, T, io_dtype) != MPA_OK) return 0;
-    return (size_t)p.splits * p.tiles * kWgTile * kWgTile * sizeof(float);
+    return (size_t)p.splits * p.tiles * wgrad_tile(io_dtype) * wgrad_tile(io_dtype) * sizeof(float);
 }
 
 extern "C" int mpa_wgrad(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_t io_dtype, void* workspace, size_t workspace_bytes,
@@ -315,7 +314,7 @@ extern "C" int mpa_wgrad(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_
     const size_t es = dtype_size(io_dtype);
     for (int i = 0; i < n; ++i) {
         if (!p.job[i].p || !p.job[i].q || !p.job[i].out) return MPA_ERR_NULL_POINTER;
-        if (!aligned_to(p.job[i].p, 4 * es) || !aligned_to(p.job[i].q, 4 * es) || !aligned_to(p.job[i].out, es)) return MPA_ERR_MISALIGNED;
+        if (!aligned_to(p.job[i].p, 16) || !aligned_to(p.job[i].q, 16) || !aligned_to(p.job[i].out, es)) return MPA_ERR_MISALIGNED;
     }
     if (!workspace) return MPA_ERR_NULL_POINTER;
     if (!aligned_to(workspace, 256)) return MPA_ERR_MISALIGNED;
@@ -323,7 +322,7 @@ extern "C" int mpa_wgrad(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_
     p.part = static_cast<float*>(workspace);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int groups = 8 / p.splits, per = (p.tiles + groups - 1) / groups;
-    const dim3 grid((unsigned)(8 * per)), sums((unsigned)(16 * p.tiles));
+    const dim3 grid((unsigned)(8 * per)), sums((unsigned)(io_dtype == MPA_F32 ? kWgTileF * kWgTileF / 4 / 256 * p.tiles : kWgTile * kWgTile / 8 / 256 * p.tiles));
     if (io_dtype == MPA_F32) {
         hipLaunchKernelGGL(wgrad_f32_kernel, grid, dim3(256), 0, st, p);
         hipLaunchKernelGGL(wgrad_sum_kernel<float>, sums, dim3(256), 0, st, p);

@@ -72,12 +72,23 @@ __device__ __forceinline__ float wave_sum(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
+// Element of the weight: float32, or bfloat16 where the caller keeps its parameters in that type (a
+// separate conversion would cost a launch per call, as long as the norm of a short sequence).
+struct NormWeight {
+    const void* p;
+    bool bf16;
+    __device__ __forceinline__ float operator[](int i) const {
+        return bf16 ? to_float(static_cast<const bf16_t*>(p)[i]) : static_cast<const float*>(p)[i];
+    }
+    __device__ __forceinline__ explicit operator bool() const { return p != nullptr; }
+};
+
 // rows x d, contiguous rows; d a multiple of the vector width, at most MAXV vectors per lane.
 // A wave takes R consecutive rows and holds all of them in registers.  With `res` the row that
 // is normalised is round(x + res), also written to `sum_out`.  rstd (rows) is optional.
 template <typename IO, int MAXV, int R>
 __global__ void __launch_bounds__(256) rmsnorm_fwd_kernel(const IO* __restrict__ x, const IO* __restrict__ res,
-                                                          const float* __restrict__ w, IO* __restrict__ y,
+                                                          const NormWeight w, IO* __restrict__ y,
                                                           IO* __restrict__ sum_out, float* __restrict__ rstd_out,
                                                           int64_t rows, int d, float eps) {
     typedef RowVec<IO> V;
@@ -156,7 +167,7 @@ __global__ void __launch_bounds__(256) rmsnorm_fwd_kernel(const IO* __restrict__
 // and read the weight from cache instead of registers.
 template <typename IO, int MAXV>
 __global__ void __launch_bounds__(kNormBwdWaves* kWave) rmsnorm_bwd_kernel(
-    const IO* __restrict__ x, const float* __restrict__ w, const IO* __restrict__ dy, const IO* __restrict__ dres,
+    const IO* __restrict__ x, const NormWeight w, const IO* __restrict__ dy, const IO* __restrict__ dres,
     IO* __restrict__ dx, float* __restrict__ part, int64_t rows, int d, float eps, int rpw) {
     typedef RowVec<IO> V;
     typedef typename V::T VT;
@@ -269,19 +280,25 @@ __global__ void __launch_bounds__(kNormBwdWaves* kWave) rmsnorm_bwd_kernel(
 
 // dweight[c] = sum over the per-block partial rows, fixed order (32 columns x 32 row groups per block)
 constexpr int kNormFinCols = 32, kNormFinRows = 32;
-__global__ void __launch_bounds__(1024) rmsnorm_bwd_finish_kernel(const float* part, float* dweight, int d,
-                                                                  int64_t nparts) {
+__global__ void __launch_bounds__(1024) rmsnorm_bwd_finish_kernel(const float* part, void* dweight, int d, int64_t nparts,
+                                                                  int bf16) {
     __shared__ float acc[kNormFinRows][kNormFinCols + 1];
     const int col = threadIdx.x % kNormFinCols, rg = threadIdx.x / kNormFinCols;
     const int c = blockIdx.x * kNormFinCols + col;
-    float s = 0.0f;
+    // (four partial rows requested at a time: one after the other they cost a memory latency each)
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (c < d)
-        for (int64_t q = rg; q < nparts; q += kNormFinRows) s += part[q * d + c];
+        for (int64_t q = rg; q < nparts; q += 4 * kNormFinRows)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (q + j * kNormFinRows < nparts) v[j] += part[(q + j * kNormFinRows) * d + c];
+    float s = (v[0] + v[1]) + (v[2] + v[3]);
     acc[rg][col] = s;
     __syncthreads();
     if (rg != 0 || c >= d) return;
     for (int r = 1; r < kNormFinRows; ++r) s += acc[r][col];
-    dweight[c] = s;
+    if (bf16) static_cast<bf16_t*>(dweight)[c] = from_float<bf16_t>(s);
+    else static_cast<float*>(dweight)[c] = s;
 }
 
 static int norm_validate(int64_t rows, int64_t d, int io_dtype) {
@@ -299,21 +316,22 @@ static int norm_maxv(int64_t d, int io_dtype) {
     return nv <= 1 ? 1 : nv <= 2 ? 2 : nv <= 4 ? 4 : 8;
 }
 
-// Backward launch: rows per wave chosen for about 4096 waves (16 per CU) when the problem has
-// that many rows, at most 16 rows per wave; one dweight partial per block.
+// Backward launch: rows per wave chosen for about 2048 waves (8 per CU) when the problem has that many
+// rows, at most 16 rows per wave; one dweight partial per block.  (4096 waves at 8000 x 768: twice the
+// partial rows, 17 + 11 us; 16 + 5.5 us this way.)
 struct NormBwdPlan {
     int rpw;
     int64_t blocks;
 };
 static NormBwdPlan norm_bwd_plan(int64_t rows) {
-    int64_t rpw = rows / 4096;
+    int64_t rpw = rows / 2048;
     rpw = rpw < 1 ? 1 : rpw > 16 ? 16 : rpw;
     const int64_t waves = (rows + rpw - 1) / rpw;
     return NormBwdPlan{(int)rpw, (waves + kNormBwdWaves - 1) / kNormBwdWaves};
 }
 
 template <typename IO, int MAXV>
-static int launch_norm_fwd(const void* x, const void* res, const float* w, void* y, void* sum_out, float* rstd,
+static int launch_norm_fwd(const void* x, const void* res, NormWeight w, void* y, void* sum_out, float* rstd,
                            int64_t rows, int d, float eps, hipStream_t st) {
     constexpr int R = MAXV <= 2 ? 4 : 1;
     const int64_t waves = (rows + R - 1) / R;
@@ -324,7 +342,7 @@ static int launch_norm_fwd(const void* x, const void* res, const float* w, void*
 }
 
 template <typename IO, int MAXV>
-static int launch_norm_bwd(const void* x, const float* w, const void* dy, const void* dsum, void* dx, float* part,
+static int launch_norm_bwd(const void* x, NormWeight w, const void* dy, const void* dsum, void* dx, float* part,
                            int64_t rows, int d, float eps, hipStream_t st) {
     const NormBwdPlan plan = norm_bwd_plan(rows);
     const size_t lds = part ? (size_t)kNormBwdWaves * d * sizeof(float) : 0;
@@ -354,17 +372,19 @@ using namespace mpa;
             : maxv == 4 ? FN<bf16_t, 4>(__VA_ARGS__)                                   \
                         : FN<bf16_t, 8>(__VA_ARGS__)))
 
-extern "C" int mpa_rmsnorm_fwd(const void* x, const void* residual, const float* weight, void* y, void* sum_out,
+extern "C" int mpa_rmsnorm_fwd(const void* x, const void* residual, const void* weight, void* y, void* sum_out,
                                float* rstd, int64_t rows, int64_t d, float eps, int32_t io_dtype, void* stream) {
+    const NormWeight nw{weight, (io_dtype & MPA_NORM_WEIGHT_BF16) != 0};
+    io_dtype &= ~MPA_NORM_WEIGHT_BF16;
     int rc = norm_validate(rows, d, io_dtype);
     if (rc != MPA_OK) return rc;
     if (!x || !y || (residual && !sum_out)) return MPA_ERR_NULL_POINTER;
-    if (!aligned_to(x, 16) || !aligned_to(y, 16) || (weight && !aligned_to(weight, 4)) ||
+    if (!aligned_to(x, 16) || !aligned_to(y, 16) || (weight && !aligned_to(weight, nw.bf16 ? 2 : 4)) ||
         (residual && (!aligned_to(residual, 16) || !aligned_to(sum_out, 16))))
         return MPA_ERR_MISALIGNED;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int maxv = norm_maxv(d, io_dtype);
-    return MPA_NORM_DISPATCH(launch_norm_fwd, x, residual, weight, y, sum_out, rstd, rows, (int)d, eps, st);
+    return MPA_NORM_DISPATCH(launch_norm_fwd, x, residual, nw, y, sum_out, rstd, rows, (int)d, eps, st);
 }
 
 extern "C" size_t mpa_rmsnorm_bwd_workspace_bytes(int64_t rows, int64_t d) {
@@ -372,14 +392,16 @@ extern "C" size_t mpa_rmsnorm_bwd_workspace_bytes(int64_t rows, int64_t d) {
     return ((size_t)norm_bwd_plan(rows).blocks * d * sizeof(float) + 255) / 256 * 256;
 }
 
-extern "C" int mpa_rmsnorm_bwd(const void* x, const float* weight, const void* dy, const void* dsum, void* dx,
-                               float* dweight, int64_t rows, int64_t d, float eps, int32_t io_dtype,
+extern "C" int mpa_rmsnorm_bwd(const void* x, const void* weight, const void* dy, const void* dsum, void* dx,
+                               void* dweight, int64_t rows, int64_t d, float eps, int32_t io_dtype,
                                void* workspace, size_t workspace_bytes, void* stream) {
+    const NormWeight nw{weight, (io_dtype & MPA_NORM_WEIGHT_BF16) != 0};
+    io_dtype &= ~MPA_NORM_WEIGHT_BF16;
     int rc = norm_validate(rows, d, io_dtype);
     if (rc != MPA_OK) return rc;
     if (!x || !dy || !dx) return MPA_ERR_NULL_POINTER;
     if (weight && (!dweight || !workspace)) return MPA_ERR_NULL_POINTER;
-    if (!aligned_to(x, 16) || !aligned_to(dy, 16) || !aligned_to(dx, 16) || (weight && !aligned_to(weight, 4)) ||
+    if (!aligned_to(x, 16) || !aligned_to(dy, 16) || !aligned_to(dx, 16) || (weight && !aligned_to(weight, nw.bf16 ? 2 : 4)) ||
         (dsum && !aligned_to(dsum, 16)) ||
         (workspace && !aligned_to(workspace, 256)))
         return MPA_ERR_MISALIGNED;
@@ -387,9 +409,9 @@ extern "C" int mpa_rmsnorm_bwd(const void* x, const float* weight, const void* d
     hipStream_t st = static_cast<hipStream_t>(stream);
     float* part = weight ? static_cast<float*>(workspace) : nullptr;
     const int maxv = norm_maxv(d, io_dtype);
-    rc = MPA_NORM_DISPATCH(launch_norm_bwd, x, weight, dy, dsum, dx, part, rows, (int)d, eps, st);
+    rc = MPA_NORM_DISPATCH(launch_norm_bwd, x, nw, dy, dsum, dx, part, rows, (int)d, eps, st);
     if (rc != MPA_OK || !weight) return rc;
     hipLaunchKernelGGL(rmsnorm_bwd_finish_kernel, dim3((unsigned)((d + kNormFinCols - 1) / kNormFinCols)),
-                       dim3(1024), 0, st, part, dweight, (int)d, norm_bwd_plan(rows).blocks);
+                       dim3(1024), 0, st, part, dweight, (int)d, norm_bwd_plan(rows).blocks, nw.bf16 ? 1 : 0);
     return check_launch();
 }

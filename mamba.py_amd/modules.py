@@ -120,7 +120,7 @@ class RMSNorm(nn.Module):
             self.weight = nn.Parameter(torch.ones(d_model))
 
     def _w(self):
-        return None if self.use_mup else _frozen_f32(self, "weight", self.weight)
+        return None if self.use_mup else self.weight
 
     def forward(self, x):
         if x.is_cuda and rmsnorm_supported(x):

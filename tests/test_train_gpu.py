@@ -16,10 +16,10 @@ def test_weight_gradients_match_float64_products(pkg, dev, dtype, tol, T):
     L = pkg._lib
     g = torch.Generator().manual_seed(T)
     # (columns of P, of Q, kept columns, first row of the gap, gap): tile edges, both tile orders, padding
-    sizes = [(4, 4, 4, 0, 0), (128, 132, 132, 0, 0), (260, 64, 17, 0, 0), (96, 388, 388, 17, 47)]
+    sizes = [(8, 8, 8, 0, 0), (128, 136, 136, 0, 0), (264, 64, 17, 0, 0), (96, 392, 392, 17, 47)]
     jobs, keep, want, outs = (L.WgradJob * 4)(), [], [], []
     for j, (M, N, kept, at, gap) in zip(jobs, sizes):
-        P = torch.randn(T, M + 8, generator=g).to(dtype).to(dev)[:, 4:4 + M]      # strided, offset
+        P = torch.randn(T, M + 16, generator=g).to(dtype).to(dev)[:, 8:8 + M]      # strided, offset
         Q = torch.randn(T, N, generator=g).to(dtype).to(dev)
         out = torch.full((M - gap, kept), float("nan"), dtype=dtype, device=dev)
         j.p, j.q, j.ldp, j.ldq, j.out = P.data_ptr(), Q.data_ptr(), P.stride(0), Q.stride(0), out.data_ptr()
@@ -34,7 +34,7 @@ def test_weight_gradients_match_float64_products(pkg, dev, dtype, tol, T):
     L.check(lib.mpa_wgrad(jobs, 4, T, io, ctypes.c_void_p(ws.data_ptr()), n, pkg.scan._stream(dev)), "mpa_wgrad")
     for got, ref in zip(outs, want):
         assert rel_err(got, ref) <= tol
-    jobs[0].rows = 6
+    jobs[0].rows = 10
     assert lib.mpa_wgrad(jobs, 4, T, io, ctypes.c_void_p(ws.data_ptr()), n, pkg.scan._stream(dev)) == 2
 
 
