@@ -477,7 +477,7 @@ __global__ void __launch_bounds__(256) sscan_bwd_finish_kernel(
 // is cut: half of the CUs or fewer covered (the first pass of a cut costs a quarter of the second)
 static constexpr int kBwdThin = 2;
 static int bwd_states_per_lane(const mpa_sscan_shape* s) {
-    const int ns = pick_states_per_lane(s->batch, s->dim, s->dstate, 4, s->plan_states_per_lane);
+    const int ns = pick_states_per_lane(s->dstate, 4, s->plan_states_per_lane);
     return ns < 0 ? 4 : ns;
 }
 // The fast kernel holds 16 states.  A wider d_state runs on it as passes over blocks of 16 states

@@ -895,21 +895,17 @@ int padded_states(int64_t n) {
     return np;
 }
 
-// States per lane (NS) for a launch.  The only parallel axes are batch*dim/64 workgroups and
-// d_state/NS scan waves inside each; a workgroup holds at most 8 scan waves.  Fewer states per
-// lane mean more waves (better latency hiding) but more LDS traffic per state; ask for about
-// two scan waves per SIMD over the chip's 1024 SIMDs when the problem offers them.  `pinned`
-// (the caller's plan_states_per_lane) wins when it is a value the kernels exist for.
-int pick_states_per_lane(int64_t batch, int64_t dim, int64_t dstate, int ns_cap, int pinned) {
+// States per lane (NS) for a launch: as few as put eight scan waves into a workgroup.  A workgroup's LDS
+// leaves no room for a second one on a CU, so its scan waves are all that hides latency there, at
+// any batch (fewer waves of more states at 16 x 500 x 8192: 934 us with 16 states per lane, 285 with 4, 272
+// with 2).  `pinned` (the caller's plan_states_per_lane) wins when it is a value the kernels exist for.
+int pick_states_per_lane(int64_t dstate, int ns_cap, int pinned) {
     const int np = padded_states(dstate);
     const int ns_min = np / 8 > 2 ? np / 8 : 2;
     const int ns_max = ns_cap < np ? ns_cap : np;
     if (ns_max < ns_min) return -1;
     if (pinned >= ns_min && pinned <= ns_max && (pinned & (pinned - 1)) == 0) return pinned;
-    const int64_t groups = batch * ((dim + kWave - 1) / kWave);
-    int ns = ns_max;
-    while (ns > ns_min && groups * (np / ns) < 2048) ns /= 2;
-    return ns;
+    return ns_min;
 }
 
 size_t bcpack_floats(const mpa_sscan_shape* s) {
@@ -963,10 +959,10 @@ extern "C" size_t mpa_sscan_fwd_workspace_bytes(const mpa_sscan_shape* s, int wi
         // passes over blocks of kFwdStateBlock states: the first block needs the most
         mpa_sscan_shape sb = *s;
         sb.dstate = kFwdStateBlock;
-        const int nsb = pick_states_per_lane(sb.batch, sb.dim, sb.dstate, 8, sb.plan_states_per_lane);
+        const int nsb = pick_states_per_lane(sb.dstate, 8, sb.plan_states_per_lane);
         return (seg_plan(&sb, nsb, kFwdThin).floats * sizeof(float) + 255) / 256 * 256 + 256;
     }
-    const int ns = pick_states_per_lane(s->batch, s->dim, s->dstate, 32, s->plan_states_per_lane);
+    const int ns = pick_states_per_lane(s->dstate, 32, s->plan_states_per_lane);
     if (ns <= 8) return (seg_plan(s, ns, kFwdThin).floats * sizeof(float) + 255) / 256 * 256 + 256;
     return (bcpack_floats(s) * sizeof(float) + 255) / 256 * 256;
 }
@@ -1043,7 +1039,7 @@ static int sscan_fwd_impl(const mpa_sscan_shape* s, const void* x, const void* d
             const int n0 = blk * kFwdStateBlock;
             mpa_sscan_shape sb = *s;
             sb.dstate = p.N - n0 < kFwdStateBlock ? p.N - n0 : kFwdStateBlock;
-            const int ns = pick_states_per_lane(sb.batch, sb.dim, sb.dstate, 8, sb.plan_states_per_lane);
+            const int ns = pick_states_per_lane(sb.dstate, 8, sb.plan_states_per_lane);
             if (ns < 0) return MPA_ERR_BAD_SHAPE;
             const int nw = padded_states(sb.dstate) / ns;
             const bool last = blk == nblk - 1;
@@ -1065,7 +1061,7 @@ static int sscan_fwd_impl(const mpa_sscan_shape* s, const void* x, const void* d
     }
 
     const int np = padded_states(s->dstate);
-    const int ns = pick_states_per_lane(s->batch, s->dim, s->dstate, 32, s->plan_states_per_lane);
+    const int ns = pick_states_per_lane(s->dstate, 32, s->plan_states_per_lane);
     if (ns < 0) return MPA_ERR_BAD_SHAPE;
     const int nw = np / ns;
     if (ns > 8) {  // !kBcastBC<NS>: B/C go through the scalar cache, repacked per scan wave
