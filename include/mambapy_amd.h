@@ -106,6 +106,8 @@ typedef struct mpa_sscan_shape {
  * (neither bit: the library picks, see mpa_sscan_fwd). */
 #define MPA_PLAN_GROUP_64 4
 #define MPA_PLAN_GROUP_48 8
+#define MPA_PLAN_GROUP_32 16
+#define MPA_PLAN_GROUP_16 32
 
 int mpa_version(void);
 /* Host string naming the GPU architecture the kernels were compiled for ("gfx950"). */

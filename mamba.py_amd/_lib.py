@@ -20,6 +20,8 @@ MPA_PLAN_BWD_GENERAL = 1
 MPA_PLAN_EXPIRE_WAITS = 2
 MPA_PLAN_GROUP_64 = 4
 MPA_PLAN_GROUP_48 = 8
+MPA_PLAN_GROUP_32 = 16
+MPA_PLAN_GROUP_16 = 32
 MPA_DELTA_F32 = 1
 MPA_CONV_SILU = 1
 MPA_CKPT_STEPS = 16

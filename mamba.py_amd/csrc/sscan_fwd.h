@@ -23,6 +23,8 @@ struct FwdParams {
     float* ckpt;
     float* hlast;
     float* dsum;     // segmented mode, first pass: sums of delta per (row, step group, channel)
+    const float* chain_hend;  // segmented mode, second pass: the first pass' end states and sums of delta; the
+    const float* chain_dsum;  // workgroup makes its initial state from those of the segments before its own
     int nseg;        // > 1: every batch row is cut into nseg segments of seg_tiles tiles, one
     int seg_tiles;   // workgroup row (blockIdx.y) per (batch row, segment)
     int batch, L, ED, N, nchunks;
@@ -33,7 +35,7 @@ struct FwdParams {
     // what `yacc` holds (strides of y) to its output before the gate.
     int a_st, h_st, ck_st;
     const void* yacc;
-    int group48;     // workgroups of 48 channels (six scan waves) instead of 64, see sscan_fwd.hip
+    int group;       // channels per workgroup: 16, 32, 48 or 64 (0: 64), see sscan_fwd.hip
     int softplus;
     int delta_f32;   // delta is float32 whatever the I/O type (MPA_DELTA_F32)
     int reverse;     // the walk runs from the last physical step to the first
@@ -64,11 +66,6 @@ struct SegPlan {
     size_t off_hend, off_h0, off_dsum, floats;
 };
 SegPlan seg_plan(const mpa_sscan_shape* s, int ns, int thin);
-// Channels per workgroup of a launch that is not cut: 48 where the kernels have that form (two states
-// per lane, d_state up to 16) and batch * ceil(dim / 48) workgroups still run in one round on the
-// chip's 256 CUs, else 64.  The plan flags pin either.
-int group_channels(const mpa_sscan_shape* s, int ns, int nseg);
-
 // Launch sscan_fwd_kernel in `mode` (FwdMode) for the (ns, nw) decomposition; the carry modes
 // exist for ns <= 8.
 int launch_fwd_any(const FwdParams& p, int io_dtype, int ns, int nw, int mode, hipStream_t stream);

@@ -104,16 +104,28 @@ constexpr bool kBcastBC = NS <= 8;
 // every row can have its own).  Batch * dim/48 workgroups fill the chip for shapes where batch *
 // dim/64 leaves CUs idle (8 x 1536: 256 instead of 192), and the six scan waves occupy two SIMDs
 // alone: the service waves are given wave numbers that land on the other two.
+//
+// 32 and 16 channels are for launches with few workgroups (a short prompt, one sequence): a tile of 16
+// channels takes a quarter of the work and little over a quarter of the time of one of 64, so a
+// walk over the sequence is as many times faster as the chip has idle CUs to take the other channels,
+// and nothing is computed twice (cutting the sequence instead costs a carry pass).  They have the form
+// of the 48-channel group: rows of 16 lanes, the four rows of a wave on different groups of states.  With
+// so few channels a service thread with four steps would be what a tile waits for (a lone wave issues
+// an instruction every 6-10 clocks): it takes CH/16 steps, so that all eight service waves have work.
 template <int NS, int NW, int CH>
-constexpr int kStateGroups = CH == 64 ? NW : 16 / NS;  // groups of NS states = partial readouts per channel
+constexpr int kStateGroups = CH == 64 ? NW : 4 * NW / (CH / 16);  // groups of NS states = partial readouts per channel
+
+template <int CH>
+constexpr int kTileRows = CH < 48 ? CH : 64;  // channels of an LDS tile
 
 template <int NS, int NW, int CH = 64>
 struct FwdLds {
+    static_assert(CH % 16 == 0, "rows of 16 lanes");
     static constexpr int NG = kStateGroups<NS, NW, CH>;
     // delta, u double-buffered (written two tiles ahead of use, read one tile ahead); D*x and
     // the gate in four buffers (written two tiles ahead, read one tile behind); readout
     // partials double-buffered per state group; B/C tiles [2][B|C][state][step] double-buffered
-    static constexpr size_t tiles = (size_t)(2 * 2 + 2 * 4 + 2 * NG) * kWave * kCP;
+    static constexpr size_t tiles = (size_t)(2 * 2 + 2 * 4 + 2 * NG) * kTileRows<CH> * kCP;
     static constexpr size_t floats = tiles + (kBcastBC<NS> ? 2 * 2 * NS * NG * kTile : 0);
 };
 
@@ -183,6 +195,36 @@ __device__ __forceinline__ float4 scan_group_bcast(const Decay4<NS>& dk, const f
     return y;
 }
 
+// steps per service item, and items per channel and tile
+template <int CH>
+constexpr int kItemSteps = CH < 48 ? CH / 16 : 4;
+// S consecutive floats in LDS
+template <int S>
+__device__ __forceinline__ void put_steps(float* dst, const float (&v)[S]) {
+    if constexpr (S == 4) *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+    else if constexpr (S == 2) *reinterpret_cast<float2*>(dst) = make_float2(v[0], v[1]);
+    else dst[0] = v[0];
+}
+template <int S>
+__device__ __forceinline__ void get_steps(const float* src, float (&v)[S]) {
+    if constexpr (S == 4) {
+        const float4 a = *reinterpret_cast<const float4*>(src);
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    } else if constexpr (S == 2) {
+        const float2 a = *reinterpret_cast<const float2*>(src);
+        v[0] = a.x; v[1] = a.y;
+    } else {
+        v[0] = src[0];
+    }
+}
+template <int S>
+__device__ __forceinline__ void add_steps(const float* src, float (&v)[S]) {
+    float a[S];
+    get_steps<S>(src, a);
+#pragma unroll
+    for (int j = 0; j < S; ++j) v[j] += a[j];
+}
+
 // waves of a workgroup: the carry modes store no output and run without reducer waves; a 48-channel
 // workgroup has sixteen wave numbers of which four do nothing (see service_role)
 template <int NW, int MODE, int CH = 64>
@@ -194,7 +236,7 @@ constexpr int kFwdWaves = CH == 48 ? 16 : NW + (MODE == kScan ? kService : kLoad
 // the wave numbers of SIMDs 2 and 3, and the numbers in between end at once.
 template <int NW, int CH>
 __device__ __forceinline__ int service_role(int w) {
-    if constexpr (CH == 64) return w - NW;
+    if constexpr (CH != 48) return w - NW;
     switch (w) {
         case 6: return 0;
         case 7: return 1;
@@ -210,12 +252,13 @@ template <typename IO, int NS, int NW, bool HAS_Z, int MODE, int CH = 64>
 __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_kernel(const FwdParams p) {
     constexpr int NQ = kTile / 4;  // step groups (of 4) per tile
     static_assert(kLoaders == NQ && kReducers == NQ, "a tile has 64 * NQ items of (channel, 4 steps)");
-    static_assert(CH == 64 || (CH == 48 && NS == 2 && NW == 6 && MODE == kScan), "48-channel groups: six scan waves of two states per lane");
+    static_assert(CH == 64 || CH < 48 || (CH == 48 && NS == 2 && NW == 6 && MODE == kScan), "48-channel groups: six scan waves of two states per lane");
     constexpr int NG = kStateGroups<NS, NW, CH>;
-    constexpr int kSvcThreads = (CH == 64 ? 4 : 3) * kWave;  // loader (and reducer) threads: one per item
+    constexpr int S = kItemSteps<CH>, QN = kTile / S;  // steps per service item, items per channel
+    constexpr int kSvcThreads = CH * QN;               // loader (and reducer) threads: one per item
 
     extern __shared__ float4 smem4[];
-    typedef float CTile[kWave][kCP];  // [channel][step]
+    typedef float CTile[kTileRows<CH>][kCP];  // [channel][step]
     CTile* sDl = reinterpret_cast<CTile*>(smem4);  // [2]
     CTile* sU = sDl + 2;                           // [2]
     CTile* sDx = sU + 2;                           // [4] D*x
@@ -266,13 +309,13 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
         if (has_z || p.softplus) __builtin_amdgcn_s_setprio(3);
         else __builtin_amdgcn_s_setprio(1);
         const int cmax = min(CH, p.ED - d0) - 1;     // last valid channel of the group
-        const int item = (sw & 3) * kWave + lane;    // 0 .. 4 * CH - 1
+        const int item = (sw & 3) * kWave + lane;    // 0 .. kSvcThreads - 1
         constexpr uint32_t kES = sizeof(IO);
         if (sw < kLoaders) {
             // ------------------------------- loaders -------------------------------
-            const int ci = p.in_tmajor ? item / NQ : item % CH;
-            const int qi = p.in_tmajor ? item % NQ : item / CH;     // walk step group of the item
-            const int qp = rev ? NQ - 1 - qi : qi;                  // its physical step group
+            const int ci = p.in_tmajor ? item / QN : item % CH;
+            const int qi = p.in_tmajor ? item % QN : item / CH;     // walk step group of the item
+            const int qp = rev ? QN - 1 - qi : qi;                  // its physical step group
             const bool ci_ok = ci <= cmax;
             const int cic = min(ci, cmax);
             const float Dv = p.D ? p.D[d0 + cic] : 0.0f;  // (NULL: a pass after the first over a wide d_state)
@@ -286,18 +329,18 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
             // byte offset of the item's lowest physical step (one vector register per tensor, see
             // ld_off); walk step j of the item is jw(j) row strides further, which goes into the
             // scalar offset of the access
-            const uint32_t offx = ((uint32_t)(4 * qp) * (uint32_t)p.u_sl + (uint32_t)cic * (uint32_t)p.u_sd) * kES;
+            const uint32_t offx = ((uint32_t)(S * qp) * (uint32_t)p.u_sl + (uint32_t)cic * (uint32_t)p.u_sd) * kES;
             // (delta may be float32 next to bfloat16 tensors: element size and conversion shift of its own)
             const bool d_wide = sizeof(IO) == 4 || p.delta_f32;
             const uint32_t kESd = d_wide ? 4u : 2u;
             const uint32_t dshift = __builtin_amdgcn_readfirstlane(d_wide ? 0u : 16u);
-            const uint32_t offd = ((uint32_t)(4 * qp) * (uint32_t)p.d_sl + (uint32_t)cic * (uint32_t)p.d_sd) * kESd;
-            const uint32_t offz = ((uint32_t)(4 * qp) * (uint32_t)p.z_sl + (uint32_t)cic * (uint32_t)p.z_sd) * kES;
-            auto jw = [&](int j) { return (uint32_t)(rev ? 3 - j : j); };
-            // scalar byte offsets of the item's four walk steps, computed once (scalar registers)
-            uint32_t sxj[4], sdj[4], szj[4];
+            const uint32_t offd = ((uint32_t)(S * qp) * (uint32_t)p.d_sl + (uint32_t)cic * (uint32_t)p.d_sd) * kESd;
+            const uint32_t offz = ((uint32_t)(S * qp) * (uint32_t)p.z_sl + (uint32_t)cic * (uint32_t)p.z_sd) * kES;
+            auto jw = [&](int j) { return (uint32_t)(rev ? S - 1 - j : j); };
+            // scalar byte offsets of the item's walk steps, computed once (scalar registers)
+            uint32_t sxj[S], sdj[S], szj[S];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 0; j < S; ++j) {
                 // (readfirstlane: told to the compiler as wave-uniform, so that they stay in scalar
                 // registers; an offset it takes for per-lane costs a loop over its values per access)
                 sxj[j] = __builtin_amdgcn_readfirstlane(jw(j) * (uint32_t)p.u_sl * kES);
@@ -337,7 +380,7 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
                 kBcast ? nullptr
                        : reinterpret_cast<const float4*>(p.bcpack) + (int64_t)b * ntiles * kPackVec + min(item, kPackVec - 1);
             float dsum = 0.0f;  // delta summed over the thread's steps of the row
-            struct Raw { IO x[4], z[4], b[kBcPer > 0 ? kBcPer : 1], c[kBcPer > 0 ? kBcPer : 1]; uint32_t d[4]; float4 warm; };
+            struct Raw { IO x[S], z[S], b[kBcPer > 0 ? kBcPer : 1], c[kBcPer > 0 ? kBcPer : 1]; uint32_t d[S]; float4 warm; };
             auto load_tile = [&](int kk, Raw& raw) {
                 // tiles beyond the last one are clamped to it; the loads are unconditional (a
                 // branch around them would force a wait on their data)
@@ -362,16 +405,16 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
                     wbc = window_bytes((p.batch - 1) * p.bc_sb + (p.L - 1) * p.bc_sl + p.N, b * p.bc_sb + tb * p.bc_sl, kES);
                 }
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
+                for (int j = 0; j < S; ++j) {
                     raw.x[j] = ld_off(xk, offx, sxj[j], wx);
                     if (has_z) raw.z[j] = ld_off(zk, offz, szj[j], wz);
                 }
                 if (d_wide) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) raw.d[j] = ld_bits32(dk, offd, sdj[j], wd);
+                    for (int j = 0; j < S; ++j) raw.d[j] = ld_bits32(dk, offd, sdj[j], wd);
                 } else {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) raw.d[j] = ld_bits16(dk, offd, sdj[j], wd);
+                    for (int j = 0; j < S; ++j) raw.d[j] = ld_bits16(dk, offd, sdj[j], wd);
                 }
 #pragma unroll
                 for (int r = 0; r < kBcPer; ++r) {
@@ -392,33 +435,36 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
                     dst[0] = ok ? to_float(raw.b[r]) : 0.0f;
                     if constexpr (MODE == kScan) dst[NP * kTile] = ok ? to_float(raw.c[r]) : 0.0f;
                 }
-                float xv[4], dv[4], gg[4];
+                float xv[S], dv[S], gg[S];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
+                for (int j = 0; j < S; ++j) {
                     xv[j] = to_float(raw.x[j]);
                     dv[j] = bits_to_float(raw.d[j], dshift);
                 }
                 if (p.softplus) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) dv[j] = softplus_f(dv[j] + bias);
+                    for (int j = 0; j < S; ++j) dv[j] = softplus_f(dv[j] + bias);
                 }
                 const int pc = phys_chunk(k);
                 if (!group_full || (ragged_seq && pc == last_chunk)) {
                     // ragged edge: delta = 0, u = 0 keeps the state of padded steps/channels
-                    const int t0 = pc * kTile + 4 * qp;
+                    const int t0 = pc * kTile + S * qp;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
+                    for (int j = 0; j < S; ++j) {
                         const bool ok = ci_ok && t0 + (int)jw(j) < p.L;
                         xv[j] = ok ? xv[j] : 0.0f;
                         dv[j] = ok ? dv[j] : 0.0f;
                     }
                 }
-                if constexpr (MODE != kScan) dsum += (dv[0] + dv[1]) + (dv[2] + dv[3]);  // only the carry needs it
-                const int q4 = 4 * qi;
-                *reinterpret_cast<float4*>(&sDl[k & 1][ci][q4]) = make_float4(dv[0], dv[1], dv[2], dv[3]);
+                if constexpr (MODE != kScan) {  // only the carry needs it
+                    if constexpr (S == 4) dsum += (dv[0] + dv[1]) + (dv[2] + dv[3]);
+                    else for (int j = 0; j < S; ++j) dsum += dv[j];
+                }
+                const int q4 = S * qi;
+                put_steps<S>(&sDl[k & 1][ci][q4], dv);
                 if (has_z) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
+                    for (int j = 0; j < S; ++j) {
                         const float zv = to_float(raw.z[j]);
                         gg[j] = zv * sigmoid_f(zv);
                     }
@@ -427,17 +473,21 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
                     // `x` is the upstream gradient dy here; the recurrence sees dy * silu(z)
                     if (has_z) {
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) xv[j] *= gg[j];
+                        for (int j = 0; j < S; ++j) xv[j] *= gg[j];
                     }
-                    *reinterpret_cast<float4*>(&sU[k & 1][ci][q4]) = make_float4(xv[0], xv[1], xv[2], xv[3]);
+                    put_steps<S>(&sU[k & 1][ci][q4], xv);
                 } else {
-                    *reinterpret_cast<float4*>(&sU[k & 1][ci][q4]) =
-                        make_float4(dv[0] * xv[0], dv[1] * xv[1], dv[2] * xv[2], dv[3] * xv[3]);
+                    float uv[S];
+#pragma unroll
+                    for (int j = 0; j < S; ++j) uv[j] = dv[j] * xv[j];
+                    put_steps<S>(&sU[k & 1][ci][q4], uv);
                 }
                 if constexpr (MODE == kScan) {
-                    *reinterpret_cast<float4*>(&sDx[k & 3][ci][q4]) =
-                        make_float4(Dv * xv[0], Dv * xv[1], Dv * xv[2], Dv * xv[3]);
-                    if (has_z) *reinterpret_cast<float4*>(&sG[k & 3][ci][q4]) = make_float4(gg[0], gg[1], gg[2], gg[3]);
+                    float dx[S];
+#pragma unroll
+                    for (int j = 0; j < S; ++j) dx[j] = Dv * xv[j];
+                    put_steps<S>(&sDx[k & 3][ci][q4], dx);
+                    if (has_z) put_steps<S>(&sG[k & 3][ci][q4], gg);
                 }
             };
             // tile j travels in register set j % 3; staging runs two tiles ahead of the scan
@@ -471,26 +521,40 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
                 __syncthreads();
                 if (k + 1 < ntiles) __syncthreads();
             }
-            if (p.dsum && ci_ok) p.dsum[((int64_t)bs * NQ + qi) * p.ED + d0 + ci] = dsum;
+            if constexpr (S == 4) {
+                if (p.dsum && ci_ok) p.dsum[((int64_t)bs * NQ + qi) * p.ED + d0 + ci] = dsum;
+            } else if (p.dsum) {
+                // more than NQ items per channel: the wave's own items of a channel are summed first (a
+                // time-contiguous layout has all of them in one wave, which then fills one of the NQ rows)
+                if (p.in_tmajor) {
+#pragma unroll
+                    for (int o = 1; o < QN; o *= 2) dsum += __shfl_xor(dsum, o);
+                    if (ci_ok && qi < NQ) p.dsum[((int64_t)bs * NQ + qi) * p.ED + d0 + ci] = qi == 0 ? dsum : 0.0f;
+                } else {
+#pragma unroll
+                    for (int o = CH; o < kWave; o *= 2) dsum += __shfl_xor(dsum, o);
+                    if (ci_ok && lane < CH) p.dsum[((int64_t)bs * NQ + sw) * p.ED + d0 + ci] = dsum;
+                }
+            }
         } else if constexpr (MODE == kScan) {
             // ------------------------------- reducers -------------------------------
-            const int co = p.out_tmajor ? item / NQ : item % CH;
-            const int qo = p.out_tmajor ? item % NQ : item / CH;     // walk step group
-            const int qpo = rev ? NQ - 1 - qo : qo;                  // physical step group
+            const int co = p.out_tmajor ? item / QN : item % CH;
+            const int qo = p.out_tmajor ? item % QN : item / CH;     // walk step group
+            const int qpo = rev ? QN - 1 - qo : qo;                  // physical step group
             const bool co_ok = co <= cmax;
-            const int q4 = 4 * qo;
-            const uint32_t offy = ((uint32_t)(4 * qpo) * (uint32_t)p.y_sl + (uint32_t)min(co, cmax) * (uint32_t)p.y_sd) * kES;
-            auto jw = [&](int j) { return (uint32_t)(rev ? 3 - j : j); };
-            uint32_t syj[4];
+            const int q4 = S * qo;
+            const uint32_t offy = ((uint32_t)(S * qpo) * (uint32_t)p.y_sl + (uint32_t)min(co, cmax) * (uint32_t)p.y_sd) * kES;
+            auto jw = [&](int j) { return (uint32_t)(rev ? S - 1 - j : j); };
+            uint32_t syj[S];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) syj[j] = __builtin_amdgcn_readfirstlane(jw(j) * (uint32_t)p.y_sl * kES);
+            for (int j = 0; j < S; ++j) syj[j] = __builtin_amdgcn_readfirstlane(jw(j) * (uint32_t)p.y_sl * kES);
             IO* const yg = static_cast<IO*>(p.y) + (b * p.y_sb + (int64_t)d0 * p.y_sd);
             IO* const ypg = static_cast<IO*>(p.ypre) + (b * p.y_sb + (int64_t)d0 * p.y_sd);
             // What is already in the output (a pass after the first over a wide d_state adds to
             // it): requested one interval before the tile is reduced, so that the wait for it
             // is not a wait for a load just issued.
             const IO* const yag = static_cast<const IO*>(p.yacc) + (b * p.y_sb + (int64_t)d0 * p.y_sd);
-            IO yav[4];
+            IO yav[S];
             auto load_yacc = [&](int kk) {
                 if (!p.yacc) return;
                 const int pc = phys_chunk(min(kk, ntiles - 1));
@@ -501,38 +565,62 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
                 }
                 const IO* yak = yag + (int64_t)pc * kTile * p.y_sl;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) yav[j] = ld_off(yak, offy, syj[j], wy);
+                for (int j = 0; j < S; ++j) yav[j] = ld_off(yak, offy, syj[j], wy);
             };
             auto reduce_store = [&](int k) {
                 const int pc = phys_chunk(k);
                 IO* yk = yg + (int64_t)pc * kTile * p.y_sl;
                 IO* ypk = ypg + (int64_t)pc * kTile * p.y_sl;
-                float4 s = *reinterpret_cast<const float4*>(&sDx[k & 3][co][q4]);
+                const int t0 = pc * kTile + S * qpo;  // lowest physical step of the item
+                const bool whole = !(ragged_seq && pc == last_chunk) || t0 + S - 1 < p.L;
+                float sv[S];
+                // (the form with four steps stays as it is written here: through the helpers of the other one the
+                // compiler issues all its LDS reads at once, in front of those of the scan waves, and the
+                // float32 kernel without a gate loses 5 %)
+                if constexpr (S == 4) {
+                    float4 s = *reinterpret_cast<const float4*>(&sDx[k & 3][co][q4]);
 #pragma unroll
-                for (int ww = 0; ww < NG; ++ww) {
-                    const float4 v = *reinterpret_cast<const float4*>(&sY[(k & 1) * NG + ww][co][q4]);
-                    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-                }
-                if (p.yacc) {
-                    s.x += to_float(yav[0]); s.y += to_float(yav[1]); s.z += to_float(yav[2]); s.w += to_float(yav[3]);
-                }
-                const int t0 = pc * kTile + 4 * qpo;  // lowest physical step of the item
-                const bool whole = !(ragged_seq && pc == last_chunk) || t0 + 3 < p.L;
-                if (has_z) {
-                    if (p.ypre) {
-                        const float pv[4] = {s.x, s.y, s.z, s.w};
-                        for (int j = 0; j < 4; ++j)
-                            if (co_ok && t0 + (int)jw(j) < p.L) st_off(ypk, offy, from_float<IO>(pv[j]), syj[j]);
+                    for (int ww = 0; ww < NG; ++ww) {
+                        const float4 v = *reinterpret_cast<const float4*>(&sY[(k & 1) * NG + ww][co][q4]);
+                        s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
                     }
-                    const float4 g = *reinterpret_cast<const float4*>(&sG[k & 3][co][q4]);
-                    s.x *= g.x; s.y *= g.y; s.z *= g.z; s.w *= g.w;
+                    if (p.yacc) {
+                        s.x += to_float(yav[0]); s.y += to_float(yav[1]); s.z += to_float(yav[2]); s.w += to_float(yav[3]);
+                    }
+                    if (has_z) {
+                        if (p.ypre) {
+                            const float pv[4] = {s.x, s.y, s.z, s.w};
+                            for (int j = 0; j < 4; ++j)
+                                if (co_ok && t0 + (int)jw(j) < p.L) st_off(ypk, offy, from_float<IO>(pv[j]), syj[j]);
+                        }
+                        const float4 g = *reinterpret_cast<const float4*>(&sG[k & 3][co][q4]);
+                        s.x *= g.x; s.y *= g.y; s.z *= g.z; s.w *= g.w;
+                    }
+                    sv[0] = s.x; sv[1] = s.y; sv[2] = s.z; sv[3] = s.w;
+                } else {
+                    get_steps<S>(&sDx[k & 3][co][q4], sv);
+#pragma unroll
+                    for (int ww = 0; ww < NG; ++ww) add_steps<S>(&sY[(k & 1) * NG + ww][co][q4], sv);
+                    if (p.yacc) {
+#pragma unroll
+                        for (int j = 0; j < S; ++j) sv[j] += to_float(yav[j]);
+                    }
+                    if (has_z) {
+                        if (p.ypre) {
+                            for (int j = 0; j < S; ++j)
+                                if (co_ok && t0 + (int)jw(j) < p.L) st_off(ypk, offy, from_float<IO>(sv[j]), syj[j]);
+                        }
+                        float g[S];
+                        get_steps<S>(&sG[k & 3][co][q4], g);
+#pragma unroll
+                        for (int j = 0; j < S; ++j) sv[j] *= g[j];
+                    }
                 }
-                const float sv[4] = {s.x, s.y, s.z, s.w};
                 if (co_ok && whole) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) st_off(yk, offy, from_float<IO>(sv[j]), syj[j]);
+                    for (int j = 0; j < S; ++j) st_off(yk, offy, from_float<IO>(sv[j]), syj[j]);
                 } else if (co_ok) {
-                    for (int j = 0; j < 4; ++j)
+                    for (int j = 0; j < S; ++j)
                         if (t0 + (int)jw(j) < p.L) st_off(yk, offy, from_float<IO>(sv[j]), syj[j]);
                 }
             };
@@ -552,13 +640,18 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
     // ================================= scan waves =================================
     // lane -> (channel inside the group, group of NS states): see FwdLds
     int ch = lane, sg = w;
-    if constexpr (CH == 48) {
+    if constexpr (CH != 64) {
+        constexpr int kRows = CH / 16;
         const int unit = 4 * w + (lane >> 4);
-        sg = unit / 3;
-        ch = (unit - 3 * sg) * 16 + (lane & 15);
+        sg = unit / kRows;
+        ch = (unit - kRows * sg) * 16 + (lane & 15);
     }
     const int d = d0 + ch;
     const bool dvalid = d < p.ED;
+    // (h0 and h_last belong to the batch row where the workgroup chains the segments itself, else to the
+    // row of the launch)
+    const bool chain = MODE == kScan && kBcast && p.chain_hend;
+    const int hrow = chain ? b : bs;
     float A2[NS], h[NS];
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
@@ -566,9 +659,37 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
         const bool ok = dvalid && n < p.N;
         const int dc = min(d, p.ED - 1), nc = min(n, p.N - 1);
         const float av = p.A[(int64_t)dc * p.a_st + nc];
-        const float hv = p.h0 ? p.h0[((int64_t)bs * p.ED + dc) * p.h_st + nc] : 0.0f;
+        const float hv = p.h0 ? p.h0[((int64_t)hrow * p.ED + dc) * p.h_st + nc] : 0.0f;
         A2[i] = ok ? av * kLog2e : 0.0f;
         h[i] = ok ? hv : 0.0f;
+    }
+    if constexpr (MODE == kScan && kBcast) {
+        if (chain) {
+            // seg_carry_kernel's chain over the segments before this one, four of them requested together
+            constexpr int kG = 4;
+            const int dc = min(d, p.ED - 1), prev = bs - b * p.nseg;
+            for (int s0 = 0; s0 < prev; s0 += kG) {
+                float e[kG][NS], sd[kG];
+#pragma unroll
+                for (int j = 0; j < kG; ++j) {
+                    const int64_t row = (int64_t)b * p.nseg + min(s0 + j, prev - 1);
+                    const float* ds = p.chain_dsum + row * (kTile / 4) * p.ED + dc;
+                    const float* eh = p.chain_hend + (row * p.ED + dc) * p.N;
+                    sd[j] = (ds[0] + ds[p.ED]) + (ds[2 * (int64_t)p.ED] + ds[3 * (int64_t)p.ED]);
+#pragma unroll
+                    for (int i = 0; i < NS; ++i) e[j][i] = eh[min(sg * NS + i, p.N - 1)];
+                }
+#pragma unroll
+                for (int j = 0; j < kG; ++j) {
+                    if (s0 + j >= prev) break;
+#pragma unroll
+                    for (int i = 0; i < NS; ++i) {
+                        const float ev = sg * NS + i < p.N ? e[j][i] : 0.0f;
+                        h[i] = h[i] == 0.0f ? ev : __builtin_fmaf(fast_exp2(A2[i] * sd[j]), h[i], ev);
+                    }
+                }
+            }
+        }
     }
     // registers of one tile: delta and u of the lane's channel and, on the broadcast path, one
     // register per state for B and for C whose lane t of every row holds step t
@@ -733,11 +854,11 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
         }
     }
 
-    if (p.hlast && dvalid) {
+    if (p.hlast && dvalid && (!chain || tile0 + ntiles == p.nchunks)) {
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
             const int n = sg * NS + i;
-            if (n < p.N) p.hlast[((int64_t)bs * p.ED + d) * p.h_st + n] = h[i];
+            if (n < p.N) p.hlast[((int64_t)hrow * p.ED + d) * p.h_st + n] = h[i];
         }
     }
 }
@@ -747,28 +868,37 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
 // P = exp(A * sum of delta) (the product of the segment's decay factors) the true end state of a
 // segment that starts from h is P*h + hend.  One thread per (batch row, channel, state) walks the
 // segments in order.
+template <int kGroup>
 __global__ void __launch_bounds__(256) seg_carry_kernel(const float* __restrict__ A, const float* __restrict__ h0,
                                                         const float* __restrict__ hend, const float* __restrict__ dsum,
                                                         float* __restrict__ segh0, float* __restrict__ hlast,
-                                                        int batch, int nseg, int ED, int N, int a_st, int h_st) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t per_b = (int64_t)ED * N;
-    if (i >= batch * per_b) return;
-    const int b = (int)(i / per_b);
-    const int64_t dn = i - b * per_b;
-    const int d = (int)(dn / N), n = (int)(dn - (int64_t)d * N);
+                                                        int nseg, int ED, int N, int a_st, int h_st) {
+    const uint32_t per_b = (uint32_t)ED * (uint32_t)N;  // (below 2^30, see validate_shape)
+    const uint32_t dn = blockIdx.x * 256u + threadIdx.x;
+    if (dn >= per_b) return;
+    const int b = (int)blockIdx.y, d = (int)(dn / (uint32_t)N), n = (int)(dn - (uint32_t)d * (uint32_t)N);
     const float a2 = A[(int64_t)d * a_st + n] * kLog2e;
     const int64_t ih = ((int64_t)b * ED + d) * h_st + n;  // in the caller's h0 / hlast
     float h = h0 ? h0[ih] : 0.0f;
-    for (int sg = 0; sg < nseg; ++sg) {
-        const int64_t row = (int64_t)b * nseg + sg;
-        segh0[row * per_b + dn] = h;
-        const float* ds = dsum + row * (kTile / 4) * ED + d;
-        const float sd = (ds[0] + ds[ED]) + (ds[2 * (int64_t)ED] + ds[3 * (int64_t)ED]);
-        // (a zero state stays out of the product: with A > 0 the factor can overflow, and 0 * inf
-        // is not what the step-by-step recurrence computes)
-        const float e = hend[row * per_b + dn];
-        h = h == 0.0f ? e : __builtin_fmaf(fast_exp2(a2 * sd), h, e);
+    // (what kGroup segments need is requested together: one segment after the other costs a memory
+    // latency each, 25 us for 64 segments)
+    for (int sg0 = 0; sg0 < nseg; sg0 += kGroup) {
+        float e[kGroup], sd[kGroup];
+#pragma unroll
+        for (int j = 0; j < kGroup; ++j) {
+            const uint32_t row = (uint32_t)b * nseg + min(sg0 + j, nseg - 1);
+            const float* ds = dsum + (int64_t)row * (kTile / 4) * ED + d;
+            e[j] = hend[(int64_t)row * per_b + dn];
+            sd[j] = (ds[0] + ds[ED]) + (ds[2 * (int64_t)ED] + ds[3 * (int64_t)ED]);
+        }
+#pragma unroll
+        for (int j = 0; j < kGroup; ++j) {
+            if (sg0 + j >= nseg) break;
+            segh0[((int64_t)b * nseg + sg0 + j) * per_b + dn] = h;
+            // (a zero state stays out of the product: with A > 0 the factor can overflow, and 0 * inf
+            // is not what the step-by-step recurrence computes)
+            h = h == 0.0f ? e[j] : __builtin_fmaf(fast_exp2(a2 * sd[j]), h, e[j]);
+        }
     }
     if (hlast) hlast[ih] = h;
 }
@@ -778,19 +908,9 @@ __global__ void __launch_bounds__(256) seg_carry_kernel(const float* __restrict_
 // segments that run side by side: up to twice the arithmetic, nseg times the parallelism.
 // `thin` is the coverage below which the cut pays: a third of the CUs for the forward (its first
 // pass costs 0.8 of the second), half of them for the backward (its first pass costs a quarter).
-SegPlan seg_plan(const mpa_sscan_shape* s, int ns, int thin) {
+static SegPlan seg_layout(const mpa_sscan_shape* s, int64_t want) {
     SegPlan sp{1, 0, 0, 0, 0, 0};
-    if (ns > 8) return sp;
     const int64_t ntiles = (s->seqlen + kTile - 1) / kTile;
-    const int64_t groups = s->batch * ((s->dim + kWave - 1) / kWave);
-    int64_t want = 1;
-    if (s->plan_segments > 0) {
-        want = s->plan_segments;
-    } else if (groups * thin <= 256 && ntiles >= 32) {
-        want = 256 / groups;
-        if (want > ntiles / 8) want = ntiles / 8;  // segments of 128 steps or more
-        if (want > 64) want = 64;
-    }
     if (want > ntiles) want = ntiles;
     if (want < 2 || s->batch * want > 65535) return sp;
     sp.seg_tiles = (int)((ntiles + want - 1) / want);
@@ -804,10 +924,72 @@ SegPlan seg_plan(const mpa_sscan_shape* s, int ns, int thin) {
     return sp;
 }
 
-int group_channels(const mpa_sscan_shape* s, int ns, int nseg) {
-    if (ns != 2 || s->dstate > 16 || nseg > 1 || (s->plan_flags & MPA_PLAN_GROUP_64)) return 64;
-    if (s->plan_flags & MPA_PLAN_GROUP_48) return 48;
-    return s->batch * ((s->dim + 47) / 48) <= 256 ? 48 : 64;
+SegPlan seg_plan(const mpa_sscan_shape* s, int ns, int thin) {
+    if (ns > 8) return SegPlan{1, 0, 0, 0, 0, 0};
+    const int64_t ntiles = (s->seqlen + kTile - 1) / kTile;
+    const int64_t groups = s->batch * ((s->dim + kWave - 1) / kWave);
+    int64_t want = 1;
+    if (s->plan_segments > 0) {
+        want = s->plan_segments;
+    } else if (groups * thin <= 256 && ntiles >= 32) {
+        want = 256 / groups;
+        if (want > ntiles / 8) want = ntiles / 8;  // segments of 128 steps or more
+        if (want > 64) want = 64;
+    }
+    return seg_layout(s, want);
+}
+
+// Decomposition of a forward call over the states of `s` (64 at most on this path): channels per workgroup
+// and segments per batch row.  An estimate of the time, in microseconds, decides: a tile of 16 steps
+// takes 0.51, 0.76, 0.90 and 0.95 with 16, 32, 48 and 64 channels and up to 16 states, in as many rounds as
+// the workgroups need on 256 CUs; cut, every tile is walked twice (1.75 times the time: the first
+// walk has no readout), for one more launch, the states of every segment written and read, and the chaining
+// of the segments.  Measured at lengths 128 to 16384 and 64 to 4096 channels the choice is the best or
+// within 10 % of it (bfloat16, gated: 1 x 512 x 1536: 27 us with 64 channels cut into eight, 19 us with 32 cut
+// into four; 4 x 512 x 1536: 35 -> 31 us with 32; 1 x 1024 x 512: 27 -> 16 us with 16 cut into eight; 4 x 2215 x
+// 832: 79 -> 71 us with the states chained in the second pass and not by a launch of their own).
+// A caller that pins segments, states per lane or a group of 48 or 64 channels keeps the rules of those.
+struct FwdPlan {
+    int group;
+    SegPlan seg;
+};
+// Up to this many segments the second pass chains the segments' states in front of its first tile (about
+// 0.9 us per segment before its own, under the loaders' latency); with more seg_carry_kernel, which reads
+// them once and takes about 7 us with its launch.
+static constexpr int kChainSegments = 8;
+static constexpr int kFwdThin = 3;  // (seg_plan) a third of the CUs or fewer covered
+static FwdPlan fwd_plan(const mpa_sscan_shape* s, int ns) {
+    const int pins = MPA_PLAN_GROUP_16 | MPA_PLAN_GROUP_32 | MPA_PLAN_GROUP_48 | MPA_PLAN_GROUP_64;
+    const bool narrow_ok = ns <= 8 && s->dstate <= 64 && s->plan_states_per_lane == 0;
+    if (narrow_ok && (s->plan_flags & (MPA_PLAN_GROUP_16 | MPA_PLAN_GROUP_32)))
+        return FwdPlan{(s->plan_flags & MPA_PLAN_GROUP_16) ? 16 : 32, seg_layout(s, s->plan_segments > 0 ? s->plan_segments : 1)};
+    const bool form48 = ns == 2 && s->dstate <= 16;  // the 48-channel kernel: not cut
+    if (!narrow_ok || s->plan_segments > 0 || (s->plan_flags & pins)) {
+        FwdPlan p{64, seg_plan(s, ns, kFwdThin)};
+        if (form48 && p.seg.nseg == 1 && !(s->plan_flags & MPA_PLAN_GROUP_64) &&
+            ((s->plan_flags & MPA_PLAN_GROUP_48) || s->batch * ((s->dim + 47) / 48) <= 256))
+            p.group = 48;
+        return p;
+    }
+    const int64_t ntiles = (s->seqlen + kTile - 1) / kTile;
+    const int wide = s->dstate <= 16 ? 0 : s->dstate <= 32 ? 1 : 2;
+    static constexpr int kCh[4] = {64, 48, 32, 16};
+    static constexpr float kTileUs[4][3] = {{0.95f, 1.55f, 2.85f}, {0.90f, 0.90f, 0.90f}, {0.76f, 0.90f, 1.50f}, {0.51f, 0.62f, 0.98f}};
+    static constexpr float kCutUs[4][3] = {{8.5f, 13.0f, 25.0f}, {0.0f, 0.0f, 0.0f}, {5.0f, 7.0f, 14.0f}, {4.5f, 8.0f, 13.0f}};
+    int group = 64;
+    int64_t nseg = 1;
+    float best = 1e30f;
+    for (int c = 0; c < 4; ++c) {
+        if (kCh[c] == 48 && !form48) continue;
+        const int64_t wg = s->batch * ((s->dim + kCh[c] - 1) / kCh[c]);
+        for (int64_t n = 1; n <= 64 && (n == 1 || (kCh[c] != 48 && n * 4 <= ntiles && wg * n <= 512)); ++n) {
+            const float rounds = (float)((wg * n + 255) / 256);
+            const float us = rounds * (float)((ntiles + n - 1) / n) * kTileUs[c][wide];
+            const float total = n == 1 ? 5.0f + us : kCutUs[c][wide] + 0.65f * (float)n + 1.75f * us + 4.0f * (rounds - 1.0f);
+            if (total < best) { best = total; group = kCh[c]; nseg = n; }
+        }
+    }
+    return FwdPlan{group, seg_layout(s, nseg)};
 }
 
 template <typename IO, int NS, int NW, bool HAS_Z, int MODE, int CH = 64>
@@ -824,10 +1006,24 @@ static int launch_fwd(const FwdParams& p, hipStream_t stream) {
 
 template <typename IO>
 static int dispatch_fwd(const FwdParams& p, int ns, int nw, int mode, hipStream_t stream) {
-    if (p.group48) {  // (chosen by the host only where this instance exists: see fwd_group_channels)
+    if (p.group == 48) {
         if (ns != 2 || mode != kScan) return MPA_ERR_BAD_SHAPE;
         return p.z ? launch_fwd<IO, 2, 6, true, kScan, 48>(p, stream) : launch_fwd<IO, 2, 6, false, kScan, 48>(p, stream);
     }
+    // narrow groups: the states per lane follow from d_state and the waves
+#define MPA_NARROW(CH_, NW_, NS_)                                                                   \
+    if (p.group == CH_ && p.N <= 4 * NW_ / (CH_ / 16) * NS_) {                                      \
+        if (mode == kCarry) return launch_fwd<IO, NS_, NW_, false, kCarry, CH_>(p, stream);         \
+        if (mode == kGCarry)                                                                        \
+            return p.z ? launch_fwd<IO, NS_, NW_, true, kGCarry, CH_>(p, stream)                    \
+                       : launch_fwd<IO, NS_, NW_, false, kGCarry, CH_>(p, stream);                  \
+        return p.z ? launch_fwd<IO, NS_, NW_, true, kScan, CH_>(p, stream)                          \
+                   : launch_fwd<IO, NS_, NW_, false, kScan, CH_>(p, stream);                        \
+    }
+    MPA_NARROW(16, 4, 1) MPA_NARROW(16, 4, 2) MPA_NARROW(16, 4, 4)
+    MPA_NARROW(32, 8, 1) MPA_NARROW(32, 8, 2) MPA_NARROW(32, 8, 4)
+#undef MPA_NARROW
+    if (p.group == 16 || p.group == 32) return MPA_ERR_BAD_SHAPE;
 #define MPA_CASE(NS_, NW_)                                                        \
     if (ns == NS_ && nw == NW_ && mode == kScan)                                  \
         return p.z ? launch_fwd<IO, NS_, NW_, true, kScan>(p, stream)             \
@@ -859,9 +1055,10 @@ int launch_fwd_any(const FwdParams& p, int io_dtype, int ns, int nw, int mode, h
 
 int launch_seg_carry(const float* A, const float* h0, const float* hend, const float* dsum, float* segh0,
                      float* hlast, int batch, int nseg, int ED, int N, int a_st, int h_st, hipStream_t st) {
-    const int64_t total = (int64_t)batch * ED * N;
-    hipLaunchKernelGGL(seg_carry_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, A, h0, hend, dsum,
-                       segh0, hlast, batch, nseg, ED, N, a_st, h_st);
+    // (the last group's missing segments are requested all the same, so few segments take the small group)
+    const dim3 grid((unsigned)(((int64_t)ED * N + 255) / 256), (unsigned)batch);
+    auto* k = nseg > 4 ? seg_carry_kernel<8> : seg_carry_kernel<4>;
+    hipLaunchKernelGGL(k, grid, dim3(256), 0, st, A, h0, hend, dsum, segh0, hlast, nseg, ED, N, a_st, h_st);
     return check_launch();
 }
 
@@ -939,9 +1136,6 @@ extern "C" int64_t mpa_sscan_ckpt_elems(const mpa_sscan_shape* s) {
     return s->batch * nchunks * s->dstate * s->dim;
 }
 
-// forward cut: a third of the CUs or fewer covered (see seg_plan)
-static constexpr int kFwdThin = 3;
-
 // d_state above 64: the states are independent given x, delta, B, C, so the call runs as passes
 // over blocks of 64 states on the broadcast path (8 states per lane, 8 scan waves; cut into segments
 // like any other launch), each pass adding its readout to the output.  A caller that pins more than
@@ -956,14 +1150,20 @@ extern "C" size_t mpa_sscan_fwd_workspace_bytes(const mpa_sscan_shape* s, int wi
     if (validate_shape(s) != MPA_OK) return 0;
     // the packed B/C exist only on the scalar-load path (more than 8 states per lane)
     if (fwd_in_state_blocks(s)) {
-        // passes over blocks of kFwdStateBlock states: the first block needs the most
-        mpa_sscan_shape sb = *s;
-        sb.dstate = kFwdStateBlock;
-        const int nsb = pick_states_per_lane(sb.dstate, 8, sb.plan_states_per_lane);
-        return (seg_plan(&sb, nsb, kFwdThin).floats * sizeof(float) + 255) / 256 * 256 + 256;
+        // passes over blocks of kFwdStateBlock states, the last of them perhaps narrower and cut otherwise
+        size_t floats = 0;
+        for (int64_t n : {(int64_t)kFwdStateBlock, s->dstate % kFwdStateBlock}) {
+            if (n == 0) continue;
+            mpa_sscan_shape sb = *s;
+            sb.dstate = n;
+            const int nsb = pick_states_per_lane(sb.dstate, 8, sb.plan_states_per_lane);
+            const size_t f = fwd_plan(&sb, nsb).seg.floats;
+            floats = f > floats ? f : floats;
+        }
+        return (floats * sizeof(float) + 255) / 256 * 256 + 256;
     }
     const int ns = pick_states_per_lane(s->dstate, 32, s->plan_states_per_lane);
-    if (ns <= 8) return (seg_plan(s, ns, kFwdThin).floats * sizeof(float) + 255) / 256 * 256 + 256;
+    if (ns <= 8) return (fwd_plan(s, ns).seg.floats * sizeof(float) + 255) / 256 * 256 + 256;
     return (bcpack_floats(s) * sizeof(float) + 255) / 256 * 256;
 }
 
@@ -1008,24 +1208,27 @@ static int sscan_fwd_impl(const mpa_sscan_shape* s, const void* x, const void* d
     // the launches for the states q describes (q.N of them, pointers at the first one): one
     // launch, or a sequence cut into segments (end states of every segment from zero, carry,
     // then the real pass)
-    auto run_states = [&](const FwdParams& q, int ns, int nw, const SegPlan& sp) -> int {
-        if (sp.nseg <= 1) {
-            FwdParams q1 = q;
-            q1.group48 = q.N == s->dstate && group_channels(s, ns, 1) == 48 ? 1 : 0;
-            return launch_fwd_any(q1, s->io_dtype, ns, nw, kScan, st);
-        }
+    auto run_states = [&](const FwdParams& q0, int ns, int nw, const FwdPlan& plan) -> int {
+        FwdParams q = q0;
+        q.group = plan.group;
+        const SegPlan& sp = plan.seg;
+        if (sp.nseg <= 1) return launch_fwd_any(q, s->io_dtype, ns, nw, kScan, st);
         FwdParams p1 = q;
         p1.nseg = sp.nseg; p1.seg_tiles = sp.seg_tiles;
         p1.z = nullptr; p1.y = nullptr; p1.ypre = nullptr; p1.yacc = nullptr; p1.h0 = nullptr; p1.ckpt = nullptr;
         p1.hlast = wsf + sp.off_hend; p1.dsum = wsf + sp.off_dsum; p1.h_st = q.N;
         int r = launch_fwd_any(p1, s->io_dtype, ns, nw, kCarry, st);
         if (r != MPA_OK) return r;
-        r = launch_seg_carry(q.A, q.h0, wsf + sp.off_hend, wsf + sp.off_dsum, wsf + sp.off_h0, q.hlast, q.batch,
-                             sp.nseg, q.ED, q.N, q.a_st, q.h_st, st);
-        if (r != MPA_OK) return r;
         FwdParams p2 = q;
         p2.nseg = sp.nseg; p2.seg_tiles = sp.seg_tiles;
-        p2.h0 = wsf + sp.off_h0; p2.hlast = nullptr; p2.h_st = q.N;
+        if (sp.nseg <= kChainSegments) {
+            p2.chain_hend = wsf + sp.off_hend; p2.chain_dsum = wsf + sp.off_dsum;
+        } else {
+            r = launch_seg_carry(q.A, q.h0, wsf + sp.off_hend, wsf + sp.off_dsum, wsf + sp.off_h0, q.hlast, q.batch,
+                                 sp.nseg, q.ED, q.N, q.a_st, q.h_st, st);
+            if (r != MPA_OK) return r;
+            p2.h0 = wsf + sp.off_h0; p2.hlast = nullptr; p2.h_st = q.N;
+        }
         return launch_fwd_any(p2, s->io_dtype, ns, nw, kScan, st);
     };
 
@@ -1054,7 +1257,7 @@ static int sscan_fwd_impl(const mpa_sscan_shape* s, const void* x, const void* d
             q.D = blk == 0 ? D : nullptr;
             q.yacc = blk > 0 ? ysum : nullptr;
             if (!last) { q.z = nullptr; q.y = ysum; q.ypre = nullptr; }
-            rc = run_states(q, ns, nw, seg_plan(&sb, ns, kFwdThin));
+            rc = run_states(q, ns, nw, fwd_plan(&sb, ns));
             if (rc != MPA_OK) return rc;
         }
         return MPA_OK;
@@ -1068,7 +1271,7 @@ static int sscan_fwd_impl(const mpa_sscan_shape* s, const void* x, const void* d
         rc = launch_pack_bc(s, B, C, wsf, ns, 1 /* FwdPack<NS>::kSS */, st);
         if (rc != MPA_OK) return rc;
     }
-    return run_states(p, ns, nw, seg_plan(s, ns, kFwdThin));
+    return run_states(p, ns, nw, fwd_plan(s, ns));
 }
 
 extern "C" int mpa_sscan_fwd(const mpa_sscan_shape* s, const void* x, const void* delta,

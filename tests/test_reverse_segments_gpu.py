@@ -469,3 +469,37 @@ def test_wide_state_256_bf16_sums_over_passes(pkg, dev, gated):
     print("wide-state bf16 N=256 gated=%s:" % gated, " ".join(f"{k} {v:.2e}" for k, v in errs.items()))
     for k, e in errs.items():
         assert e <= TOL[dt], f"N=256 bf16 gated={gated}: {k} rel err {e:.3e}"
+
+
+@pytest.mark.parametrize("ch", [16, 32])
+@pytest.mark.parametrize("case", [
+    # (B, L, ED, N, dtype, gated, reverse, time-contiguous, segments)
+    (2, 1, 16, 16, torch.float32, False, False, False, None), (1, 33, 17, 3, torch.float32, True, False, False, None),
+    (2, 160, 48, 16, torch.bfloat16, True, True, False, None), (1, 95, 40, 17, torch.float32, True, False, True, None),
+    (1, 130, 33, 64, torch.float32, True, True, False, None), (1, 200, 47, 32, torch.float32, True, False, False, 3),
+    (2, 257, 16, 16, torch.float32, False, True, True, 5), (1, 97, 64, 64, torch.bfloat16, True, False, False, 2),
+    (1, 300, 33, 20, torch.float32, True, False, False, 10),
+])
+def test_narrow_channel_groups_match_the_wide_form(pkg, dev, ch, case):
+    # workgroups of 16 or 32 channels: ragged groups and tiles, every count of states per lane, both directions and
+    # layouts, cut sequences; output, last state and (through the gradients) checkpoints
+    Bs, L, ED, N, dtype, gated, reverse, tmajor, nseg = case
+    inp = so.make_inputs(Bs, L, ED, N, seed=ch + L)
+    g = torch.Generator().manual_seed(L)
+    z, bias = torch.randn(Bs, L, ED, generator=g), torch.randn(ED, generator=g) * 0.2
+    h0 = torch.randn(Bs, ED, N, generator=g).to(dev)
+
+    def run(**plan):
+        lay = (lambda t: t.transpose(1, 2).contiguous().transpose(1, 2)) if tmajor else (lambda t: t)
+        leaf = {k: lay(inp[k].to(dev).to(dtype)).requires_grad_() for k in ("x", "delta")}
+        leaf.update({k: inp[k].to(dev).to(dtype).requires_grad_() for k in ("B", "C")})
+        leaf.update({k: inp[k].to(dev).requires_grad_() for k in ("A", "D")})
+        kw = dict(z=lay(z.to(dev).to(dtype)).requires_grad_(), delta_bias=bias.to(dev), delta_softplus=True) if gated else {}
+        with pkg.plan_override(**plan):
+            y, h = pkg.selective_scan_fn(**leaf, **kw, h0=h0, return_last_state=True, reverse=reverse)
+            y.backward(inp["dy"].to(dev).to(dtype))
+        return [y, h] + [t.grad for t in leaf.values()]
+
+    tol = 1e-5 if dtype == torch.float32 else 1e-2
+    for a, b in zip(run(group_channels=ch, fwd_segments=nseg), run(group_channels=64, fwd_segments=1, bwd_segments=1)):
+        assert rel_err(a, b.double()) <= tol
