@@ -28,7 +28,7 @@ struct BwdParams {
     float* partD;   // [rows][ED]
     float* partDb;  // [rows][ED]  (ddelta_bias)
     // sequence cut into nseg segments of seg_tiles tiles, counted from the END of the forward
-    // walk (the order in which the backward visits them); ag0 [rows][ED][N] = a*g flowing into
+    // walk (the order in which the backward visits them); ag0 [rows][ED][Nst] = a*g flowing into
     // every segment from the one visited before it (NULL = zeros: not cut)
     const float* ag0;
     int nseg, seg_tiles;

@@ -393,6 +393,22 @@ __global__ void __launch_bounds__(NW* kWave) sscan_bwd_kernel(const BwdParams p)
     }
 }
 
+// sum of `rows` values `stride` apart, in order; sixteen are requested together (one after the other, 64 rows
+// of a cut sequence with four passes over the states took 25 us)
+__device__ __forceinline__ float sum_rows(const float* v, int rows, int64_t stride) {
+    constexpr int kRound = 16;
+    float s = 0.0f;
+    for (int r0 = 0; r0 < rows; r0 += kRound) {
+        float t[kRound];
+#pragma unroll
+        for (int r = 0; r < kRound; ++r) t[r] = v[min(r0 + r, rows - 1) * stride];
+#pragma unroll
+        for (int r = 0; r < kRound; ++r)
+            if (r0 + r < rows) s += t[r];
+    }
+    return s;
+}
+
 // Sums the partial buffers: dB/dC over channel groups, dA over its rows_a rows (batch rows, or
 // their segments), dD/ddelta_bias over their rows_d rows (the same, or batch rows times the state
 // blocks of a wide d_state).  V = 4: d_state is a multiple of 4, a thread sums
@@ -458,18 +474,11 @@ __global__ void __launch_bounds__(256) sscan_bwd_finish_kernel(
         }
     } else if (i < bln + edn) {
         const int64_t j = i - bln;
-        float s = 0.0f;
-        for (int bb = 0; bb < rows_a; ++bb) s += partA[bb * edn + j];
-        dA[j] = s;
+        dA[j] = sum_rows(partA + j, rows_a, edn);
     } else if (i < bln + edn + ED) {
         const int64_t j = i - bln - edn;
-        float s = 0.0f, sdb = 0.0f;
-        for (int bb = 0; bb < rows_d; ++bb) {
-            s += partD[(int64_t)bb * ED + j];
-            if (dDb) sdb += partDb[(int64_t)bb * ED + j];
-        }
-        dD[j] = s;
-        if (dDb) dDb[j] = sdb;
+        dD[j] = sum_rows(partD + j, rows_d, ED);
+        if (dDb) dDb[j] = sum_rows(partDb + j, rows_d, ED);
     }
 }
 
@@ -495,9 +504,10 @@ static SegPlan bwd_seg_plan(const mpa_sscan_shape* s) {
     const int ns = bwd_states_per_lane(&blk);
     if (!bwd_fast_supported(ns, padded_states(blk.dstate) / ns) || (s->plan_flags & MPA_PLAN_BWD_GENERAL))
         return SegPlan{1, 0, 0, 0, 0, 0};
-    return seg_plan(&blk, ns, kBwdThin);
+    return seg_layout(s, seg_plan(&blk, ns, kBwdThin).nseg);  // (buffers for all states)
 }
 
+constexpr int kCarryStates = 64;  // states one launch of the carry kernel holds (8 per lane, 8 waves)
 constexpr int kStateBlock = 64;  // states one launch of the general kernel holds (4 per lane, 16 waves)
 
 struct BwdWorkspace {
@@ -637,6 +647,41 @@ extern "C" int mpa_sscan_bwd(const mpa_sscan_shape* s, const void* x, const void
         const int nseg = ws.seg.nseg > 1 ? ws.seg.nseg : 1;
         const int nblk = (p.N + kFastStates - 1) / kFastStates;
         const size_t es_ = dtype_size(s->io_dtype);
+        float* const seg = wsf + ws.offSeg;
+        if (nseg > 1) {
+            // Sequence cut into segments that run side by side.  The reverse recurrence
+            // ag[t] = a[t] * (ag[t+1] + C[t]*dy[t]) is linear in its state like the forward one,
+            // so the forward kernel in its carry mode, walking against the forward direction,
+            // finds every segment's end value from zero and its sum of delta; seg_carry_kernel chains
+            // them into the values that flow into the segments.  It holds 64 states where the kernel below holds
+            // 16 (1 x 3001 x 1000 with 64 states, float32: 25 us in one launch, 68 in four).
+            FwdParams g{};
+            g.x = dy; g.delta = delta; g.z = z; g.D = D; g.dbias = delta_bias;
+            g.bc_sb = s->bc_sb; g.bc_sl = s->bc_sl;
+            g.dsum = seg + ws.seg.off_dsum;
+            g.nseg = nseg; g.seg_tiles = ws.seg.seg_tiles;
+            g.batch = p.batch; g.L = p.L; g.ED = p.ED; g.nchunks = p.nchunks;
+            g.a_st = g.h_st = g.ck_st = p.N;
+            g.softplus = p.softplus; g.delta_f32 = p.delta_f32; g.reverse = p.reverse ? 0 : 1;
+            g.u_sb = s->y_sb; g.u_sl = s->y_sl; g.u_sd = s->y_sd;
+            g.z_sb = s->z_sb; g.z_sl = s->z_sl; g.z_sd = s->z_sd;
+            g.d_sb = s->d_sb; g.d_sl = s->d_sl; g.d_sd = s->d_sd;
+            g.in_tmajor = (s->d_sd != 1 && s->d_sl == 1) ? 1 : 0;
+            for (int n0 = 0; n0 < p.N; n0 += kCarryStates) {
+                g.N = p.N - n0 < kCarryStates ? p.N - n0 : kCarryStates;
+                g.A = A + n0;
+                g.Bm = g.C = static_cast<const char*>(C) + n0 * es_;
+                g.hlast = seg + ws.seg.off_hend + n0;
+                const int cns = pick_states_per_lane(g.N, 8, s->plan_states_per_lane);
+                rc = launch_fwd_any(g, s->io_dtype, cns, padded_states(g.N) / cns, kGCarry, st);
+                if (rc != MPA_OK) return rc;
+            }
+            // (chained by seg_carry_kernel for any number of segments: in front of the kernel below, which has no
+            // registers to spare, the chain cost the uncut call 6 %)
+            rc = launch_seg_carry(A, nullptr, seg + ws.seg.off_hend, seg + ws.seg.off_dsum, seg + ws.seg.off_h0, nullptr, p.batch,
+                                  nseg, p.ED, p.N, p.N, p.N, st);
+            if (rc != MPA_OK) return rc;
+        }
         for (int sb = 0; sb < nblk && rc == MPA_OK; ++sb) {
             const int n0 = sb * kFastStates;
             BwdParams q = p;
@@ -650,30 +695,8 @@ extern "C" int mpa_sscan_bwd(const mpa_sscan_shape* s, const void* x, const void
             q.accumulate = sb > 0 ? 1 : 0;
             q.row0 = sb * p.batch * nseg;
             if (nseg > 1) {
-                // Sequence cut into segments that run side by side.  The reverse recurrence
-                // ag[t] = a[t] * (ag[t+1] + C[t]*dy[t]) is linear in its state like the forward one,
-                // so the forward kernel in its carry mode, walking against the forward direction,
-                // finds every segment's end value from zero and its sum of delta; seg_carry_kernel
-                // chains them into the value that flows into each segment.
-                float* seg = wsf + ws.offSeg;
-                FwdParams g{};
-                g.x = dy; g.delta = delta; g.z = z; g.A = q.A; g.D = D; g.dbias = delta_bias;
-                g.Bm = q.C; g.C = q.C; g.bc_sb = s->bc_sb; g.bc_sl = s->bc_sl;
-                g.hlast = seg + ws.seg.off_hend; g.dsum = seg + ws.seg.off_dsum;
-                g.nseg = nseg; g.seg_tiles = ws.seg.seg_tiles;
-                g.batch = p.batch; g.L = p.L; g.ED = p.ED; g.N = q.N; g.nchunks = p.nchunks;
-                g.a_st = p.N; g.h_st = q.N; g.ck_st = q.N;
-                g.softplus = p.softplus; g.delta_f32 = p.delta_f32; g.reverse = p.reverse ? 0 : 1;
-                g.u_sb = s->y_sb; g.u_sl = s->y_sl; g.u_sd = s->y_sd;
-                g.z_sb = s->z_sb; g.z_sl = s->z_sl; g.z_sd = s->z_sd;
-                g.d_sb = s->d_sb; g.d_sl = s->d_sl; g.d_sd = s->d_sd;
-                g.in_tmajor = (s->d_sd != 1 && s->d_sl == 1) ? 1 : 0;
-                rc = launch_fwd_any(g, s->io_dtype, fns, fnw, kGCarry, st);
-                if (rc != MPA_OK) return rc;
-                rc = launch_seg_carry(q.A, nullptr, seg + ws.seg.off_hend, seg + ws.seg.off_dsum, seg + ws.seg.off_h0,
-                                      nullptr, p.batch, nseg, p.ED, q.N, p.N, q.N, st);
-                if (rc != MPA_OK) return rc;
-                q.nseg = nseg; q.seg_tiles = ws.seg.seg_tiles; q.ag0 = seg + ws.seg.off_h0;
+                q.nseg = nseg; q.seg_tiles = ws.seg.seg_tiles;
+                q.ag0 = seg + ws.seg.off_h0 + n0;
             }
             rc = launch_bwd_fast(q, fns, fnw, s->io_dtype, st);
         }

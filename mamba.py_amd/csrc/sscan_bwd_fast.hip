@@ -670,12 +670,12 @@ __global__ void __launch_bounds__((NW + kSvc) * kWave) sscan_bwd_fast_kernel(con
         const int n = w * NS + i;
         // (A, h0, the checkpoints and the dA partials are rows of Nst states, the states of the whole
         // call; this launch works on N of them, starting where the host put the pointers)
-        const int64_t dn = (int64_t)min(d, p.ED - 1) * p.N + min(n, p.N - 1);
-        const float av = p.A[(int64_t)min(d, p.ED - 1) * p.Nst + min(n, p.N - 1)];
+        const int64_t dn = (int64_t)min(d, p.ED - 1) * p.Nst + min(n, p.N - 1);
+        const float av = p.A[dn];
         const bool ok = dvalid && n < p.N;
         A2[i] = ok ? av * kLog2e : 0.0f;
         // a*g flowing in from the steps after this row's last one (zero at the sequence end)
-        const float ag_in = p.ag0 ? p.ag0[(int64_t)bs * p.ED * p.N + dn] : 0.0f;
+        const float ag_in = p.ag0 ? p.ag0[(int64_t)bs * p.ED * p.Nst + dn] : 0.0f;
         ag[i] = ok ? ag_in : 0.0f;
         dAacc[i] = 0.0f;
     }

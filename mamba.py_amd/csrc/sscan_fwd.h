@@ -66,6 +66,7 @@ struct SegPlan {
     size_t off_hend, off_h0, off_dsum, floats;
 };
 SegPlan seg_plan(const mpa_sscan_shape* s, int ns, int thin);
+SegPlan seg_layout(const mpa_sscan_shape* s, int64_t want);
 // Launch sscan_fwd_kernel in `mode` (FwdMode) for the (ns, nw) decomposition; the carry modes
 // exist for ns <= 8.
 int launch_fwd_any(const FwdParams& p, int io_dtype, int ns, int nw, int mode, hipStream_t stream);

@@ -248,6 +248,40 @@ __device__ __forceinline__ int service_role(int w) {
     }
 }
 
+// The state that flows into a segment of a cut sequence, from the segments the walk visits before it (`prev` of
+// them, rows row0 .. row0+prev-1): each ran from a zero state to its end state hend and summed its delta
+// (dsum, kTile/4 partial sums), so the state after it is 2^(A2 * sum of delta) * state before + hend.  On entry h
+// is the state before the first of them; a lane has states n0 .. n0+NS-1 of channel d.  Four segments are
+// requested together.
+template <int NS>
+__device__ __forceinline__ void chain_segments(const float* hend, const float* dsum, int64_t row0, int prev, int ED, int d, int st,
+                                               int n0, int N, const float (&A2)[NS], float (&h)[NS]) {
+    constexpr int kG = 4;
+    for (int s0 = 0; s0 < prev; s0 += kG) {
+        float e[kG][NS], sd[kG];
+#pragma unroll
+        for (int j = 0; j < kG; ++j) {
+            const int64_t row = row0 + min(s0 + j, prev - 1);
+            const float* ds = dsum + row * (kTile / 4) * ED + d;
+            const float* eh = hend + (row * ED + d) * st;
+            sd[j] = (ds[0] + ds[ED]) + (ds[2 * (int64_t)ED] + ds[3 * (int64_t)ED]);
+#pragma unroll
+            for (int i = 0; i < NS; ++i) e[j][i] = eh[min(n0 + i, N - 1)];
+        }
+#pragma unroll
+        for (int j = 0; j < kG; ++j) {
+            if (s0 + j >= prev) break;
+#pragma unroll
+            for (int i = 0; i < NS; ++i) {
+                const float ev = n0 + i < N ? e[j][i] : 0.0f;
+                // (a zero state stays out of the product: with A > 0 the factor can overflow, and 0 * inf
+                // is not what the step-by-step recurrence computes)
+                h[i] = h[i] == 0.0f ? ev : __builtin_fmaf(fast_exp2(A2[i] * sd[j]), h[i], ev);
+            }
+        }
+    }
+}
+
 template <typename IO, int NS, int NW, bool HAS_Z, int MODE, int CH = 64>
 __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_kernel(const FwdParams p) {
     constexpr int NQ = kTile / 4;  // step groups (of 4) per tile
@@ -664,32 +698,9 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
         h[i] = ok ? hv : 0.0f;
     }
     if constexpr (MODE == kScan && kBcast) {
-        if (chain) {
-            // seg_carry_kernel's chain over the segments before this one, four of them requested together
-            constexpr int kG = 4;
-            const int dc = min(d, p.ED - 1), prev = bs - b * p.nseg;
-            for (int s0 = 0; s0 < prev; s0 += kG) {
-                float e[kG][NS], sd[kG];
-#pragma unroll
-                for (int j = 0; j < kG; ++j) {
-                    const int64_t row = (int64_t)b * p.nseg + min(s0 + j, prev - 1);
-                    const float* ds = p.chain_dsum + row * (kTile / 4) * p.ED + dc;
-                    const float* eh = p.chain_hend + (row * p.ED + dc) * p.N;
-                    sd[j] = (ds[0] + ds[p.ED]) + (ds[2 * (int64_t)p.ED] + ds[3 * (int64_t)p.ED]);
-#pragma unroll
-                    for (int i = 0; i < NS; ++i) e[j][i] = eh[min(sg * NS + i, p.N - 1)];
-                }
-#pragma unroll
-                for (int j = 0; j < kG; ++j) {
-                    if (s0 + j >= prev) break;
-#pragma unroll
-                    for (int i = 0; i < NS; ++i) {
-                        const float ev = sg * NS + i < p.N ? e[j][i] : 0.0f;
-                        h[i] = h[i] == 0.0f ? ev : __builtin_fmaf(fast_exp2(A2[i] * sd[j]), h[i], ev);
-                    }
-                }
-            }
-        }
+        if (chain)
+            chain_segments<NS>(p.chain_hend, p.chain_dsum, (int64_t)b * p.nseg, bs - b * p.nseg, p.ED, min(d, p.ED - 1), p.N,
+                               sg * NS, p.N, A2, h);
     }
     // registers of one tile: delta and u of the lane's channel and, on the broadcast path, one
     // register per state for B and for C whose lane t of every row holds step t
@@ -908,7 +919,7 @@ __global__ void __launch_bounds__(256) seg_carry_kernel(const float* __restrict_
 // segments that run side by side: up to twice the arithmetic, nseg times the parallelism.
 // `thin` is the coverage below which the cut pays: a third of the CUs for the forward (its first
 // pass costs 0.8 of the second), half of them for the backward (its first pass costs a quarter).
-static SegPlan seg_layout(const mpa_sscan_shape* s, int64_t want) {
+SegPlan seg_layout(const mpa_sscan_shape* s, int64_t want) {
     SegPlan sp{1, 0, 0, 0, 0, 0};
     const int64_t ntiles = (s->seqlen + kTile - 1) / kTile;
     if (want > ntiles) want = ntiles;

@@ -503,3 +503,22 @@ def test_narrow_channel_groups_match_the_wide_form(pkg, dev, ch, case):
     tol = 1e-5 if dtype == torch.float32 else 1e-2
     for a, b in zip(run(group_channels=ch, fwd_segments=nseg), run(group_channels=64, fwd_segments=1, bwd_segments=1)):
         assert rel_err(a, b.double()) <= tol
+
+
+@pytest.mark.parametrize("nseg", [2, 9])
+@pytest.mark.parametrize("N,gated,reverse", [(16, True, False), (40, False, True), (80, True, False)])
+def test_cut_backward_carries_every_state_block(pkg, dev, nseg, N, gated, reverse):
+    # the carry runs for 64 states at a time, the backward for 16
+    Bs, L, ED = 2, 301, 70
+    inp = so.make_inputs(Bs, L, ED, N, seed=nseg)
+    z = torch.randn(Bs, L, ED, generator=torch.Generator().manual_seed(N))
+
+    def run(n):
+        leaf = {k: inp[k].to(dev).requires_grad_() for k in ("x", "delta", "A", "B", "C", "D")}
+        kw = dict(z=z.to(dev).requires_grad_()) if gated else {}
+        with pkg.plan_override(fwd_segments=1, bwd_segments=n):
+            pkg.selective_scan_fn(**leaf, **kw, reverse=reverse).backward(inp["dy"].to(dev))
+        return [t.grad for t in (*leaf.values(), *kw.values())]
+
+    for a, b in zip(run(nseg), run(1)):
+        assert rel_err(a, b.double()) <= 1e-5
