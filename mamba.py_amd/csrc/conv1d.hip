@@ -248,17 +248,31 @@ static int conv_validate(const mpa_conv_shape* s) {
     return MPA_OK;
 }
 
-// Steps per lane: longer spans mean fewer halo reads and fewer dweight partials, shorter spans
-// more waves; 128 steps when that still leaves 16 waves per CU.
+// Steps per lane of the backward kernel: longer spans mean fewer halo reads and fewer dweight partials, shorter
+// spans more waves; 128 steps when that still leaves 16 waves per CU, fewer than 64 below six (1 x 512 x 1536,
+// bfloat16: 14.1 us in spans of 64, 8.8 in spans of 16; 8 x 1000 x 1536: 29.6 and 46 with the sums).
 static int conv_span(const mpa_conv_shape* s) {
-    const int64_t waves128 = s->batch * ((s->seqlen + 2 * kConvSpan - 1) / (2 * kConvSpan)) * ((s->dim + kWave - 1) / kWave);
-    return waves128 >= 4096 ? 2 * kConvSpan : kConvSpan;
+    const int64_t cols = s->batch * ((s->dim + kWave - 1) / kWave);
+    if (cols * ((s->seqlen + 2 * kConvSpan - 1) / (2 * kConvSpan)) >= 4096) return 2 * kConvSpan;
+    int span = kConvSpan;
+    while (span > kConvGroup && cols * ((s->seqlen + span - 1) / span) < 1500) span /= 2;
+    return span;
 }
 
-static ConvParams conv_params(const mpa_conv_shape* s) {
+// Of the forward kernel, which leaves no partials behind: the longest that keeps 6000 waves, at least one group of
+// loads (the three steps before a span come from the L2).  Bfloat16, 1 x 512 x 1536: 8.4 us in spans of 64,
+// 4.5 in spans of 16; 8 x 3000 x 1536: 33.6, 29.2, 30.2, 33.2 us in spans of 128, 64, 32, 16.
+static int conv_fwd_span(const mpa_conv_shape* s) {
+    const int64_t cols = s->batch * ((s->dim + kWave - 1) / kWave);
+    int span = kConvSpan;
+    while (span > kConvGroup && cols * ((s->seqlen + span - 1) / span) < 6000) span /= 2;
+    return (s->seqlen + span - 1) / span > 65535 ? kConvSpan : span;  // (the grid's y axis)
+}
+
+static ConvParams conv_params(const mpa_conv_shape* s, int span) {
     ConvParams p{};
     p.batch = (int)s->batch; p.L = (int)s->seqlen; p.ED = (int)s->dim; p.K = s->kernel;
-    p.span = conv_span(s);
+    p.span = span;
     p.nspan = (p.L + p.span - 1) / p.span;
     p.silu = (s->flags & MPA_CONV_SILU) ? 1 : 0;
     p.x_sb = s->x_sb; p.x_sl = s->x_sl; p.x_sd = s->x_sd;
@@ -281,7 +295,7 @@ extern "C" int mpa_conv1d_fwd(const mpa_conv_shape* s, const void* x, const floa
     if (!aligned_to(x, es) || !aligned_to(y, es) || !aligned_to(weight, 4) || (bias && !aligned_to(bias, 4)) ||
         (window_in && !aligned_to(window_in, es)) || (window_out && !aligned_to(window_out, es)))
         return MPA_ERR_MISALIGNED;
-    ConvParams p = conv_params(s);
+    ConvParams p = conv_params(s, conv_fwd_span(s));
     p.x = x; p.w = weight; p.bias = bias; p.win = window_in; p.y = y; p.wout = window_out;
     dim3 grid((p.ED + 255) / 256, p.nspan, p.batch), block(256);
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -316,7 +330,7 @@ extern "C" int mpa_conv1d_bwd(const mpa_conv_shape* s, const void* x, const floa
         (window_in && !aligned_to(window_in, es)) || !aligned_to(workspace, 256))
         return MPA_ERR_MISALIGNED;
     if (workspace_bytes < mpa_conv1d_bwd_workspace_bytes(s)) return MPA_ERR_WORKSPACE;
-    ConvParams p = conv_params(s);
+    ConvParams p = conv_params(s, conv_span(s));
     p.x = x; p.w = weight; p.bias = bias; p.win = window_in; p.dy = dy; p.dx = dx;
     p.part = static_cast<float*>(workspace);
     dim3 grid((p.ED + 255) / 256, p.nspan, p.batch), block(256);
