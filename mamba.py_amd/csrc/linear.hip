@@ -1,0 +1,259 @@
+// y (T x M) = x (T x K) . W (M x K)^T for the projections of a layer over a short sequence, bfloat16, for
+// gfx950.
+//
+// A prompt of a few hundred steps gives products of a few GFLOP: what they cost is latency (a library
+// call of 8-12 us on the device and 18 us on the host each), not arithmetic.  The kernels here
+// run one tile per workgroup, as many workgroups as the shape offers, and take over the element-wise work around
+// the product: with `residual` the sum y + residual is stored, with `ssq_out` the partial sums of squares of its rows;
+// with `ssq`, those of x, the rows of x are normalised on their way into LDS (x * rstd * weight, rounded to bfloat16, as
+// the norm kernel rounds: a factor of the finished product would be cheaper, but rounds elsewhere).
+//
+// Tile: BT steps x BM rows of W per workgroup, each wave 32 x 32 of it (2 x 2 MFMA tiles of 16 x 16, W as the left
+// operand, so that a lane's four results are neighbours in y) over its share of K.  K runs in stages of 64 per share:
+// a stage is staged in LDS in 16-byte parts, rotated by the row (part ^ (row & 7)) so that the operand reads, one row
+// per lane, fall on different banks; D stages are in registers on their way in, two in LDS.
+//
+// At 512 steps the kernels are as fast as the library's in a queue that never runs dry (9.0 / 6.7 / 3.7 / 7.9 us for
+// in_proj, x_proj, dt_proj and out_proj of width 768, the library 9.3 / 5.1 / 5.2 / 8.2 us); what they save is
+// the norm between the layers (6 us) and three quarters of the host time (24 layers: 2.1 ms, all of it host).
+#include "common.h"
+
+namespace mpa {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+struct LinearParams {
+    const bf16_t *x, *w, *bias;
+    int64_t x_pitch, y_pitch;
+    int T, M, K;
+    bf16_t* y;
+    const float* ssq;  // [in_parts][T]
+    int in_parts;
+    float inv_d, eps;
+    const float* norm_w;  // [K], with ssq
+    const bf16_t* residual;
+    float* ssq_out;  // [M/32 rounded up][T]
+};
+
+template <int BT, int BM, int KS, int D, bool NORM>
+__global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kernel(const LinearParams p) {
+    constexpr int kThreads = BT / 32 * (BM / 32) * KS * kWave;
+    static_assert(BM * 8 * KS % kThreads == 0, "a load instruction reads W or x");
+    constexpr int kRows = BT + BM, kParts = 8 * KS, kLoads = kRows * kParts / kThreads, kStage = kRows * kParts;  // 16-byte parts
+    static_assert(D % 2 == 0, "a set of registers always goes to the same buffer");
+    __shared__ u32x4 lds[2][kStage];
+    // blocks of one XCD (every eighth) share rows of W: they walk the steps of a tile of W first
+    const int nt = (p.T + BT - 1) / BT, nm = (p.M + BM - 1) / BM, per = (nt * nm + 7) / 8;
+    const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || tile >= nt * nm) return;  // uniform over the block
+    const int m0 = tile / nt * BM, t0 = tile % nt * BT;
+    const int lane = threadIdx.x & (kWave - 1), wave = wave_id();
+    const int ks = wave % KS, wm = wave / KS % (BM / 32), wt = wave / KS / (BM / 32);
+
+    // (buffer loads: a part beyond K gets an offset beyond the window and reads as zero without a branch, which
+    // would make every wait one for all loads in flight)
+    const rsrc_t rw = make_rsrc(p.w, (uint32_t)p.M * (uint32_t)p.K * 2u);
+    const rsrc_t rx = make_rsrc(p.x, ((uint32_t)(p.T - 1) * (uint32_t)p.x_pitch + (uint32_t)p.K) * 2u);
+    uint32_t off[kLoads];
+    int koff[kLoads], at[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        const int c = threadIdx.x + i * kThreads, row = c / kParts, part = c % kParts;
+        koff[i] = part * 8;
+        off[i] = 2u * (koff[i] + (row < BM ? (uint32_t)min(m0 + row, p.M - 1) * (uint32_t)p.K
+                                           : (uint32_t)min(t0 + row - BM, p.T - 1) * (uint32_t)p.x_pitch));
+        at[i] = (part >> 3) * (kRows * 8) + row * 8 + ((part & 7) ^ (row & 7));
+    }
+    const int steps = (p.K + 64 * KS - 1) / (64 * KS);
+    constexpr int kWLoads = BM * kParts / kThreads;  // the loads of W; those of x follow
+    struct Stage {
+        u32x4 v[kLoads];
+        f32x4 w[NORM ? 2 : 1];  // norm weight of the thread's eight k (the same in all its parts)
+    };
+    const rsrc_t rn = make_rsrc(p.norm_w, (uint32_t)p.K * 4u);
+    float rs[kLoads - kWLoads];  // rstd of the rows of x the thread stages
+    Stage r[D];
+    auto load = [&](Stage& st, int s) {
+        u32x4(&v)[kLoads] = st.v;
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const int k = s * 64 * KS;
+            v[i] = __builtin_amdgcn_raw_buffer_load_b128(i * kThreads / kParts < BM ? rw : rx, k + koff[i] < p.K ? off[i] + 2u * k : 0xffffffffu, 0, 0);
+        }
+        if constexpr (NORM) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                st.w[h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rn, 4u * (uint32_t)(s * 64 * KS + koff[0] + 4 * h), 0, 0));
+        }
+    };
+    auto store = [&](const Stage& st, int buf) {
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            u32x4 v = st.v[i];
+            if (NORM && i >= kWLoads) {
+                bf16x8 x = __builtin_bit_cast(bf16x8, v);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = static_cast<__bf16>(static_cast<float>(x[e]) * rs[i - kWLoads] * st.w[e >> 2][e & 3]);
+                v = __builtin_bit_cast(u32x4, x);
+            }
+            lds[buf][at[i]] = v;
+        }
+    };
+    f32x4 acc[2][2] = {};  // [rows of W][steps]
+    const int fr = lane & 15, fq = lane >> 4;
+    auto compute = [&](int buf) {
+        const u32x4* base = lds[buf] + ks * (kRows * 8);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            const int part = (kk * 4 + fq) ^ (fr & 7);
+            bf16x8 a[2], b[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                a[i] = __builtin_bit_cast(bf16x8, base[(wm * 32 + i * 16 + fr) * 8 + part]);
+                b[i] = __builtin_bit_cast(bf16x8, base[(BM + wt * 32 + i * 16 + fr) * 8 + part]);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < D; ++i) load(r[i], i);
+    if constexpr (NORM) {
+#pragma unroll
+        for (int i = kWLoads; i < kLoads; ++i) {
+            const int t = min(t0 + (int)(threadIdx.x + i * kThreads) / kParts - BM, p.T - 1), q0 = threadIdx.x % 8;
+            float s = 0.0f;  // (the eight lanes of a row share its partial sums)
+            for (int q = q0; q < p.in_parts; q += 8) s += p.ssq[(int64_t)q * p.T + t];
+            s += __shfl_xor(s, 1);
+            s += __shfl_xor(s, 2);
+            s += __shfl_xor(s, 4);
+            rs[i - kWLoads] = __builtin_amdgcn_rsqf(s * p.inv_d + p.eps);
+        }
+    }
+    store(r[0], 0);
+    load(r[0], D);
+    __syncthreads();
+    // (whole groups of D stages without a branch, so that every wait is for the one stage it needs; loads and
+    // stores beyond the last stage are of zeros)
+    int s0 = 0;
+    for (; s0 + D <= steps; s0 += D) {
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+            store(r[(i + 1) % D], (i + 1) & 1);
+            load(r[(i + 1) % D], s0 + i + 1 + D);
+            compute(i & 1);
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < D - 1; ++i) {
+        if (s0 + i >= steps) break;
+        store(r[(i + 1) % D], (i + 1) & 1);
+        compute(i & 1);
+        __syncthreads();
+    }
+    if constexpr (KS > 1) {
+        // (the stages are done with: the last barrier)
+        f32x4* part = reinterpret_cast<f32x4*>(&lds[0][0]);
+        if (ks > 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) part[(wave * 4 + i) * kWave + lane] = acc[i >> 1][i & 1];
+        }
+        __syncthreads();
+        if (ks > 0) return;
+#pragma unroll
+        for (int q = 1; q < KS; ++q)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i >> 1][i & 1] += part[((wave + q) * 4 + i) * kWave + lane];
+    }
+    float ss[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int m = m0 + wm * 32 + i * 16 + fq * 4;
+        if (m >= p.M) continue;
+        bf16x4 bias = {};
+        if (p.bias) bias = *reinterpret_cast<const bf16x4*>(p.bias + m);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int t = t0 + wt * 32 + j * 16 + fr;
+            if (t >= p.T) continue;
+            const int64_t o = (int64_t)t * p.y_pitch + m;
+            bf16x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = static_cast<__bf16>(acc[i][j][e] + static_cast<float>(bias[e]));
+            if (p.residual) {
+                const bf16x4 res = *reinterpret_cast<const bf16x4*>(p.residual + o);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = static_cast<__bf16>(static_cast<float>(v[e]) + static_cast<float>(res[e]));
+            }
+            *reinterpret_cast<bf16x4*>(p.y + o) = v;
+            if (p.ssq_out) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) ss[j] = __builtin_fmaf(static_cast<float>(v[e]), static_cast<float>(v[e]), ss[j]);
+            }
+        }
+    }
+    if (p.ssq_out) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int t = t0 + wt * 32 + j * 16 + fr, q = (m0 + wm * 32) / 32;
+            float s = ss[j];
+            s += __shfl_xor(s, 16);
+            s += __shfl_xor(s, 32);
+            if (fq == 0 && t < p.T && q * 32 < p.M) p.ssq_out[(int64_t)q * p.T + t] = s;
+        }
+    }
+}
+
+template <int BT, int BM, int KS>
+static int launch_linear(const LinearParams& p, hipStream_t st) {
+    const int nt = (p.T + BT - 1) / BT, nm = (p.M + BM - 1) / BM, per = (nt * nm + 7) / 8;
+    const dim3 grid((unsigned)per * 8), block(BT / 32 * (BM / 32) * KS * kWave);
+    if (p.ssq) hipLaunchKernelGGL((linear_kernel<BT, BM, KS, 2, true>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((linear_kernel<BT, BM, KS, 2, false>), grid, block, 0, st, p);
+    return check_launch();
+}
+
+// The largest tile that gives most CUs one (a tile's traffic per product falls with its size), smaller ones
+// with K split over more waves (512 steps of a layer of width 768: in_proj 9.0 us with 64 x 128, 9.9 with 64 x
+// 64, 15 with 32 x 32; out_proj 7.9 us with 64 x 32 on eight waves, 10.8 with 64 x 64; x_proj 6.7 and 10.2 us).
+static int dispatch_linear(const LinearParams& p, hipStream_t st) {
+    auto tiles = [&](int bt, int bm) { return (int64_t)((p.T + bt - 1) / bt) * ((p.M + bm - 1) / bm); };
+    constexpr int kFull = 160;
+    if (tiles(64, 128) >= kFull) return launch_linear<64, 128, 1>(p, st);
+    if (p.K <= 128) return launch_linear<64, 64, 1>(p, st);  // (one or two stages: nothing to split)
+    if (tiles(64, 64) >= kFull) return p.K >= 1024 ? launch_linear<64, 64, 2>(p, st) : launch_linear<64, 64, 1>(p, st);
+    if (tiles(64, 32) >= kFull) return p.K >= 1024 ? launch_linear<64, 32, 4>(p, st) : launch_linear<64, 32, 2>(p, st);
+    return launch_linear<32, 32, 4>(p, st);
+}
+
+}  // namespace mpa
+
+using namespace mpa;
+
+extern "C" int mpa_linear_bf16(const mpa_linear* s, void* stream) {
+    if (!s || !s->x || !s->weight || !s->y) return MPA_ERR_NULL_POINTER;
+    if (s->x_ssq && !s->norm_weight) return MPA_ERR_NULL_POINTER;
+    // (x and the weight are addressed with 32-bit byte offsets)
+    if (s->T <= 0 || s->M <= 0 || s->K <= 0 || s->K % 8 || s->x_pitch % 8 || s->M % 4 || s->y_pitch % 4 || s->x_pitch < s->K ||
+        s->y_pitch < s->M || s->T > 1 << 24 || s->M > 1 << 24 || s->K > 1 << 24 || s->T * s->x_pitch >= (int64_t)1 << 30 ||
+        s->M * s->K >= (int64_t)1 << 30 || (s->x_ssq && (s->ssq_parts <= 0 || s->ssq_parts > 1 << 20)))
+        return MPA_ERR_BAD_SHAPE;
+    if (!aligned_to(s->x, 16) || !aligned_to(s->weight, 16) || !aligned_to(s->bias, 8) || !aligned_to(s->y, 8) ||
+        !aligned_to(s->residual, 8) || !aligned_to(s->norm_weight, 16) || !aligned_to(s->x_ssq, 4) || !aligned_to(s->y_ssq, 4))
+        return MPA_ERR_MISALIGNED;
+    LinearParams p{};
+    p.x = static_cast<const bf16_t*>(s->x); p.w = static_cast<const bf16_t*>(s->weight); p.bias = static_cast<const bf16_t*>(s->bias);
+    p.x_pitch = s->x_pitch; p.y_pitch = s->y_pitch;
+    p.T = (int)s->T; p.M = (int)s->M; p.K = (int)s->K;
+    p.y = static_cast<bf16_t*>(s->y);
+    p.ssq = s->x_ssq; p.in_parts = (int)s->ssq_parts;
+    p.inv_d = 1.0f / (float)s->K; p.eps = s->eps; p.norm_w = s->norm_weight;
+    p.residual = static_cast<const bf16_t*>(s->residual);
+    p.ssq_out = s->y_ssq;
+    return dispatch_linear(p, static_cast<hipStream_t>(stream));
+}

@@ -1,0 +1,41 @@
+"""The bfloat16 projection kernel of short sequences against float64 products."""
+import ctypes
+
+import pytest
+import torch
+from util import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+class Linear(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int64) for n in ("T", "M", "K", "x_pitch", "y_pitch")] + \
+               [(n, ctypes.c_void_p) for n in ("x", "weight", "bias", "y", "norm_weight", "x_ssq")] + \
+               [("ssq_parts", ctypes.c_int64), ("eps", ctypes.c_float), ("residual", ctypes.c_void_p), ("y_ssq", ctypes.c_void_p)]
+
+
+# tiles of every size (few to many rows and columns, short and long K) with remainders in T, M and K
+@pytest.mark.parametrize("T,M,K,pitch", [(1, 4, 8, 8), (33, 100, 72, 80), (65, 520, 1032, 1032), (500, 1540, 264, 264), (700, 1000, 1096, 1096),
+                                         (1000, 1288, 64, 128), (2047, 900, 136, 144)])
+@pytest.mark.parametrize("fused", [False, True])
+def test_linear_matches_product(pkg, dev, T, M, K, pitch, fused):
+    L, lib = pkg._lib, pkg._lib.load()
+    g = torch.Generator().manual_seed(T)
+    rand = lambda *s: torch.randn(*s, generator=g).to(dev)
+    x, w = rand(T, pitch).bfloat16(), rand(M, K).bfloat16()
+    q = Linear(T=T, M=M, K=K, x_pitch=pitch, y_pitch=M, x=x.data_ptr(), weight=w.data_ptr())
+    y = torch.full((T, M), float("nan"), device=dev, dtype=torch.bfloat16)
+    q.y = y.data_ptr()
+    want = x[:, :K].double() @ w.double().t()
+    if fused:
+        bias, res, nw = rand(M).bfloat16(), rand(T, M).bfloat16(), rand(K)
+        ssq, eps = rand(5, T).square() * K / 5, 1e-5
+        out_ssq = torch.empty((M + 31) // 32, T, device=dev)
+        q.bias, q.residual, q.y_ssq = bias.data_ptr(), res.data_ptr(), out_ssq.data_ptr()
+        q.norm_weight, q.x_ssq, q.ssq_parts, q.eps = nw.data_ptr(), ssq.data_ptr(), 5, eps
+        normed = x[:, :K].double() * (ssq.double().sum(0) / K + eps).rsqrt()[:, None] * nw.double()
+        want = normed @ w.double().t() + bias.double() + res.double()
+    L.check(lib.mpa_linear_bf16(ctypes.byref(q), pkg.scan._stream(dev)), "mpa_linear_bf16")
+    assert rel_err(y.float(), want) <= 1e-2  # (rounded twice with a residual)
+    if fused:
+        assert rel_err(out_ssq.sum(0), y.double().square().sum(1)) <= 1e-5
