@@ -381,6 +381,32 @@ __global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams
     }
 }
 
+// Rows of x times the norm weight in operand order, and their sums of squares: what decode_out of a layer before
+// would have left.  One workgroup per sequence.
+template <typename IO>
+__global__ void __launch_bounds__(256) decode_scale_kernel(const DecodeParams p, void* xw, float* ssq) {
+    constexpr int kVec = Frag<IO>::kVec;
+    __shared__ float part[4];
+    const int b = blockIdx.x;
+    const IO* row = static_cast<const IO*>(p.x) + (int64_t)b * p.d;
+    float ss = 0.0f;
+    for (int k = threadIdx.x * kVec; k < p.d; k += 256 * kVec) {
+        float f[kVec];
+        Frag<IO>::unpack(ld16(row + k), f);
+#pragma unroll
+        for (int i = 0; i < kVec; ++i) {
+            ss = __builtin_fmaf(f[i], f[i], ss);
+            if (p.norm_w) f[i] *= p.norm_w[k + i];
+        }
+        *reinterpret_cast<u32x4*>(static_cast<IO*>(xw) + frag_at<IO>(b, k, p.d)) = Frag<IO>::pack(f);
+    }
+#pragma unroll
+    for (int o = 1; o < kWave; o *= 2) ss += __shfl_xor(ss, o);
+    if ((threadIdx.x & (kWave - 1)) == 0) part[wave_id()] = ss;
+    __syncthreads();
+    if (threadIdx.x == 0) ssq[b] = (part[0] + part[1]) + (part[2] + part[3]);
+}
+
 template <typename IO, int NW>
 __global__ void __launch_bounds__(NW* kWave) decode_xproj_kernel(const DecodeParams p, int row_tiles, int groups) {
     __shared__ WaveLds tile[NW];
@@ -572,10 +598,11 @@ static dim3 decode_grid(int64_t row_tiles, int64_t groups, int splits) {
 // per CU, which hides more (in_proj at 64 x 768, bfloat16: 6.1 us, 8.7 us with U = 2).  in_proj with more
 // than 1536 tiles takes two batch tiles per workgroup (128 x 768: 8.6 us on four waves, 10.0 with one
 // tile), on eight waves where K is long (64 x 2560, float32: 55 us, 62 on four).
+constexpr int kManyTiles = 1536;
 template <typename IO, int MODE>
 static int launch_in(const DecodeParams& p, hipStream_t st) {
     const int rt = (2 * p.ED + 15) / 16, bt = (p.batch + 15) / 16;
-    if (rt * bt < 1536) {
+    if (rt * bt < kManyTiles) {
         hipLaunchKernelGGL((decode_in_kernel<IO, 1, 8, 1, MODE>), decode_grid(rt, bt, 1), dim3(512), 0, st, p, rt, bt);
     } else {
         const int groups = (bt + 1) / 2;
@@ -617,8 +644,18 @@ static int launch_ssm(const DecodeParams& p, hipStream_t st) {
     return check_launch();
 }
 
+// A first layer whose in_proj has many tiles: each of them would normalise its sequences again, and read them by
+// rows (64 x 2560, float32: 88 us, 62 + 4 with the rows prepared).
+static bool scale_first(int ED, int batch) { return (2 * ED + 15) / 16 * ((batch + 15) / 16) >= kManyTiles; }
+
 template <typename IO>
-static int decode_launch(const DecodeParams& p, bool norm, hipStream_t st) {
+static int decode_launch(DecodeParams p, bool norm, void* xw, float* ssq, hipStream_t st) {
+    if (norm && !p.xw && scale_first(p.ED, p.batch)) {
+        hipLaunchKernelGGL((decode_scale_kernel<IO>), dim3(p.batch), dim3(256), 0, st, p, xw, ssq);
+        const int e = check_launch();
+        if (e != MPA_OK) return e;
+        p.xw = xw; p.ssq = ssq; p.ssq_tiles = 1;
+    }
     int rc = !norm ? launch_in<IO, kInPlain>(p, st) : p.xw ? launch_in<IO, kInReady>(p, st) : launch_in<IO, kInNorm>(p, st);
     if (rc != MPA_OK) return rc;
     rc = launch_xproj<IO>(p, st);
@@ -640,10 +677,15 @@ extern "C" size_t mpa_decode_scaled_bytes(const mpa_decode_layer* s) {
     return decode_validate(s) == MPA_OK ? (size_t)frag_bytes(s->batch, s->d_model, (int)dtype_size(s->io_dtype)) : 0;
 }
 
+static size_t decode_scaled_ws(const mpa_decode_layer* s) {
+    return s->norm && scale_first((int)s->dim, (int)s->batch)
+               ? (size_t)frag_bytes(s->batch, s->d_model, (int)dtype_size(s->io_dtype)) + round256(s->batch * sizeof(float)) : 0;
+}
+
 extern "C" size_t mpa_decode_layer_workspace_bytes(const mpa_decode_layer* s) {
     if (decode_validate(s) != MPA_OK) return 0;
     const size_t act = (size_t)frag_bytes(s->batch, s->dim, (int)dtype_size(s->io_dtype));
-    return 3 * act + round256((size_t)decode_splits(s) * s->batch * (s->dt_rank + 2 * s->dstate) * sizeof(float));
+    return 3 * act + round256((size_t)decode_splits(s) * s->batch * (s->dt_rank + 2 * s->dstate) * sizeof(float)) + decode_scaled_ws(s);
 }
 
 extern "C" int mpa_decode_layer_step(const mpa_decode_layer* s, const void* x, const void* x_scaled, const float* x_ssq, void* y,
@@ -680,5 +722,7 @@ extern "C" int mpa_decode_layer_step(const mpa_decode_layer* s, const void* x, c
     char* ws = static_cast<char*>(workspace);
     p.xs = ws; p.z = ws + act; p.g = ws + 2 * act; p.dbc = reinterpret_cast<float*>(ws + 3 * act);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    return s->io_dtype == MPA_F32 ? decode_launch<float>(p, s->norm != 0, st) : decode_launch<bf16_t>(p, s->norm != 0, st);
+    char* const xw = ws + mpa_decode_layer_workspace_bytes(s) - decode_scaled_ws(s);
+    float* const ssq = reinterpret_cast<float*>(xw + frag_bytes(s->batch, s->d_model, (int)es));
+    return s->io_dtype == MPA_F32 ? decode_launch<float>(p, s->norm != 0, xw, ssq, st) : decode_launch<bf16_t>(p, s->norm != 0, xw, ssq, st);
 }
