@@ -1,5 +1,5 @@
 // One decode step of a whole residual layer (norm, in_proj, convolution, x_proj, dt_proj, state
-// update, gate, out_proj) in four launches, for gfx950.
+// update, gate, out_proj) in three or four launches, for gfx950.
 //
 // At decode batch sizes every operation of a layer is a pass over a weight matrix of a few MB or
 // over the recurrent state: 2-3 us of memory time next to ~1.6 us of launch time per graph node.
@@ -9,7 +9,7 @@
 //
 //   decode_in_kernel   RMSNorm, in_proj, and for the x half the convolution over the rolling
 //                      window with bias and silu
-//   decode_xproj_kernel  x_proj (float32 partial sums over ranges of K)
+//   decode_xproj_kernel  x_proj (float32 partial sums over ranges of K); in a small call decode_in does it
 //   decode_ssm_kernel  dt_proj, softplus, state update, readout, gate
 //   decode_out_kernel  out_proj, residual add, and what the next layer's norm needs
 //
@@ -286,11 +286,14 @@ __device__ __forceinline__ void decode_tile(int row_tiles, int groups, int& rt, 
     bt = (in >> 3) * NT;
 }
 
-template <typename IO, int NT, int NW, int U, int MODE>
+// XP: also the workgroup's share of x_proj, its 16 channels' product with all rows of x_proj's weight, as one
+// more partial sum of dbc; a thread owns one row and every so many sequences.
+template <typename IO, int NT, int NW, int U, int MODE, bool XP = false>
 __global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams p, int row_tiles, int groups) {
     constexpr int kThreads = NW * kWave, kAll = NT * 256, kOuts = (kAll + kThreads - 1) / kThreads;
     __shared__ WaveLds tile[NW];
     __shared__ float ssq[NW][NT][16];
+    __shared__ float xl[XP ? NT * 16 : 1][16];  // convolved x of the tile
     int rt, bt;
     decode_tile<NT>(row_tiles, groups, rt, bt);
     if (rt >= row_tiles) return;  // uniform over the block
@@ -301,7 +304,18 @@ __global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams
     IO win[kOuts][3];
     float cw[kOuts][4], cb[kOuts], ib[kOuts];
     float ss[NT] = {};
+    const int P = p.R + 2 * p.N;
+    u32x4 xw[XP ? 16 / Frag<IO>::kVec : 1];
     auto more = [&] {
+        if constexpr (XP) {
+            // (a part beyond the last channel is read at the row's start and meets zeros)
+            const IO* row = static_cast<const IO*>(p.xp_w) + (int64_t)(threadIdx.x % P) * p.ED;
+#pragma unroll
+            for (int i = 0; i < 16 / Frag<IO>::kVec; ++i) {
+                const int k = n0 + i * Frag<IO>::kVec;
+                xw[i] = ld16(row + (k < p.ED ? k : 0));
+            }
+        }
 #pragma unroll
         for (int i = 0; i < kOuts; ++i) {
             const int o = threadIdx.x + i * kThreads, n = n0 + o % 16, b = b0 + o / 16;
@@ -377,7 +391,29 @@ __global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams
         for (int j = 0; j < 3; ++j)
             if (j <= last) wo[j] = j < last ? win[i][j < 2 ? j + 1 : 2] : vr;
         c *= sigmoid_f(c);
-        static_cast<IO*>(p.xs)[frag_at<IO>(b, n, p.ED)] = from_float<IO>(c);
+        const IO cr = from_float<IO>(c);
+        static_cast<IO*>(p.xs)[frag_at<IO>(b, n, p.ED)] = cr;
+        if constexpr (XP) xl[bl][row] = to_float(cr);
+    }
+    if constexpr (XP) {
+        if (n0 >= p.ED) return;  // uniform over the block
+        if (n0 + 16 > p.ED)
+            for (int o = threadIdx.x; o < kAll; o += kThreads)
+                if (n0 + o % 16 >= p.ED) xl[o / 16][o % 16] = 0.0f;
+        __syncthreads();
+        const int G = kThreads / P, g = threadIdx.x / P, nb = min(p.batch - b0, NT * 16);
+        if (g >= G) return;
+        for (int b = g; b < nb; b += G) {
+            float s = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 16 / Frag<IO>::kVec; ++i) {
+                float w[Frag<IO>::kVec];
+                Frag<IO>::unpack(xw[i], w);
+#pragma unroll
+                for (int e = 0; e < Frag<IO>::kVec; ++e) s = __builtin_fmaf(w[e], xl[b][i * Frag<IO>::kVec + e], s);
+            }
+            p.dbc[((int64_t)rt * p.batch + b0 + b) * P + threadIdx.x % P] = s;
+        }
     }
 }
 
@@ -474,12 +510,41 @@ __global__ void __launch_bounds__(NW* kWave) decode_out_kernel(const DecodeParam
     }
 }
 
+// DTV consecutive values of a row of dt_proj
+template <typename IO, int DTV>
+struct DtVec {  // one element
+    typedef IO Raw;
+    static __device__ __forceinline__ Raw load(const IO* p) { return *p; }
+    static __device__ __forceinline__ void unpack(const Raw& r, float (&w)[DTV]) { w[0] = to_float(r); }
+};
+template <>
+struct DtVec<bf16_t, 4> {
+    typedef u32x2 Raw;
+    static __device__ __forceinline__ Raw load(const bf16_t* p) { return *reinterpret_cast<const u32x2*>(p); }
+    static __device__ __forceinline__ void unpack(const Raw& v, float (&w)[4]) {
+        w[0] = __uint_as_float(v[0] << 16);
+        w[1] = __uint_as_float(v[0] & 0xffff0000u);
+        w[2] = __uint_as_float(v[1] << 16);
+        w[3] = __uint_as_float(v[1] & 0xffff0000u);
+    }
+};
+template <>
+struct DtVec<float, 4> {
+    typedef u32x4 Raw;
+    static __device__ __forceinline__ Raw load(const float* p) { return ld16(p); }
+    static __device__ __forceinline__ void unpack(const Raw& v, float (&w)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = __uint_as_float(v[i]);
+    }
+};
+
 // A thread owns a quarter of the states and of the dt_rank of one channel, for BT sequences: the
 // quarter sums of dt_proj meet in a quad (two exchanges), after which every lane of the quad has
 // delta and goes on with its own states.  State loads are issued before the dt_proj sum.
-template <typename IO, int BT, bool N16, int DTV>
+// MANY: dbc comes as many partial sums (see xproj_fused).
+template <typename IO, int BT, bool N16, int DTV, bool MANY>
 __global__ void __launch_bounds__(256) decode_ssm_kernel(const DecodeParams p) {
-    extern __shared__ float dbc[];  // [BT][R + 2N]
+    extern __shared__ float dbc[];  // [BT][R + 2N], as many times as threads allow while it is summed
     const int P = p.R + 2 * p.N;
     const int b0 = blockIdx.y * BT;
     const int part = threadIdx.x & 3, ch = blockIdx.x * 64 + (threadIdx.x >> 2);
@@ -497,36 +562,63 @@ __global__ void __launch_bounds__(256) decode_ssm_kernel(const DecodeParams p) {
         zv[t] = load_as_float<IO>(p.z, row);
     }
     const float Dv = p.D[d], bias = p.dt_b ? p.dt_b[d] : 0.0f;
-    for (int i = threadIdx.x; i < BT * P; i += 256) {
-        const int t = i / P, b = b0 + t;
-        float s = 0.0f;
-        if (b < p.batch)
-            for (int q = 0; q < p.splits; ++q) s += p.dbc[((int64_t)q * p.batch + b) * P + (i - t * P)];
-        dbc[i] = s;
-    }
-    __syncthreads();
-    float dl[BT] = {};
+    // the first rows of dt_proj are requested here, ahead of the barriers
+    typedef DtVec<IO, DTV> Dt;
+    constexpr int kPre = 3;
     const IO* wr = static_cast<const IO*>(p.dt_w) + (int64_t)d * p.R;
-    for (int r = DTV * part; r < p.R; r += 4 * DTV) {
-        float w[DTV];
-        if constexpr (DTV == 4 && sizeof(IO) == 2) {
-            const u32x2 v = *reinterpret_cast<const u32x2*>(wr + r);
-            w[0] = __uint_as_float(v[0] << 16);
-            w[1] = __uint_as_float(v[0] & 0xffff0000u);
-            w[2] = __uint_as_float(v[1] << 16);
-            w[3] = __uint_as_float(v[1] & 0xffff0000u);
-        } else if constexpr (DTV == 4) {
-            const u32x4 v = ld16(wr + r);
+    typename Dt::Raw pre[kPre];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) w[i] = __uint_as_float(v[i]);
-        } else {
-            w[0] = to_float(wr[r]);
+    for (int i = 0; i < kPre; ++i) pre[i] = Dt::load(wr + min(DTV * (part + 4 * i), p.R - DTV));
+    if constexpr (!MANY) {
+        for (int i = threadIdx.x; i < BT * P; i += 256) {
+            const int t = i / P, b = b0 + t;
+            float s = 0.0f;
+            if (b < p.batch)
+                for (int q = 0; q < p.splits; ++q) s += p.dbc[((int64_t)q * p.batch + b) * P + (i - t * P)];
+            dbc[i] = s;
         }
+        __syncthreads();
+    } else {
+        static_assert(BT == 1, "small calls take one sequence per workgroup");
+        // thread -> (output, every G-th of the partial sums), sixteen requested together
+        const int G = max(256 / P, 1), g = G > 1 ? threadIdx.x / P : 0;
+        for (int i = G > 1 ? threadIdx.x % P : threadIdx.x; i < P && g < G; i += 256) {
+            const float* src = p.dbc + (int64_t)b0 * P + i;
+            const int64_t pitch = (int64_t)p.batch * P;
+            float s = 0.0f;
+            for (int q0 = g; q0 < p.splits; q0 += 16 * G) {
+                float v[16];
+#pragma unroll
+                for (int j = 0; j < 16; ++j) v[j] = src[min(q0 + j * G, p.splits - 1) * pitch];
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    if (q0 + j * G < p.splits) s += v[j];
+            }
+            dbc[g * P + i] = s;
+        }
+        __syncthreads();
+        if (G > 1) {
+            float s = 0.0f;
+            if ((int)threadIdx.x < P)
+                for (int q = 0; q < G; ++q) s += dbc[q * P + threadIdx.x];
+            __syncthreads();
+            if ((int)threadIdx.x < P) dbc[threadIdx.x] = s;
+            __syncthreads();
+        }
+    }
+    float dl[BT] = {};
+    auto dt_dot = [&](const typename Dt::Raw& raw, int r) {
+        float w[DTV];
+        Dt::unpack(raw, w);
 #pragma unroll
         for (int t = 0; t < BT; ++t)
 #pragma unroll
             for (int i = 0; i < DTV; ++i) dl[t] = __builtin_fmaf(w[i], dbc[t * P + r + i], dl[t]);
-    }
+    };
+#pragma unroll
+    for (int i = 0; i < kPre; ++i)
+        if (DTV * (part + 4 * i) < p.R) dt_dot(pre[i], DTV * (part + 4 * i));
+    for (int r = DTV * (part + 4 * kPre); r < p.R; r += 4 * DTV) dt_dot(Dt::load(wr + r), r);
 #pragma unroll
     for (int t = 0; t < BT; ++t) {
         const int b = b0 + t;
@@ -577,7 +669,9 @@ static int decode_validate(const mpa_decode_layer* s) {
 // K ranges of x_proj: its few rows give few workgroups, so K is cut until about 128 of them run
 // (each with at least one piece per wave); the state kernel adds the partial sums as it reads them.
 constexpr int kXprojWaves = 8;
+static bool xproj_fused(int ED, int P, int batch);
 static int decode_splits(const mpa_decode_layer* s) {
+    if (xproj_fused((int)s->dim, (int)(s->dt_rank + 2 * s->dstate), (int)s->batch)) return (int)((s->dim + 15) / 16);
     const int64_t piece = s->io_dtype == MPA_BF16 ? 64 : 32;
     const int64_t tiles = ((s->dt_rank + 2 * s->dstate + 15) / 16) * ((s->batch + 15) / 16);
     const int64_t by_k = (s->dim + piece * kXprojWaves - 1) / (piece * kXprojWaves);
@@ -599,10 +693,19 @@ static dim3 decode_grid(int64_t row_tiles, int64_t groups, int splits) {
 // than 1536 tiles takes two batch tiles per workgroup (128 x 768: 8.6 us on four waves, 10.0 with one
 // tile), on eight waves where K is long (64 x 2560, float32: 55 us, 62 on four).
 constexpr int kManyTiles = 1536;
+
+// in_proj does its share of x_proj for one batch tile while the partial sums that it leaves, one per 16 channels, are
+// few: they cost the state kernel less than a launch then (a layer of width 768 in bfloat16, one sequence: 16.3 ->
+// 14.9 us, 16 sequences 18.2 -> 17.1; width 256 13.1 -> 11.3; but width 2560 in float32, eight times the partial
+// sums, 56 -> 72).
+static bool xproj_fused(int ED, int P, int batch) { return batch <= 16 && P <= 512 && (int64_t)((ED + 15) / 16) * P <= 16384; }
+
 template <typename IO, int MODE>
 static int launch_in(const DecodeParams& p, hipStream_t st) {
     const int rt = (2 * p.ED + 15) / 16, bt = (p.batch + 15) / 16;
-    if (rt * bt < kManyTiles) {
+    if (xproj_fused(p.ED, p.R + 2 * p.N, p.batch)) {
+        hipLaunchKernelGGL((decode_in_kernel<IO, 1, 8, 1, MODE, true>), decode_grid(rt, bt, 1), dim3(512), 0, st, p, rt, bt);
+    } else if (rt * bt < kManyTiles) {
         hipLaunchKernelGGL((decode_in_kernel<IO, 1, 8, 1, MODE>), decode_grid(rt, bt, 1), dim3(512), 0, st, p, rt, bt);
     } else {
         const int groups = (bt + 1) / 2;
@@ -634,10 +737,16 @@ static int launch_out(const DecodeParams& p, hipStream_t st) {
 template <typename IO, int BT>
 static int launch_ssm(const DecodeParams& p, hipStream_t st) {
     const dim3 grid((p.ED + 63) / 64, (p.batch + BT - 1) / BT);
-    const size_t lds = (size_t)BT * (p.R + 2 * p.N) * sizeof(float);
+    const int outs = BT * (p.R + 2 * p.N);
+    const size_t lds = (size_t)(outs < 256 ? 256 : outs) * sizeof(float);
     if (lds > 48 * 1024) return MPA_ERR_BAD_SHAPE;
     const bool v4 = p.R % 4 == 0 && aligned_to(p.dt_w, 4 * sizeof(IO));
-#define MPA_SSM(N16_, V_) hipLaunchKernelGGL((decode_ssm_kernel<IO, BT, N16_, V_>), grid, dim3(256), lds, st, p)
+    const bool many = BT == 1 && xproj_fused(p.ED, p.R + 2 * p.N, p.batch);
+#define MPA_SSM(N16_, V_)                                                                                              \
+    do {                                                                                                               \
+        if (many) hipLaunchKernelGGL((decode_ssm_kernel<IO, 1, N16_, V_, true>), grid, dim3(256), lds, st, p);         \
+        else hipLaunchKernelGGL((decode_ssm_kernel<IO, BT, N16_, V_, false>), grid, dim3(256), lds, st, p);            \
+    } while (0)
     if (p.N == 16) { if (v4) MPA_SSM(true, 4); else MPA_SSM(true, 1); }
     else { if (v4) MPA_SSM(false, 4); else MPA_SSM(false, 1); }
 #undef MPA_SSM
@@ -658,7 +767,7 @@ static int decode_launch(DecodeParams p, bool norm, void* xw, float* ssq, hipStr
     }
     int rc = !norm ? launch_in<IO, kInPlain>(p, st) : p.xw ? launch_in<IO, kInReady>(p, st) : launch_in<IO, kInNorm>(p, st);
     if (rc != MPA_OK) return rc;
-    rc = launch_xproj<IO>(p, st);
+    if (!xproj_fused(p.ED, p.R + 2 * p.N, p.batch)) rc = launch_xproj<IO>(p, st);
     if (rc != MPA_OK) return rc;
     // sequences per workgroup: four (weights and A read once for them) while that leaves two
     // workgroups per CU

@@ -34,6 +34,7 @@ def layer_step_ref(layer, x, h, win):
     (33, 40, dict(d_state=4, expand_factor=1)),                   # 40 channels: the last row tile is half empty
     (64, 136, dict(d_state=20, dt_rank=5, bias=True)), (65, 64, dict(d_state=64)),
     (128, 1288, dict(d_state=8)),                                 # several batch tiles per workgroup
+    (16, 520, dict(d_state=32, dt_rank=200)), (16, 1032, {}),     # x_proj within in_proj: most rows; not any more
     (129, 64, {}), (2, 64, dict(d_state=6)), (2, 64, dict(d_conv=5)),   # not taken by the kernels
 ])
 def test_stack_step_matches_float64_layers(pkg, dev, dtype, batch, width, kw):
