@@ -123,13 +123,6 @@ py::object block_step(const py::object& block, const Tensor& x_in, const Opt& h_
 
 // ---- forward without gradients ------------------------------------------------------------------
 
-// Up to this many steps a bfloat16 stack runs on mpa_linear_bf16, which takes the norms and the residual adds
-// between the layers along: width 768 and 512 steps 1.2 ms for 24 layers, 2.1 with library calls, which cost the host 18 us
-// each.  At 2048 steps both keep the device busy and the library's large tiles begin to win.
-constexpr int64_t kLinearSteps = 2048;
-
-bool aligned(const void* p, size_t a) { return reinterpret_cast<uintptr_t>(p) % a == 0; }
-
 // A sequence through the residual blocks: (y, list of caches or None), or None.  The activations of a
 // layer live in buffers that every layer uses again.
 py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::object& caches, bool return_caches,
@@ -165,22 +158,19 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
                  dbc = empty({T, P}, dt, x), delta = empty({T, ED}, dt, x), y = empty({T, ED}, dt, x), hidden = empty({T, d}, dt, x);
     Tensor sum[2];
     if (n > 1) { sum[0] = empty({T, d}, dt, x); sum[1] = empty({T, d}, dt, x); }
-    bool own = dt == at::kBFloat16 && T <= kLinearSteps && ED % 8 == 0 && P % 4 == 0 && aligned(ptr(x), 16);
-    for (const LayerHandle* l : hs) {
-        for (const Tensor* w : {&l->p[kInW].t, &l->p[kOutW].t, &l->xp, &l->dtp, &l->norm_w.t, &l->p[kInB].t, &l->p[kOutB].t})
-            own &= !w->defined() || aligned(w->const_data_ptr(), 16);
-        own &= l->norm_w.t.defined();
-    }
+    bool own = use_linear(dt, T, d, ED, P, {&x});
+    for (const LayerHandle* l : hs)
+        own &= l->norm_w.t.defined() &&
+               use_linear(dt, T, d, ED, P, {&l->p[kInW].t, &l->p[kOutW].t, &l->xp, &l->dtp, &l->norm_w.t, &l->p[kInB].t, &l->p[kOutB].t});
     const int64_t parts = (d + 31) / 32;
     const Tensor ssq = own ? empty({parts, T}, at::kFloat, x) : Tensor();
     auto linear = [&](const void* in, int64_t pitch, int64_t K, const Tensor& weight, const Tensor& bias, const Tensor& out) {
-        mpa_linear q{};
-        q.T = T; q.M = weight.size(0); q.K = K;
-        q.x_pitch = pitch; q.y_pitch = q.M;
-        q.x = in; q.weight = ptr(weight); q.bias = ptr(bias); q.y = ptr(out);
+        const int64_t M = weight.size(0);
+        mpa_linear q = linear_of(T, in, pitch, K, ptr(weight), M, ptr(out), M);
+        q.bias = ptr(bias);
         return q;
     };
-    auto run = [&](const mpa_linear& q) { check(mpa_linear_bf16(&q, stream), "mpa_linear_bf16"); };
+    auto run = [&](const mpa_linear& q) { run_linear(q, stream); };
     const Tensor xs2 = xs.view({T, ED}), dlow = dbc.narrow(1, 0, a.Rp);
 
     mpa_conv_shape cv{};

@@ -104,7 +104,18 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
         const int64_t T = m.Bs * m.L, ED = m.ED, N = m.N;
         const Tensor x2 = x.view({T, m.d});
         void* stream = stream_of(x);
-        m.xz = l->p[kInB].t.defined() ? at::addmm(l->p[kInB].t, x2, l->in_wt) : at::mm(x2, l->in_wt);
+        const int64_t P = l->xp.size(0);
+        const bool own = use_linear(dt, T, m.d, ED, P, {&x, &l->p[kInW].t, &l->p[kOutW].t, &l->xp, &l->dtp, &l->p[kInB].t, &l->p[kOutB].t});
+        auto product = [&](const Tensor& in, int64_t K, const Tensor& weight, const Tensor& bias) {
+            const int64_t M = weight.size(0);
+            const Tensor y = empty({T, M}, dt, x);
+            mpa_linear q = linear_of(T, ptr(in), in.size(1), K, ptr(weight), M, ptr(y), M);
+            q.bias = ptr(bias);
+            run_linear(q, stream);
+            return y;
+        };
+        m.xz = own ? product(x2, m.d, l->p[kInW].t, l->p[kInB].t)
+               : l->p[kInB].t.defined() ? at::addmm(l->p[kInB].t, x2, l->in_wt) : at::mm(x2, l->in_wt);
         m.xs = empty({T, ED}, dt, x);
         if (return_cache) {
             window = empty({m.Bs, ED, m.K - 1}, dt, x);
@@ -112,8 +123,8 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
         }
         const mpa_conv_shape cv = mixer_conv_shape(m, io, false);
         check(mpa_conv1d_fwd(&cv, ptr(m.xz), fptr(m.conv_w), fptr(m.conv_b), ptr(wc), ptr(m.xs), ptr(window), stream), "mpa_conv1d_fwd");
-        m.dbc = at::mm(m.xs, l->xp_t);
-        m.delta = at::mm(m.dbc.narrow(1, 0, m.Rp), l->dtp_t);
+        m.dbc = own ? product(m.xs, ED, l->xp, Tensor()) : at::mm(m.xs, l->xp_t);
+        m.delta = own ? product(m.dbc, m.Rp, l->dtp, Tensor()) : at::mm(m.dbc.narrow(1, 0, m.Rp), l->dtp_t);
         m.y = empty({T, ED}, dt, x);
         m.y_pre = empty({T, ED}, dt, x);
         const mpa_sscan_shape sc = mixer_scan_shape(m, io, false);
@@ -124,7 +135,8 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
         check(mpa_sscan_fwd(&sc, ptr(m.xs), ptr(m.delta), fptr(m.A), bc, bc + N * es, fptr(m.D), static_cast<const char*>(ptr(m.xz)) + ED * es,
                             fptr(m.dt_b), fptr(hc), ptr(m.y), ptr(m.y_pre), fptr(m.ckpt), fptr(h_last), ptr(ws), nbytes, stream),
               "mpa_sscan_fwd");
-        out = (l->p[kOutB].t.defined() ? at::addmm(l->p[kOutB].t, m.y, l->out_wt) : at::mm(m.y, l->out_wt)).view({m.Bs, m.L, m.d});
+        out = (own ? product(m.y, ED, l->p[kOutW].t, l->p[kOutB].t)
+               : l->p[kOutB].t.defined() ? at::addmm(l->p[kOutB].t, m.y, l->out_wt) : at::mm(m.y, l->out_wt)).view({m.Bs, m.L, m.d});
         m.x = keep(x);
         m.win = keep(wc);
         m.h0 = keep(hc);
@@ -153,10 +165,22 @@ variable_list MixerBackward::apply(variable_list&& grads) {
     auto at_col = [&](const Tensor& t, int64_t col) { return static_cast<char*>(ptr(t)) + col * es; };
     const Tensor x2 = x_.view({T, d}), dout = cast(grads[0], dt).contiguous().view({T, d});
 
-    const Tensor dy = at::mm(dout, w[kIOutW]);
+    const bool own = use_linear(dt, T, d, ED, P, {&dout, &w[kIOutW], &w[kIInW], &xp, &dtp});
+    // out (T x M) = in (T x K) . weight (K x M), or added to out
+    auto product = [&](const void* in, int64_t in_pitch, int64_t K, const Tensor& weight, void* out, int64_t out_pitch, bool add) {
+        mpa_linear q = linear_of(T, in, in_pitch, K, ptr(weight), weight.size(1), out, out_pitch);
+        q.weight_kxm = 1;
+        if (add) { q.residual = out; q.accumulate = 1; }
+        run_linear(q, stream);
+    };
+    Tensor dy;
+    if (own) {
+        dy = empty({T, ED}, dt, x_);
+        product(ptr(dout), d, d, w[kIOutW], ptr(dy), ED, false);
+    } else {
+        dy = at::mm(dout, w[kIOutW]);
+    }
     const Tensor dxz = empty({T, 2 * ED}, dt, x_), dxs_ddelta = empty({T, 2 * ED}, dt, x_), ddbc = empty({T, P}, dt, x_);
-    Tensor dxs = dxs_ddelta.narrow(1, 0, ED);
-    const Tensor ddelta = dxs_ddelta.narrow(1, ED, ED);
     const Tensor dA = empty({ED, N}, at::kFloat, x_), dD = empty({ED}, at::kFloat, x_), ddt_b = empty({ED}, at::kFloat, x_);
     {
         const mpa_sscan_shape s = mixer_scan_shape(*this, io, true);
@@ -167,10 +191,15 @@ variable_list MixerBackward::apply(variable_list&& grads) {
                             at_col(ddbc, Rp + N), fptr(dD), at_col(dxz, ED), fptr(ddt_b), ptr(ws), nbytes, stream),
               "mpa_sscan_bwd");
     }
-    Tensor ddlow = ddbc.narrow(1, 0, Rp);
-    at::mm_out(ddlow, ddelta, dtp);
-    // (the columns past `used` were never written)
-    at::addmm_out(dxs, dxs, ddbc.narrow(1, 0, used), xp.narrow(0, 0, used));
+    // (the columns of ddbc past `used` were never written)
+    if (own) {
+        product(at_col(dxs_ddelta, ED), 2 * ED, ED, dtp, ptr(ddbc), P, false);
+        product(ptr(ddbc), P, used, xp, ptr(dxs_ddelta), 2 * ED, true);
+    } else {
+        Tensor dxs = dxs_ddelta.narrow(1, 0, ED), ddlow = ddbc.narrow(1, 0, Rp);
+        at::mm_out(ddlow, dxs_ddelta.narrow(1, ED, ED), dtp);
+        at::addmm_out(dxs, dxs, ddbc.narrow(1, 0, used), xp.narrow(0, 0, used));
+    }
     const Tensor dconv_w = empty({ED, K}, at::kFloat, x_), dconv_b = conv_b.defined() ? empty({ED}, at::kFloat, x_) : Tensor();
     {
         const mpa_conv_shape s = mixer_conv_shape(*this, io, true);
@@ -180,7 +209,14 @@ variable_list MixerBackward::apply(variable_list&& grads) {
                              ptr(ws), nbytes, stream),
               "mpa_conv1d_bwd");
     }
-    if (task_should_compute_output(kIX)) g[kIX] = at::mm(dxz, w[kIInW]).view({Bs, L, d});
+    if (task_should_compute_output(kIX)) {
+        if (own) {
+            g[kIX] = empty({Bs, L, d}, dt, x_);
+            product(ptr(dxz), 2 * ED, 2 * ED, w[kIInW], ptr(g[kIX]), d, false);
+        } else {
+            g[kIX] = at::mm(dxz, w[kIInW]).view({Bs, L, d});
+        }
+    }
 
     // weight gradients.  float32: the wide ones are compute bound and stay with the GEMM library
     std::vector<mpa_wgrad_job> jobs;

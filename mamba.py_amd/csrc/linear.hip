@@ -34,10 +34,11 @@ struct LinearParams {
     float inv_d, eps;
     const float* norm_w;  // [K], with ssq
     const bf16_t* residual;
+    int accumulate;
     float* ssq_out;  // [M/32 rounded up][T]
 };
 
-template <int BT, int BM, int KS, int D, bool NORM>
+template <int BT, int BM, int KS, int D, bool NORM, bool NN>
 __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kernel(const LinearParams p) {
     constexpr int kThreads = BT / 32 * (BM / 32) * KS * kWave;
     static_assert(BM * 8 * KS % kThreads == 0, "a load instruction reads W or x");
@@ -54,20 +55,28 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
 
     // (buffer loads: a part beyond K gets an offset beyond the window and reads as zero without a branch, which
     // would make every wait one for all loads in flight)
-    const rsrc_t rw = make_rsrc(p.w, (uint32_t)p.M * (uint32_t)p.K * 2u);
+    const rsrc_t rw = make_rsrc(p.w, (uint32_t)p.M * (uint32_t)p.K * 2u);  // (both forms of W are dense)
     const rsrc_t rx = make_rsrc(p.x, ((uint32_t)(p.T - 1) * (uint32_t)p.x_pitch + (uint32_t)p.K) * 2u);
+    constexpr int kWLoads = BM * kParts / kThreads;  // the loads of W; those of x follow
     uint32_t off[kLoads];
     int koff[kLoads], at[kLoads];
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
         const int c = threadIdx.x + i * kThreads, row = c / kParts, part = c % kParts;
+        if (NN && i < kWLoads) {
+            // two neighbouring rows of W (K x M), eight columns: see store_transposed
+            const int pair = threadIdx.x + i / 2 * kThreads, col = pair % (BM / 8) * 8;
+            koff[i] = pair / (BM / 8) * 2 + i % 2;
+            off[i] = 2u * ((uint32_t)koff[i] * (uint32_t)p.M + (uint32_t)min(m0 + col, p.M - 8));
+            at[i] = 0;
+            continue;
+        }
         koff[i] = part * 8;
         off[i] = 2u * (koff[i] + (row < BM ? (uint32_t)min(m0 + row, p.M - 1) * (uint32_t)p.K
                                            : (uint32_t)min(t0 + row - BM, p.T - 1) * (uint32_t)p.x_pitch));
         at[i] = (part >> 3) * (kRows * 8) + row * 8 + ((part & 7) ^ (row & 7));
     }
     const int steps = (p.K + 64 * KS - 1) / (64 * KS);
-    constexpr int kWLoads = BM * kParts / kThreads;  // the loads of W; those of x follow
     struct Stage {
         u32x4 v[kLoads];
         f32x4 w[NORM ? 2 : 1];  // norm weight of the thread's eight k (the same in all its parts)
@@ -80,7 +89,7 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
             const int k = s * 64 * KS;
-            v[i] = __builtin_amdgcn_raw_buffer_load_b128(i * kThreads / kParts < BM ? rw : rx, k + koff[i] < p.K ? off[i] + 2u * k : 0xffffffffu, 0, 0);
+            v[i] = __builtin_amdgcn_raw_buffer_load_b128(i * kThreads / kParts < BM ? rw : rx, k + koff[i] < p.K ? off[i] + 2u * k * (NN && i < kWLoads ? (uint32_t)p.M : 1u) : 0xffffffffu, 0, 0);
         }
         if constexpr (NORM) {
 #pragma unroll
@@ -88,10 +97,28 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
                 st.w[h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rn, 4u * (uint32_t)(s * 64 * KS + koff[0] + 4 * h), 0, 0));
         }
     };
+    // W with K as its slow dimension: the two rows of a pair make one word of each of the eight columns' rows in LDS.
+    // Column 8*c + 4*h + e goes to row h*BM/2 + 4*c + e, so that a lane's four results are neighbours again, and the
+    // parts of that row are rotated by row ^ row/4: the words of a wave's 8 x 8 columns and pairs then meet two to a
+    // bank, the operand reads as without.
+    auto store_transposed = [&](const u32x4& k0, const u32x4& k1, int buf, int pair) {
+        const int c = pair % (BM / 8), kp = pair / (BM / 8);
+        uint32_t* const words = reinterpret_cast<uint32_t*>(lds[buf] + kp / 32 * (kRows * 8));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int u = (e >> 2) * (BM / 2) + 4 * c + (e & 3);
+            words[u * 32 + ((kp % 32 >> 2) ^ ((u ^ u >> 2) & 7)) * 4 + (kp & 3)] =
+                __builtin_amdgcn_perm(k1[e >> 1], k0[e >> 1], e & 1 ? 0x07060302u : 0x05040100u);
+        }
+    };
     auto store = [&](const Stage& st, int buf) {
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
             u32x4 v = st.v[i];
+            if (NN && i < kWLoads) {
+                if (i % 2 == 0) store_transposed(v, st.v[i + 1], buf, threadIdx.x + i / 2 * kThreads);
+                continue;
+            }
             if (NORM && i >= kWLoads) {
                 bf16x8 x = __builtin_bit_cast(bf16x8, v);
 #pragma unroll
@@ -107,11 +134,12 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
         const u32x4* base = lds[buf] + ks * (kRows * 8);
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
-            const int part = (kk * 4 + fq) ^ (fr & 7);
+            const int part = (kk * 4 + fq) ^ (fr & 7);  // of x, and of W unless it is transposed
             bf16x8 a[2], b[2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                a[i] = __builtin_bit_cast(bf16x8, base[(wm * 32 + i * 16 + fr) * 8 + part]);
+                const int u = wm * 32 + i * 16 + fr;
+                a[i] = __builtin_bit_cast(bf16x8, base[u * 8 + (NN ? (kk * 4 + fq) ^ ((u ^ u >> 2) & 7) : part)]);
                 b[i] = __builtin_bit_cast(bf16x8, base[(BM + wt * 32 + i * 16 + fr) * 8 + part]);
             }
 #pragma unroll
@@ -173,7 +201,8 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
     float ss[2] = {0.0f, 0.0f};
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const int m = m0 + wm * 32 + i * 16 + fq * 4;
+        const int u = wm * 32 + i * 16 + fq * 4;
+        const int m = m0 + (NN ? u % (BM / 2) * 2 + u / (BM / 2) * 4 : u);
         if (m >= p.M) continue;
         bf16x4 bias = {};
         if (p.bias) bias = *reinterpret_cast<const bf16x4*>(p.bias + m);
@@ -187,6 +216,10 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
             for (int e = 0; e < 4; ++e) v[e] = static_cast<__bf16>(acc[i][j][e] + static_cast<float>(bias[e]));
             if (p.residual) {
                 const bf16x4 res = *reinterpret_cast<const bf16x4*>(p.residual + o);
+                if (p.accumulate) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = static_cast<__bf16>(acc[i][j][e] + static_cast<float>(bias[e]) + static_cast<float>(res[e]));
+                } else
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = static_cast<__bf16>(static_cast<float>(v[e]) + static_cast<float>(res[e]));
             }
@@ -210,25 +243,26 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
 }
 
 template <int BT, int BM, int KS>
-static int launch_linear(const LinearParams& p, hipStream_t st) {
+static int launch_linear(const LinearParams& p, bool nn, hipStream_t st) {
     const int nt = (p.T + BT - 1) / BT, nm = (p.M + BM - 1) / BM, per = (nt * nm + 7) / 8;
     const dim3 grid((unsigned)per * 8), block(BT / 32 * (BM / 32) * KS * kWave);
-    if (p.ssq) hipLaunchKernelGGL((linear_kernel<BT, BM, KS, 2, true>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((linear_kernel<BT, BM, KS, 2, false>), grid, block, 0, st, p);
+    if (nn) hipLaunchKernelGGL((linear_kernel<BT, BM, KS, 2, false, true>), grid, block, 0, st, p);
+    else if (p.ssq) hipLaunchKernelGGL((linear_kernel<BT, BM, KS, 2, true, false>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((linear_kernel<BT, BM, KS, 2, false, false>), grid, block, 0, st, p);
     return check_launch();
 }
 
 // The largest tile that gives most CUs one (a tile's traffic per product falls with its size), smaller ones
 // with K split over more waves (512 steps of a layer of width 768: in_proj 9.0 us with 64 x 128, 9.9 with 64 x
 // 64, 15 with 32 x 32; out_proj 7.9 us with 64 x 32 on eight waves, 10.8 with 64 x 64; x_proj 6.7 and 10.2 us).
-static int dispatch_linear(const LinearParams& p, hipStream_t st) {
+static int dispatch_linear(const LinearParams& p, bool nn, hipStream_t st) {
     auto tiles = [&](int bt, int bm) { return (int64_t)((p.T + bt - 1) / bt) * ((p.M + bm - 1) / bm); };
     constexpr int kFull = 160;
-    if (tiles(64, 128) >= kFull) return launch_linear<64, 128, 1>(p, st);
-    if (p.K <= 128) return launch_linear<64, 64, 1>(p, st);  // (one or two stages: nothing to split)
-    if (tiles(64, 64) >= kFull) return p.K >= 1024 ? launch_linear<64, 64, 2>(p, st) : launch_linear<64, 64, 1>(p, st);
-    if (tiles(64, 32) >= kFull) return p.K >= 1024 ? launch_linear<64, 32, 4>(p, st) : launch_linear<64, 32, 2>(p, st);
-    return launch_linear<32, 32, 4>(p, st);
+    if (tiles(64, 128) >= kFull) return launch_linear<64, 128, 1>(p, nn, st);
+    if (p.K <= 128) return launch_linear<64, 64, 1>(p, nn, st);  // (one or two stages: nothing to split)
+    if (tiles(64, 64) >= kFull) return p.K >= 1024 ? launch_linear<64, 64, 2>(p, nn, st) : launch_linear<64, 64, 1>(p, nn, st);
+    if (tiles(64, 32) >= kFull) return p.K >= 1024 ? launch_linear<64, 32, 4>(p, nn, st) : launch_linear<64, 32, 2>(p, nn, st);
+    return launch_linear<32, 32, 4>(p, nn, st);
 }
 
 }  // namespace mpa
@@ -238,6 +272,7 @@ using namespace mpa;
 extern "C" int mpa_linear_bf16(const mpa_linear* s, void* stream) {
     if (!s || !s->x || !s->weight || !s->y) return MPA_ERR_NULL_POINTER;
     if (s->x_ssq && !s->norm_weight) return MPA_ERR_NULL_POINTER;
+    if (s->weight_kxm && (s->x_ssq || s->y_ssq || s->M % 8)) return MPA_ERR_BAD_SHAPE;
     // (x and the weight are addressed with 32-bit byte offsets)
     if (s->T <= 0 || s->M <= 0 || s->K <= 0 || s->K % 8 || s->x_pitch % 8 || s->M % 4 || s->y_pitch % 4 || s->x_pitch < s->K ||
         s->y_pitch < s->M || s->T > 1 << 24 || s->M > 1 << 24 || s->K > 1 << 24 || s->T * s->x_pitch >= (int64_t)1 << 30 ||
@@ -254,6 +289,6 @@ extern "C" int mpa_linear_bf16(const mpa_linear* s, void* stream) {
     p.ssq = s->x_ssq; p.in_parts = (int)s->ssq_parts;
     p.inv_d = 1.0f / (float)s->K; p.eps = s->eps; p.norm_w = s->norm_weight;
     p.residual = static_cast<const bf16_t*>(s->residual);
-    p.ssq_out = s->y_ssq;
-    return dispatch_linear(p, static_cast<hipStream_t>(stream));
+    p.accumulate = s->accumulate; p.ssq_out = s->y_ssq;
+    return dispatch_linear(p, s->weight_kxm != 0, static_cast<hipStream_t>(stream));
 }

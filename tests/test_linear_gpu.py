@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 class Linear(ctypes.Structure):
     _fields_ = [(n, ctypes.c_int64) for n in ("T", "M", "K", "x_pitch", "y_pitch")] + \
                [(n, ctypes.c_void_p) for n in ("x", "weight", "bias", "y", "norm_weight", "x_ssq")] + \
-               [("ssq_parts", ctypes.c_int64), ("eps", ctypes.c_float), ("residual", ctypes.c_void_p), ("y_ssq", ctypes.c_void_p)]
+               [("ssq_parts", ctypes.c_int64), ("eps", ctypes.c_float), ("weight_kxm", ctypes.c_int32), ("accumulate", ctypes.c_int32), ("residual", ctypes.c_void_p), ("y_ssq", ctypes.c_void_p)]
 
 
 # tiles of every size (few to many rows and columns, short and long K) with remainders in T, M and K
@@ -39,3 +39,18 @@ def test_linear_matches_product(pkg, dev, T, M, K, pitch, fused):
     assert rel_err(y.float(), want) <= 1e-2  # (rounded twice with a residual)
     if fused:
         assert rel_err(out_ssq.sum(0), y.double().square().sum(1)) <= 1e-5
+
+
+@pytest.mark.parametrize("T,M,K,pitch", [(1, 8, 8, 8), (33, 104, 72, 80), (65, 520, 1032, 1032), (500, 1544, 264, 264), (700, 1000, 1096, 1096),
+                                         (1000, 1288, 64, 128), (2047, 904, 136, 144)])
+def test_linear_with_the_weight_transposed(pkg, dev, T, M, K, pitch):
+    L, lib = pkg._lib, pkg._lib.load()
+    g = torch.Generator().manual_seed(M)
+    rand = lambda *s: torch.randn(*s, generator=g).to(dev).bfloat16()
+    x, w, y = rand(T, pitch), rand(K, M), rand(T, M + 8)
+    want = x[:, :K].double() @ w.double() + y[:, :M].double()
+    pad = y[:, M:].clone()
+    q = Linear(T=T, M=M, K=K, x_pitch=pitch, y_pitch=M + 8, x=x.data_ptr(), weight=w.data_ptr(), y=y.data_ptr(), residual=y.data_ptr(),
+               weight_kxm=1, accumulate=1)
+    L.check(lib.mpa_linear_bf16(ctypes.byref(q), pkg.scan._stream(dev)), "mpa_linear_bf16")
+    assert rel_err(y[:, :M].float(), want) <= 5e-3 and torch.equal(y[:, M:], pad)
