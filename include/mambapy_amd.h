@@ -356,16 +356,16 @@ int mpa_decode_layer_step(const mpa_decode_layer* s, const void* x, const void* 
                           void* stream);
 
 /* ---- projections of a short sequence -----------------------------------------------------------
- * y (T x M) = x (T x K) . weight (M x K)^T + bias, bfloat16 with float32 sums, around it the norm and the
+ * y (T x M) = x (T x K) . weight (M x K)^T + bias, io_dtype with float32 sums, around it the norm and the
  * residual add of a pre-norm stack (mambapy/mamba.py:114-125):
  *   norm_weight, x_ssq  optional: `ssq_parts` rows of T partial sums of squares of the rows of x, which are
  *     multiplied by 1 / sqrt(sum / K + eps) and by norm_weight (K, float32) and rounded before the product.
- *   weight_kxm  the weight is (K x M), M a multiple of 8: y = x . weight, the product of a projection's backward;
+ *   weight_kxm  the weight is (K x M), M a multiple of 4 (float32) / 8: y = x . weight, the product of a projection's backward;
  *     without norm_weight and y_ssq.
  *   residual  optional: (T x M), added to the rounded product or, with `accumulate`, before it is rounded; may be y.
  *   y_ssq  optional: ceil(M / 32) rows of T partial sums of squares of y.
- * Rows of x are x_pitch apart, those of y and residual y_pitch.  K and x_pitch are multiples of 8, M and y_pitch
- * of 4; x, weight and norm_weight 16-byte aligned, the other matrices and the bias 8-byte.
+ * Rows of x are x_pitch apart, those of y and residual y_pitch.  K and x_pitch are multiples of 4 (float32) / 8
+ * (bfloat16), M and y_pitch of 4; x, weight and norm_weight 16-byte aligned, the rest four elements.
  */
 typedef struct mpa_linear {
     int64_t T, M, K, x_pitch, y_pitch;
@@ -374,11 +374,11 @@ typedef struct mpa_linear {
     const float *norm_weight, *x_ssq;
     int64_t ssq_parts;
     float eps;
-    int32_t weight_kxm, accumulate;
+    int32_t io_dtype, weight_kxm, accumulate;
     const void* residual;
     float* y_ssq;
 } mpa_linear;
-int mpa_linear_bf16(const mpa_linear* s, void* stream);
+int mpa_linear_run(const mpa_linear* s, void* stream);
 
 /* ---- weight gradients --------------------------------------------------------------------------
  * out = P^T . Q for up to MPA_WGRAD_MAX_JOBS pairs of matrices of T rows: what autograd forms for the

@@ -35,7 +35,7 @@ EXPORTS = ("mpa_version", "mpa_arch", "mpa_source_hash", "mpa_status_string", "m
            "mpa_conv1d_fwd", "mpa_conv1d_bwd", "mpa_conv1d_bwd_workspace_bytes",
            "mpa_rmsnorm_fwd", "mpa_rmsnorm_bwd", "mpa_rmsnorm_bwd_workspace_bytes",
            "mpa_decode_layer_workspace_bytes", "mpa_decode_scaled_bytes", "mpa_decode_layer_step",
-           "mpa_wgrad_workspace_bytes", "mpa_wgrad", "mpa_cast", "mpa_linear_bf16")
+           "mpa_wgrad_workspace_bytes", "mpa_wgrad", "mpa_cast", "mpa_linear_run")
 
 
 class SscanShape(ctypes.Structure):
@@ -134,7 +134,7 @@ def load():
     lib.mpa_wgrad_workspace_bytes.restype = sz
     lib.mpa_wgrad.argtypes = [wp, i32, i64, i32, vp, sz, vp]
     lib.mpa_cast.argtypes = [vp, i32, vp]
-    lib.mpa_linear_bf16.argtypes = [vp, vp]
+    lib.mpa_linear_run.argtypes = [vp, vp]
     for name in EXPORTS:
         getattr(lib, name)
     _lib = lib

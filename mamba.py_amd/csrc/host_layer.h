@@ -323,26 +323,33 @@ struct LayerHandle {
     }
 };
 
-// Up to this many steps x width the products of a bfloat16 layer run on mpa_linear_bf16, which costs the host a
-// quarter of a library call (18 us) and takes norms and residual adds along: a stack of width 768 without gradients,
-// 512 steps, 1.4 ms for 24 layers, 2.1 with library calls.  At 2048 steps both keep the device busy and the
-// library's large tiles begin to win.
-constexpr int64_t kLinearWork = 2048 * 768;
+// The products of a layer run on mpa_linear_run while they are small: it costs the host a quarter of a library call
+// (18 us) and takes norms and residual adds along: a bfloat16 stack of width 768 without gradients, 512 steps, 1.4 ms
+// for 24 layers, 2.1 with library calls.  The line is steps x width^2, which the products' arithmetic goes with.  Over
+// 50 shapes of widths 64 to 968 bfloat16 stacks below it are 1.0 to 1.6 times faster than with library calls, float32
+// ones too; at twice the float32 line (1342 steps of width 896, a quarter of the bfloat16 rate) the library's
+// large tiles win 1.1 times.  kLinearSteps bounds what was measured.
+constexpr int64_t kLinearWorkBf16 = 2048LL * 768 * 768, kLinearWorkF32 = 1024LL * 704 * 704, kLinearSteps = 3072 * 768;
 inline bool aligned(const void* p, size_t a) { return reinterpret_cast<uintptr_t>(p) % a == 0; }
 inline bool use_linear(at::ScalarType dt, int64_t T, int64_t d, int64_t ED, int64_t P, std::initializer_list<const Tensor*> operands) {
-    bool ok = dt == at::kBFloat16 && T * d <= kLinearWork && ED % 8 == 0 && P % 8 == 0;
+    const bool bf16 = dt == at::kBFloat16;
+    if (!bf16 && dt != at::kFloat) return false;
+    const int64_t vec = bf16 ? 8 : 4, span = (int64_t)1 << 28;  // (32-bit byte offsets in the kernel)
+    bool ok = T * d <= kLinearSteps && T * d * d <= (bf16 ? kLinearWorkBf16 : kLinearWorkF32) && d % vec == 0 && ED % vec == 0 && P % vec == 0 &&
+              ED * d < span && ED * P < span && T * std::max(ED, P) < span;
     for (const Tensor* t : operands) ok &= !t->defined() || aligned(t->const_data_ptr(), 16);
     return ok;
 }
 // out (T x M, rows y_pitch apart) = in (T x K, rows x_pitch apart) . weight^T
-inline mpa_linear linear_of(int64_t T, const void* in, int64_t x_pitch, int64_t K, const void* weight, int64_t M, void* out, int64_t y_pitch) {
+inline mpa_linear linear_of(int io, int64_t T, const void* in, int64_t x_pitch, int64_t K, const void* weight, int64_t M, void* out, int64_t y_pitch) {
     mpa_linear q{};
     q.T = T; q.M = M; q.K = K;
     q.x_pitch = x_pitch; q.y_pitch = y_pitch;
     q.x = in; q.weight = weight; q.y = out;
+    q.io_dtype = io;
     return q;
 }
-inline void run_linear(const mpa_linear& q, void* stream) { check(mpa_linear_bf16(&q, stream), "mpa_linear_bf16"); }
+inline void run_linear(const mpa_linear& q, void* stream) { check(mpa_linear_run(&q, stream), "mpa_linear_run"); }
 
 struct Types {  // the exact Python classes that a handle is made for
     py::object block, norm;

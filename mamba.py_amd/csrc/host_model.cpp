@@ -166,7 +166,7 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
     const Tensor ssq = own ? empty({parts, T}, at::kFloat, x) : Tensor();
     auto linear = [&](const void* in, int64_t pitch, int64_t K, const Tensor& weight, const Tensor& bias, const Tensor& out) {
         const int64_t M = weight.size(0);
-        mpa_linear q = linear_of(T, in, pitch, K, ptr(weight), M, ptr(out), M);
+        mpa_linear q = linear_of(io, T, in, pitch, K, ptr(weight), M, ptr(out), M);
         q.bias = ptr(bias);
         return q;
     };

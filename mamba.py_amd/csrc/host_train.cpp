@@ -109,7 +109,7 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
         auto product = [&](const Tensor& in, int64_t K, const Tensor& weight, const Tensor& bias) {
             const int64_t M = weight.size(0);
             const Tensor y = empty({T, M}, dt, x);
-            mpa_linear q = linear_of(T, ptr(in), in.size(1), K, ptr(weight), M, ptr(y), M);
+            mpa_linear q = linear_of(io, T, ptr(in), in.size(1), K, ptr(weight), M, ptr(y), M);
             q.bias = ptr(bias);
             run_linear(q, stream);
             return y;
@@ -168,7 +168,7 @@ variable_list MixerBackward::apply(variable_list&& grads) {
     const bool own = use_linear(dt, T, d, ED, P, {&dout, &w[kIOutW], &w[kIInW], &xp, &dtp});
     // out (T x M) = in (T x K) . weight (K x M), or added to out
     auto product = [&](const void* in, int64_t in_pitch, int64_t K, const Tensor& weight, void* out, int64_t out_pitch, bool add) {
-        mpa_linear q = linear_of(T, in, in_pitch, K, ptr(weight), weight.size(1), out, out_pitch);
+        mpa_linear q = linear_of(io, T, in, in_pitch, K, ptr(weight), weight.size(1), out, out_pitch);
         q.weight_kxm = 1;
         if (add) { q.residual = out; q.accumulate = 1; }
         run_linear(q, stream);

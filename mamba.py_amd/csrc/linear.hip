@@ -1,21 +1,23 @@
-// y (T x M) = x (T x K) . W (M x K)^T for the projections of a layer over a short sequence, bfloat16, for
-// gfx950.
+// y (T x M) = x (T x K) . W (M x K)^T for the projections of a layer over a short sequence, for gfx950.
 //
 // A prompt of a few hundred steps gives products of a few GFLOP: what they cost is latency (a library
 // call of 8-12 us on the device and 18 us on the host each), not arithmetic.  The kernels here
 // run one tile per workgroup, as many workgroups as the shape offers, and take over the element-wise work around
 // the product: with `residual` the sum y + residual is stored, with `ssq_out` the partial sums of squares of its rows;
-// with `ssq`, those of x, the rows of x are normalised on their way into LDS (x * rstd * weight, rounded to bfloat16, as
+// with `ssq`, those of x, the rows of x are normalised on their way into LDS (x * rstd * weight, rounded, as
 // the norm kernel rounds: a factor of the finished product would be cheaper, but rounds elsewhere).
 //
 // Tile: BT steps x BM rows of W per workgroup, each wave 32 x 32 of it (2 x 2 MFMA tiles of 16 x 16, W as the left
-// operand, so that a lane's four results are neighbours in y) over its share of K.  K runs in stages of 64 per share:
-// a stage is staged in LDS in 16-byte parts, rotated by the row (part ^ (row & 7)) so that the operand reads, one row
+// operand, so that a lane's four results are neighbours in y) over its share of K.  K runs in stages of 128 bytes per
+// share: a stage is staged in LDS in 16-byte parts, rotated by the row (part ^ (row & 7)) so that the operand reads, one row
 // per lane, fall on different banks; D stages are in registers on their way in, two in LDS.
 //
 // At 512 steps the kernels are as fast as the library's in a queue that never runs dry (9.0 / 6.7 / 3.7 / 7.9 us for
 // in_proj, x_proj, dt_proj and out_proj of width 768, the library 9.3 / 5.1 / 5.2 / 8.2 us); what they save is
 // the norm between the layers (6 us) and three quarters of the host time (24 layers: 2.1 ms, all of it host).
+// float32 runs the same tiles with sixteen times less of the matrix unit's rate (16x16x4, 150 TFLOP/s): the same host
+// time is saved, until the product itself is longer than a library call (a training layer of 1614 steps and width 424
+// 0.69 ms, 0.81 with library calls; 168 steps of ten layers of width 640 without gradients 0.63 and 0.85 ms).
 #include "common.h"
 
 namespace mpa {
@@ -24,22 +26,64 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
+// What a 16-byte part holds: kVec elements; a stage is 8 parts of every row.
+template <typename IO>
+struct LinearOps;
+template <>
+struct LinearOps<bf16_t> {
+    static constexpr int kVec = 8;
+    typedef bf16x4 Out;
+    static __device__ __forceinline__ float get(const Out& v, int e) { return static_cast<float>(v[e]); }
+    static __device__ __forceinline__ void set(Out& v, int e, float f) { v[e] = static_cast<__bf16>(f); }
+    static __device__ __forceinline__ void mma(const u32x4& a, const u32x4& b, f32x4& c) {
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ u32x4 scale(const u32x4& v, float rs, const f32x4 (&w)[2]) {
+        bf16x8 x = __builtin_bit_cast(bf16x8, v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = static_cast<__bf16>(static_cast<float>(x[e]) * rs * w[e >> 2][e & 3]);
+        return __builtin_bit_cast(u32x4, x);
+    }
+};
+template <>
+struct LinearOps<float> {
+    static constexpr int kVec = 4;
+    typedef f32x4 Out;
+    static __device__ __forceinline__ float get(const Out& v, int e) { return v[e]; }
+    static __device__ __forceinline__ void set(Out& v, int e, float f) { v[e] = f; }
+    // (four products of one k per lane group; the groups' k are those of the part, whatever their order)
+    static __device__ __forceinline__ void mma(const u32x4& a, const u32x4& b, f32x4& c) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[e]), __uint_as_float(b[e]), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ u32x4 scale(const u32x4& v, float rs, const f32x4 (&w)[1]) {
+        u32x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = __float_as_uint(__uint_as_float(v[e]) * rs * w[0][e]);
+        return x;
+    }
+};
+
 struct LinearParams {
-    const bf16_t *x, *w, *bias;
+    const void *x, *w, *bias;
     int64_t x_pitch, y_pitch;
     int T, M, K;
-    bf16_t* y;
+    void* y;
     const float* ssq;  // [in_parts][T]
     int in_parts;
     float inv_d, eps;
     const float* norm_w;  // [K], with ssq
-    const bf16_t* residual;
+    const void* residual;
     int accumulate;
     float* ssq_out;  // [M/32 rounded up][T]
 };
 
-template <int BT, int BM, int KS, int D, bool NORM, bool NN>
+template <typename IO, int BT, int BM, int KS, int D, bool NORM, bool NN>
 __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kernel(const LinearParams p) {
+    typedef LinearOps<IO> Ops;
+    constexpr int kVec = Ops::kVec, kStep = 8 * kVec;  // k of a stage and share
+    constexpr uint32_t kES = sizeof(IO);
     constexpr int kThreads = BT / 32 * (BM / 32) * KS * kWave;
     static_assert(BM * 8 * KS % kThreads == 0, "a load instruction reads W or x");
     constexpr int kRows = BT + BM, kParts = 8 * KS, kLoads = kRows * kParts / kThreads, kStage = kRows * kParts;  // 16-byte parts
@@ -55,31 +99,32 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
 
     // (buffer loads: a part beyond K gets an offset beyond the window and reads as zero without a branch, which
     // would make every wait one for all loads in flight)
-    const rsrc_t rw = make_rsrc(p.w, (uint32_t)p.M * (uint32_t)p.K * 2u);  // (both forms of W are dense)
-    const rsrc_t rx = make_rsrc(p.x, ((uint32_t)(p.T - 1) * (uint32_t)p.x_pitch + (uint32_t)p.K) * 2u);
+    const rsrc_t rw = make_rsrc(p.w, (uint32_t)p.M * (uint32_t)p.K * kES);  // (both forms of W are dense)
+    const rsrc_t rx = make_rsrc(p.x, ((uint32_t)(p.T - 1) * (uint32_t)p.x_pitch + (uint32_t)p.K) * kES);
     constexpr int kWLoads = BM * kParts / kThreads;  // the loads of W; those of x follow
+    constexpr int kRowsPer = sizeof(IO) == 2 ? 2 : 1;  // rows of W that make a word in LDS
     uint32_t off[kLoads];
     int koff[kLoads], at[kLoads];
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
         const int c = threadIdx.x + i * kThreads, row = c / kParts, part = c % kParts;
         if (NN && i < kWLoads) {
-            // two neighbouring rows of W (K x M), eight columns: see store_transposed
-            const int pair = threadIdx.x + i / 2 * kThreads, col = pair % (BM / 8) * 8;
-            koff[i] = pair / (BM / 8) * 2 + i % 2;
-            off[i] = 2u * ((uint32_t)koff[i] * (uint32_t)p.M + (uint32_t)min(m0 + col, p.M - 8));
+            // eight columns of two neighbouring rows of W (K x M), or four of one: see store_transposed
+            const int item = threadIdx.x + i / kRowsPer * kThreads, col = item % (BM / kVec) * kVec;
+            koff[i] = item / (BM / kVec) * kRowsPer + i % kRowsPer;
+            off[i] = kES * ((uint32_t)koff[i] * (uint32_t)p.M + (uint32_t)min(m0 + col, p.M - kVec));
             at[i] = 0;
             continue;
         }
-        koff[i] = part * 8;
-        off[i] = 2u * (koff[i] + (row < BM ? (uint32_t)min(m0 + row, p.M - 1) * (uint32_t)p.K
+        koff[i] = part * kVec;
+        off[i] = kES * (koff[i] + (row < BM ? (uint32_t)min(m0 + row, p.M - 1) * (uint32_t)p.K
                                            : (uint32_t)min(t0 + row - BM, p.T - 1) * (uint32_t)p.x_pitch));
         at[i] = (part >> 3) * (kRows * 8) + row * 8 + ((part & 7) ^ (row & 7));
     }
-    const int steps = (p.K + 64 * KS - 1) / (64 * KS);
+    const int steps = (p.K + kStep * KS - 1) / (kStep * KS);
     struct Stage {
         u32x4 v[kLoads];
-        f32x4 w[NORM ? 2 : 1];  // norm weight of the thread's eight k (the same in all its parts)
+        f32x4 w[kVec / 4];  // NORM: norm weight of the thread's k (the same in all its parts)
     };
     const rsrc_t rn = make_rsrc(p.norm_w, (uint32_t)p.K * 4u);
     float rs[kLoads - kWLoads];  // rstd of the rows of x the thread stages
@@ -88,27 +133,31 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
         u32x4(&v)[kLoads] = st.v;
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
-            const int k = s * 64 * KS;
-            v[i] = __builtin_amdgcn_raw_buffer_load_b128(i * kThreads / kParts < BM ? rw : rx, k + koff[i] < p.K ? off[i] + 2u * k * (NN && i < kWLoads ? (uint32_t)p.M : 1u) : 0xffffffffu, 0, 0);
+            const int k = s * kStep * KS;
+            const uint32_t at_k = kES * (uint32_t)k * (NN && i < kWLoads ? (uint32_t)p.M : 1u);
+            v[i] = __builtin_amdgcn_raw_buffer_load_b128(i < kWLoads ? rw : rx, k + koff[i] < p.K ? off[i] + at_k : 0xffffffffu, 0, 0);
         }
         if constexpr (NORM) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
-                st.w[h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rn, 4u * (uint32_t)(s * 64 * KS + koff[0] + 4 * h), 0, 0));
+            for (int h = 0; h < kVec / 4; ++h)
+                st.w[h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rn, 4u * (uint32_t)(s * kStep * KS + koff[0] + 4 * h), 0, 0));
         }
     };
-    // W with K as its slow dimension: the two rows of a pair make one word of each of the eight columns' rows in LDS.
-    // Column 8*c + 4*h + e goes to row h*BM/2 + 4*c + e, so that a lane's four results are neighbours again, and the
-    // parts of that row are rotated by row ^ row/4: the words of a wave's 8 x 8 columns and pairs then meet two to a
-    // bank, the operand reads as without.
-    auto store_transposed = [&](const u32x4& k0, const u32x4& k1, int buf, int pair) {
-        const int c = pair % (BM / 8), kp = pair / (BM / 8);
-        uint32_t* const words = reinterpret_cast<uint32_t*>(lds[buf] + kp / 32 * (kRows * 8));
+    // W with K as its slow dimension: a word of LDS holds two neighbouring k of a column, or one in float32; a lane writes
+    // those of its eight (four) columns.  Column 8*c + 4*h + e goes to row h*BM/2 + 4*c + e (4*c + e to row 4*c + e), so
+    // that a lane's four results are neighbours again, and the parts of that row are rotated by row ^ row/4: the words
+    // of a wave then meet two to a bank, the operand reads as without.
+    auto store_transposed = [&](const Stage& st, int i, int buf) {
+        const int item = threadIdx.x + i / kRowsPer * kThreads, c = item % (BM / kVec), kw = item / (BM / kVec);
+        uint32_t* const words = reinterpret_cast<uint32_t*>(lds[buf] + kw / 32 * (kRows * 8));
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < kVec; ++e) {
             const int u = (e >> 2) * (BM / 2) + 4 * c + (e & 3);
-            words[u * 32 + ((kp % 32 >> 2) ^ ((u ^ u >> 2) & 7)) * 4 + (kp & 3)] =
-                __builtin_amdgcn_perm(k1[e >> 1], k0[e >> 1], e & 1 ? 0x07060302u : 0x05040100u);
+            uint32_t v;
+            if constexpr (sizeof(IO) == 2)
+                v = __builtin_amdgcn_perm(st.v[i + 1][e >> 1], st.v[i][e >> 1], e & 1 ? 0x07060302u : 0x05040100u);
+            else v = st.v[i][e];
+            words[u * 32 + ((kw % 32 >> 2) ^ ((u ^ u >> 2) & 7)) * 4 + (kw & 3)] = v;
         }
     };
     auto store = [&](const Stage& st, int buf) {
@@ -116,15 +165,10 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
         for (int i = 0; i < kLoads; ++i) {
             u32x4 v = st.v[i];
             if (NN && i < kWLoads) {
-                if (i % 2 == 0) store_transposed(v, st.v[i + 1], buf, threadIdx.x + i / 2 * kThreads);
+                if (i % kRowsPer == 0) store_transposed(st, i, buf);
                 continue;
             }
-            if (NORM && i >= kWLoads) {
-                bf16x8 x = __builtin_bit_cast(bf16x8, v);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] = static_cast<__bf16>(static_cast<float>(x[e]) * rs[i - kWLoads] * st.w[e >> 2][e & 3]);
-                v = __builtin_bit_cast(u32x4, x);
-            }
+            if (NORM && i >= kWLoads) v = Ops::scale(v, rs[i - kWLoads], st.w);
             lds[buf][at[i]] = v;
         }
     };
@@ -135,17 +179,17 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             const int part = (kk * 4 + fq) ^ (fr & 7);  // of x, and of W unless it is transposed
-            bf16x8 a[2], b[2];
+            u32x4 a[2], b[2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int u = wm * 32 + i * 16 + fr;
-                a[i] = __builtin_bit_cast(bf16x8, base[u * 8 + (NN ? (kk * 4 + fq) ^ ((u ^ u >> 2) & 7) : part)]);
-                b[i] = __builtin_bit_cast(bf16x8, base[(BM + wt * 32 + i * 16 + fr) * 8 + part]);
+                a[i] = base[u * 8 + (NN ? (kk * 4 + fq) ^ ((u ^ u >> 2) & 7) : part)];
+                b[i] = base[(BM + wt * 32 + i * 16 + fr) * 8 + part];
             }
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < 2; ++j) Ops::mma(a[i], b[j], acc[i][j]);
         }
     };
 #pragma unroll
@@ -202,31 +246,27 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int u = wm * 32 + i * 16 + fq * 4;
-        const int m = m0 + (NN ? u % (BM / 2) * 2 + u / (BM / 2) * 4 : u);
+        const int m = m0 + (NN && kVec == 8 ? u % (BM / 2) * 2 + u / (BM / 2) * 4 : u);
         if (m >= p.M) continue;
-        bf16x4 bias = {};
-        if (p.bias) bias = *reinterpret_cast<const bf16x4*>(p.bias + m);
+        typename Ops::Out bias = {};
+        if (p.bias) bias = *reinterpret_cast<const typename Ops::Out*>(static_cast<const IO*>(p.bias) + m);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int t = t0 + wt * 32 + j * 16 + fr;
             if (t >= p.T) continue;
             const int64_t o = (int64_t)t * p.y_pitch + m;
-            bf16x4 v;
+            typename Ops::Out v, res = {};
+            if (p.residual) res = *reinterpret_cast<const typename Ops::Out*>(static_cast<const IO*>(p.residual) + o);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = static_cast<__bf16>(acc[i][j][e] + static_cast<float>(bias[e]));
-            if (p.residual) {
-                const bf16x4 res = *reinterpret_cast<const bf16x4*>(p.residual + o);
-                if (p.accumulate) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = static_cast<__bf16>(acc[i][j][e] + static_cast<float>(bias[e]) + static_cast<float>(res[e]));
-                } else
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = static_cast<__bf16>(static_cast<float>(v[e]) + static_cast<float>(res[e]));
+            for (int e = 0; e < 4; ++e) {
+                const float f = acc[i][j][e] + Ops::get(bias, e);
+                Ops::set(v, e, p.accumulate ? f + Ops::get(res, e) : f);
+                if (p.residual && !p.accumulate) Ops::set(v, e, Ops::get(v, e) + Ops::get(res, e));
             }
-            *reinterpret_cast<bf16x4*>(p.y + o) = v;
+            *reinterpret_cast<typename Ops::Out*>(static_cast<IO*>(p.y) + o) = v;
             if (p.ssq_out) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) ss[j] = __builtin_fmaf(static_cast<float>(v[e]), static_cast<float>(v[e]), ss[j]);
+                for (int e = 0; e < 4; ++e) ss[j] = __builtin_fmaf(Ops::get(v, e), Ops::get(v, e), ss[j]);
             }
         }
     }
@@ -242,53 +282,58 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
     }
 }
 
-template <int BT, int BM, int KS>
+template <typename IO, int BT, int BM, int KS>
 static int launch_linear(const LinearParams& p, bool nn, hipStream_t st) {
     const int nt = (p.T + BT - 1) / BT, nm = (p.M + BM - 1) / BM, per = (nt * nm + 7) / 8;
     const dim3 grid((unsigned)per * 8), block(BT / 32 * (BM / 32) * KS * kWave);
-    if (nn) hipLaunchKernelGGL((linear_kernel<BT, BM, KS, 2, false, true>), grid, block, 0, st, p);
-    else if (p.ssq) hipLaunchKernelGGL((linear_kernel<BT, BM, KS, 2, true, false>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((linear_kernel<BT, BM, KS, 2, false, false>), grid, block, 0, st, p);
+    if (nn) hipLaunchKernelGGL((linear_kernel<IO, BT, BM, KS, 2, false, true>), grid, block, 0, st, p);
+    else if (p.ssq) hipLaunchKernelGGL((linear_kernel<IO, BT, BM, KS, 2, true, false>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((linear_kernel<IO, BT, BM, KS, 2, false, false>), grid, block, 0, st, p);
     return check_launch();
 }
 
 // The largest tile that gives most CUs one (a tile's traffic per product falls with its size), smaller ones
 // with K split over more waves (512 steps of a layer of width 768: in_proj 9.0 us with 64 x 128, 9.9 with 64 x
 // 64, 15 with 32 x 32; out_proj 7.9 us with 64 x 32 on eight waves, 10.8 with 64 x 64; x_proj 6.7 and 10.2 us).
+template <typename IO>
 static int dispatch_linear(const LinearParams& p, bool nn, hipStream_t st) {
     auto tiles = [&](int bt, int bm) { return (int64_t)((p.T + bt - 1) / bt) * ((p.M + bm - 1) / bm); };
     constexpr int kFull = 160;
-    if (tiles(64, 128) >= kFull) return launch_linear<64, 128, 1>(p, nn, st);
-    if (p.K <= 128) return launch_linear<64, 64, 1>(p, nn, st);  // (one or two stages: nothing to split)
-    if (tiles(64, 64) >= kFull) return p.K >= 1024 ? launch_linear<64, 64, 2>(p, nn, st) : launch_linear<64, 64, 1>(p, nn, st);
-    if (tiles(64, 32) >= kFull) return p.K >= 1024 ? launch_linear<64, 32, 4>(p, nn, st) : launch_linear<64, 32, 2>(p, nn, st);
-    return launch_linear<32, 32, 4>(p, nn, st);
+    if (tiles(64, 128) >= kFull) return launch_linear<IO, 64, 128, 1>(p, nn, st);
+    if (p.K <= 128) return launch_linear<IO, 64, 64, 1>(p, nn, st);  // (one or two stages: nothing to split)
+    if (tiles(64, 64) >= kFull) return p.K >= 1024 ? launch_linear<IO, 64, 64, 2>(p, nn, st) : launch_linear<IO, 64, 64, 1>(p, nn, st);
+    if (tiles(64, 32) >= kFull) return p.K >= 1024 ? launch_linear<IO, 64, 32, 4>(p, nn, st) : launch_linear<IO, 64, 32, 2>(p, nn, st);
+    return launch_linear<IO, 32, 32, 4>(p, nn, st);
 }
 
 }  // namespace mpa
 
 using namespace mpa;
 
-extern "C" int mpa_linear_bf16(const mpa_linear* s, void* stream) {
+extern "C" int mpa_linear_run(const mpa_linear* s, void* stream) {
     if (!s || !s->x || !s->weight || !s->y) return MPA_ERR_NULL_POINTER;
     if (s->x_ssq && !s->norm_weight) return MPA_ERR_NULL_POINTER;
-    if (s->weight_kxm && (s->x_ssq || s->y_ssq || s->M % 8)) return MPA_ERR_BAD_SHAPE;
+    if (s->io_dtype != MPA_F32 && s->io_dtype != MPA_BF16) return MPA_ERR_BAD_DTYPE;
+    const bool f32 = s->io_dtype == MPA_F32;
+    const int vec = f32 ? 4 : 8;
+    if (s->weight_kxm && (s->x_ssq || s->y_ssq || s->M % vec)) return MPA_ERR_BAD_SHAPE;
     // (x and the weight are addressed with 32-bit byte offsets)
-    if (s->T <= 0 || s->M <= 0 || s->K <= 0 || s->K % 8 || s->x_pitch % 8 || s->M % 4 || s->y_pitch % 4 || s->x_pitch < s->K ||
-        s->y_pitch < s->M || s->T > 1 << 24 || s->M > 1 << 24 || s->K > 1 << 24 || s->T * s->x_pitch >= (int64_t)1 << 30 ||
-        s->M * s->K >= (int64_t)1 << 30 || (s->x_ssq && (s->ssq_parts <= 0 || s->ssq_parts > 1 << 20)))
+    if (s->T <= 0 || s->M <= 0 || s->K <= 0 || s->K % vec || s->x_pitch % vec || s->M % 4 || s->y_pitch % 4 || s->x_pitch < s->K ||
+        s->y_pitch < s->M || s->T > 1 << 24 || s->M > 1 << 24 || s->K > 1 << 24 || s->T * s->x_pitch >= (int64_t)1 << 29 ||
+        s->M * s->K >= (int64_t)1 << 29 || (s->x_ssq && (s->ssq_parts <= 0 || s->ssq_parts > 1 << 20)))
         return MPA_ERR_BAD_SHAPE;
-    if (!aligned_to(s->x, 16) || !aligned_to(s->weight, 16) || !aligned_to(s->bias, 8) || !aligned_to(s->y, 8) ||
-        !aligned_to(s->residual, 8) || !aligned_to(s->norm_weight, 16) || !aligned_to(s->x_ssq, 4) || !aligned_to(s->y_ssq, 4))
+    if (!aligned_to(s->x, 16) || !aligned_to(s->weight, 16) || !aligned_to(s->bias, f32 ? 16 : 8) || !aligned_to(s->y, f32 ? 16 : 8) ||
+        !aligned_to(s->residual, f32 ? 16 : 8) || !aligned_to(s->norm_weight, 16) || !aligned_to(s->x_ssq, 4) || !aligned_to(s->y_ssq, 4))
         return MPA_ERR_MISALIGNED;
     LinearParams p{};
-    p.x = static_cast<const bf16_t*>(s->x); p.w = static_cast<const bf16_t*>(s->weight); p.bias = static_cast<const bf16_t*>(s->bias);
+    p.x = s->x; p.w = s->weight; p.bias = s->bias;
     p.x_pitch = s->x_pitch; p.y_pitch = s->y_pitch;
     p.T = (int)s->T; p.M = (int)s->M; p.K = (int)s->K;
-    p.y = static_cast<bf16_t*>(s->y);
+    p.y = s->y;
     p.ssq = s->x_ssq; p.in_parts = (int)s->ssq_parts;
     p.inv_d = 1.0f / (float)s->K; p.eps = s->eps; p.norm_w = s->norm_weight;
-    p.residual = static_cast<const bf16_t*>(s->residual);
+    p.residual = s->residual;
     p.accumulate = s->accumulate; p.ssq_out = s->y_ssq;
-    return dispatch_linear(p, s->weight_kxm != 0, static_cast<hipStream_t>(stream));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    return f32 ? dispatch_linear<float>(p, s->weight_kxm != 0, st) : dispatch_linear<bf16_t>(p, s->weight_kxm != 0, st);
 }
