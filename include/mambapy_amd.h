@@ -401,10 +401,11 @@ int mpa_wgrad(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_t io_dtype,
 
 /* ---- conversions of small matrices ----------------------------------------------------------------
  * Up to MPA_CAST_MAX_JOBS copies of rows x cols elements between float32 and bfloat16 in one launch, each
- * optionally through -exp(v) (A from A_log, mambapy/mamba.py:239) or v * factor (float32, contiguous).
+ * optionally through -exp(v) (A from A_log, mambapy/mamba.py:239) or v * factor (float32, contiguous);
+ * MPA_CAST_ZERO writes zeros (src is not read).
  */
-#define MPA_CAST_MAX_JOBS 10
-enum mpa_cast_op { MPA_CAST_COPY = 0, MPA_CAST_NEG_EXP = 1, MPA_CAST_TIMES = 2 };
+#define MPA_CAST_MAX_JOBS 12
+enum mpa_cast_op { MPA_CAST_COPY = 0, MPA_CAST_NEG_EXP = 1, MPA_CAST_TIMES = 2, MPA_CAST_ZERO = 3 };
 typedef struct mpa_cast_job {
     const void* src;
     void* dst;

@@ -1,8 +1,8 @@
 // A residual block or mixer of the package as C++ sees it: which parameters it has, whether it is of the
 // plain kind, and the forms of its weights that the kernels take.
 //
-// What a layer needs from its modules is looked up once and kept in a LayerHandle in the
-// block's __dict__.  Every call checks, by comparing pointers and version counters, that the parameters are
+// What a layer needs from its modules is looked up once and kept in handles, a MixerHandle in the mixer's
+// __dict__ and a NormHandle in the residual block's.  Every call checks, by comparing pointers and version counters, that the parameters are
 // the ones the handle was made from and that nothing (a hook, a wrapped or replaced submodule, autocast) wants
 // to see the calls that are skipped; a block that fails the check is run module by module in Python.
 #pragma once
@@ -109,12 +109,12 @@ struct Param {
     }
 };
 
-enum { kNormW, kInW, kInB, kConvW, kConvB, kXW, kDtW, kDtB, kALog, kD, kOutW, kOutB, kParams };
+enum { kInW, kInB, kConvW, kConvB, kXW, kDtW, kDtB, kALog, kD, kOutW, kOutB, kParams };
 
-// A tensor derived from a parameter.  It is refreshed in place, so that a captured graph goes on reading
-// current values from the same memory, unless somebody else (the backward of an earlier forward) holds it.
+// A tensor derived from a parameter for the calls without gradients.  It is refreshed in place, so that a captured
+// graph goes on reading current values from the same memory.
 inline const Tensor& derived(Tensor& kept, at::IntArrayRef shape, at::ScalarType dt, const Tensor& like) {
-    if (!kept.defined() || kept.use_count() > 1 || kept.sizes() != shape || kept.device() != like.device() || kept.scalar_type() != dt)
+    if (!kept.defined() || kept.sizes() != shape || kept.device() != like.device() || kept.scalar_type() != dt)
         kept = at::zeros(shape, at::TensorOptions().dtype(dt).device(like.device()));
     return kept;
 }
@@ -131,6 +131,18 @@ inline mpa_cast_job cast_job(const Tensor& src, const Tensor& dst, int64_t rows,
     j.op = op;
     return j;
 }
+inline void run_casts(const std::vector<mpa_cast_job>& jobs, const Tensor& like) {
+    if (!jobs.empty()) check(mpa_cast(jobs.data(), (int)jobs.size(), stream_of(like)), "mpa_cast");
+}
+// the elements of a small parameter as one row
+inline mpa_cast_job row_job(const Tensor& src, const Tensor& dst) {
+    mpa_cast_job j = cast_job(src, dst, 1, src.numel());
+    j.src_pitch = j.dst_pitch = src.numel();
+    return j;
+}
+inline mpa_cast_job zero_job(const Tensor& dst, int64_t rows, int64_t cols, int64_t dst_at) {
+    return cast_job(dst, dst, rows, cols, 0, dst_at, MPA_CAST_ZERO);
+}
 // float32 form of a small parameter: the parameter itself when it is that already, else a buffer
 struct F32 {
     Tensor t, own;
@@ -138,59 +150,47 @@ struct F32 {
         t = Tensor();
         if (!p.defined()) return;
         if (p.scalar_type() == at::kFloat) { t = p.detach(); return; }
-        t = Tensor();
-        derived(own, p.sizes(), at::kFloat, p);
-        jobs.push_back(cast_job(p, own, 1, p.numel()));
-        jobs.back().src_pitch = jobs.back().dst_pitch = p.numel();
-        t = own;
+        t = derived(own, p.sizes(), at::kFloat, p);
+        jobs.push_back(row_job(p, own));
     }
 };
 
-struct LayerHandle {
+struct MixerHandle {
     bool usable = false;      // the block has the plain structure
     bool decode_ok = false;   // ... and shapes that mpa_decode_layer_step takes
-    bool forward_ok = false;  // ... and that stack_forward takes
-    bool with_norm = false;
-    Ref block_modules, mixer_modules, mixer, mixer_params;
-    Hooks mixer_hooks;
-    Sub norm, in_proj, conv1d, x_proj, dt_proj, out_proj;
+    bool forward_ok = false;  // ... and that stack_forward and block_train take
+    Ref modules, params;
+    Hooks hooks;
+    Sub in_proj, conv1d, x_proj, dt_proj, out_proj;
     Param p[kParams];
-    int64_t d = 0, ED = 0, N = 0, R = 0, K = 0;
-    double eps = 0;
-    bool fused_softplus = true, stale = true;
-    F32 norm_w, conv_w, conv_b, dt_b, D;
-    Tensor A;                                    // -exp(A_log), float32
-    Tensor in_wt, out_wt, xp, dtp, xp_t, dtp_t;  // (transposed views of) the GEMM weights
-    int64_t Rp = 0;
-    bool padded = false;  // xp .. dtp_t are up to date
+    int64_t d = 0, ED = 0, N = 0, R = 0, K = 0, Rp = 0;
+    bool fused_softplus = true;
     at::ScalarType dt = at::kFloat;
     c10::Device device{at::kCPU};
+    // Forms kept for calls without gradients, and the epoch they are of.  Version counters do not show every change
+    // of a parameter (writes through .data), and a training loop makes one after each of its calls: a call with
+    // gradients forms its own (TrainForms) and begins an epoch.
+    uint64_t epoch = 1, formed = 0;
+    bool padded = false;  // xp .. dtp_t are up to date
+    F32 conv_w, conv_b, dt_b, D;
+    Tensor A;                                    // -exp(A_log), float32
+    Tensor in_wt, out_wt, xp, dtp, xp_t, dtp_t;  // (transposed views of) the GEMM weights
 
-    // `block`: a ResidualBlock (norm + mixer) or a bare MambaBlock; types: the exact classes expected
-    LayerHandle(const py::object& block, const py::object& block_type, const py::object& norm_type, bool residual) {
-        with_norm = residual;
-        PyObject* bm = get(dict_of(block.ptr()), keys().modules);
-        if (!bm) return;
+    MixerHandle(const py::object& block, const py::object& block_type) {
         PyObject* mx = block.ptr();
-        if (residual) {
-            block_modules = Ref(bm);
-            mx = get(bm, keys().mixer);
-            if (!norm.open(bm, "norm", norm_type.ptr(), false)) return;
-        }
-        if (!mx || (PyObject*)Py_TYPE(mx) != block_type.ptr()) return;
-        if (residual) mixer = Ref(mx);  // (a bare block's handle sits in its own __dict__: no reference to itself)
+        if ((PyObject*)Py_TYPE(mx) != block_type.ptr()) return;
         PyObject* md = dict_of(mx);
         PyObject* mm = get(md, keys().modules);
-        mixer_modules = Ref(mm);
-        mixer_params = Ref(get(md, keys().params));
+        modules = Ref(mm);
+        params = Ref(get(md, keys().params));
         const py::module_ nn = py::module_::import("torch.nn");
         PyObject* linear = nn.attr("Linear").ptr();
-        if (!mm || !mixer_params.o || !mixer_hooks.open(md) || get(md, keys().forward)) return;
+        if (!mm || !params.o || !hooks.open(md) || get(md, keys().forward)) return;
         if (!in_proj.open(mm, "in_proj", linear, true) || !conv1d.open(mm, "conv1d", nn.attr("Conv1d").ptr(), false) ||
             !x_proj.open(mm, "x_proj", linear, true) || !dt_proj.open(mm, "dt_proj", linear, false) ||
             !out_proj.open(mm, "out_proj", linear, true))
             return;
-        const py::object cfg = py::reinterpret_borrow<py::object>(mx).attr("config");
+        const py::object cfg = block.attr("config");
         if (cfg.attr("inner_layernorms").cast<bool>()) return;
         d = cfg.attr("d_model").cast<int64_t>();
         ED = cfg.attr("d_inner").cast<int64_t>();
@@ -199,10 +199,7 @@ struct LayerHandle {
         K = cfg.attr("d_conv").cast<int64_t>();
         Rp = (R + 63) / 64 * 64;
         fused_softplus = cfg.attr("fused_softplus").cast<bool>();
-        if (residual) eps = py::reinterpret_borrow<py::object>(norm.mod.o).attr("eps").cast<double>();
         const Keys& k = keys();
-        if (residual) p[kNormW] = Param{norm.params.o, k.weight};
-        else p[kNormW] = Param{mixer_params.o, k.weight};  // no such parameter: stays undefined
         p[kInW] = Param{in_proj.params.o, k.weight};
         p[kInB] = Param{in_proj.params.o, k.bias};
         p[kConvW] = Param{conv1d.params.o, k.weight};
@@ -210,86 +207,95 @@ struct LayerHandle {
         p[kXW] = Param{x_proj.params.o, k.weight};
         p[kDtW] = Param{dt_proj.params.o, k.weight};
         p[kDtB] = Param{dt_proj.params.o, k.bias};
-        p[kALog] = Param{mixer_params.o, k.A_log};
-        p[kD] = Param{mixer_params.o, k.D};
+        p[kALog] = Param{params.o, k.A_log};
+        p[kD] = Param{params.o, k.D};
         p[kOutW] = Param{out_proj.params.o, k.weight};
         p[kOutB] = Param{out_proj.params.o, k.bias};
         usable = true;
     }
 
     // the dictionaries are those of this block (a shallow copy brings the handle of its original along)
-    bool belongs_to(PyObject* dict) const {
-        return !usable || get(dict, keys().modules) == (with_norm ? block_modules.o : mixer_modules.o);
-    }
+    bool belongs_to(PyObject* dict) const { return !usable || get(dict, keys().modules) == modules.o; }
 
     bool same_modules() const {
-        if (with_norm && (!norm.same(block_modules.o) || get(block_modules.o, keys().mixer) != mixer.o)) return false;
-        PyObject* mm = mixer_modules.o;
-        return in_proj.same(mm) && conv1d.same(mm) && x_proj.same(mm) && dt_proj.same(mm) && out_proj.same(mm) && mixer_hooks.none();
+        PyObject* mm = modules.o;
+        return in_proj.same(mm) && conv1d.same(mm) && x_proj.same(mm) && dt_proj.same(mm) && out_proj.same(mm) && hooks.none();
     }
 
-    // Whether the block can run here with activations like x; brings the derived weights up to date.
+    // Whether the block can run here with activations like x.
     bool ready(const Tensor& x) {
         if (!usable || !same_modules()) return false;
-        bool changed = stale;
+        bool changed = false;
         for (Param& q : p) changed |= q.changed();
         if (changed) {
-            stale = true;
+            ++epoch;
             decode_ok = forward_ok = false;
-            if (!prepare()) return false;
-            stale = false;
+            look_over();
         }
         return (decode_ok || forward_ok) && x.scalar_type() == dt && x.device() == device && x.size(-1) == d;
     }
 
-    bool prepare() {
+    void expire() { ++epoch; }
+
+    void look_over() {
         const Tensor& w = p[kInW].t;
-        if (!w.defined() || !w.is_cuda() || (w.scalar_type() != at::kFloat && w.scalar_type() != at::kBFloat16)) return false;
+        if (!w.defined() || !w.is_cuda() || (w.scalar_type() != at::kFloat && w.scalar_type() != at::kBFloat16)) return;
         dt = w.scalar_type();
         device = w.device();
         for (int i : {kInW, kXW, kDtW, kOutW, kInB, kOutB}) {
             const Tensor& t = p[i].t;
             const bool optional = i == kInB || i == kOutB;
             if (!t.defined() && optional) continue;
-            if (!t.defined() || t.scalar_type() != dt || t.device() != device || !t.is_contiguous()) return false;
+            if (!t.defined() || t.scalar_type() != dt || t.device() != device || !t.is_contiguous()) return;
         }
-        for (int i : {kNormW, kConvW, kConvB, kDtB, kALog, kD}) {
-            const Tensor& t = p[i].t;
-            if (t.defined() && (t.device() != device || !t.is_contiguous() ||
-                                (t.scalar_type() != at::kFloat && t.scalar_type() != at::kBFloat16)))
-                return false;
-        }
-        if (!p[kConvW].t.defined() || !p[kALog].t.defined() || !p[kD].t.defined()) return false;
+        for (int i : {kConvW, kConvB, kDtB, kALog, kD})
+            if (p[i].t.defined() && !small_ok(p[i].t, device)) return;
+        if (!p[kConvW].t.defined() || !p[kALog].t.defined() || !p[kD].t.defined()) return;
         if (p[kInW].t.sizes() != at::IntArrayRef({2 * ED, d}) || p[kXW].t.sizes() != at::IntArrayRef({R + 2 * N, ED}) ||
             p[kDtW].t.sizes() != at::IntArrayRef({ED, R}) || p[kOutW].t.sizes() != at::IntArrayRef({d, ED}) ||
             p[kConvW].t.numel() != ED * K || p[kALog].t.sizes() != at::IntArrayRef({ED, N}) || p[kD].t.numel() != ED)
-            return false;
+            return;
+        for (const auto& [i, n] : {std::pair<int, int64_t>{kInB, 2 * ED}, {kConvB, ED}, {kDtB, ED}, {kOutB, d}})
+            if (p[i].t.defined() && p[i].t.numel() != n) return;
+        const int64_t vec = dt == at::kFloat ? 4 : 8;
+        decode_ok = K >= 2 && K <= 4 && d % vec == 0 && ED % vec == 0 && N % 4 == 0 && N <= MPA_MAX_DSTATE && R <= 2048;
+        for (int i : {kInW, kXW, kOutW}) decode_ok &= reinterpret_cast<uintptr_t>(p[i].data) % 16 == 0;
+        forward_ok = K >= 2 && K <= 4 && N <= MPA_MAX_DSTATE && fused_softplus && d % vec == 0 && d <= 512 * vec && p[kDtB].t.defined();
+    }
+    static bool small_ok(const Tensor& t, const c10::Device& device) {
+        return t.device() == device && t.is_contiguous() && (t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16);
+    }
+
+    // brings the kept forms up to date; after ready()
+    void form() {
+        if (formed == epoch) return;
+        const Tensor& w = p[kInW].t;
         std::vector<mpa_cast_job> jobs;
-        norm_w.take(p[kNormW].t, jobs);
         conv_w.take(p[kConvW].t, jobs);
         conv_b.take(p[kConvB].t, jobs);
         dt_b.take(p[kDtB].t, jobs);
         D.take(p[kD].t, jobs);
         derived(A, {ED, N}, at::kFloat, w);
         jobs.push_back(cast_job(p[kALog].t, A, ED, N, 0, 0, MPA_CAST_NEG_EXP));
-        check(mpa_cast(jobs.data(), (int)jobs.size(), stream_of(w)), "mpa_cast");
+        run_casts(jobs, w);
         in_wt = p[kInW].t.detach().t();
         out_wt = p[kOutW].t.detach().t();
         padded = false;
-        const int64_t vec = dt == at::kFloat ? 4 : 8;
-        decode_ok = K >= 2 && K <= 4 && d % vec == 0 && ED % vec == 0 && N % 4 == 0 && N <= MPA_MAX_DSTATE && R <= 2048;
-        for (int i : {kInW, kXW, kOutW}) decode_ok &= reinterpret_cast<uintptr_t>(p[i].data) % 16 == 0;
-        for (const Tensor* t : {&norm_w.t, &A})
-            decode_ok &= !t->defined() || reinterpret_cast<uintptr_t>(t->const_data_ptr()) % 16 == 0;
-        forward_ok = K >= 2 && K <= 4 && N <= MPA_MAX_DSTATE && fused_softplus && d % vec == 0 && d <= 512 * vec && dt_b.t.defined();
-        return true;
+        formed = epoch;
     }
 
     // x_proj and dt_proj in the shape the GEMM library serves best: the low-rank width R is the K of
     // dt_proj and R + 2N the rows of x_proj, both odd for its tiles (48 and 80 at width 768).  With R
     // rounded up to a multiple of 64 by zeros and the rows regrouped as [delta | 0 | B | C | 0], the two
     // products take 21 + 26 us instead of 25 + 38 us at 32768 rows in bfloat16.
-    void pad() {
+    int64_t padded_rows() const { return Rp == R ? R + 2 * N : (Rp + 2 * N + 63) / 64 * 64; }
+    void pad_jobs(const Tensor& xp, const Tensor& dtp, std::vector<mpa_cast_job>& jobs) const {
+        const Tensor &xw = p[kXW].t, &dw = p[kDtW].t;
+        jobs.push_back(cast_job(xw, xp, R, ED));
+        jobs.push_back(cast_job(xw, xp, 2 * N, ED, R * ED, Rp * ED));
+        jobs.push_back(cast_job(dw, dtp, ED, R));
+    }
+    void pad() {  // after form()
         if (padded) return;
         padded = true;
         const Tensor &xw = p[kXW].t, &dw = p[kDtW].t;
@@ -297,13 +303,51 @@ struct LayerHandle {
             xp = xw.detach();
             dtp = dw.detach();
         } else {
-            derived(xp, {(Rp + 2 * N + 63) / 64 * 64, ED}, dt, xw);
+            derived(xp, {padded_rows(), ED}, dt, xw);
             derived(dtp, {ED, Rp}, dt, dw);
-            const mpa_cast_job jobs[] = {cast_job(xw, xp, R, ED), cast_job(xw, xp, 2 * N, ED, R * ED, Rp * ED), cast_job(dw, dtp, ED, R)};
-            check(mpa_cast(jobs, 3, stream_of(xw)), "mpa_cast");
+            std::vector<mpa_cast_job> jobs;
+            pad_jobs(xp, dtp, jobs);
+            run_casts(jobs, xw);
         }
         xp_t = xp.t();
         dtp_t = dtp.t();
+    }
+
+    // What a call with gradients takes in place of the kept forms: made in the call, on its stream, from the parameters
+    // as they are, and held by its graph node; one launch.
+    struct TrainForms {
+        Tensor A, D, dt_b, conv_w, conv_b, xp, dtp;
+    };
+    TrainForms train_forms() const {
+        const Tensor& w = p[kInW].t;
+        TrainForms f;
+        std::vector<mpa_cast_job> jobs;
+        auto f32 = [&](const Tensor& q) {
+            if (!q.defined() || q.scalar_type() == at::kFloat) return q.defined() ? q.detach() : q;
+            const Tensor t = empty(q.sizes(), at::kFloat, q);
+            jobs.push_back(row_job(q, t));
+            return t;
+        };
+        f.conv_w = f32(p[kConvW].t);
+        f.conv_b = f32(p[kConvB].t);
+        f.dt_b = f32(p[kDtB].t);
+        f.D = f32(p[kD].t);
+        f.A = empty({ED, N}, at::kFloat, w);
+        jobs.push_back(cast_job(p[kALog].t, f.A, ED, N, 0, 0, MPA_CAST_NEG_EXP));
+        if (Rp == R) {
+            f.xp = p[kXW].t.detach();
+            f.dtp = p[kDtW].t.detach();
+        } else {
+            const int64_t rows = padded_rows(), used = Rp + 2 * N;
+            f.xp = empty({rows, ED}, dt, w);
+            f.dtp = empty({ED, Rp}, dt, w);
+            pad_jobs(f.xp, f.dtp, jobs);
+            jobs.push_back(zero_job(f.xp, Rp - R, ED, R * ED));
+            if (rows > used) jobs.push_back(zero_job(f.xp, rows - used, ED, used * ED));
+            jobs.push_back(zero_job(f.dtp, ED, Rp - R, R));
+        }
+        run_casts(jobs, w);
+        return f;
     }
 
     mpa_decode_layer desc(int64_t batch) const {
@@ -311,15 +355,47 @@ struct LayerHandle {
         s.batch = batch; s.d_model = d; s.dim = ED; s.dstate = N; s.dt_rank = R;
         s.d_conv = (int)K;
         s.io_dtype = dt == at::kFloat ? MPA_F32 : MPA_BF16;
-        s.norm = with_norm;
-        s.eps = (float)eps;
-        s.norm_weight = fptr(norm_w.t);
         s.in_weight = p[kInW].data; s.in_bias = p[kInB].data;
         s.conv_weight = fptr(conv_w.t); s.conv_bias = fptr(conv_b.t);
         s.x_weight = p[kXW].data; s.dt_weight = p[kDtW].data;
         s.dt_bias = fptr(dt_b.t); s.A = fptr(A); s.D = fptr(D.t);
         s.out_weight = p[kOutW].data; s.out_bias = p[kOutB].data;
         return s;
+    }
+};
+
+// The norm in front of a mixer.
+struct NormHandle {
+    bool usable = false, ok = false, changed = false;
+    Ref modules;
+    Sub norm;
+    Param p;
+    double eps = 0;
+    F32 w;
+    uint64_t formed = 0;  // epoch of the mixer's handle that w is of
+
+    NormHandle(const py::object& block, const py::object& norm_type) {
+        PyObject* bm = get(dict_of(block.ptr()), keys().modules);
+        modules = Ref(bm);
+        if (!bm || !norm.open(bm, "norm", norm_type.ptr(), false)) return;
+        eps = py::reinterpret_borrow<py::object>(norm.mod.o).attr("eps").cast<double>();
+        p = Param{norm.params.o, keys().weight};
+        usable = true;
+    }
+    bool belongs_to(PyObject* dict) const { return !usable || get(dict, keys().modules) == modules.o; }
+    bool ready(const MixerHandle& m) {
+        if (!usable || !norm.same(modules.o)) return false;
+        changed |= p.changed();
+        const Tensor& t = p.t;
+        return !t.defined() || (t.numel() == m.d && MixerHandle::small_ok(t, m.device) && reinterpret_cast<uintptr_t>(p.data) % 16 == 0);
+    }
+    void form(const MixerHandle& m) {
+        if (!changed && formed == m.epoch) return;
+        std::vector<mpa_cast_job> jobs;
+        w.take(p.t, jobs);
+        run_casts(jobs, m.p[kInW].t);
+        changed = false;
+        formed = m.epoch;
     }
 };
 
@@ -356,17 +432,33 @@ struct Types {  // the exact Python classes that a handle is made for
 };
 inline Types* types = nullptr;  // set by register_types, kept for the interpreter's lifetime
 
-inline LayerHandle* handle_of(PyObject* block, bool residual) {
-    PyObject* dict = dict_of(block);
-    if (!dict || !types) return nullptr;
+template <typename H>
+inline H* handle_in(PyObject* module, const py::object& type) {
+    PyObject* dict = dict_of(module);
+    if (!dict) return nullptr;
     PyObject* o = get(dict, keys().handle);
-    if (!o || o == Py_None || !py::cast<LayerHandle*>(py::handle(o))->belongs_to(dict)) {
-        const py::object h = py::cast(new LayerHandle(py::reinterpret_borrow<py::object>(block), types->block, types->norm, residual),
-                                      py::return_value_policy::take_ownership);
+    if (!o || o == Py_None || !py::cast<H*>(py::handle(o))->belongs_to(dict)) {
+        const py::object h = py::cast(new H(py::reinterpret_borrow<py::object>(module), type), py::return_value_policy::take_ownership);
         PyDict_SetItem(dict, keys().handle, h.ptr());
         o = h.ptr();
     }
-    return py::cast<LayerHandle*>(py::handle(o));
+    return py::cast<H*>(py::handle(o));
+}
+inline MixerHandle* mixer_handle(PyObject* mixer) {
+    return mixer && types && (PyObject*)Py_TYPE(mixer) == types->block.ptr() ? handle_in<MixerHandle>(mixer, types->block) : nullptr;
+}
+
+// A residual block: its norm and its mixer.
+struct Layer {
+    NormHandle* n = nullptr;
+    MixerHandle* m = nullptr;
+};
+inline bool find_layer(PyObject* block, const Tensor& x, Layer& l) {
+    PyObject* mods = get(dict_of(block), keys().modules);
+    l.m = mixer_handle(get(mods, keys().mixer));
+    if (!l.m || !l.m->ready(x)) return false;
+    l.n = handle_in<NormHandle>(block, types->norm);
+    return l.n && l.n->ready(*l.m);
 }
 
 // Whether the calls a native path replaces would be rewritten by autocast.

@@ -21,7 +21,7 @@ bool read_cache(PyObject* pair, Cache& c) {
     c.window = THPVariable_Unpack(w);
     return true;
 }
-bool cache_fits(const Cache& c, const LayerHandle& l, int64_t batch, bool need_h) {
+bool cache_fits(const Cache& c, const MixerHandle& l, int64_t batch, bool need_h) {
     if (!c.h.defined() ? need_h : !fits(c.h, {batch, l.ED, l.N}, at::kFloat, l.device)) return false;
     return c.window.scalar_type() == l.dt && c.window.device() == l.device && c.window.is_contiguous() &&
            c.window.sizes() == at::IntArrayRef({batch, l.ED, l.K - 1});
@@ -39,31 +39,35 @@ py::object stack_step(const py::list& layers, const Tensor& x_in, const py::list
         x_in.size(0) > MPA_DECODE_MAX_BATCH || x_in.size(0) == 0)
         return py::none();
     const int64_t batch = x_in.size(0);
-    std::vector<LayerHandle*> hs(n);
+    std::vector<Layer> hs(n);
     std::vector<Cache> cs(n);
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard guard(x_in.device());
     for (size_t i = 0; i < n; ++i) {
-        hs[i] = handle_of(layers[i].ptr(), true);
-        if (!hs[i] || !hs[i]->ready(x_in) || !hs[i]->decode_ok || hs[i]->d != hs[0]->d) return py::none();
-        if (!read_cache(caches[i].ptr(), cs[i]) || !cache_fits(cs[i], *hs[i], batch, inplace)) return py::none();
+        if (!find_layer(layers[i].ptr(), x_in, hs[i]) || !hs[i].m->decode_ok || hs[i].m->d != hs[0].m->d) return py::none();
+        if (!read_cache(caches[i].ptr(), cs[i]) || !cache_fits(cs[i], *hs[i].m, batch, inplace)) return py::none();
     }
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
+    std::vector<mpa_decode_layer> desc(n);
+    for (size_t i = 0; i < n; ++i) {
+        hs[i].m->form();
+        hs[i].n->form(*hs[i].m);
+        desc[i] = hs[i].m->desc(batch);
+        desc[i].norm = 1;
+        desc[i].eps = (float)hs[i].n->eps;
+        desc[i].norm_weight = fptr(hs[i].n->w.t);
+    }
     const auto dt = x.scalar_type();
     const int64_t d = x.size(1);
     // two rows per sequence and two scaled rows, used in turn (a kernel never writes what it reads), with
     // the partial sums of squares of the latter
     const int64_t tiles = (d + 15) / 16;
-    const mpa_decode_layer any = hs[0]->desc(batch);
-    const size_t scaled_bytes = mpa_decode_scaled_bytes(&any);
+    const size_t scaled_bytes = mpa_decode_scaled_bytes(&desc[0]);
     const Tensor spare = empty({batch, d}, dt, x), y = empty({batch, d}, dt, x), scaled_rows = scratch(2 * scaled_bytes, x),
                  ssq = empty({2, tiles * batch}, at::kFloat, x);
     size_t ws_bytes = 0;
-    for (LayerHandle* h : hs) {
-        const mpa_decode_layer s = h->desc(batch);
-        ws_bytes = std::max(ws_bytes, mpa_decode_layer_workspace_bytes(&s));
-    }
+    for (const mpa_decode_layer& s : desc) ws_bytes = std::max(ws_bytes, mpa_decode_layer_workspace_bytes(&s));
     const Tensor ws = scratch(ws_bytes, x);
     void* stream = stream_of(x);
     // the last layer writes y, the others y and a spare row in turn
@@ -71,19 +75,18 @@ py::object stack_step(const py::list& layers, const Tensor& x_in, const py::list
     const void* scaled = nullptr;
     const float* sums = nullptr;
     for (size_t i = 0; i < n; ++i) {
-        LayerHandle& l = *hs[i];
+        const MixerHandle& l = *hs[i].m;
         Cache out = cs[i];
         if (!inplace) {
             out.h = empty({batch, l.ED, l.N}, at::kFloat, x);
             out.window = empty({batch, l.ED, l.K - 1}, dt, x);
         }
-        const mpa_decode_layer s = l.desc(batch);
         void* to = (n - 1 - i) % 2 == 0 ? ptr(y) : ptr(spare);
         // (a norm without a weight has nothing to scale by: the next layer forms its own sums)
-        const float* next_w = i + 1 < n ? fptr(hs[i + 1]->norm_w.t) : nullptr;
+        const float* next_w = i + 1 < n ? desc[i + 1].norm_weight : nullptr;
         void* to_scaled = static_cast<char*>(ptr(scaled_rows)) + (i % 2) * scaled_bytes;
         float* to_sums = fptr(ssq) + (i % 2) * tiles * batch;
-        check(mpa_decode_layer_step(&s, in, scaled, sums, to, next_w, to_scaled, to_sums, fptr(cs[i].h), fptr(out.h), ptr(cs[i].window),
+        check(mpa_decode_layer_step(&desc[i], in, scaled, sums, to, next_w, to_scaled, to_sums, fptr(cs[i].h), fptr(out.h), ptr(cs[i].window),
                                     ptr(out.window), ptr(ws), ws_bytes, stream),
               "mpa_decode_layer_step");
         in = to;
@@ -100,12 +103,13 @@ py::object block_step(const py::object& block, const Tensor& x_in, const Opt& h_
         return py::none();
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard guard(x_in.device());
-    LayerHandle* l = handle_of(block.ptr(), false);
+    MixerHandle* l = mixer_handle(block.ptr());
     const int64_t batch = x_in.size(0);
     const Cache in{val(h_in), window};
     if (!l || !l->ready(x_in) || !l->decode_ok || !cache_fits(in, *l, batch, inplace)) return py::none();
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
+    l->form();
     Cache out = in;
     if (!inplace) {
         out.h = empty({batch, l->ED, l->N}, at::kFloat, x);
@@ -130,25 +134,28 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
     const size_t n = layers.size();
     if (at::GradMode::is_enabled() || autocast_on() || !x_in.is_cuda() || x_in.dim() != 3 || n == 0 || x_in.numel() == 0) return py::none();
     const int64_t Bs = x_in.size(0), L = x_in.size(1), T = Bs * L;
-    std::vector<LayerHandle*> hs(n);
+    std::vector<Layer> hs(n);
     std::vector<Cache> cs(n);
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard guard(x_in.device());
     for (size_t i = 0; i < n; ++i) {
-        hs[i] = handle_of(layers[i].ptr(), true);
-        const LayerHandle& a = *hs[0];
-        if (!hs[i] || !hs[i]->ready(x_in) || !hs[i]->forward_ok) return py::none();
-        hs[i]->pad();
-        if (hs[i]->d != a.d || hs[i]->ED != a.ED || hs[i]->N != a.N || hs[i]->Rp != a.Rp) return py::none();
+        if (!find_layer(layers[i].ptr(), x_in, hs[i]) || !hs[i].m->forward_ok) return py::none();
+        const MixerHandle &l = *hs[i].m, &a = *hs[0].m;
+        if (l.d != a.d || l.ED != a.ED || l.N != a.N || l.Rp != a.Rp || l.padded_rows() != a.padded_rows()) return py::none();
         if (!caches.is_none()) {
             const py::object c = caches[py::int_(i)];
-            if (!read_cache(c.ptr(), cs[i]) || !cache_fits(cs[i], *hs[i], Bs, false)) return py::none();
+            if (!read_cache(c.ptr(), cs[i]) || !cache_fits(cs[i], l, Bs, false)) return py::none();
         }
     }
     const Plan plan = unpack(packed);
-    const LayerHandle& a = *hs[0];
+    const MixerHandle& a = *hs[0].m;
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
+    for (const Layer& l : hs) {
+        l.m->form();
+        l.m->pad();
+        l.n->form(*l.m);
+    }
     const auto dt = x.scalar_type();
     const int io = io_dtype(dt);
     const int64_t d = a.d, ED = a.ED, N = a.N, P = a.xp.size(0);
@@ -159,9 +166,9 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
     Tensor sum[2];
     if (n > 1) { sum[0] = empty({T, d}, dt, x); sum[1] = empty({T, d}, dt, x); }
     bool own = use_linear(dt, T, d, ED, P, {&x});
-    for (const LayerHandle* l : hs)
-        own &= l->norm_w.t.defined() &&
-               use_linear(dt, T, d, ED, P, {&l->p[kInW].t, &l->p[kOutW].t, &l->xp, &l->dtp, &l->norm_w.t, &l->p[kInB].t, &l->p[kOutB].t});
+    for (const auto& [norm, l] : hs)
+        own &= norm->w.t.defined() &&
+               use_linear(dt, T, d, ED, P, {&l->p[kInW].t, &l->p[kOutW].t, &l->xp, &l->dtp, &norm->w.t, &l->p[kInB].t, &l->p[kOutB].t});
     const int64_t parts = (d + 31) / 32;
     const Tensor ssq = own ? empty({parts, T}, at::kFloat, x) : Tensor();
     auto linear = [&](const void* in, int64_t pitch, int64_t K, const Tensor& weight, const Tensor& bias, const Tensor& out) {
@@ -195,17 +202,18 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
     const void* in = ptr(x);
     const void* residual = nullptr;
     for (size_t i = 0; i < n; ++i) {
-        LayerHandle& l = *hs[i];
+        const MixerHandle& l = *hs[i].m;
+        const float* norm_w = fptr(hs[i].n->w.t);
+        const float eps = (float)hs[i].n->eps;
         const Tensor& s = sum[i % 2];
         if (!own || i == 0)
-            check(mpa_rmsnorm_fwd(in, residual, fptr(l.norm_w.t), ptr(normed), residual ? ptr(s) : nullptr, nullptr, T, d, (float)l.eps, io,
-                                  stream),
+            check(mpa_rmsnorm_fwd(in, residual, norm_w, ptr(normed), residual ? ptr(s) : nullptr, nullptr, T, d, eps, io, stream),
                   "mpa_rmsnorm_fwd");
         if (!own) residual = residual ? ptr(s) : in;
         Tensor out = xz;
         if (own) {
             mpa_linear q = linear(i == 0 ? ptr(normed) : ptr(sum[(i - 1) % 2]), d, d, l.p[kInW].t, l.p[kInB].t, xz);
-            if (i > 0) { q.norm_weight = fptr(l.norm_w.t); q.x_ssq = fptr(ssq); q.ssq_parts = parts; q.eps = (float)l.eps; }
+            if (i > 0) { q.norm_weight = norm_w; q.x_ssq = fptr(ssq); q.ssq_parts = parts; q.eps = eps; }
             run(q);
         } else if (l.p[kInB].t.defined()) {
             at::addmm_out(out, l.p[kInB].t.detach(), normed, l.in_wt);
@@ -257,11 +265,17 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
 }  // namespace
 
 void bind_model(py::module_& m) {
-    // copies of a module (copy.deepcopy, pickle) take None in its place and make their own
-    const auto gone = [](const LayerHandle&) { return py::make_tuple(py::type::of(py::none()), py::tuple()); };
-    py::class_<LayerHandle>(m, "LayerHandle")
-        .def("__reduce__", gone)
-        .def("__deepcopy__", [](const LayerHandle&, const py::object&) { return py::none(); });
+    // copies of a module (copy.deepcopy, pickle) take None in a handle's place and make their own
+    const auto copies = [](auto& cls) {
+        typedef typename std::remove_reference_t<decltype(cls)>::type H;
+        cls.def("__reduce__", [](const H&) { return py::make_tuple(py::type::of(py::none()), py::tuple()); })
+            .def("__deepcopy__", [](const H&, const py::object&) { return py::none(); });
+    };
+    py::class_<MixerHandle> mixer(m, "MixerHandle");
+    copies(mixer);
+    mixer.def("expire", &MixerHandle::expire);
+    py::class_<NormHandle> norm(m, "NormHandle");
+    copies(norm);
     m.def("register_types", [](const py::object& block, const py::object& norm) {
         if (!types) types = new Types();
         types->block = block;

@@ -66,7 +66,7 @@ mpa_conv_shape mixer_conv_shape(const MixerBackward& m, int io, bool backward) {
 py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h_in, const Opt& win_in, bool return_cache,
                        const PackedPlan& packed) {
     if (!at::GradMode::is_enabled() || autocast_on() || !x_in.is_cuda() || x_in.dim() != 3 || x_in.numel() == 0) return py::none();
-    LayerHandle* l = handle_of(block.ptr(), false);
+    MixerHandle* l = mixer_handle(block.ptr());
     const Tensor hc = val(h_in), wc = val(win_in);
     {
         at::AutoDispatchBelowADInplaceOrView below;
@@ -76,7 +76,6 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
         const int64_t Bs = x_in.size(0);
         if (hc.defined() && !fits(hc, {Bs, l->ED, l->N}, at::kFloat, l->device)) return py::none();
         if (wc.defined() && !fits(wc, {Bs, l->ED, l->K - 1}, l->dt, l->device)) return py::none();
-        l->pad();
     }
     const std::array<int, kInputs> from = {-1, kInW, kInB, kConvW, kConvB, kXW, kDtW, kDtB, kALog, kD, kOutW, kOutB};
     const Tensor none;
@@ -100,12 +99,13 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
         const size_t es = x.element_size();
         m.Bs = x.size(0); m.L = x.size(1); m.d = l->d; m.ED = l->ED; m.N = l->N; m.R = l->R; m.Rp = l->Rp; m.K = l->K;
         m.plan = unpack(packed);
-        m.A = l->A; m.D = l->D.t; m.dt_b = l->dt_b.t; m.conv_w = l->conv_w.t; m.conv_b = l->conv_b.t; m.xp = l->xp; m.dtp = l->dtp;
+        const MixerHandle::TrainForms f = l->train_forms();
+        m.A = f.A; m.D = f.D; m.dt_b = f.dt_b; m.conv_w = f.conv_w; m.conv_b = f.conv_b; m.xp = f.xp; m.dtp = f.dtp;
         const int64_t T = m.Bs * m.L, ED = m.ED, N = m.N;
         const Tensor x2 = x.view({T, m.d});
         void* stream = stream_of(x);
-        const int64_t P = l->xp.size(0);
-        const bool own = use_linear(dt, T, m.d, ED, P, {&x, &l->p[kInW].t, &l->p[kOutW].t, &l->xp, &l->dtp, &l->p[kInB].t, &l->p[kOutB].t});
+        const int64_t P = m.xp.size(0);
+        const bool own = use_linear(dt, T, m.d, ED, P, {&x, &l->p[kInW].t, &l->p[kOutW].t, &m.xp, &m.dtp, &l->p[kInB].t, &l->p[kOutB].t});
         auto product = [&](const Tensor& in, int64_t K, const Tensor& weight, const Tensor& bias) {
             const int64_t M = weight.size(0);
             const Tensor y = empty({T, M}, dt, x);
@@ -115,7 +115,7 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
             return y;
         };
         m.xz = own ? product(x2, m.d, l->p[kInW].t, l->p[kInB].t)
-               : l->p[kInB].t.defined() ? at::addmm(l->p[kInB].t, x2, l->in_wt) : at::mm(x2, l->in_wt);
+               : l->p[kInB].t.defined() ? at::addmm(l->p[kInB].t, x2, l->p[kInW].t.t()) : at::mm(x2, l->p[kInW].t.t());
         m.xs = empty({T, ED}, dt, x);
         if (return_cache) {
             window = empty({m.Bs, ED, m.K - 1}, dt, x);
@@ -123,8 +123,8 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
         }
         const mpa_conv_shape cv = mixer_conv_shape(m, io, false);
         check(mpa_conv1d_fwd(&cv, ptr(m.xz), fptr(m.conv_w), fptr(m.conv_b), ptr(wc), ptr(m.xs), ptr(window), stream), "mpa_conv1d_fwd");
-        m.dbc = own ? product(m.xs, ED, l->xp, Tensor()) : at::mm(m.xs, l->xp_t);
-        m.delta = own ? product(m.dbc, m.Rp, l->dtp, Tensor()) : at::mm(m.dbc.narrow(1, 0, m.Rp), l->dtp_t);
+        m.dbc = own ? product(m.xs, ED, m.xp, Tensor()) : at::mm(m.xs, m.xp.t());
+        m.delta = own ? product(m.dbc, m.Rp, m.dtp, Tensor()) : at::mm(m.dbc.narrow(1, 0, m.Rp), m.dtp.t());
         m.y = empty({T, ED}, dt, x);
         m.y_pre = empty({T, ED}, dt, x);
         const mpa_sscan_shape sc = mixer_scan_shape(m, io, false);
@@ -136,7 +136,7 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
                             fptr(m.dt_b), fptr(hc), ptr(m.y), ptr(m.y_pre), fptr(m.ckpt), fptr(h_last), ptr(ws), nbytes, stream),
               "mpa_sscan_fwd");
         out = (own ? product(m.y, ED, l->p[kOutW].t, l->p[kOutB].t)
-               : l->p[kOutB].t.defined() ? at::addmm(l->p[kOutB].t, m.y, l->out_wt) : at::mm(m.y, l->out_wt)).view({m.Bs, m.L, m.d});
+               : l->p[kOutB].t.defined() ? at::addmm(l->p[kOutB].t, m.y, l->p[kOutW].t.t()) : at::mm(m.y, l->p[kOutW].t.t())).view({m.Bs, m.L, m.d});
         m.x = keep(x);
         m.win = keep(wc);
         m.h0 = keep(hc);

@@ -287,7 +287,7 @@ __global__ void __launch_bounds__(256) cast_kernel(const CastParams p) {
     const int64_t n = j.rows * j.cols;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
         const int64_t r = i / j.cols, c = i - r * j.cols;
-        float v = load_any(j.src, r * j.src_pitch + c, j.src_dtype);
+        float v = j.op == MPA_CAST_ZERO ? 0.0f : load_any(j.src, r * j.src_pitch + c, j.src_dtype);
         if (j.op == MPA_CAST_NEG_EXP) v = -expf(v);
         if (j.op == MPA_CAST_TIMES) v *= static_cast<const float*>(j.factor)[i];
         const int64_t at = r * j.dst_pitch + c;

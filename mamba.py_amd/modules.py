@@ -87,8 +87,8 @@ def _frozen_f32(owner, key, p, fn=None):
     float32 constants.  Inside autograd the parameter itself is returned and the conversion is
     part of the graph.  Outside it (decode, prefill) the converted value is kept in one
     persistent buffer per (module, key) that is refreshed in place when the parameter has
-    changed: a forward pass then spends no kernels on these conversions and a captured HIP graph
-    keeps reading the same memory."""
+    changed, or may have (_expire_forms): a forward pass then spends no kernels on these conversions and a
+    captured HIP graph keeps reading the same memory."""
     if p is None:
         return None
     if torch.is_grad_enabled() and p.requires_grad:
@@ -105,8 +105,21 @@ def _frozen_f32(owner, key, p, fn=None):
                     and hit[1].dtype == fresh.dtype:
                 hit[1].copy_(fresh)
                 fresh = hit[1]
-        cache[key] = (tag, fresh)
+        cache[key] = (tag, fresh, p.requires_grad)
     return cache[key][1]
+
+
+def _expire_forms(block):
+    """After a call with gradients the parameters will change, and not always in a way that their version
+    counters show (writes through .data): the next call without gradients converts those that train again."""
+    kept = block.__dict__.get("_f32_cache")
+    if kept:
+        for key, (_, form, trains) in kept.items():
+            if trains:
+                kept[key] = (None, form, trains)
+    handle = block.__dict__.get("_mpa_handle")
+    if handle is not None:
+        handle.expire()
 
 
 class RMSNorm(nn.Module):
@@ -243,6 +256,7 @@ class MambaBlock(nn.Module):
             # a block of the plain kind: one graph node
             h_in, win_in = cache if cache is not None else (None, None)
             out = _host().block_train(self, x, h_in, win_in, bool(return_cache), plan.packed)
+            _expire_forms(self)
             if out is not None:
                 return (out[0], out[1:]) if return_cache else out[0]
         xz = self.in_proj(x)

@@ -1,0 +1,111 @@
+"""Layers read their parameters as they are at the call: changed through .data (which leaves version counters
+alone), under a captured graph, on another stream.  The yardstick is a deep copy made at the time of the call: it has
+kept nothing from earlier ones, and runs the same kernels, so results are equal bit for bit."""
+import copy
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float32, torch.bfloat16]
+
+
+def train_pass(m, x, dy):
+    y = m(x)
+    return [y.detach()] + list(torch.autograd.grad(y, [x] + list(m.parameters()), dy))
+
+
+def change(m, by=0.05):
+    for i, p in enumerate(m.parameters()):
+        p.data.add_(torch.full_like(p, by * (1 + i % 3)))
+
+
+def same(a, b):
+    return len(a) == len(b) and all(torch.equal(u, v) for u, v in zip(a, b))
+
+
+# dt_rank: rounded up by zero rows and columns; a multiple of 64 as it is
+@pytest.mark.parametrize("dt_rank", [5, 64])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_training_sees_writes_through_data(pkg, dev, dtype, dt_rank):
+    torch.manual_seed(dt_rank)
+    blk = pkg.MambaBlock(pkg.MambaConfig(d_model=64, n_layers=1, dt_rank=dt_rank)).to(dev).to(dtype)
+    x = torch.randn(2, 70, 64, device=dev).to(dtype).requires_grad_()
+    dy = torch.randn(2, 70, 64, device=dev).to(dtype)
+    first = train_pass(blk, x, dy)
+    versions = [p._version for p in blk.parameters()]
+    for _ in range(2):
+        change(blk)
+        got, want = train_pass(blk, x, dy), train_pass(copy.deepcopy(blk), x, dy)
+        assert same(got, want) and not torch.equal(got[0], first[0])
+    assert versions == [p._version for p in blk.parameters()]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_calls_without_gradients_see_what_training_wrote(pkg, dev, dtype):
+    torch.manual_seed(2)
+    m = pkg.Mamba(pkg.MambaConfig(d_model=64, n_layers=2)).to(dev).to(dtype)
+    x = torch.randn(2, 70, 64, device=dev).to(dtype)
+    xr = x.clone().requires_grad_()
+
+    @torch.no_grad()
+    def frozen(m):
+        y, caches = m.step(x[:, 0], m.empty_caches(2))
+        y1, h, w = m.layers[0].mixer.step(x[:, 0], m.empty_caches(2)[0])[0], *caches[1]
+        return [m(x), y, y1, h, w]
+
+    first = frozen(m)
+    for _ in range(2):
+        train_pass(m, xr, torch.ones_like(x))
+        change(m)
+        got = frozen(m)
+        assert same(got, frozen(copy.deepcopy(m))) and not torch.equal(got[0], first[0])
+
+
+def test_captured_training_pass_sees_new_weights(pkg, dev):
+    """Recorded once after warm-up passes, replayed after the weights have changed outside the graph."""
+    torch.manual_seed(3)
+    dtype = torch.bfloat16      # (no library products in either direction at this size)
+    m = pkg.Mamba(pkg.MambaConfig(d_model=64, n_layers=2)).to(dev).to(dtype)
+    x = torch.randn(2, 70, 64, device=dev).to(dtype).requires_grad_()
+    dy = torch.randn(2, 70, 64, device=dev).to(dtype)
+    side = torch.cuda.Stream(device=dev)
+    side.wait_stream(torch.cuda.current_stream(dev))
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            train_pass(m, x, dy)
+    torch.cuda.current_stream(dev).wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = train_pass(m, x, dy)
+    for rep in range(3):
+        with torch.no_grad():
+            for i, p in enumerate(m.parameters()):
+                p.add_(0.05 * (1 + (i + rep) % 3))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in out]
+        assert same(got, train_pass(copy.deepcopy(m), x, dy)), rep
+        torch.cuda.synchronize()
+
+
+def test_training_on_two_streams(pkg, dev):
+    """The second stream's call waits for nothing of the first one's, whose stream is busy."""
+    torch.manual_seed(4)
+    blk = pkg.MambaBlock(pkg.MambaConfig(d_model=64, n_layers=1)).to(dev).to(torch.bfloat16)
+    x = torch.randn(2, 70, 64, device=dev).to(torch.bfloat16).requires_grad_()
+    dy = torch.randn(2, 70, 64, device=dev).to(torch.bfloat16)
+    want = train_pass(copy.deepcopy(blk), x, dy)
+    busy = torch.randn(2048, 2048, device=dev)
+    one, two = torch.cuda.Stream(device=dev), torch.cuda.Stream(device=dev)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(one):
+        for _ in range(40):
+            busy = (busy @ busy).clamp_(-1, 1)
+        a = train_pass(blk, x, dy)
+    with torch.cuda.stream(two):
+        b = train_pass(blk, x, dy)
+    torch.cuda.synchronize()
+    assert same(a, want) and same(b, want)
