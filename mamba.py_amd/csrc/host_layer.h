@@ -89,8 +89,7 @@ struct Param {
     const void* impl = nullptr;
     const void* data = nullptr;
     uint32_t version = 0;
-    static uint32_t version_of(const Tensor& t) { return t.is_inference() ? 0 : t._version(); }
-    bool changed() {  // also takes the new state over
+    bool changed() {  // also takes the new state over; an inference tensor has no version counter and may always have changed
         PyObject* o = get(params, name);
         const bool there = o && THPVariable_Check(o);
         if (!there) {
@@ -100,11 +99,12 @@ struct Param {
         }
         const Tensor& now = THPVariable_Unpack(o);
         const void* im = now.unsafeGetTensorImpl();
-        if (im == impl && now.const_data_ptr() == data && version_of(now) == version) return false;
+        const bool counted = !now.is_inference();
+        if (counted && im == impl && now.const_data_ptr() == data && now._version() == version) return false;
         t = now;
         impl = im;
         data = now.const_data_ptr();
-        version = version_of(now);
+        version = counted ? now._version() : 0;
         return true;
     }
 };

@@ -109,3 +109,18 @@ def test_training_on_two_streams(pkg, dev):
         b = train_pass(blk, x, dy)
     torch.cuda.synchronize()
     assert same(a, want) and same(b, want)
+
+
+def test_inference_tensors_are_read_in_every_call(pkg, dev):
+    """Parameters made under inference_mode have no version counter."""
+    torch.manual_seed(5)
+    with torch.inference_mode():
+        m = pkg.Mamba(pkg.MambaConfig(d_model=64, n_layers=2)).to(dev).to(torch.bfloat16)
+        x = torch.randn(2, 30, 64, device=dev).to(torch.bfloat16)
+        run = lambda m: [m(x), m.step(x[:, 0], m.empty_caches(2))[0]]
+        first = run(m)
+        for _ in range(2):
+            for p in m.parameters():
+                p.add_(0.05)
+            got = run(m)
+            assert same(got, run(copy.deepcopy(m))) and not torch.equal(got[0], first[0])
