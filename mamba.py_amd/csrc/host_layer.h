@@ -8,6 +8,8 @@
 #pragma once
 
 #include <ATen/autocast_mode.h>
+#include <c10/core/Event.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 
 #include "host.h"
 
@@ -155,6 +157,30 @@ struct F32 {
     }
 };
 
+inline c10::Stream current_stream(const c10::Device& device) { return c10::impl::VirtualGuardImpl(device.type()).getStream(device); }
+inline bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
+
+// Orders the streams that read kept forms after the one that last wrote them, and tells the allocator of them.
+// (A capture cannot wait for an event from outside; torch synchronises the device before it begins one.)
+struct Written {
+    std::optional<c10::Event> event;
+    std::optional<c10::Stream> last;  // the stream that wrote, or one that has waited since
+    void before(const c10::Stream& s) const {
+        if (event && last != s && !capturing()) event->block(s);
+    }
+    void after(const c10::Stream& s, bool wrote, std::initializer_list<const Tensor*> forms) {
+        if (last && last != s)
+            for (const Tensor* t : forms)
+                if (t->defined()) t->record_stream(s);
+        if (capturing()) return;
+        if (wrote) {
+            if (!event || event->device_index() != s.device_index()) event.emplace(s.device_type());
+            event->record(s);
+        }
+        last = s;
+    }
+};
+
 struct MixerHandle {
     bool usable = false;      // the block has the plain structure
     bool decode_ok = false;   // ... and shapes that mpa_decode_layer_step takes
@@ -170,8 +196,8 @@ struct MixerHandle {
     // Forms kept for calls without gradients, and the epoch they are of.  Version counters do not show every change
     // of a parameter (writes through .data), and a training loop makes one after each of its calls: a call with
     // gradients forms its own (TrainForms) and begins an epoch.
-    uint64_t epoch = 1, formed = 0;
-    bool padded = false;  // xp .. dtp_t are up to date
+    uint64_t epoch = 1, formed = 0, padded = 0;  // padded: that of xp .. dtp_t
+    Written written;
     F32 conv_w, conv_b, dt_b, D;
     Tensor A;                                    // -exp(A_log), float32
     Tensor in_wt, out_wt, xp, dtp, xp_t, dtp_t;  // (transposed views of) the GEMM weights
@@ -266,9 +292,22 @@ struct MixerHandle {
         return t.device() == device && t.is_contiguous() && (t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16);
     }
 
-    // brings the kept forms up to date; after ready()
-    void form() {
-        if (formed == epoch) return;
+    // Brings the kept forms up to date, xp .. dtp_t among them for a sequence; after ready().  Within a capture nothing
+    // runs yet: the next call still finds them old.
+    void form(bool sequence) {
+        const c10::Stream s = current_stream(device);
+        written.before(s);
+        const bool small = formed != epoch, wide = sequence && padded != epoch;
+        if (small) form_small();
+        if (wide) form_padded();
+        if (small || wide) {
+            const uint64_t of = capturing() ? 0 : epoch;
+            if (small) formed = of;
+            if (wide) padded = of;
+        }
+        written.after(s, small || wide, {&conv_w.own, &conv_b.own, &dt_b.own, &D.own, &A, &xp, &dtp});
+    }
+    void form_small() {
         const Tensor& w = p[kInW].t;
         std::vector<mpa_cast_job> jobs;
         conv_w.take(p[kConvW].t, jobs);
@@ -280,8 +319,6 @@ struct MixerHandle {
         run_casts(jobs, w);
         in_wt = p[kInW].t.detach().t();
         out_wt = p[kOutW].t.detach().t();
-        padded = false;
-        formed = epoch;
     }
 
     // x_proj and dt_proj in the shape the GEMM library serves best: the low-rank width R is the K of
@@ -295,9 +332,7 @@ struct MixerHandle {
         jobs.push_back(cast_job(xw, xp, 2 * N, ED, R * ED, Rp * ED));
         jobs.push_back(cast_job(dw, dtp, ED, R));
     }
-    void pad() {  // after form()
-        if (padded) return;
-        padded = true;
+    void form_padded() {
         const Tensor &xw = p[kXW].t, &dw = p[kDtW].t;
         if (Rp == R) {
             xp = xw.detach();
@@ -373,6 +408,7 @@ struct NormHandle {
     double eps = 0;
     F32 w;
     uint64_t formed = 0;  // epoch of the mixer's handle that w is of
+    Written written;
 
     NormHandle(const py::object& block, const py::object& norm_type) {
         PyObject* bm = get(dict_of(block.ptr()), keys().modules);
@@ -390,12 +426,17 @@ struct NormHandle {
         return !t.defined() || (t.numel() == m.d && MixerHandle::small_ok(t, m.device) && reinterpret_cast<uintptr_t>(p.data) % 16 == 0);
     }
     void form(const MixerHandle& m) {
-        if (!changed && formed == m.epoch) return;
-        std::vector<mpa_cast_job> jobs;
-        w.take(p.t, jobs);
-        run_casts(jobs, m.p[kInW].t);
-        changed = false;
-        formed = m.epoch;
+        const c10::Stream s = current_stream(m.device);
+        written.before(s);
+        const bool old = changed || formed != m.epoch;
+        if (old) {
+            std::vector<mpa_cast_job> jobs;
+            w.take(p.t, jobs);
+            run_casts(jobs, m.p[kInW].t);
+            changed = false;
+            formed = capturing() ? 0 : m.epoch;
+        }
+        written.after(s, old, {&w.own});
     }
 };
 

@@ -51,7 +51,7 @@ py::object stack_step(const py::list& layers, const Tensor& x_in, const py::list
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
     std::vector<mpa_decode_layer> desc(n);
     for (size_t i = 0; i < n; ++i) {
-        hs[i].m->form();
+        hs[i].m->form(false);
         hs[i].n->form(*hs[i].m);
         desc[i] = hs[i].m->desc(batch);
         desc[i].norm = 1;
@@ -109,7 +109,7 @@ py::object block_step(const py::object& block, const Tensor& x_in, const Opt& h_
     if (!l || !l->ready(x_in) || !l->decode_ok || !cache_fits(in, *l, batch, inplace)) return py::none();
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
-    l->form();
+    l->form(false);
     Cache out = in;
     if (!inplace) {
         out.h = empty({batch, l->ED, l->N}, at::kFloat, x);
@@ -152,8 +152,7 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
     for (const Layer& l : hs) {
-        l.m->form();
-        l.m->pad();
+        l.m->form(true);
         l.n->form(*l.m);
     }
     const auto dt = x.scalar_type();

@@ -124,3 +124,49 @@ def test_inference_tensors_are_read_in_every_call(pkg, dev):
                 p.add_(0.05)
             got = run(m)
             assert same(got, run(copy.deepcopy(m))) and not torch.equal(got[0], first[0])
+
+
+@torch.no_grad()
+def forward_and_step(m, x):
+    y, caches = m.step(x[:, 0], m.empty_caches(x.shape[0]))
+    return [m(x), y] + [t for pair in caches for t in pair]
+
+
+def test_a_stream_waits_for_the_forms_another_one_makes(pkg, dev):
+    torch.manual_seed(6)
+    m = pkg.Mamba(pkg.MambaConfig(d_model=64, n_layers=2)).to(dev).to(torch.bfloat16)
+    x = torch.randn(2, 70, 64, device=dev).to(torch.bfloat16)
+    want = forward_and_step(copy.deepcopy(m), x)
+    one, two = torch.cuda.Stream(device=dev), torch.cuda.Stream(device=dev)
+    busy = torch.randn(2048, 2048, device=dev)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(one):
+        for _ in range(40):
+            busy = (busy @ busy).clamp_(-1, 1)
+        a = forward_and_step(m, x)
+    with torch.cuda.stream(two):
+        b = forward_and_step(m, x)
+    c = forward_and_step(m, x)
+    torch.cuda.synchronize()
+    assert same(a, want) and same(b, want) and same(c, want)
+
+
+def test_a_capture_does_not_pass_for_a_run(pkg, dev):
+    """Recorded on a model that has not run yet: the calls after it, before any replay, form the weights themselves."""
+    torch.manual_seed(7)
+    cfg = pkg.MambaConfig(d_model=64, n_layers=2)
+    x = torch.randn(2, 70, 64, device=dev).to(torch.bfloat16)
+    warm, m = (pkg.Mamba(cfg).to(dev).to(torch.bfloat16) for _ in range(2))
+    forward_and_step(warm, x)
+    want = forward_and_step(copy.deepcopy(m), x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = forward_and_step(m, x)
+    assert same(forward_and_step(m, x), want)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert same(out, want)
+        forward_and_step(warm, x)
+        torch.cuda.synchronize()
