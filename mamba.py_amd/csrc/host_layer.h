@@ -1,10 +1,10 @@
 // A residual block or mixer of the package as C++ sees it: which parameters it has, whether it is of the
 // plain kind, and the forms of its weights that the kernels take.
 //
-// What a layer needs from its modules is looked up once and kept in handles, a MixerHandle in the mixer's
-// __dict__ and a NormHandle in the residual block's.  Every call checks, by comparing pointers and version counters, that the parameters are
-// the ones the handle was made from and that nothing (a hook, a wrapped or replaced submodule, autocast) wants
-// to see the calls that are skipped; a block that fails the check is run module by module in Python.
+// What is made from a layer's parameters is kept in handles, a MixerHandle in the mixer's __dict__ and a NormHandle
+// in the residual block's.  Nothing about the modules is: every call looks whether the submodules are of the plain
+// types and nothing (a hook, a method put on an instance or a class, autocast) wants to see the calls that are skipped,
+// and takes the parameters from where they are.  A block that fails is run module by module in Python.
 #pragma once
 
 #include <ATen/autocast_mode.h>
@@ -29,10 +29,13 @@ struct Ref {  // an owned PyObject*
 
 inline PyObject* key(const char* s) { return PyUnicode_InternFromString(s); }
 struct Keys {
-    PyObject *modules = key("_modules"), *params = key("_parameters"), *fwd = key("_forward_hooks"), *pre = key("_forward_pre_hooks"),
-             *bwd = key("_backward_hooks"), *bpre = key("_backward_pre_hooks"),
-             *handle = key("_mpa_handle"), *mixer = key("mixer"), *norm = key("norm"), *weight = key("weight"), *bias = key("bias"),
-             *A_log = key("A_log"), *D = key("D"), *forward = key("forward");
+    PyObject *modules = key("_modules"), *params = key("_parameters"), *handle = key("_mpa_handle"), *config = key("config"),
+             *mixer = key("mixer"), *norm = key("norm"), *weight = key("weight"), *bias = key("bias"), *A_log = key("A_log"), *D = key("D"),
+             *in_proj = key("in_proj"), *conv1d = key("conv1d"), *x_proj = key("x_proj"), *dt_proj = key("dt_proj"), *out_proj = key("out_proj"),
+             *dt_layernorm = key("dt_layernorm"), *eps = key("eps"), *use_mup = key("use_mup");
+    PyObject* const hooks[4] = {key("_forward_hooks"), key("_forward_pre_hooks"), key("_backward_hooks"), key("_backward_pre_hooks")};
+    PyObject* const sizes[7] = {key("d_model"), key("d_inner"), key("d_state"), key("dt_rank"), key("d_conv"), key("inner_layernorms"),
+                                key("fused_softplus")};
 };
 inline const Keys& keys() {
     static const Keys k;
@@ -45,64 +48,69 @@ inline PyObject* dict_of(PyObject* module) {
 }
 inline PyObject* get(PyObject* dict, PyObject* k) { return dict ? PyDict_GetItem(dict, k) : nullptr; }
 
-struct Hooks {
-    Ref dicts[4];
-    bool open(PyObject* module_dict) {
-        const Keys& k = keys();
-        PyObject* const names[4] = {k.fwd, k.pre, k.bwd, k.bpre};
-        for (int i = 0; i < 4; ++i) {
-            dicts[i] = Ref(get(module_dict, names[i]));
-            if (!dicts[i].o) return false;
-        }
-        return true;
-    }
-    bool none() const {
-        for (const Ref& d : dicts)
-            if (PyDict_Size(d.o) != 0) return false;
-        return true;
-    }
-};
+inline bool empty_dict(PyObject* o) { return o && PyDict_Check(o) && PyDict_Size(o) == 0; }
 
-// A submodule: found under its name, of exactly the expected type, without hooks.
-struct Sub {
-    PyObject* name = nullptr;
-    bool called = false;  // through __call__, so that hooks would run
-    Ref mod, params;
-    Hooks hooks;
-    bool open(PyObject* modules, const char* n, PyObject* type, bool is_called) {
-        name = key(n);
-        called = is_called;
-        PyObject* m = get(modules, name);
-        if (!m || (PyObject*)Py_TYPE(m) != type) return false;
-        PyObject* d = dict_of(m);
-        mod = Ref(m);
-        params = Ref(get(d, keys().params));
-        return hooks.open(d) && params.o && !get(d, keys().forward);
-    }
-    bool same(PyObject* modules) const {
-        return get(modules, name) == mod.o && (!called || hooks.none());
+// The exact Python classes that handles are made for, the methods of theirs that a native call stands in for, and
+// torch's hooks on all modules.
+struct Types {
+    struct Method {
+        Ref dict, name, was;  // the class's __dict__, and what was under the name
+    };
+    py::object block, norm, linear, conv;
+    std::vector<Method> methods;
+    std::vector<Ref> block_names, norm_names, linear_names;  // not to be found on an instance
+    std::vector<Ref> global_hooks;
+    bool plain() const {
+        for (const Method& m : methods)
+            if (get(m.dict.o, m.name.o) != m.was.o) return false;
+        for (const Ref& h : global_hooks)
+            if (!empty_dict(h.o)) return false;
+        return true;
     }
 };
+inline Types* types = nullptr;  // set by register_types, kept for the interpreter's lifetime
+
+// nothing on the module itself changes or watches its calls
+inline bool plain_instance(PyObject* dict, const std::vector<Ref>& names) {
+    if (!dict) return false;
+    for (const Ref& n : names)
+        if (get(dict, n.o)) return false;
+    for (PyObject* k : keys().hooks)
+        if (!empty_dict(get(dict, k))) return false;
+    return true;
+}
+// the instance dictionary of the plain submodule under `name`, or null
+inline PyObject* plain_sub(PyObject* modules, PyObject* name, const py::object& type, const std::vector<Ref>& names) {
+    PyObject* m = get(modules, name);
+    if (!m || (PyObject*)Py_TYPE(m) != type.ptr()) return nullptr;
+    PyObject* d = dict_of(m);
+    return plain_instance(d, names) ? d : nullptr;
+}
 
 // A parameter and the state it was last seen in.
 struct Param {
-    PyObject *params = nullptr, *name = nullptr;
     Tensor t;
     const void* impl = nullptr;
     const void* data = nullptr;
     uint32_t version = 0;
-    bool changed() {  // also takes the new state over; an inference tensor has no version counter and may always have changed
+    // Takes over what `params` holds under `name`, None for no parameter; false if it holds neither that nor a plain tensor
+    // (pruning and parametrisation take the name away).  An inference tensor has no version counter and may
+    // always have changed.
+    bool look(PyObject* params, PyObject* name, bool& changed) {
         PyObject* o = get(params, name);
-        const bool there = o && THPVariable_Check(o);
-        if (!there) {
-            const bool was = impl != nullptr;
-            *this = Param{params, name};
-            return was;
+        if (o == Py_None) {
+            if (impl) {
+                changed = true;
+                *this = Param{};
+            }
+            return true;
         }
+        if (!o || !THPVariable_CheckExact(o)) return false;
         const Tensor& now = THPVariable_Unpack(o);
         const void* im = now.unsafeGetTensorImpl();
         const bool counted = !now.is_inference();
-        if (counted && im == impl && now.const_data_ptr() == data && now._version() == version) return false;
+        if (counted && im == impl && now.const_data_ptr() == data && now._version() == version) return true;
+        changed = true;
         t = now;
         impl = im;
         data = now.const_data_ptr();
@@ -111,7 +119,7 @@ struct Param {
     }
 };
 
-enum { kInW, kInB, kConvW, kConvB, kXW, kDtW, kDtB, kALog, kD, kOutW, kOutB, kParams };
+enum { kInW, kInB, kConvW, kConvB, kXW, kXB, kDtW, kDtB, kALog, kD, kOutW, kOutB, kParams };
 
 // A tensor derived from a parameter for the calls without gradients.  It is refreshed in place, so that a captured
 // graph goes on reading current values from the same memory.
@@ -182,12 +190,10 @@ struct Written {
 };
 
 struct MixerHandle {
-    bool usable = false;      // the block has the plain structure
-    bool decode_ok = false;   // ... and shapes that mpa_decode_layer_step takes
-    bool forward_ok = false;  // ... and that stack_forward and block_train take
-    Ref modules, params;
-    Hooks hooks;
-    Sub in_proj, conv1d, x_proj, dt_proj, out_proj;
+    bool decode_ok = false;   // the shapes are such as mpa_decode_layer_step takes
+    bool forward_ok = false;  // ... as stack_forward and block_train take
+    Ref modules;
+    Ref sizes[7];  // values of the config, by Keys::sizes
     Param p[kParams];
     int64_t d = 0, ED = 0, N = 0, R = 0, K = 0, Rp = 0;
     bool fused_softplus = true;
@@ -202,70 +208,68 @@ struct MixerHandle {
     Tensor A;                                    // -exp(A_log), float32
     Tensor in_wt, out_wt, xp, dtp, xp_t, dtp_t;  // (transposed views of) the GEMM weights
 
-    MixerHandle(const py::object& block, const py::object& block_type) {
-        PyObject* mx = block.ptr();
-        if ((PyObject*)Py_TYPE(mx) != block_type.ptr()) return;
-        PyObject* md = dict_of(mx);
-        PyObject* mm = get(md, keys().modules);
-        modules = Ref(mm);
-        params = Ref(get(md, keys().params));
-        const py::module_ nn = py::module_::import("torch.nn");
-        PyObject* linear = nn.attr("Linear").ptr();
-        if (!mm || !params.o || !hooks.open(md) || get(md, keys().forward)) return;
-        if (!in_proj.open(mm, "in_proj", linear, true) || !conv1d.open(mm, "conv1d", nn.attr("Conv1d").ptr(), false) ||
-            !x_proj.open(mm, "x_proj", linear, true) || !dt_proj.open(mm, "dt_proj", linear, false) ||
-            !out_proj.open(mm, "out_proj", linear, true))
-            return;
-        const py::object cfg = block.attr("config");
-        if (cfg.attr("inner_layernorms").cast<bool>()) return;
-        d = cfg.attr("d_model").cast<int64_t>();
-        ED = cfg.attr("d_inner").cast<int64_t>();
-        N = cfg.attr("d_state").cast<int64_t>();
-        R = cfg.attr("dt_rank").cast<int64_t>();
-        K = cfg.attr("d_conv").cast<int64_t>();
-        Rp = (R + 63) / 64 * 64;
-        fused_softplus = cfg.attr("fused_softplus").cast<bool>();
-        const Keys& k = keys();
-        p[kInW] = Param{in_proj.params.o, k.weight};
-        p[kInB] = Param{in_proj.params.o, k.bias};
-        p[kConvW] = Param{conv1d.params.o, k.weight};
-        p[kConvB] = Param{conv1d.params.o, k.bias};
-        p[kXW] = Param{x_proj.params.o, k.weight};
-        p[kDtW] = Param{dt_proj.params.o, k.weight};
-        p[kDtB] = Param{dt_proj.params.o, k.bias};
-        p[kALog] = Param{params.o, k.A_log};
-        p[kD] = Param{params.o, k.D};
-        p[kOutW] = Param{out_proj.params.o, k.weight};
-        p[kOutB] = Param{out_proj.params.o, k.bias};
-        usable = true;
-    }
-
+    explicit MixerHandle(PyObject* dict) : modules(get(dict, keys().modules)) {}
     // the dictionaries are those of this block (a shallow copy brings the handle of its original along)
-    bool belongs_to(PyObject* dict) const { return !usable || get(dict, keys().modules) == modules.o; }
+    bool belongs_to(PyObject* dict) const { return get(dict, keys().modules) == modules.o; }
 
-    bool same_modules() const {
+    // Whether the block with this __dict__ can run here with activations like x.
+    bool ready(PyObject* dict, const Tensor& x) {
+        const Keys& k = keys();
+        if (!plain_instance(dict, types->block_names) || get(dict, k.dt_layernorm) != Py_None) return false;
         PyObject* mm = modules.o;
-        return in_proj.same(mm) && conv1d.same(mm) && x_proj.same(mm) && dt_proj.same(mm) && out_proj.same(mm) && hooks.none();
-    }
-
-    // Whether the block can run here with activations like x.
-    bool ready(const Tensor& x) {
-        if (!usable || !same_modules()) return false;
+        PyObject* const in = plain_sub(mm, k.in_proj, types->linear, types->linear_names);
+        PyObject* const conv = plain_sub(mm, k.conv1d, types->conv, types->linear_names);
+        PyObject* const xp = plain_sub(mm, k.x_proj, types->linear, types->linear_names);
+        PyObject* const dtp = plain_sub(mm, k.dt_proj, types->linear, types->linear_names);
+        PyObject* const out = plain_sub(mm, k.out_proj, types->linear, types->linear_names);
+        if (!in || !conv || !xp || !dtp || !out) return false;
         bool changed = false;
-        for (Param& q : p) changed |= q.changed();
+        if (!read_config(get(dict, k.config), changed)) return false;
+        PyObject* const params = get(dict, k.params);
+        const bool there = both(in, kInW, kInB, changed) && both(conv, kConvW, kConvB, changed) && both(xp, kXW, kXB, changed) &&
+                           both(dtp, kDtW, kDtB, changed) && both(out, kOutW, kOutB, changed) && p[kALog].look(params, k.A_log, changed) &&
+                           p[kD].look(params, k.D, changed);
         if (changed) {
             ++epoch;
             decode_ok = forward_ok = false;
-            look_over();
+            if (there) look_over();
+            else forget();
         }
-        return (decode_ok || forward_ok) && x.scalar_type() == dt && x.device() == device && x.size(-1) == d;
+        return there && (decode_ok || forward_ok) && x.scalar_type() == dt && x.device() == device && x.size(-1) == d;
+    }
+    bool both(PyObject* dict, int weight, int bias, bool& changed) {
+        PyObject* params = get(dict, keys().params);
+        return p[weight].look(params, keys().weight, changed) && p[bias].look(params, keys().bias, changed);
+    }
+    // (what has been taken over before a parameter was found missing is looked over again once it is back)
+    void forget() {
+        for (Param& q : p) q = Param{};
+    }
+    bool read_config(PyObject* config, bool& changed) {
+        PyObject* dict = config ? dict_of(config) : nullptr;
+        PyObject* v[7];
+        bool same = true;
+        for (int i = 0; i < 7; ++i) {
+            v[i] = get(dict, keys().sizes[i]);
+            if (!v[i] || (i < 5 && !PyLong_Check(v[i]))) return false;
+            same &= v[i] == sizes[i].o;
+        }
+        if (!same) {
+            changed = true;
+            int64_t* const to[] = {&d, &ED, &N, &R, &K};
+            for (int i = 0; i < 5; ++i) *to[i] = PyLong_AsLongLong(v[i]);
+            for (int i = 0; i < 7; ++i) sizes[i] = Ref(v[i]);
+            Rp = (R + 63) / 64 * 64;
+            fused_softplus = PyObject_IsTrue(sizes[6].o) == 1;
+        }
+        return PyObject_IsTrue(sizes[5].o) == 0;
     }
 
     void expire() { ++epoch; }
 
     void look_over() {
         const Tensor& w = p[kInW].t;
-        if (!w.defined() || !w.is_cuda() || (w.scalar_type() != at::kFloat && w.scalar_type() != at::kBFloat16)) return;
+        if (d <= 0 || R <= 0 || N <= 0 || !w.defined() || !w.is_cuda() || (w.scalar_type() != at::kFloat && w.scalar_type() != at::kBFloat16)) return;
         dt = w.scalar_type();
         device = w.device();
         for (int i : {kInW, kXW, kDtW, kOutW, kInB, kOutB}) {
@@ -276,7 +280,7 @@ struct MixerHandle {
         }
         for (int i : {kConvW, kConvB, kDtB, kALog, kD})
             if (p[i].t.defined() && !small_ok(p[i].t, device)) return;
-        if (!p[kConvW].t.defined() || !p[kALog].t.defined() || !p[kD].t.defined()) return;
+        if (!p[kConvW].t.defined() || !p[kALog].t.defined() || !p[kD].t.defined() || p[kXB].t.defined()) return;
         if (p[kInW].t.sizes() != at::IntArrayRef({2 * ED, d}) || p[kXW].t.sizes() != at::IntArrayRef({R + 2 * N, ED}) ||
             p[kDtW].t.sizes() != at::IntArrayRef({ED, R}) || p[kOutW].t.sizes() != at::IntArrayRef({d, ED}) ||
             p[kConvW].t.numel() != ED * K || p[kALog].t.sizes() != at::IntArrayRef({ED, N}) || p[kD].t.numel() != ED)
@@ -401,27 +405,32 @@ struct MixerHandle {
 
 // The norm in front of a mixer.
 struct NormHandle {
-    bool usable = false, ok = false, changed = false;
-    Ref modules;
-    Sub norm;
+    bool changed = false;
+    Ref modules, eps_seen;
     Param p;
     double eps = 0;
     F32 w;
     uint64_t formed = 0;  // epoch of the mixer's handle that w is of
     Written written;
 
-    NormHandle(const py::object& block, const py::object& norm_type) {
-        PyObject* bm = get(dict_of(block.ptr()), keys().modules);
-        modules = Ref(bm);
-        if (!bm || !norm.open(bm, "norm", norm_type.ptr(), false)) return;
-        eps = py::reinterpret_borrow<py::object>(norm.mod.o).attr("eps").cast<double>();
-        p = Param{norm.params.o, keys().weight};
-        usable = true;
-    }
-    bool belongs_to(PyObject* dict) const { return !usable || get(dict, keys().modules) == modules.o; }
+    explicit NormHandle(PyObject* dict) : modules(get(dict, keys().modules)) {}
+    bool belongs_to(PyObject* dict) const { return get(dict, keys().modules) == modules.o; }
     bool ready(const MixerHandle& m) {
-        if (!usable || !norm.same(modules.o)) return false;
-        changed |= p.changed();
+        const Keys& k = keys();
+        PyObject* const d = plain_sub(modules.o, k.norm, types->norm, types->norm_names);
+        if (!d) return false;
+        PyObject *const e = get(d, k.eps), *const gainless = get(d, k.use_mup);
+        if (!e || !gainless) return false;
+        if (e != eps_seen.o) {
+            eps_seen = Ref(e);
+            eps = py::handle(e).cast<double>();
+        }
+        if (PyObject_IsTrue(gainless) == 1) {
+            changed |= p.impl != nullptr;
+            p = Param{};
+        } else if (!p.look(get(d, k.params), k.weight, changed)) {
+            return false;
+        }
         const Tensor& t = p.t;
         return !t.defined() || (t.numel() == m.d && MixerHandle::small_ok(t, m.device) && reinterpret_cast<uintptr_t>(p.data) % 16 == 0);
     }
@@ -468,25 +477,23 @@ inline mpa_linear linear_of(int io, int64_t T, const void* in, int64_t x_pitch, 
 }
 inline void run_linear(const mpa_linear& q, void* stream) { check(mpa_linear_run(&q, stream), "mpa_linear_run"); }
 
-struct Types {  // the exact Python classes that a handle is made for
-    py::object block, norm;
-};
-inline Types* types = nullptr;  // set by register_types, kept for the interpreter's lifetime
-
 template <typename H>
-inline H* handle_in(PyObject* module, const py::object& type) {
-    PyObject* dict = dict_of(module);
-    if (!dict) return nullptr;
+inline H* handle_in(PyObject* dict) {
     PyObject* o = get(dict, keys().handle);
     if (!o || o == Py_None || !py::cast<H*>(py::handle(o))->belongs_to(dict)) {
-        const py::object h = py::cast(new H(py::reinterpret_borrow<py::object>(module), type), py::return_value_policy::take_ownership);
+        const py::object h = py::cast(new H(dict), py::return_value_policy::take_ownership);
         PyDict_SetItem(dict, keys().handle, h.ptr());
         o = h.ptr();
     }
     return py::cast<H*>(py::handle(o));
 }
-inline MixerHandle* mixer_handle(PyObject* mixer) {
-    return mixer && types && (PyObject*)Py_TYPE(mixer) == types->block.ptr() ? handle_in<MixerHandle>(mixer, types->block) : nullptr;
+
+// The handle of a mixer that can run here, or null.
+inline MixerHandle* ready_mixer(PyObject* mixer, const Tensor& x) {
+    if (!mixer || (PyObject*)Py_TYPE(mixer) != types->block.ptr()) return nullptr;
+    PyObject* dict = dict_of(mixer);
+    MixerHandle* m = dict ? handle_in<MixerHandle>(dict) : nullptr;
+    return m && m->ready(dict, x) ? m : nullptr;
 }
 
 // A residual block: its norm and its mixer.
@@ -495,11 +502,11 @@ struct Layer {
     MixerHandle* m = nullptr;
 };
 inline bool find_layer(PyObject* block, const Tensor& x, Layer& l) {
-    PyObject* mods = get(dict_of(block), keys().modules);
-    l.m = mixer_handle(get(mods, keys().mixer));
-    if (!l.m || !l.m->ready(x)) return false;
-    l.n = handle_in<NormHandle>(block, types->norm);
-    return l.n && l.n->ready(*l.m);
+    PyObject* dict = dict_of(block);
+    l.m = ready_mixer(get(get(dict, keys().modules), keys().mixer), x);
+    if (!l.m) return false;
+    l.n = handle_in<NormHandle>(dict);
+    return l.n->ready(*l.m);
 }
 
 // Whether the calls a native path replaces would be rewritten by autocast.

@@ -35,7 +35,7 @@ py::object pair(const Tensor& h, const Tensor& w) { return py::make_tuple(h, w);
 // list.  None: not a stack that can run here (the caller goes on in Python).
 py::object stack_step(const py::list& layers, const Tensor& x_in, const py::list& caches, bool inplace) {
     const size_t n = layers.size();
-    if (at::GradMode::is_enabled() || autocast_on() || !x_in.is_cuda() || x_in.dim() != 2 || n == 0 || caches.size() < n ||
+    if (at::GradMode::is_enabled() || autocast_on() || !types || !types->plain() || !x_in.is_cuda() || x_in.dim() != 2 || n == 0 || caches.size() < n ||
         x_in.size(0) > MPA_DECODE_MAX_BATCH || x_in.size(0) == 0)
         return py::none();
     const int64_t batch = x_in.size(0);
@@ -99,14 +99,14 @@ py::object stack_step(const py::list& layers, const Tensor& x_in, const py::list
 
 // One token through one MambaBlock (no norm, no residual): (y, h, window) or None.
 py::object block_step(const py::object& block, const Tensor& x_in, const Opt& h_in, const Tensor& window, bool inplace) {
-    if (at::GradMode::is_enabled() || autocast_on() || !x_in.is_cuda() || x_in.dim() != 2 || x_in.size(0) > MPA_DECODE_MAX_BATCH || x_in.size(0) == 0)
+    if (at::GradMode::is_enabled() || autocast_on() || !types || !types->plain() || !x_in.is_cuda() || x_in.dim() != 2 || x_in.size(0) > MPA_DECODE_MAX_BATCH || x_in.size(0) == 0)
         return py::none();
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard guard(x_in.device());
-    MixerHandle* l = mixer_handle(block.ptr());
+    MixerHandle* l = ready_mixer(block.ptr(), x_in);
     const int64_t batch = x_in.size(0);
     const Cache in{val(h_in), window};
-    if (!l || !l->ready(x_in) || !l->decode_ok || !cache_fits(in, *l, batch, inplace)) return py::none();
+    if (!l || !l->decode_ok || !cache_fits(in, *l, batch, inplace)) return py::none();
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
     l->form(false);
@@ -132,7 +132,7 @@ py::object block_step(const py::object& block, const Tensor& x_in, const Opt& h_
 py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::object& caches, bool return_caches,
                          const PackedPlan& packed) {
     const size_t n = layers.size();
-    if (at::GradMode::is_enabled() || autocast_on() || !x_in.is_cuda() || x_in.dim() != 3 || n == 0 || x_in.numel() == 0) return py::none();
+    if (at::GradMode::is_enabled() || autocast_on() || !types || !types->plain() || !x_in.is_cuda() || x_in.dim() != 3 || n == 0 || x_in.numel() == 0) return py::none();
     const int64_t Bs = x_in.size(0), L = x_in.size(1), T = Bs * L;
     std::vector<Layer> hs(n);
     std::vector<Cache> cs(n);
@@ -275,10 +275,28 @@ void bind_model(py::module_& m) {
     mixer.def("expire", &MixerHandle::expire);
     py::class_<NormHandle> norm(m, "NormHandle");
     copies(norm);
-    m.def("register_types", [](const py::object& block, const py::object& norm) {
-        if (!types) types = new Types();
-        types->block = block;
-        types->norm = norm;
+    // {method: what it was when the package was imported} of each class that native calls stand in for
+    m.def("register_types", [](const py::object& block, const py::dict& block_methods, const py::object& norm, const py::dict& norm_methods,
+                               const py::object& linear, const py::dict& linear_methods, const py::object& module, const py::dict& module_methods,
+                               const py::object& conv, const py::list& global_hooks) {
+        Types* t = new Types();
+        t->block = block;
+        t->norm = norm;
+        t->linear = linear;
+        t->conv = conv;
+        auto watch = [&](const py::object& cls, const py::dict& methods, std::vector<Ref>* names) {
+            PyObject* dict = reinterpret_cast<PyTypeObject*>(cls.ptr())->tp_dict;
+            for (const auto& [name, was] : methods) {
+                t->methods.push_back({Ref(dict), Ref(name.ptr()), Ref(was.ptr())});
+                if (names) names->push_back(Ref(name.ptr()));
+            }
+        };
+        watch(block, block_methods, &t->block_names);
+        watch(norm, norm_methods, &t->norm_names);
+        watch(linear, linear_methods, &t->linear_names);
+        watch(module, module_methods, nullptr);
+        for (const auto& h : global_hooks) t->global_hooks.push_back(Ref(h.ptr()));
+        types = t;
     });
     m.def("stack_step", &stack_step);
     m.def("block_step", &block_step);

@@ -65,13 +65,15 @@ mpa_conv_shape mixer_conv_shape(const MixerBackward& m, int io, bool backward) {
 // (y, h_last or None, window or None), or None: not a block that can run here
 py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h_in, const Opt& win_in, bool return_cache,
                        const PackedPlan& packed) {
-    if (!at::GradMode::is_enabled() || autocast_on() || !x_in.is_cuda() || x_in.dim() != 3 || x_in.numel() == 0) return py::none();
-    MixerHandle* l = mixer_handle(block.ptr());
+    if (!at::GradMode::is_enabled() || autocast_on() || !types || !types->plain() || !x_in.is_cuda() || x_in.dim() != 3 || x_in.numel() == 0)
+        return py::none();
+    MixerHandle* l = nullptr;
     const Tensor hc = val(h_in), wc = val(win_in);
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::DeviceGuard guard(x_in.device());
-        if (!l || !l->ready(x_in) || !l->forward_ok || l->N % 4) return py::none();
+        l = ready_mixer(block.ptr(), x_in);
+        if (!l || !l->forward_ok || l->N % 4) return py::none();
         if (unpack(packed).flags & MPA_PLAN_BWD_GENERAL) return py::none();
         const int64_t Bs = x_in.size(0);
         if (hc.defined() && !fits(hc, {Bs, l->ED, l->N}, at::kFloat, l->device)) return py::none();

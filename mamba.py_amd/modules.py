@@ -76,9 +76,8 @@ def _host():
     """The compiled layer code (csrc/host_model.cpp), told once which classes it stands in for."""
     global _HOST
     if _HOST is None:
-        host = _lib.host()
-        host.register_types(MambaBlock, RMSNorm)
-        _HOST = host
+        _HOST = _lib.host()
+        _HOST.register_types(*_STOOD_IN_FOR)
     return _HOST
 
 
@@ -255,7 +254,7 @@ class MambaBlock(nn.Module):
         if x.is_cuda and torch.is_grad_enabled():
             # a block of the plain kind: one graph node
             h_in, win_in = cache if cache is not None else (None, None)
-            out = _host().block_train(self, x, h_in, win_in, bool(return_cache), plan.packed)
+            out = _host().block_train(self, x, h_in, win_in, bool(return_cache), plan.packed) if PAD_PROJECTIONS else None
             _expire_forms(self)
             if out is not None:
                 return (out[0], out[1:]) if return_cache else out[0]
@@ -383,6 +382,23 @@ class MambaBlock(nn.Module):
         return self.out_proj(y)
 
 
+def _methods(cls, *names):
+    return {name: cls.__dict__[name] for name in names}
+
+
+# The methods that native calls stand in for, as they are now: one that is replaced later, on its class or on an
+# instance, is called.  So are torch's hooks on all modules.
+_STOOD_IN_FOR = (
+    MambaBlock, _methods(MambaBlock, "forward", "ssm", "step", "ssm_step", "step_", "_A", "_D", "_dt_bias", "_conv_wb", "_split_projection",
+                         "_padded_projections"),
+    RMSNorm, _methods(RMSNorm, "forward", "add_norm", "_w"),
+    nn.Linear, _methods(nn.Linear, "forward"),
+    nn.Module, _methods(nn.Module, "__call__", "_wrapped_call_impl", "_call_impl"),
+    nn.Conv1d,
+    [getattr(nn.modules.module, "_global_" + hooks) for hooks in ("forward_hooks", "forward_pre_hooks", "backward_hooks",
+                                                                  "backward_pre_hooks")])
+
+
 class ResidualBlock(nn.Module):
     """mixer(norm(x)) + x  (mambapy/mamba.py:99-125); keys: mixer.*, norm.weight."""
 
@@ -417,7 +433,7 @@ class Mamba(nn.Module):
         """x : (B, L, D) -> (B, L, D) [, caches].  `caches` (one (h, inputs) pair per layer, as
         returned by an earlier call with return_caches=True, by step() or by empty_caches()) makes
         the call continue that sequence."""
-        if x.is_cuda and not torch.is_grad_enabled():
+        if x.is_cuda and not torch.is_grad_enabled() and PAD_PROJECTIONS:
             # layers of the plain kind: the whole stack in one call
             out = _host().stack_forward(list(self.layers), x, caches, bool(return_caches), plan.packed)
             if out is not None:
