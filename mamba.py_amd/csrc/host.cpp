@@ -50,9 +50,12 @@ variable_list ScanBackward::apply(variable_list&& grads) {
     variable_list out(8);
     Tensor dy = grads[0];
     if (!dy.defined()) return out;
+    // (unpacked outside of the guard, here and in the other nodes: a hook may run a whole forward pass)
+    const Tensor x_ = x.unpack(), delta_ = delta.unpack(), A_ = dense(A.unpack()), D_ = dense(D.unpack()), z_ = z.unpack(),
+                 bias_ = dense(bias.unpack()), h0_ = dense(h0.unpack()), ckpt_ = dense(ckpt.unpack()), y_pre_ = y_pre.unpack();
+    Tensor B_ = unit_rows(B.unpack()), C_ = unit_rows(C.unpack());
+    if (B_.strides() != C_.strides()) { B_ = B_.contiguous(); C_ = C_.contiguous(); }
     at::AutoDispatchBelowADInplaceOrView below;
-    const Tensor x_ = x.unpack(), delta_ = delta.unpack(), A_ = A.unpack(), B_ = B.unpack(), C_ = C.unpack(), D_ = D.unpack(),
-                 z_ = z.unpack(), bias_ = bias.unpack(), h0_ = h0.unpack(), ckpt_ = ckpt.unpack(), y_pre_ = y_pre.unpack();
     const c10::DeviceGuard guard(x_.device());
     const auto dt = x_.scalar_type();
     const int64_t Bs = x_.size(0), L = x_.size(1), ED = x_.size(2), N = A_.size(1);
@@ -100,19 +103,24 @@ std::tuple<Tensor, Opt> scan_fwd(const Tensor& x, const Tensor& delta_in, const 
     std::shared_ptr<ScanBackward> node;
     if (need_grad) node = make_node<ScanBackward>({&x, &delta_in, &A_in, &B_in, &C_in, &D_in, &zc, &bc});
     Tensor y, h_last;
+    Tensor delta, A, B, C, D, z, bias, h0, ckpt, y_pre;
+    const int flags = (softplus ? MPA_SSCAN_DELTA_SOFTPLUS : 0) | (reverse ? MPA_SSCAN_REVERSE : 0);
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::DeviceGuard guard(x.device());
         // the general backward kernel, which only a pinned plan selects, has no float32 delta
         const bool wide = delta_in.scalar_type() == at::kFloat && dt == at::kBFloat16 && !(plan.flags & MPA_PLAN_BWD_GENERAL);
-        const Tensor delta = wide ? delta_in : cast(delta_in, dt);
-        Tensor B = unit_rows(cast(B_in, dt)), C = unit_rows(cast(C_in, dt));
+        delta = wide ? delta_in : cast(delta_in, dt);
+        B = unit_rows(cast(B_in, dt));
+        C = unit_rows(cast(C_in, dt));
         if (B.strides() != C.strides()) { B = B.contiguous(); C = C.contiguous(); }
-        const Tensor z = cast(zc, dt), A = f32c(A_in), D = f32c(D_in), bias = f32c(bc), h0 = f32c(hc);
+        z = cast(zc, dt);
+        A = f32c(A_in);
+        D = f32c(D_in);
+        bias = f32c(bc);
+        h0 = f32c(hc);
         y = empty({Bs, L, ED}, dt, x);
-        const int flags = (softplus ? MPA_SSCAN_DELTA_SOFTPLUS : 0) | (reverse ? MPA_SSCAN_REVERSE : 0);
         const mpa_sscan_shape s = sscan_shape(x, delta, B, y, y, B, N, flags, z, plan, false);
-        Tensor ckpt, y_pre;
         if (need_grad) {
             ckpt = empty({mpa_sscan_ckpt_elems(&s)}, at::kFloat, x);
             if (z.defined()) y_pre = empty({Bs, L, ED}, dt, x);  // output before the gate, read again by the backward
@@ -123,16 +131,16 @@ std::tuple<Tensor, Opt> scan_fwd(const Tensor& x, const Tensor& delta_in, const 
         check(mpa_sscan_fwd(&s, ptr(x), ptr(delta), fptr(A), ptr(B), ptr(C), fptr(D), ptr(z), fptr(bias), fptr(h0), ptr(y), ptr(y_pre),
                             fptr(ckpt), fptr(h_last), ptr(ws), nbytes, stream_of(x)),
               "mpa_sscan_fwd");
-        if (node) {
-            node->flags = flags;
-            node->plan = plan;
-            node->x = keep(x); node->delta = keep(delta); node->A = keep(A); node->B = keep(B); node->C = keep(C); node->D = keep(D);
-            node->z = keep(z); node->bias = keep(bias); node->h0 = keep(h0); node->ckpt = keep(ckpt); node->y_pre = keep(y_pre);
-            const std::array<const Tensor*, 8> in = {&x, &delta_in, &A_in, &B_in, &C_in, &D_in, &zc, &bc};
-            for (size_t i = 0; i < 8; ++i) node->dtypes[i] = in[i]->defined() ? in[i]->scalar_type() : at::kFloat;
-        }
     }
-    if (node) torch::autograd::set_history(y, node);
+    if (node) {
+        node->flags = flags;
+        node->plan = plan;
+        node->x = keep(x); node->delta = keep(delta); node->A = keep(A); node->B = keep(B); node->C = keep(C); node->D = keep(D);
+        node->z = keep(z); node->bias = keep(bias); node->h0 = keep(h0); node->ckpt = keep(ckpt); node->y_pre = keep(y_pre);
+        const std::array<const Tensor*, 8> in = {&x, &delta_in, &A_in, &B_in, &C_in, &D_in, &zc, &bc};
+        for (size_t i = 0; i < 8; ++i) node->dtypes[i] = in[i]->defined() ? in[i]->scalar_type() : at::kFloat;
+        torch::autograd::set_history(y, node);
+    }
     return {y, return_last ? Opt(h_last) : Opt()};
 }
 
@@ -237,8 +245,8 @@ struct ConvBackward : public Node {
     variable_list apply(variable_list&& grads) override {
         variable_list out(3);
         if (!grads[0].defined()) return out;
+        const Tensor x_ = x.unpack(), w_ = dense(w.unpack()), b_ = dense(b.unpack()), win_ = dense(win.unpack());
         at::AutoDispatchBelowADInplaceOrView below;
-        const Tensor x_ = x.unpack(), w_ = w.unpack(), b_ = b.unpack(), win_ = win.unpack();
         const c10::DeviceGuard guard(x_.device());
         const int64_t ED = x_.size(2), K = w_.size(1);
         const Tensor dy = cast(grads[0], x_.scalar_type());
@@ -268,25 +276,26 @@ std::tuple<Tensor, Opt> conv(const Tensor& x, const Tensor& w_in, const Opt& b_i
     io_dtype(dt);
     std::shared_ptr<ConvBackward> node;
     if (tracked({&x, &w_in, &bc})) node = make_node<ConvBackward>({&x, &w_in, &bc});
-    Tensor y, wout;
+    Tensor y, wout, w, b, win;
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::DeviceGuard guard(x.device());
-        const Tensor w = f32c(w_in).view({ED, K}), b = f32c(bc);
-        const Tensor win = wc.defined() ? cast(wc, dt).contiguous() : wc;
+        w = f32c(w_in).view({ED, K});
+        b = f32c(bc);
+        win = wc.defined() ? cast(wc, dt).contiguous() : wc;
         y = empty({Bs, L, ED}, dt, x);
         if (return_window) wout = empty({Bs, ED, K - 1}, dt, x);
         const mpa_conv_shape s = conv_shape(x, y, y, K, silu);
         check(mpa_conv1d_fwd(&s, ptr(x), fptr(w), fptr(b), ptr(win), ptr(y), ptr(wout), stream_of(x)), "mpa_conv1d_fwd");
-        if (node) {
-            node->silu = silu;
-            node->wshape = w_in.sizes().vec();
-            node->tw = w_in.scalar_type();
-            node->tb = bc.defined() ? bc.scalar_type() : at::kFloat;
-            node->x = keep(x); node->w = keep(w); node->b = keep(b); node->win = keep(win);
-        }
     }
-    if (node) torch::autograd::set_history(y, node);
+    if (node) {
+        node->silu = silu;
+        node->wshape = w_in.sizes().vec();
+        node->tw = w_in.scalar_type();
+        node->tb = bc.defined() ? bc.scalar_type() : at::kFloat;
+        node->x = keep(x); node->w = keep(w); node->b = keep(b); node->win = keep(win);
+        torch::autograd::set_history(y, node);
+    }
     return {y, return_window ? Opt(wout) : Opt()};
 }
 
@@ -321,7 +330,7 @@ struct NormBackward : public Node {
         variable_list out(3);
         const bool has_dy = grads[0].defined(), has_ds = with_sum && grads[1].defined();
         if (!has_dy && !has_ds) return out;
-        const Tensor x_ = with_sum ? x.unpack(shared_from_this()) : x.unpack(), w_ = w.unpack();
+        const Tensor x_ = dense(with_sum ? x.unpack(shared_from_this()) : x.unpack()), w_ = dense(w.unpack());
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::DeviceGuard guard(x_.device());
         const auto dt = x_.scalar_type();

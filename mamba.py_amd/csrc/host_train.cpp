@@ -14,26 +14,26 @@ namespace {
 
 enum { kIX, kIInW, kIInB, kIConvW, kIConvB, kIXW, kIDtW, kIDtB, kIALog, kID, kIOutW, kIOutB, kInputs };
 
+// What the node keeps: inputs, activations and derived weights, all of them as saved variables, so that hooks on saved
+// tensors (checkpointing, offloading) have them; and the parameters the derived ones are made from, whose version
+// counters are checked when they are unpacked.
+enum { kSWin, kSH0, kSXz, kSXs, kSDbc, kSDelta, kSY, kSYPre, kSCkpt, kSA, kSD, kSDtB, kSConvW, kSConvB, kSXp, kSDtp, kSaved };
+
 struct MixerBackward : public Node {
-    // inputs and activations; originals of the parameters whose derived forms are used (their
-    // version counters are checked when they are unpacked)
-    SavedVariable x, win, h0, params[kInputs];
-    Tensor xz, xs, dbc, delta, y, y_pre, ckpt;  // made here, seen by nobody else
-    Tensor A, D, dt_b, conv_w, conv_b, xp, dtp;
-    int64_t Bs = 0, L = 0, d = 0, ED = 0, N = 0, R = 0, Rp = 0, K = 0;
+    SavedVariable inputs[kInputs], saved[kSaved];
+    int64_t Bs = 0, L = 0, d = 0, ED = 0, N = 0, R = 0, Rp = 0, K = 0, P = 0;
     Plan plan;
     std::string name() const override { return "MambaBlockBackward"; }
     void release_variables() override {
-        x.reset_data(); win.reset_data(); h0.reset_data();
-        for (SavedVariable& v : params) v.reset_data();
-        for (Tensor* t : {&xz, &xs, &dbc, &delta, &y, &y_pre, &ckpt, &A, &D, &dt_b, &conv_w, &conv_b, &xp, &dtp}) t->reset();
+        for (SavedVariable& v : inputs) v.reset_data();
+        for (SavedVariable& v : saved) v.reset_data();
     }
     variable_list apply(variable_list&& grads) override;
 };
 
 mpa_sscan_shape mixer_scan_shape(const MixerBackward& m, int io, bool backward) {
     mpa_sscan_shape s{};
-    const int64_t L = m.L, ED = m.ED, P = m.dbc.size(1);
+    const int64_t L = m.L, ED = m.ED, P = m.P;
     s.batch = m.Bs; s.seqlen = L; s.dim = ED; s.dstate = m.N;
     s.io_dtype = io;
     s.flags = MPA_SSCAN_DELTA_SOFTPLUS;
@@ -90,24 +90,23 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
     }
     if (!any) return py::none();
     auto node = make_node<MixerBackward>({in[0], in[1], in[2], in[3], in[4], in[5], in[6], in[7], in[8], in[9], in[10], in[11]});
-    Tensor out, h_last, window;
+    Tensor x, out, h_last, window, t[kSaved];
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::DeviceGuard guard(x_in.device());
         MixerBackward& m = *node;
-        const Tensor x = x_in.contiguous();
+        x = x_in.contiguous();
         const auto dt = x.scalar_type();
         const int io = io_dtype(dt);
         const size_t es = x.element_size();
         m.Bs = x.size(0); m.L = x.size(1); m.d = l->d; m.ED = l->ED; m.N = l->N; m.R = l->R; m.Rp = l->Rp; m.K = l->K;
+        m.P = l->padded_rows();
         m.plan = unpack(packed);
         const MixerHandle::TrainForms f = l->train_forms();
-        m.A = f.A; m.D = f.D; m.dt_b = f.dt_b; m.conv_w = f.conv_w; m.conv_b = f.conv_b; m.xp = f.xp; m.dtp = f.dtp;
-        const int64_t T = m.Bs * m.L, ED = m.ED, N = m.N;
+        const int64_t T = m.Bs * m.L, ED = m.ED, N = m.N, P = m.P;
         const Tensor x2 = x.view({T, m.d});
         void* stream = stream_of(x);
-        const int64_t P = m.xp.size(0);
-        const bool own = use_linear(dt, T, m.d, ED, P, {&x, &l->p[kInW].t, &l->p[kOutW].t, &m.xp, &m.dtp, &l->p[kInB].t, &l->p[kOutB].t});
+        const bool own = use_linear(dt, T, m.d, ED, P, {&x, &l->p[kInW].t, &l->p[kOutW].t, &f.xp, &f.dtp, &l->p[kInB].t, &l->p[kOutB].t});
         auto product = [&](const Tensor& in, int64_t K, const Tensor& weight, const Tensor& bias) {
             const int64_t M = weight.size(0);
             const Tensor y = empty({T, M}, dt, x);
@@ -116,34 +115,36 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
             run_linear(q, stream);
             return y;
         };
-        m.xz = own ? product(x2, m.d, l->p[kInW].t, l->p[kInB].t)
-               : l->p[kInB].t.defined() ? at::addmm(l->p[kInB].t, x2, l->p[kInW].t.t()) : at::mm(x2, l->p[kInW].t.t());
-        m.xs = empty({T, ED}, dt, x);
+        const Tensor xz = own ? product(x2, m.d, l->p[kInW].t, l->p[kInB].t)
+                          : l->p[kInB].t.defined() ? at::addmm(l->p[kInB].t, x2, l->p[kInW].t.t()) : at::mm(x2, l->p[kInW].t.t());
+        const Tensor xs = empty({T, ED}, dt, x);
         if (return_cache) {
             window = empty({m.Bs, ED, m.K - 1}, dt, x);
             h_last = empty({m.Bs, ED, N}, at::kFloat, x);
         }
         const mpa_conv_shape cv = mixer_conv_shape(m, io, false);
-        check(mpa_conv1d_fwd(&cv, ptr(m.xz), fptr(m.conv_w), fptr(m.conv_b), ptr(wc), ptr(m.xs), ptr(window), stream), "mpa_conv1d_fwd");
-        m.dbc = own ? product(m.xs, ED, m.xp, Tensor()) : at::mm(m.xs, m.xp.t());
-        m.delta = own ? product(m.dbc, m.Rp, m.dtp, Tensor()) : at::mm(m.dbc.narrow(1, 0, m.Rp), m.dtp.t());
-        m.y = empty({T, ED}, dt, x);
-        m.y_pre = empty({T, ED}, dt, x);
+        check(mpa_conv1d_fwd(&cv, ptr(xz), fptr(f.conv_w), fptr(f.conv_b), ptr(wc), ptr(xs), ptr(window), stream), "mpa_conv1d_fwd");
+        const Tensor dbc = own ? product(xs, ED, f.xp, Tensor()) : at::mm(xs, f.xp.t());
+        const Tensor delta = own ? product(dbc, m.Rp, f.dtp, Tensor()) : at::mm(dbc.narrow(1, 0, m.Rp), f.dtp.t());
+        const Tensor y = empty({T, ED}, dt, x), y_pre = empty({T, ED}, dt, x);
         const mpa_sscan_shape sc = mixer_scan_shape(m, io, false);
-        m.ckpt = empty({mpa_sscan_ckpt_elems(&sc)}, at::kFloat, x);
+        const Tensor ckpt = empty({mpa_sscan_ckpt_elems(&sc)}, at::kFloat, x);
         const size_t nbytes = mpa_sscan_fwd_workspace_bytes(&sc, 1);
         const Tensor ws = scratch(nbytes, x);
-        const char* bc = static_cast<const char*>(ptr(m.dbc)) + m.Rp * es;
-        check(mpa_sscan_fwd(&sc, ptr(m.xs), ptr(m.delta), fptr(m.A), bc, bc + N * es, fptr(m.D), static_cast<const char*>(ptr(m.xz)) + ED * es,
-                            fptr(m.dt_b), fptr(hc), ptr(m.y), ptr(m.y_pre), fptr(m.ckpt), fptr(h_last), ptr(ws), nbytes, stream),
+        const char* bc = static_cast<const char*>(ptr(dbc)) + m.Rp * es;
+        check(mpa_sscan_fwd(&sc, ptr(xs), ptr(delta), fptr(f.A), bc, bc + N * es, fptr(f.D), static_cast<const char*>(ptr(xz)) + ED * es,
+                            fptr(f.dt_b), fptr(hc), ptr(y), ptr(y_pre), fptr(ckpt), fptr(h_last), ptr(ws), nbytes, stream),
               "mpa_sscan_fwd");
-        out = (own ? product(m.y, ED, l->p[kOutW].t, l->p[kOutB].t)
-               : l->p[kOutB].t.defined() ? at::addmm(l->p[kOutB].t, m.y, l->p[kOutW].t.t()) : at::mm(m.y, l->p[kOutW].t.t())).view({m.Bs, m.L, m.d});
-        m.x = keep(x);
-        m.win = keep(wc);
-        m.h0 = keep(hc);
-        for (int i = 1; i < kInputs; ++i) m.params[i] = keep(*in[i]);
+        out = (own ? product(y, ED, l->p[kOutW].t, l->p[kOutB].t)
+               : l->p[kOutB].t.defined() ? at::addmm(l->p[kOutB].t, y, l->p[kOutW].t.t()) : at::mm(y, l->p[kOutW].t.t())).view({m.Bs, m.L, m.d});
+        const std::array<const Tensor*, kSaved> made = {&wc, &hc, &xz, &xs, &dbc, &delta, &y, &y_pre, &ckpt, &f.A, &f.D, &f.dt_b, &f.conv_w,
+                                                        &f.conv_b, &f.xp, &f.dtp};
+        for (int i = 0; i < kSaved; ++i) t[i] = *made[i];
     }
+    // (outside of the guard: hooks on saved tensors are called here)
+    node->inputs[kIX] = keep(x);
+    for (int i = 1; i < kInputs; ++i) node->inputs[i] = keep(*in[i]);
+    for (int i = 0; i < kSaved; ++i) node->saved[i] = keep(t[i]);
     torch::autograd::set_history(out, node);
     return py::make_tuple(out, return_cache ? py::cast(h_last) : py::object(py::none()),
                           return_cache ? py::cast(window) : py::object(py::none()));
@@ -152,17 +153,36 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
 variable_list MixerBackward::apply(variable_list&& grads) {
     variable_list g(kInputs);
     if (!grads[0].defined()) return g;
+    // (unpacked outside of the guard: a hook may run a whole forward pass)
+    Tensor w[kInputs], t[kSaved];
+    for (int i = 0; i < kInputs; ++i) w[i] = inputs[i].unpack();
+    for (int i = 0; i < kSaved; ++i) t[i] = saved[i].unpack();
+    const int64_t T = Bs * L, used = Rp + 2 * N;
+    const auto dt = w[kIX].scalar_type();
+    const auto f32 = at::kFloat;
+    // (a hook may also give back another tensor than it was given: the kernels rely on these)
+    const auto given = [&](Tensor& v, at::IntArrayRef shape, at::ScalarType type) {
+        if (!v.defined()) return;
+        TORCH_CHECK(v.sizes() == shape && v.scalar_type() == type && v.device() == w[kIX].device(), "a saved tensor of a MambaBlock came back as ",
+                    v.scalar_type(), v.sizes(), " on ", v.device(), ", was ", type, shape);
+        v = v.contiguous();
+    };
+    given(w[kIX], {Bs, L, d}, dt); given(w[kIInW], {2 * ED, d}, dt); given(w[kIOutW], {d, ED}, dt);
+    given(t[kSWin], {Bs, ED, K - 1}, dt); given(t[kSH0], {Bs, ED, N}, f32);
+    given(t[kSXz], {T, 2 * ED}, dt); given(t[kSDbc], {T, P}, dt);
+    for (int i : {kSXs, kSDelta, kSY, kSYPre}) given(t[i], {T, ED}, dt);
+    given(t[kSCkpt], {Bs * ((L + MPA_CKPT_STEPS - 1) / MPA_CKPT_STEPS) * N * ED}, f32);
+    given(t[kSA], {ED, N}, f32);
+    for (int i : {kSD, kSDtB, kSConvB}) given(t[i], {ED}, f32);
+    given(t[kSConvW], {ED, 1, K}, f32);
+    given(t[kSXp], {P, ED}, dt); given(t[kSDtp], {ED, Rp}, dt);
+    const Tensor &x_ = w[kIX], &win_ = t[kSWin], &h0_ = t[kSH0], &xz = t[kSXz], &xs = t[kSXs], &dbc = t[kSDbc], &delta = t[kSDelta], &y = t[kSY],
+                 &y_pre = t[kSYPre], &ckpt = t[kSCkpt], &A = t[kSA], &D = t[kSD], &dt_b = t[kSDtB], &conv_w = t[kSConvW], &conv_b = t[kSConvB],
+                 &xp = t[kSXp], &dtp = t[kSDtp];
     at::AutoDispatchBelowADInplaceOrView below;
-    const Tensor x_ = x.unpack(), win_ = win.unpack(), h0_ = h0.unpack();
-    TORCH_CHECK(xz.defined(), "Trying to backward through the graph a second time: the saved tensors have been freed "
-                              "(specify retain_graph=True)");
-    Tensor w[kInputs];
-    for (int i = 1; i < kInputs; ++i) w[i] = params[i].unpack();
     const c10::DeviceGuard guard(x_.device());
-    const auto dt = x_.scalar_type();
     const int io = io_dtype(dt);
     const size_t es = x_.element_size();
-    const int64_t T = Bs * L, P = dbc.size(1), used = Rp + 2 * N;
     void* stream = stream_of(x_);
     auto at_col = [&](const Tensor& t, int64_t col) { return static_cast<char*>(ptr(t)) + col * es; };
     const Tensor x2 = x_.view({T, d}), dout = cast(grads[0], dt).contiguous().view({T, d});
