@@ -84,6 +84,7 @@ std::tuple<Tensor, Opt> scan_fwd(const Tensor& x, const Tensor& delta_in, const 
                                  bool return_last, bool reverse, const PackedPlan& packed) {
     const Tensor zc = val(z_in), bc = val(bias_in), hc = val(h0_in);
     require_gpu({&x, &delta_in, &A_in, &B_in, &C_in, &D_in, &zc, &bc, &hc});
+    require_plain({&x, &delta_in, &A_in, &B_in, &C_in, &D_in, &zc, &bc, &hc});
     const Plan plan = unpack(packed);
     const auto dt = x.scalar_type();
     io_dtype(dt);
@@ -188,6 +189,7 @@ struct PScanBackward : public Node {
 
 Tensor pscan(const Tensor& A_in, const Tensor& X_in, bool reverse, const PackedPlan& packed) {
     require_gpu({&A_in, &X_in});
+    require_plain({&A_in, &X_in});
     TORCH_CHECK(A_in.sizes() == X_in.sizes() && X_in.dim() == 4, "pscan expects two (B, L, D, N) tensors, got ", A_in.sizes(), " and ",
                 X_in.sizes());
     const auto dt = at::promote_types(A_in.scalar_type(), X_in.scalar_type());
@@ -268,6 +270,7 @@ struct ConvBackward : public Node {
 std::tuple<Tensor, Opt> conv(const Tensor& x, const Tensor& w_in, const Opt& b_in, const Opt& win_in, bool silu, bool return_window) {
     const Tensor bc = val(b_in), wc = val(win_in);
     require_gpu({&x, &w_in, &bc, &wc});
+    require_plain({&x, &w_in, &bc, &wc});
     TORCH_CHECK(x.dim() == 3, "x must be (B, L, ED)");
     const int64_t Bs = x.size(0), L = x.size(1), ED = x.size(2), K = w_in.size(-1);
     TORCH_CHECK(w_in.numel() == ED * K, "weight must be (ED, 1, K) or (ED, K), got ", w_in.sizes());
@@ -358,6 +361,7 @@ struct NormBackward : public Node {
 std::tuple<Tensor, Opt> rmsnorm(const Tensor& x_in, const Opt& res_in, const Opt& w_in, double eps) {
     const Tensor rc = val(res_in), wc = val(w_in);
     require_gpu({&x_in, &rc, &wc});
+    require_plain({&x_in, &rc, &wc});
     TORCH_CHECK(!rc.defined() || (rc.sizes() == x_in.sizes() && rc.scalar_type() == x_in.scalar_type()),
                 "residual must have the shape and dtype of x");
     const int io = io_dtype(x_in.scalar_type());

@@ -7,6 +7,7 @@
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
@@ -69,6 +70,22 @@ inline bool tracked(std::initializer_list<const Tensor*> ts) {
     for (const Tensor* t : ts)
         if (t->defined() && t->requires_grad()) return true;
     return false;
+}
+
+// Forward-mode derivatives: the entry points run below autograd and have no rule for them.  Operators refuse a dual
+// tensor; layers leave it to the composed path, whose operators do.  (functorch's wrapped tensors, of vmap and of its own
+// grad and jvp, have no memory of their own and are refused with them.)
+inline bool forward_mode() { return torch::autograd::ForwardADLevel::try_get_by_idx(0) != nullptr; }  // (no tangents outside of a level)
+inline bool wrapped(const Tensor& t) {
+    return t.defined() && (t.key_set().has(c10::DispatchKey::FuncTorchBatched) || t.key_set().has(c10::DispatchKey::FuncTorchGradWrapper));
+}
+inline void require_plain(std::initializer_list<const Tensor*> ts) {
+    const bool tangents = forward_mode();
+    for (const Tensor* t : ts) {
+        TORCH_CHECK_NOT_IMPLEMENTED(!tangents || !t->defined() || !t->_fw_grad(/*level=*/0).defined(),
+                                    "forward-mode derivatives are not implemented for the operators of mambapy_amd");
+        TORCH_CHECK(!wrapped(*t), "functorch transforms (vmap, grad, jvp) are not implemented for the operators of mambapy_amd");
+    }
 }
 
 inline SavedVariable keep(const Tensor& t) { return SavedVariable(t, false); }

@@ -107,6 +107,7 @@ struct Param {
         }
         if (!o || !THPVariable_CheckExact(o)) return false;
         const Tensor& now = THPVariable_Unpack(o);
+        if (wrapped(now)) return false;
         const void* im = now.unsafeGetTensorImpl();
         const bool counted = !now.is_inference();
         if (counted && im == impl && now.const_data_ptr() == data && now._version() == version) return true;
@@ -509,8 +510,11 @@ inline bool find_layer(PyObject* block, const Tensor& x, Layer& l) {
     return l.n->ready(*l.m);
 }
 
-// Whether the calls a native path replaces would be rewritten by autocast.
-inline bool autocast_on() { return at::autocast::is_autocast_enabled(at::kCUDA); }
+// Whether a native call may run at all: nothing replaces or rewrites the calls it stands in for (autocast does), and x is
+// an ordinary tensor without a tangent.
+inline bool native_call(const Tensor& x) {
+    return types && types->plain() && !at::autocast::is_autocast_enabled(at::kCUDA) && !forward_mode() && x.is_cuda() && !wrapped(x);
+}
 
 inline bool fits(const Tensor& t, at::IntArrayRef shape, at::ScalarType dt, const c10::Device& dev) {
     return t.scalar_type() == dt && t.device() == dev && t.sizes() == shape && t.is_contiguous() &&

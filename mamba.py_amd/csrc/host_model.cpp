@@ -35,7 +35,7 @@ py::object pair(const Tensor& h, const Tensor& w) { return py::make_tuple(h, w);
 // list.  None: not a stack that can run here (the caller goes on in Python).
 py::object stack_step(const py::list& layers, const Tensor& x_in, const py::list& caches, bool inplace) {
     const size_t n = layers.size();
-    if (at::GradMode::is_enabled() || autocast_on() || !types || !types->plain() || !x_in.is_cuda() || x_in.dim() != 2 || n == 0 || caches.size() < n ||
+    if (at::GradMode::is_enabled() || !native_call(x_in) || x_in.dim() != 2 || n == 0 || caches.size() < n ||
         x_in.size(0) > MPA_DECODE_MAX_BATCH || x_in.size(0) == 0)
         return py::none();
     const int64_t batch = x_in.size(0);
@@ -99,7 +99,7 @@ py::object stack_step(const py::list& layers, const Tensor& x_in, const py::list
 
 // One token through one MambaBlock (no norm, no residual): (y, h, window) or None.
 py::object block_step(const py::object& block, const Tensor& x_in, const Opt& h_in, const Tensor& window, bool inplace) {
-    if (at::GradMode::is_enabled() || autocast_on() || !types || !types->plain() || !x_in.is_cuda() || x_in.dim() != 2 || x_in.size(0) > MPA_DECODE_MAX_BATCH || x_in.size(0) == 0)
+    if (at::GradMode::is_enabled() || !native_call(x_in) || x_in.dim() != 2 || x_in.size(0) > MPA_DECODE_MAX_BATCH || x_in.size(0) == 0)
         return py::none();
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard guard(x_in.device());
@@ -132,7 +132,7 @@ py::object block_step(const py::object& block, const Tensor& x_in, const Opt& h_
 py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::object& caches, bool return_caches,
                          const PackedPlan& packed) {
     const size_t n = layers.size();
-    if (at::GradMode::is_enabled() || autocast_on() || !types || !types->plain() || !x_in.is_cuda() || x_in.dim() != 3 || n == 0 || x_in.numel() == 0) return py::none();
+    if (at::GradMode::is_enabled() || !native_call(x_in) || x_in.dim() != 3 || n == 0 || x_in.numel() == 0) return py::none();
     const int64_t Bs = x_in.size(0), L = x_in.size(1), T = Bs * L;
     std::vector<Layer> hs(n);
     std::vector<Cache> cs(n);

@@ -65,8 +65,7 @@ mpa_conv_shape mixer_conv_shape(const MixerBackward& m, int io, bool backward) {
 // (y, h_last or None, window or None), or None: not a block that can run here
 py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h_in, const Opt& win_in, bool return_cache,
                        const PackedPlan& packed) {
-    if (!at::GradMode::is_enabled() || autocast_on() || !types || !types->plain() || !x_in.is_cuda() || x_in.dim() != 3 || x_in.numel() == 0)
-        return py::none();
+    if (!at::GradMode::is_enabled() || !native_call(x_in) || x_in.dim() != 3 || x_in.numel() == 0) return py::none();
     MixerHandle* l = nullptr;
     const Tensor hc = val(h_in), wc = val(win_in);
     {

@@ -15,6 +15,7 @@ from typing import Optional, Tuple, Union
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _lib
 from .conv import causal_conv1d_fn, causal_conv1d_update
@@ -90,8 +91,8 @@ def _frozen_f32(owner, key, p, fn=None):
     captured HIP graph keeps reading the same memory."""
     if p is None:
         return None
-    if torch.is_grad_enabled() and p.requires_grad:
-        return p if fn is None else fn(p)
+    if (torch.is_grad_enabled() and p.requires_grad) or forward_ad._current_level >= 0:
+        return p if fn is None else fn(p)      # (forward mode: a tangent of p is not in a kept value)
     if fn is None and p.dtype == torch.float32:
         return p
     cache = owner.__dict__.setdefault("_f32_cache", {})
