@@ -168,8 +168,9 @@ size_t mpa_sscan_fwd_workspace_bytes(const mpa_sscan_shape* s, int with_ckpt);
  * every GPU it runs on, held until the process ends.  The call allocates and frees nothing.
  * A shape whose mpa_sscan_fwd_workspace_bytes() exceeds MPA_NOALLOC_SCRATCH_BYTES is refused with
  * MPA_ERR_WORKSPACE before anything is launched (sequences cut into segments need
- * 2 * batch * segments * dim * min(dstate, 64) floats and a little more; a caller that pins 16 or
- * 32 states per lane needs the packed B/C of the whole sequence).  All calls on one GPU share that GPU's array: calls that overlap
+ * 2 * batch * segments * dim * min(dstate, 64) floats and a little more, which fits for any shape unless the
+ * caller pins the segments; one that pins 16 or 32 states per lane needs the packed B/C of the whole
+ * sequence).  All calls on one GPU share that GPU's array: calls that overlap
  * on one GPU (different streams or threads) race; calls on one stream are ordered.
  * The first call on a device looks up the array's address and raises the kernels' dynamic-LDS limit
  * (host calls that do not belong into a stream capture): make one call per device and kernel variant

@@ -987,13 +987,16 @@ static FwdPlan fwd_plan(const mpa_sscan_shape* s, int ns) {
     static constexpr int kCh[4] = {64, 48, 32, 16};
     static constexpr float kTileUs[4][3] = {{0.95f, 1.55f, 2.85f}, {0.90f, 0.90f, 0.90f}, {0.76f, 0.90f, 1.50f}, {0.51f, 0.62f, 0.98f}};
     static constexpr float kCutUs[4][3] = {{8.5f, 13.0f, 25.0f}, {0.0f, 0.0f, 0.0f}, {5.0f, 7.0f, 14.0f}, {4.5f, 8.0f, 13.0f}};
+    // (the static scratch of mpa_sscan_fwd_noalloc holds the states of any number of segments chosen here; the bound
+    // is met with 61 and more states by cuts into the last 5 % of 512 workgroups of 64 channels)
+    const int64_t fit = ((int64_t)MPA_NOALLOC_SCRATCH_BYTES - 512) / (4 * s->batch * s->dim * (2 * s->dstate + kTile / 4));
     int group = 64;
     int64_t nseg = 1;
     float best = 1e30f;
     for (int c = 0; c < 4; ++c) {
         if (kCh[c] == 48 && !form48) continue;
         const int64_t wg = s->batch * ((s->dim + kCh[c] - 1) / kCh[c]);
-        for (int64_t n = 1; n <= 64 && (n == 1 || (kCh[c] != 48 && n * 4 <= ntiles && wg * n <= 512)); ++n) {
+        for (int64_t n = 1; n <= 64 && (n == 1 || (kCh[c] != 48 && n * 4 <= ntiles && wg * n <= 512 && n <= fit)); ++n) {
             const float rounds = (float)((wg * n + 255) / 256);
             const float us = rounds * (float)((ntiles + n - 1) / n) * kTileUs[c][wide];
             const float total = n == 1 ? 5.0f + us : kCutUs[c][wide] + 0.65f * (float)n + 1.75f * us + 4.0f * (rounds - 1.0f);

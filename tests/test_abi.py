@@ -125,3 +125,22 @@ def test_launch_plan_reads_the_environment_once_in_python(pkg, monkeypatch):
     with pytest.raises(TypeError):
         with pkg.plan_override(nonsense=1):
             pass
+
+
+def test_noalloc_scratch_holds_every_plan_of_the_library(pkg):
+    """Whatever the library chooses by itself fits the static scratch of mpa_sscan_fwd_noalloc."""
+    import random
+    L = pkg._lib
+    lib = L.load()
+    rng = random.Random(5)
+    log = lambda lo, hi: int(round(lo * (hi / lo) ** rng.random()))
+    shapes = [(1, 16384, 1280, 64), (3, 4096, 832, 64), (1, 16384, 1280, 128), (1, 16384, 1280, 256), (1, 1 << 20, 32768, 64), (512, 4096, 64, 64)]
+    shapes += [(log(1, 64), log(1, 1 << 17), log(1, 16384), rng.choice([1, 4, 16, 17, 33, 60, 61, 63, 64, 65, 100, 128, 192, 256]))
+               for _ in range(20000)]
+    cut = 0
+    for batch, seqlen, dim, dstate in shapes:
+        s = L.SscanShape(batch=batch, seqlen=seqlen, dim=dim, dstate=dstate)
+        need = [lib.mpa_sscan_fwd_workspace_bytes(ctypes.byref(s), k) for k in (0, 1)]
+        assert 0 < max(need) <= L.MPA_NOALLOC_SCRATCH_BYTES, (batch, seqlen, dim, dstate, need)
+        cut += need[0] > 256
+    assert cut > 1000       # (calls that are cut are among them)
