@@ -190,24 +190,93 @@ struct Written {
     }
 };
 
-struct MixerHandle {
+struct LayerSizes {
+    int64_t d = 0, ED = 0, N = 0, R = 0, K = 0, Rp = 0;
+    at::ScalarType dt = at::kFloat;
+    c10::Device device{at::kCPU};
+    int64_t padded_rows() const { return Rp == R ? R + 2 * N : (Rp + 2 * N + 63) / 64 * 64; }
+};
+
+// The parameters of a mixer and the forms of them that the kernels take.  A call takes one along when it lets go of the
+// interpreter: handles change under the interpreter's lock, these not at all.
+struct Weights : LayerSizes {
+    Tensor p[kParams];
+    Tensor conv_w, conv_b, dt_b, D;              // float32
+    Tensor A;                                    // -exp(A_log), float32
+    Tensor in_wt, out_wt, xp, dtp, xp_t, dtp_t;  // (transposed views of) the GEMM weights
+
+    // x_proj and dt_proj in the shape the GEMM library serves best: the low-rank width R is the K of
+    // dt_proj and R + 2N the rows of x_proj, both odd for its tiles (48 and 80 at width 768).  With R
+    // rounded up to a multiple of 64 by zeros and the rows regrouped as [delta | 0 | B | C | 0], the two
+    // products take 21 + 26 us instead of 25 + 38 us at 32768 rows in bfloat16.
+    void pad_jobs(std::vector<mpa_cast_job>& jobs) const {
+        const Tensor &xw = p[kXW], &dw = p[kDtW];
+        jobs.push_back(cast_job(xw, xp, R, ED));
+        jobs.push_back(cast_job(xw, xp, 2 * N, ED, R * ED, Rp * ED));
+        jobs.push_back(cast_job(dw, dtp, ED, R));
+    }
+
+    // What a call with gradients takes in place of the kept forms: made in the call, on its stream, from the parameters
+    // as they are, and held by its graph node; one launch.
+    void form_for_training() {
+        const Tensor& w = p[kInW];
+        std::vector<mpa_cast_job> jobs;
+        auto f32 = [&](const Tensor& q) {
+            if (!q.defined() || q.scalar_type() == at::kFloat) return q.defined() ? q.detach() : q;
+            const Tensor t = empty(q.sizes(), at::kFloat, q);
+            jobs.push_back(row_job(q, t));
+            return t;
+        };
+        conv_w = f32(p[kConvW]);
+        conv_b = f32(p[kConvB]);
+        dt_b = f32(p[kDtB]);
+        D = f32(p[kD]);
+        A = empty({ED, N}, at::kFloat, w);
+        jobs.push_back(cast_job(p[kALog], A, ED, N, 0, 0, MPA_CAST_NEG_EXP));
+        if (Rp == R) {
+            xp = p[kXW].detach();
+            dtp = p[kDtW].detach();
+        } else {
+            const int64_t rows = padded_rows(), used = Rp + 2 * N;
+            xp = empty({rows, ED}, dt, w);
+            dtp = empty({ED, Rp}, dt, w);
+            pad_jobs(jobs);
+            jobs.push_back(zero_job(xp, Rp - R, ED, R * ED));
+            if (rows > used) jobs.push_back(zero_job(xp, rows - used, ED, used * ED));
+            jobs.push_back(zero_job(dtp, ED, Rp - R, R));
+        }
+        run_casts(jobs, w);
+    }
+
+    mpa_decode_layer desc(int64_t batch) const {
+        mpa_decode_layer s{};
+        s.batch = batch; s.d_model = d; s.dim = ED; s.dstate = N; s.dt_rank = R;
+        s.d_conv = (int)K;
+        s.io_dtype = dt == at::kFloat ? MPA_F32 : MPA_BF16;
+        s.in_weight = ptr(p[kInW]); s.in_bias = ptr(p[kInB]);
+        s.conv_weight = fptr(conv_w); s.conv_bias = fptr(conv_b);
+        s.x_weight = ptr(p[kXW]); s.dt_weight = ptr(p[kDtW]);
+        s.dt_bias = fptr(dt_b); s.A = fptr(A); s.D = fptr(D);
+        s.out_weight = ptr(p[kOutW]); s.out_bias = ptr(p[kOutB]);
+        return s;
+    }
+};
+
+struct MixerHandle : LayerSizes {
     bool decode_ok = false;   // the shapes are such as mpa_decode_layer_step takes
     bool forward_ok = false;  // ... as stack_forward and block_train take
     Ref modules;
     Ref sizes[7];  // values of the config, by Keys::sizes
     Param p[kParams];
-    int64_t d = 0, ED = 0, N = 0, R = 0, K = 0, Rp = 0;
     bool fused_softplus = true;
-    at::ScalarType dt = at::kFloat;
-    c10::Device device{at::kCPU};
     // Forms kept for calls without gradients, and the epoch they are of.  Version counters do not show every change
     // of a parameter (writes through .data), and a training loop makes one after each of its calls: a call with
-    // gradients forms its own (TrainForms) and begins an epoch.
+    // gradients forms its own and begins an epoch.
     uint64_t epoch = 1, formed = 0, padded = 0;  // padded: that of xp .. dtp_t
     Written written;
     F32 conv_w, conv_b, dt_b, D;
-    Tensor A;                                    // -exp(A_log), float32
-    Tensor in_wt, out_wt, xp, dtp, xp_t, dtp_t;  // (transposed views of) the GEMM weights
+    Tensor A, xp, dtp;  // (xp and dtp: where the layer's own shapes are padded)
+    std::shared_ptr<const Weights> kept;
 
     explicit MixerHandle(PyObject* dict) : modules(get(dict, keys().modules)) {}
     // the dictionaries are those of this block (a shallow copy brings the handle of its original along)
@@ -230,13 +299,11 @@ struct MixerHandle {
         const bool there = both(in, kInW, kInB, changed) && both(conv, kConvW, kConvB, changed) && both(xp, kXW, kXB, changed) &&
                            both(dtp, kDtW, kDtB, changed) && both(out, kOutW, kOutB, changed) && p[kALog].look(params, k.A_log, changed) &&
                            p[kD].look(params, k.D, changed);
-        if (changed) {
-            ++epoch;
-            decode_ok = forward_ok = false;
-            if (there) look_over();
-            else forget();
-        }
-        return there && (decode_ok || forward_ok) && x.scalar_type() == dt && x.device() == device && x.size(-1) == d;
+        if (changed) ++epoch;
+        if (changed && !there) forget();
+        decode_ok = forward_ok = false;
+        if (there) look_over();
+        return (decode_ok || forward_ok) && x.scalar_type() == dt && x.device() == device && x.size(-1) == d;
     }
     bool both(PyObject* dict, int weight, int bias, bool& changed) {
         PyObject* params = get(dict, keys().params);
@@ -262,6 +329,7 @@ struct MixerHandle {
             for (int i = 0; i < 7; ++i) sizes[i] = Ref(v[i]);
             Rp = (R + 63) / 64 * 64;
             fused_softplus = PyObject_IsTrue(sizes[6].o) == 1;
+            xp = dtp = Tensor();  // (their zeros are elsewhere)
         }
         return PyObject_IsTrue(sizes[5].o) == 0;
     }
@@ -297,110 +365,50 @@ struct MixerHandle {
         return t.device() == device && t.is_contiguous() && (t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16);
     }
 
-    // Brings the kept forms up to date, xp .. dtp_t among them for a sequence; after ready().  Within a capture nothing
+    Weights parameters() const {
+        Weights w;
+        static_cast<LayerSizes&>(w) = *this;
+        for (int i = 0; i < kParams; ++i) w.p[i] = p[i].t;
+        return w;
+    }
+
+    // The kept forms, up to date, xp .. dtp_t among them for a sequence; after ready().  Within a capture nothing
     // runs yet: the next call still finds them old.
-    void form(bool sequence) {
+    std::shared_ptr<const Weights> form(bool sequence) {
         const c10::Stream s = current_stream(device);
         written.before(s);
         const bool small = formed != epoch, wide = sequence && padded != epoch;
-        if (small) form_small();
-        if (wide) form_padded();
         if (small || wide) {
+            auto w = std::make_shared<Weights>(parameters());
+            std::vector<mpa_cast_job> jobs;
+            auto f32 = [&](F32& form, int i) {
+                if (small) form.take(p[i].t, jobs);
+                return form.t;
+            };
+            w->conv_w = f32(conv_w, kConvW);
+            w->conv_b = f32(conv_b, kConvB);
+            w->dt_b = f32(dt_b, kDtB);
+            w->D = f32(D, kD);
+            w->A = derived(A, {ED, N}, at::kFloat, w->p[kInW]);
+            if (small) jobs.push_back(cast_job(p[kALog].t, A, ED, N, 0, 0, MPA_CAST_NEG_EXP));
+            w->in_wt = w->p[kInW].detach().t();
+            w->out_wt = w->p[kOutW].detach().t();
+            if (sequence) {
+                const Tensor &xw = w->p[kXW], &dw = w->p[kDtW];
+                w->xp = Rp == R ? xw.detach() : derived(xp, {padded_rows(), ED}, dt, xw);
+                w->dtp = Rp == R ? dw.detach() : derived(dtp, {ED, Rp}, dt, dw);
+                w->xp_t = w->xp.t();
+                w->dtp_t = w->dtp.t();
+                if (wide && Rp != R) w->pad_jobs(jobs);
+            }
+            run_casts(jobs, w->p[kInW]);
+            kept = w;
             const uint64_t of = capturing() ? 0 : epoch;
             if (small) formed = of;
-            if (wide) padded = of;
+            padded = sequence ? of : 0;  // (xp .. dtp_t are not in `kept` otherwise)
         }
         written.after(s, small || wide, {&conv_w.own, &conv_b.own, &dt_b.own, &D.own, &A, &xp, &dtp});
-    }
-    void form_small() {
-        const Tensor& w = p[kInW].t;
-        std::vector<mpa_cast_job> jobs;
-        conv_w.take(p[kConvW].t, jobs);
-        conv_b.take(p[kConvB].t, jobs);
-        dt_b.take(p[kDtB].t, jobs);
-        D.take(p[kD].t, jobs);
-        derived(A, {ED, N}, at::kFloat, w);
-        jobs.push_back(cast_job(p[kALog].t, A, ED, N, 0, 0, MPA_CAST_NEG_EXP));
-        run_casts(jobs, w);
-        in_wt = p[kInW].t.detach().t();
-        out_wt = p[kOutW].t.detach().t();
-    }
-
-    // x_proj and dt_proj in the shape the GEMM library serves best: the low-rank width R is the K of
-    // dt_proj and R + 2N the rows of x_proj, both odd for its tiles (48 and 80 at width 768).  With R
-    // rounded up to a multiple of 64 by zeros and the rows regrouped as [delta | 0 | B | C | 0], the two
-    // products take 21 + 26 us instead of 25 + 38 us at 32768 rows in bfloat16.
-    int64_t padded_rows() const { return Rp == R ? R + 2 * N : (Rp + 2 * N + 63) / 64 * 64; }
-    void pad_jobs(const Tensor& xp, const Tensor& dtp, std::vector<mpa_cast_job>& jobs) const {
-        const Tensor &xw = p[kXW].t, &dw = p[kDtW].t;
-        jobs.push_back(cast_job(xw, xp, R, ED));
-        jobs.push_back(cast_job(xw, xp, 2 * N, ED, R * ED, Rp * ED));
-        jobs.push_back(cast_job(dw, dtp, ED, R));
-    }
-    void form_padded() {
-        const Tensor &xw = p[kXW].t, &dw = p[kDtW].t;
-        if (Rp == R) {
-            xp = xw.detach();
-            dtp = dw.detach();
-        } else {
-            derived(xp, {padded_rows(), ED}, dt, xw);
-            derived(dtp, {ED, Rp}, dt, dw);
-            std::vector<mpa_cast_job> jobs;
-            pad_jobs(xp, dtp, jobs);
-            run_casts(jobs, xw);
-        }
-        xp_t = xp.t();
-        dtp_t = dtp.t();
-    }
-
-    // What a call with gradients takes in place of the kept forms: made in the call, on its stream, from the parameters
-    // as they are, and held by its graph node; one launch.
-    struct TrainForms {
-        Tensor A, D, dt_b, conv_w, conv_b, xp, dtp;
-    };
-    TrainForms train_forms() const {
-        const Tensor& w = p[kInW].t;
-        TrainForms f;
-        std::vector<mpa_cast_job> jobs;
-        auto f32 = [&](const Tensor& q) {
-            if (!q.defined() || q.scalar_type() == at::kFloat) return q.defined() ? q.detach() : q;
-            const Tensor t = empty(q.sizes(), at::kFloat, q);
-            jobs.push_back(row_job(q, t));
-            return t;
-        };
-        f.conv_w = f32(p[kConvW].t);
-        f.conv_b = f32(p[kConvB].t);
-        f.dt_b = f32(p[kDtB].t);
-        f.D = f32(p[kD].t);
-        f.A = empty({ED, N}, at::kFloat, w);
-        jobs.push_back(cast_job(p[kALog].t, f.A, ED, N, 0, 0, MPA_CAST_NEG_EXP));
-        if (Rp == R) {
-            f.xp = p[kXW].t.detach();
-            f.dtp = p[kDtW].t.detach();
-        } else {
-            const int64_t rows = padded_rows(), used = Rp + 2 * N;
-            f.xp = empty({rows, ED}, dt, w);
-            f.dtp = empty({ED, Rp}, dt, w);
-            pad_jobs(f.xp, f.dtp, jobs);
-            jobs.push_back(zero_job(f.xp, Rp - R, ED, R * ED));
-            if (rows > used) jobs.push_back(zero_job(f.xp, rows - used, ED, used * ED));
-            jobs.push_back(zero_job(f.dtp, ED, Rp - R, R));
-        }
-        run_casts(jobs, w);
-        return f;
-    }
-
-    mpa_decode_layer desc(int64_t batch) const {
-        mpa_decode_layer s{};
-        s.batch = batch; s.d_model = d; s.dim = ED; s.dstate = N; s.dt_rank = R;
-        s.d_conv = (int)K;
-        s.io_dtype = dt == at::kFloat ? MPA_F32 : MPA_BF16;
-        s.in_weight = p[kInW].data; s.in_bias = p[kInB].data;
-        s.conv_weight = fptr(conv_w.t); s.conv_bias = fptr(conv_b.t);
-        s.x_weight = p[kXW].data; s.dt_weight = p[kDtW].data;
-        s.dt_bias = fptr(dt_b.t); s.A = fptr(A); s.D = fptr(D.t);
-        s.out_weight = p[kOutW].data; s.out_bias = p[kOutB].data;
-        return s;
+        return kept;
     }
 };
 
@@ -435,7 +443,7 @@ struct NormHandle {
         const Tensor& t = p.t;
         return !t.defined() || (t.numel() == m.d && MixerHandle::small_ok(t, m.device) && reinterpret_cast<uintptr_t>(p.data) % 16 == 0);
     }
-    void form(const MixerHandle& m) {
+    Tensor form(const MixerHandle& m) {
         const c10::Stream s = current_stream(m.device);
         written.before(s);
         const bool old = changed || formed != m.epoch;
@@ -447,6 +455,7 @@ struct NormHandle {
             formed = capturing() ? 0 : m.epoch;
         }
         written.after(s, old, {&w.own});
+        return w.t;
     }
 };
 

@@ -21,15 +21,72 @@ bool read_cache(PyObject* pair, Cache& c) {
     c.window = THPVariable_Unpack(w);
     return true;
 }
-bool cache_fits(const Cache& c, const MixerHandle& l, int64_t batch, bool need_h) {
+bool cache_fits(const Cache& c, const LayerSizes& l, int64_t batch, bool need_h) {
     if (!c.h.defined() ? need_h : !fits(c.h, {batch, l.ED, l.N}, at::kFloat, l.device)) return false;
     return c.window.scalar_type() == l.dt && c.window.device() == l.device && c.window.is_contiguous() &&
            c.window.sizes() == at::IntArrayRef({batch, l.ED, l.K - 1});
 }
 
+// What a layer's kernels read.
+struct LayerWeights {
+    std::shared_ptr<const Weights> m;
+    Tensor norm_w;
+    double eps = 0;
+};
+
 py::object pair(const Tensor& h, const Tensor& w) { return py::make_tuple(h, w); }
 
 // ---- decode -------------------------------------------------------------------------------------
+
+// The launches of a step, without the interpreter's lock; `cs` becomes the caches after it.
+Tensor run_steps(const std::vector<LayerWeights>& layers, const Tensor& x, std::vector<Cache>& cs, bool inplace) {
+    const size_t n = layers.size();
+    const int64_t batch = x.size(0);
+    std::vector<mpa_decode_layer> desc(n);
+    for (size_t i = 0; i < n; ++i) {
+        desc[i] = layers[i].m->desc(batch);
+        desc[i].norm = 1;
+        desc[i].eps = (float)layers[i].eps;
+        desc[i].norm_weight = fptr(layers[i].norm_w);
+    }
+    const auto dt = x.scalar_type();
+    const int64_t d = x.size(1);
+    // two rows per sequence and two scaled rows, used in turn (a kernel never writes what it reads), with
+    // the partial sums of squares of the latter
+    const int64_t tiles = (d + 15) / 16;
+    const size_t scaled_bytes = mpa_decode_scaled_bytes(&desc[0]);
+    const Tensor spare = empty({batch, d}, dt, x), y = empty({batch, d}, dt, x), scaled_rows = scratch(2 * scaled_bytes, x),
+                 ssq = empty({2, tiles * batch}, at::kFloat, x);
+    size_t ws_bytes = 0;
+    for (const mpa_decode_layer& s : desc) ws_bytes = std::max(ws_bytes, mpa_decode_layer_workspace_bytes(&s));
+    const Tensor ws = scratch(ws_bytes, x);
+    void* stream = stream_of(x);
+    // the last layer writes y, the others y and a spare row in turn
+    const void* in = ptr(x);
+    const void* scaled = nullptr;
+    const float* sums = nullptr;
+    for (size_t i = 0; i < n; ++i) {
+        const Weights& l = *layers[i].m;
+        Cache out = cs[i];
+        if (!inplace) {
+            out.h = empty({batch, l.ED, l.N}, at::kFloat, x);
+            out.window = empty({batch, l.ED, l.K - 1}, dt, x);
+        }
+        void* to = (n - 1 - i) % 2 == 0 ? ptr(y) : ptr(spare);
+        // (a norm without a weight has nothing to scale by: the next layer forms its own sums)
+        const float* next_w = i + 1 < n ? desc[i + 1].norm_weight : nullptr;
+        void* to_scaled = static_cast<char*>(ptr(scaled_rows)) + (i % 2) * scaled_bytes;
+        float* to_sums = fptr(ssq) + (i % 2) * tiles * batch;
+        check(mpa_decode_layer_step(&desc[i], in, scaled, sums, to, next_w, to_scaled, to_sums, fptr(cs[i].h), fptr(out.h), ptr(cs[i].window),
+                                    ptr(out.window), ptr(ws), ws_bytes, stream),
+              "mpa_decode_layer_step");
+        in = to;
+        scaled = next_w ? to_scaled : nullptr;
+        sums = next_w ? to_sums : nullptr;
+        cs[i] = out;
+    }
+    return y;
+}
 
 // One token through the residual blocks `layers`; the caches are updated in place or replaced in the
 // list.  None: not a stack that can run here (the caller goes on in Python).
@@ -49,51 +106,15 @@ py::object stack_step(const py::list& layers, const Tensor& x_in, const py::list
     }
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
-    std::vector<mpa_decode_layer> desc(n);
-    for (size_t i = 0; i < n; ++i) {
-        hs[i].m->form(false);
-        hs[i].n->form(*hs[i].m);
-        desc[i] = hs[i].m->desc(batch);
-        desc[i].norm = 1;
-        desc[i].eps = (float)hs[i].n->eps;
-        desc[i].norm_weight = fptr(hs[i].n->w.t);
+    std::vector<LayerWeights> ws(n);
+    for (size_t i = 0; i < n; ++i) ws[i] = {hs[i].m->form(false), hs[i].n->form(*hs[i].m), hs[i].n->eps};
+    Tensor y;
+    {
+        const py::gil_scoped_release nogil;
+        y = run_steps(ws, x, cs, inplace);
     }
-    const auto dt = x.scalar_type();
-    const int64_t d = x.size(1);
-    // two rows per sequence and two scaled rows, used in turn (a kernel never writes what it reads), with
-    // the partial sums of squares of the latter
-    const int64_t tiles = (d + 15) / 16;
-    const size_t scaled_bytes = mpa_decode_scaled_bytes(&desc[0]);
-    const Tensor spare = empty({batch, d}, dt, x), y = empty({batch, d}, dt, x), scaled_rows = scratch(2 * scaled_bytes, x),
-                 ssq = empty({2, tiles * batch}, at::kFloat, x);
-    size_t ws_bytes = 0;
-    for (const mpa_decode_layer& s : desc) ws_bytes = std::max(ws_bytes, mpa_decode_layer_workspace_bytes(&s));
-    const Tensor ws = scratch(ws_bytes, x);
-    void* stream = stream_of(x);
-    // the last layer writes y, the others y and a spare row in turn
-    const void* in = ptr(x);
-    const void* scaled = nullptr;
-    const float* sums = nullptr;
-    for (size_t i = 0; i < n; ++i) {
-        const MixerHandle& l = *hs[i].m;
-        Cache out = cs[i];
-        if (!inplace) {
-            out.h = empty({batch, l.ED, l.N}, at::kFloat, x);
-            out.window = empty({batch, l.ED, l.K - 1}, dt, x);
-        }
-        void* to = (n - 1 - i) % 2 == 0 ? ptr(y) : ptr(spare);
-        // (a norm without a weight has nothing to scale by: the next layer forms its own sums)
-        const float* next_w = i + 1 < n ? desc[i + 1].norm_weight : nullptr;
-        void* to_scaled = static_cast<char*>(ptr(scaled_rows)) + (i % 2) * scaled_bytes;
-        float* to_sums = fptr(ssq) + (i % 2) * tiles * batch;
-        check(mpa_decode_layer_step(&desc[i], in, scaled, sums, to, next_w, to_scaled, to_sums, fptr(cs[i].h), fptr(out.h), ptr(cs[i].window),
-                                    ptr(out.window), ptr(ws), ws_bytes, stream),
-              "mpa_decode_layer_step");
-        in = to;
-        scaled = next_w ? to_scaled : nullptr;
-        sums = next_w ? to_sums : nullptr;
-        if (!inplace) caches[i] = pair(out.h, out.window);
-    }
+    if (!inplace)
+        for (size_t i = 0; i < n; ++i) caches[i] = pair(cs[i].h, cs[i].window);
     return py::cast(y);
 }
 
@@ -109,52 +130,32 @@ py::object block_step(const py::object& block, const Tensor& x_in, const Opt& h_
     if (!l || !l->decode_ok || !cache_fits(in, *l, batch, inplace)) return py::none();
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
-    l->form(false);
+    const std::shared_ptr<const Weights> w = l->form(false);
+    py::gil_scoped_release nogil;
     Cache out = in;
     if (!inplace) {
-        out.h = empty({batch, l->ED, l->N}, at::kFloat, x);
-        out.window = empty({batch, l->ED, l->K - 1}, x.scalar_type(), x);
+        out.h = empty({batch, w->ED, w->N}, at::kFloat, x);
+        out.window = empty({batch, w->ED, w->K - 1}, x.scalar_type(), x);
     }
-    const Tensor y = empty({batch, l->d}, x.scalar_type(), x);
-    const mpa_decode_layer s = l->desc(batch);
+    const Tensor y = empty({batch, w->d}, x.scalar_type(), x);
+    const mpa_decode_layer s = w->desc(batch);
     const size_t nbytes = mpa_decode_layer_workspace_bytes(&s);
     const Tensor ws = scratch(nbytes, x);
     check(mpa_decode_layer_step(&s, ptr(x), nullptr, nullptr, ptr(y), nullptr, nullptr, nullptr, fptr(in.h), fptr(out.h), ptr(in.window),
                                 ptr(out.window), ptr(ws), nbytes, stream_of(x)),
           "mpa_decode_layer_step");
+    const py::gil_scoped_acquire gil;
     return py::make_tuple(y, out.h, out.window);
 }
 
 // ---- forward without gradients ------------------------------------------------------------------
 
-// A sequence through the residual blocks: (y, list of caches or None), or None.  The activations of a
-// layer live in buffers that every layer uses again.
-py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::object& caches, bool return_caches,
-                         const PackedPlan& packed) {
-    const size_t n = layers.size();
-    if (at::GradMode::is_enabled() || !native_call(x_in) || x_in.dim() != 3 || n == 0 || x_in.numel() == 0) return py::none();
-    const int64_t Bs = x_in.size(0), L = x_in.size(1), T = Bs * L;
-    std::vector<Layer> hs(n);
-    std::vector<Cache> cs(n);
-    at::AutoDispatchBelowADInplaceOrView below;
-    const c10::DeviceGuard guard(x_in.device());
-    for (size_t i = 0; i < n; ++i) {
-        if (!find_layer(layers[i].ptr(), x_in, hs[i]) || !hs[i].m->forward_ok) return py::none();
-        const MixerHandle &l = *hs[i].m, &a = *hs[0].m;
-        if (l.d != a.d || l.ED != a.ED || l.N != a.N || l.Rp != a.Rp || l.padded_rows() != a.padded_rows()) return py::none();
-        if (!caches.is_none()) {
-            const py::object c = caches[py::int_(i)];
-            if (!read_cache(c.ptr(), cs[i]) || !cache_fits(cs[i], l, Bs, false)) return py::none();
-        }
-    }
-    const Plan plan = unpack(packed);
-    const MixerHandle& a = *hs[0].m;
-    const Tensor x = x_in.contiguous();
-    if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
-    for (const Layer& l : hs) {
-        l.m->form(true);
-        l.n->form(*l.m);
-    }
+// The launches of a sequence, without the interpreter's lock; with `keep`, `cs` becomes the caches after it.
+// The activations of a layer live in buffers that every layer uses again.
+Tensor run_sequence(const std::vector<LayerWeights>& hs, const Tensor& x, std::vector<Cache>& cs, bool keep, const Plan& plan) {
+    const size_t n = hs.size();
+    const int64_t Bs = x.size(0), L = x.size(1), T = Bs * L;
+    const Weights& a = *hs[0].m;
     const auto dt = x.scalar_type();
     const int io = io_dtype(dt);
     const int64_t d = a.d, ED = a.ED, N = a.N, P = a.xp.size(0);
@@ -165,9 +166,9 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
     Tensor sum[2];
     if (n > 1) { sum[0] = empty({T, d}, dt, x); sum[1] = empty({T, d}, dt, x); }
     bool own = use_linear(dt, T, d, ED, P, {&x});
-    for (const auto& [norm, l] : hs)
-        own &= norm->w.t.defined() &&
-               use_linear(dt, T, d, ED, P, {&l->p[kInW].t, &l->p[kOutW].t, &l->xp, &l->dtp, &norm->w.t, &l->p[kInB].t, &l->p[kOutB].t});
+    for (const LayerWeights& h : hs)
+        own &= h.norm_w.defined() &&
+               use_linear(dt, T, d, ED, P, {&h.m->p[kInW], &h.m->p[kOutW], &h.m->xp, &h.m->dtp, &h.norm_w, &h.m->p[kInB], &h.m->p[kOutB]});
     const int64_t parts = (d + 31) / 32;
     const Tensor ssq = own ? empty({parts, T}, at::kFloat, x) : Tensor();
     auto linear = [&](const void* in, int64_t pitch, int64_t K, const Tensor& weight, const Tensor& bias, const Tensor& out) {
@@ -196,14 +197,13 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
     const size_t ws_bytes = mpa_sscan_fwd_workspace_bytes(&sc, 0);
     const Tensor ws = scratch(ws_bytes, x);
 
-    py::list new_caches;
     const Tensor result = own ? empty({Bs, L, d}, dt, x) : Tensor();
     const void* in = ptr(x);
     const void* residual = nullptr;
     for (size_t i = 0; i < n; ++i) {
-        const MixerHandle& l = *hs[i].m;
-        const float* norm_w = fptr(hs[i].n->w.t);
-        const float eps = (float)hs[i].n->eps;
+        const Weights& l = *hs[i].m;
+        const float* norm_w = fptr(hs[i].norm_w);
+        const float eps = (float)hs[i].eps;
         const Tensor& s = sum[i % 2];
         if (!own || i == 0)
             check(mpa_rmsnorm_fwd(in, residual, norm_w, ptr(normed), residual ? ptr(s) : nullptr, nullptr, T, d, eps, io, stream),
@@ -211,21 +211,21 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
         if (!own) residual = residual ? ptr(s) : in;
         Tensor out = xz;
         if (own) {
-            mpa_linear q = linear(i == 0 ? ptr(normed) : ptr(sum[(i - 1) % 2]), d, d, l.p[kInW].t, l.p[kInB].t, xz);
+            mpa_linear q = linear(i == 0 ? ptr(normed) : ptr(sum[(i - 1) % 2]), d, d, l.p[kInW], l.p[kInB], xz);
             if (i > 0) { q.norm_weight = norm_w; q.x_ssq = fptr(ssq); q.ssq_parts = parts; q.eps = eps; }
             run(q);
-        } else if (l.p[kInB].t.defined()) {
-            at::addmm_out(out, l.p[kInB].t.detach(), normed, l.in_wt);
+        } else if (l.p[kInB].defined()) {
+            at::addmm_out(out, l.p[kInB].detach(), normed, l.in_wt);
         } else {
             at::mm_out(out, normed, l.in_wt);
         }
         Tensor window, h_last;
-        if (return_caches) {
+        if (keep) {
             window = empty({Bs, ED, l.K - 1}, dt, x);
             h_last = empty({Bs, ED, N}, at::kFloat, x);
         }
         cv.kernel = (int)l.K;
-        check(mpa_conv1d_fwd(&cv, ptr(xz), fptr(l.conv_w.t), fptr(l.conv_b.t), ptr(cs[i].window), ptr(xs), ptr(window), stream),
+        check(mpa_conv1d_fwd(&cv, ptr(xz), fptr(l.conv_w), fptr(l.conv_b), ptr(cs[i].window), ptr(xs), ptr(window), stream),
               "mpa_conv1d_fwd");
         if (own) {
             run(linear(ptr(xs), ED, ED, l.xp, Tensor(), dbc));
@@ -237,28 +237,61 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
             at::mm_out(out, dlow, l.dtp_t);
         }
         const char* bc = static_cast<const char*>(ptr(dbc)) + l.Rp * es;
-        check(mpa_sscan_fwd(&sc, ptr(xs), ptr(delta), fptr(l.A), bc, bc + N * es, fptr(l.D.t), static_cast<const char*>(ptr(xz)) + ED * es,
-                            fptr(l.dt_b.t), fptr(cs[i].h), ptr(y), nullptr, nullptr, fptr(h_last), ptr(ws), ws_bytes, stream),
+        check(mpa_sscan_fwd(&sc, ptr(xs), ptr(delta), fptr(l.A), bc, bc + N * es, fptr(l.D), static_cast<const char*>(ptr(xz)) + ED * es,
+                            fptr(l.dt_b), fptr(cs[i].h), ptr(y), nullptr, nullptr, fptr(h_last), ptr(ws), ws_bytes, stream),
               "mpa_sscan_fwd");
         out = hidden;
         if (own) {
             const bool last = i + 1 == n;
-            mpa_linear q = linear(ptr(y), ED, ED, l.p[kOutW].t, l.p[kOutB].t, last ? result : s);
+            mpa_linear q = linear(ptr(y), ED, ED, l.p[kOutW], l.p[kOutB], last ? result : s);
             q.residual = i == 0 ? ptr(x) : ptr(sum[(i - 1) % 2]);
             if (!last) q.y_ssq = fptr(ssq);
             run(q);
-        } else if (l.p[kOutB].t.defined()) {
-            at::addmm_out(out, l.p[kOutB].t.detach(), y, l.out_wt);
+        } else if (l.p[kOutB].defined()) {
+            at::addmm_out(out, l.p[kOutB].detach(), y, l.out_wt);
         } else {
             at::mm_out(out, y, l.out_wt);
         }
         in = ptr(hidden);
-        if (return_caches) new_caches.append(pair(h_last, window));
+        if (keep) cs[i] = {h_last, window};
     }
-    const py::object kept = return_caches ? py::object(new_caches) : py::object(py::none());
-    if (own) return py::make_tuple(result, kept);
+    if (own) return result;
     const Tensor last = n > 1 ? sum[(n - 1) % 2] : x.view({T, d});
-    return py::make_tuple(at::add(hidden, last).view({Bs, L, d}), kept);
+    return at::add(hidden, last).view({Bs, L, d});
+}
+
+// A sequence through the residual blocks: (y, list of caches or None), or None.
+py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::object& caches, bool return_caches,
+                         const PackedPlan& packed) {
+    const size_t n = layers.size();
+    if (at::GradMode::is_enabled() || !native_call(x_in) || x_in.dim() != 3 || n == 0 || x_in.numel() == 0) return py::none();
+    const int64_t Bs = x_in.size(0);
+    std::vector<Layer> hs(n);
+    std::vector<Cache> cs(n);
+    at::AutoDispatchBelowADInplaceOrView below;
+    const c10::DeviceGuard guard(x_in.device());
+    for (size_t i = 0; i < n; ++i) {
+        if (!find_layer(layers[i].ptr(), x_in, hs[i]) || !hs[i].m->forward_ok) return py::none();
+        const MixerHandle &l = *hs[i].m, &a = *hs[0].m;
+        if (l.d != a.d || l.ED != a.ED || l.N != a.N || l.Rp != a.Rp || l.padded_rows() != a.padded_rows()) return py::none();
+        if (!caches.is_none()) {
+            const py::object c = caches[py::int_(i)];
+            if (!read_cache(c.ptr(), cs[i]) || !cache_fits(cs[i], l, Bs, false)) return py::none();
+        }
+    }
+    const Tensor x = x_in.contiguous();
+    if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
+    std::vector<LayerWeights> ws(n);
+    for (size_t i = 0; i < n; ++i) ws[i] = {hs[i].m->form(true), hs[i].n->form(*hs[i].m), hs[i].n->eps};
+    Tensor y;
+    {
+        const py::gil_scoped_release nogil;
+        y = run_sequence(ws, x, cs, return_caches, unpack(packed));
+    }
+    if (!return_caches) return py::make_tuple(y, py::none());
+    py::list after;
+    for (const Cache& c : cs) after.append(pair(c.h, c.window));
+    return py::make_tuple(y, after);
 }
 
 }  // namespace

@@ -62,32 +62,10 @@ mpa_conv_shape mixer_conv_shape(const MixerBackward& m, int io, bool backward) {
     return s;
 }
 
-// (y, h_last or None, window or None), or None: not a block that can run here
-py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h_in, const Opt& win_in, bool return_cache,
-                       const PackedPlan& packed) {
-    if (!at::GradMode::is_enabled() || !native_call(x_in) || x_in.dim() != 3 || x_in.numel() == 0) return py::none();
-    MixerHandle* l = nullptr;
-    const Tensor hc = val(h_in), wc = val(win_in);
-    {
-        at::AutoDispatchBelowADInplaceOrView below;
-        const c10::DeviceGuard guard(x_in.device());
-        l = ready_mixer(block.ptr(), x_in);
-        if (!l || !l->forward_ok || l->N % 4) return py::none();
-        if (unpack(packed).flags & MPA_PLAN_BWD_GENERAL) return py::none();
-        const int64_t Bs = x_in.size(0);
-        if (hc.defined() && !fits(hc, {Bs, l->ED, l->N}, at::kFloat, l->device)) return py::none();
-        if (wc.defined() && !fits(wc, {Bs, l->ED, l->K - 1}, l->dt, l->device)) return py::none();
-    }
-    const std::array<int, kInputs> from = {-1, kInW, kInB, kConvW, kConvB, kXW, kDtW, kDtB, kALog, kD, kOutW, kOutB};
-    const Tensor none;
-    std::array<const Tensor*, kInputs> in;
-    in[kIX] = &x_in;
-    bool any = x_in.requires_grad();
-    for (int i = 1; i < kInputs; ++i) {
-        in[i] = &l->p[from[i]].t;
-        any |= in[i]->defined() && in[i]->requires_grad();
-    }
-    if (!any) return py::none();
+// The forward pass and its node; (y, h_last, window), the latter two if asked for.  Runs without the interpreter's lock.
+std::tuple<Tensor, Tensor, Tensor> mixer_forward(Weights& l, const std::array<const Tensor*, kInputs>& in, const Tensor& hc, const Tensor& wc,
+                                                 bool return_cache, const Plan& plan) {
+    const Tensor& x_in = *in[kIX];
     auto node = make_node<MixerBackward>({in[0], in[1], in[2], in[3], in[4], in[5], in[6], in[7], in[8], in[9], in[10], in[11]});
     Tensor x, out, h_last, window, t[kSaved];
     {
@@ -98,14 +76,14 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
         const auto dt = x.scalar_type();
         const int io = io_dtype(dt);
         const size_t es = x.element_size();
-        m.Bs = x.size(0); m.L = x.size(1); m.d = l->d; m.ED = l->ED; m.N = l->N; m.R = l->R; m.Rp = l->Rp; m.K = l->K;
-        m.P = l->padded_rows();
-        m.plan = unpack(packed);
-        const MixerHandle::TrainForms f = l->train_forms();
+        m.Bs = x.size(0); m.L = x.size(1); m.d = l.d; m.ED = l.ED; m.N = l.N; m.R = l.R; m.Rp = l.Rp; m.K = l.K;
+        m.P = l.padded_rows();
+        m.plan = plan;
+        l.form_for_training();
         const int64_t T = m.Bs * m.L, ED = m.ED, N = m.N, P = m.P;
         const Tensor x2 = x.view({T, m.d});
         void* stream = stream_of(x);
-        const bool own = use_linear(dt, T, m.d, ED, P, {&x, &l->p[kInW].t, &l->p[kOutW].t, &f.xp, &f.dtp, &l->p[kInB].t, &l->p[kOutB].t});
+        const bool own = use_linear(dt, T, m.d, ED, P, {&x, &l.p[kInW], &l.p[kOutW], &l.xp, &l.dtp, &l.p[kInB], &l.p[kOutB]});
         auto product = [&](const Tensor& in, int64_t K, const Tensor& weight, const Tensor& bias) {
             const int64_t M = weight.size(0);
             const Tensor y = empty({T, M}, dt, x);
@@ -114,30 +92,30 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
             run_linear(q, stream);
             return y;
         };
-        const Tensor xz = own ? product(x2, m.d, l->p[kInW].t, l->p[kInB].t)
-                          : l->p[kInB].t.defined() ? at::addmm(l->p[kInB].t, x2, l->p[kInW].t.t()) : at::mm(x2, l->p[kInW].t.t());
+        const Tensor xz = own ? product(x2, m.d, l.p[kInW], l.p[kInB])
+                          : l.p[kInB].defined() ? at::addmm(l.p[kInB], x2, l.p[kInW].t()) : at::mm(x2, l.p[kInW].t());
         const Tensor xs = empty({T, ED}, dt, x);
         if (return_cache) {
             window = empty({m.Bs, ED, m.K - 1}, dt, x);
             h_last = empty({m.Bs, ED, N}, at::kFloat, x);
         }
         const mpa_conv_shape cv = mixer_conv_shape(m, io, false);
-        check(mpa_conv1d_fwd(&cv, ptr(xz), fptr(f.conv_w), fptr(f.conv_b), ptr(wc), ptr(xs), ptr(window), stream), "mpa_conv1d_fwd");
-        const Tensor dbc = own ? product(xs, ED, f.xp, Tensor()) : at::mm(xs, f.xp.t());
-        const Tensor delta = own ? product(dbc, m.Rp, f.dtp, Tensor()) : at::mm(dbc.narrow(1, 0, m.Rp), f.dtp.t());
+        check(mpa_conv1d_fwd(&cv, ptr(xz), fptr(l.conv_w), fptr(l.conv_b), ptr(wc), ptr(xs), ptr(window), stream), "mpa_conv1d_fwd");
+        const Tensor dbc = own ? product(xs, ED, l.xp, Tensor()) : at::mm(xs, l.xp.t());
+        const Tensor delta = own ? product(dbc, m.Rp, l.dtp, Tensor()) : at::mm(dbc.narrow(1, 0, m.Rp), l.dtp.t());
         const Tensor y = empty({T, ED}, dt, x), y_pre = empty({T, ED}, dt, x);
         const mpa_sscan_shape sc = mixer_scan_shape(m, io, false);
         const Tensor ckpt = empty({mpa_sscan_ckpt_elems(&sc)}, at::kFloat, x);
         const size_t nbytes = mpa_sscan_fwd_workspace_bytes(&sc, 1);
         const Tensor ws = scratch(nbytes, x);
         const char* bc = static_cast<const char*>(ptr(dbc)) + m.Rp * es;
-        check(mpa_sscan_fwd(&sc, ptr(xs), ptr(delta), fptr(f.A), bc, bc + N * es, fptr(f.D), static_cast<const char*>(ptr(xz)) + ED * es,
-                            fptr(f.dt_b), fptr(hc), ptr(y), ptr(y_pre), fptr(ckpt), fptr(h_last), ptr(ws), nbytes, stream),
+        check(mpa_sscan_fwd(&sc, ptr(xs), ptr(delta), fptr(l.A), bc, bc + N * es, fptr(l.D), static_cast<const char*>(ptr(xz)) + ED * es,
+                            fptr(l.dt_b), fptr(hc), ptr(y), ptr(y_pre), fptr(ckpt), fptr(h_last), ptr(ws), nbytes, stream),
               "mpa_sscan_fwd");
-        out = (own ? product(y, ED, l->p[kOutW].t, l->p[kOutB].t)
-               : l->p[kOutB].t.defined() ? at::addmm(l->p[kOutB].t, y, l->p[kOutW].t.t()) : at::mm(y, l->p[kOutW].t.t())).view({m.Bs, m.L, m.d});
-        const std::array<const Tensor*, kSaved> made = {&wc, &hc, &xz, &xs, &dbc, &delta, &y, &y_pre, &ckpt, &f.A, &f.D, &f.dt_b, &f.conv_w,
-                                                        &f.conv_b, &f.xp, &f.dtp};
+        out = (own ? product(y, ED, l.p[kOutW], l.p[kOutB])
+               : l.p[kOutB].defined() ? at::addmm(l.p[kOutB], y, l.p[kOutW].t()) : at::mm(y, l.p[kOutW].t())).view({m.Bs, m.L, m.d});
+        const std::array<const Tensor*, kSaved> made = {&wc, &hc, &xz, &xs, &dbc, &delta, &y, &y_pre, &ckpt, &l.A, &l.D, &l.dt_b, &l.conv_w,
+                                                        &l.conv_b, &l.xp, &l.dtp};
         for (int i = 0; i < kSaved; ++i) t[i] = *made[i];
     }
     // (outside of the guard: hooks on saved tensors are called here)
@@ -145,6 +123,40 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
     for (int i = 1; i < kInputs; ++i) node->inputs[i] = keep(*in[i]);
     for (int i = 0; i < kSaved; ++i) node->saved[i] = keep(t[i]);
     torch::autograd::set_history(out, node);
+    return {out, h_last, window};
+}
+
+// (y, h_last or None, window or None), or None: not a block that can run here
+py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h_in, const Opt& win_in, bool return_cache,
+                       const PackedPlan& packed) {
+    if (!at::GradMode::is_enabled() || !native_call(x_in) || x_in.dim() != 3 || x_in.numel() == 0) return py::none();
+    Weights l;
+    const Tensor hc = val(h_in), wc = val(win_in);
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::DeviceGuard guard(x_in.device());
+        MixerHandle* handle = ready_mixer(block.ptr(), x_in);
+        if (!handle || !handle->forward_ok || handle->N % 4) return py::none();
+        if (unpack(packed).flags & MPA_PLAN_BWD_GENERAL) return py::none();
+        l = handle->parameters();
+        const int64_t Bs = x_in.size(0);
+        if (hc.defined() && !fits(hc, {Bs, l.ED, l.N}, at::kFloat, l.device)) return py::none();
+        if (wc.defined() && !fits(wc, {Bs, l.ED, l.K - 1}, l.dt, l.device)) return py::none();
+    }
+    const std::array<int, kInputs> from = {-1, kInW, kInB, kConvW, kConvB, kXW, kDtW, kDtB, kALog, kD, kOutW, kOutB};
+    std::array<const Tensor*, kInputs> in;
+    in[kIX] = &x_in;
+    bool any = x_in.requires_grad();
+    for (int i = 1; i < kInputs; ++i) {
+        in[i] = &l.p[from[i]];
+        any |= in[i]->defined() && in[i]->requires_grad();
+    }
+    if (!any) return py::none();
+    Tensor out, h_last, window;
+    {
+        const py::gil_scoped_release nogil;
+        std::tie(out, h_last, window) = mixer_forward(l, in, hc, wc, return_cache, unpack(packed));
+    }
     return py::make_tuple(out, return_cache ? py::cast(h_last) : py::object(py::none()),
                           return_cache ? py::cast(window) : py::object(py::none()));
 }

@@ -6,6 +6,7 @@ backward is called from the autograd engine's own thread (mambapy/pscan.py:151-2
 wait for nothing itself, and give the same bits when several host threads call it at once.
 All streams here have the default priority."""
 import threading
+import time
 
 import pytest
 import torch
@@ -172,3 +173,96 @@ def test_forward_backward_captured_in_a_hip_graph(pkg, dev, gated):
         torch.cuda.synchronize()
         for i, (a, b) in enumerate(zip(got, want)):
             assert torch.equal(a, b), (rep, i)
+
+
+def test_layer_calls_let_other_threads_run(pkg, dev):
+    """The interpreter is free while a stack's launches are enqueued: another thread runs in the middle of a native call.
+    (Threads hand it over on their own at most once in ten seconds here.)"""
+    import sys
+    torch.manual_seed(9)
+    m = pkg.Mamba(pkg.MambaConfig(d_model=64, n_layers=24)).to(dev)
+    x = torch.randn(2, 40, 64, device=dev)
+    caches = m.empty_caches(2)
+    layers, mixer, host, packed = list(m.layers), m.layers[0].mixer, pkg.modules._host(), pkg.plan.packed
+    with torch.no_grad():
+        m(x)
+        m.step(x[:, 0], list(caches))
+    mixer(x)
+    ticks, stop = [], threading.Event()
+
+    def ticking():
+        while not stop.is_set():
+            ticks.append(time.perf_counter())
+            time.sleep(0)       # lets go of the interpreter
+
+    def forward():
+        with torch.no_grad():
+            return host.stack_forward(layers, x, None, False, packed)
+
+    x0 = x[:, 0].contiguous()
+
+    def step():
+        with torch.no_grad():
+            return host.stack_step(layers, x0, list(caches), False)
+
+    def train():
+        return host.block_train(mixer, x, None, None, False, packed)
+
+    interval = sys.getswitchinterval()
+    thread = threading.Thread(target=ticking, daemon=True)
+    try:
+        sys.setswitchinterval(10.0)
+        thread.start()
+        for call in (forward, step, train):
+            seen, results = 0, []
+            for _ in range(20):
+                t0 = time.perf_counter()
+                results.append(call())
+                t1 = time.perf_counter()
+                mid = (0.7 * t0 + 0.3 * t1, 0.3 * t0 + 0.7 * t1)
+                seen += sum(mid[0] < t < mid[1] for t in ticks)
+                ticks.clear()
+            assert None not in results and seen > 0, call.__name__
+    finally:
+        stop.set()
+        sys.setswitchinterval(interval)
+        thread.join(timeout=30)
+    assert not thread.is_alive()
+
+
+def test_layer_calls_from_several_threads(pkg, dev):
+    """One model on four threads and streams, its forms made anew by each of them in turn: the serial bits."""
+    torch.manual_seed(10)
+    m = pkg.Mamba(pkg.MambaConfig(d_model=64, n_layers=3)).to(dev).to(torch.bfloat16)
+    xs = [torch.randn(2, 40 + i, 64, device=dev).to(torch.bfloat16) for i in range(4)]
+
+    def run(i):
+        with torch.no_grad():
+            y, caches = m(xs[i], return_caches=True)
+            out = [y, m.step(xs[i][:, 0], list(caches))[0]]
+        z = m(xs[i])
+        return out + [z.detach()] + list(torch.autograd.grad(z.float().sum(), list(m.parameters())))
+
+    serial = [run(i) for i in range(4)]
+    torch.cuda.synchronize()
+    errors, barrier = [], threading.Barrier(4)
+
+    def worker(i):
+        try:
+            stream = torch.cuda.Stream(device=dev)
+            barrier.wait(timeout=60)
+            with torch.cuda.stream(stream):
+                for _ in range(20):
+                    got = run(i)
+                    stream.synchronize()
+                    errors.extend((i, j) for j, (a, b) in enumerate(zip(got, serial[i])) if not torch.equal(a, b))
+        except Exception as exc:
+            errors.append((i, repr(exc)))
+
+    threads = [threading.Thread(target=worker, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=100)
+    assert not any(t.is_alive() for t in threads)
+    assert errors == []
