@@ -172,22 +172,36 @@ inline bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx(
 // Orders the streams that read kept forms after the one that last wrote them, and tells the allocator of them.
 // (A capture cannot wait for an event from outside; torch synchronises the device before it begins one.)
 struct Written {
-    std::optional<c10::Event> event;
+    std::shared_ptr<c10::Event> event;
     std::optional<c10::Stream> last;  // the stream that wrote, or one that has waited since
-    void before(const c10::Stream& s) const {
-        if (event && last != s && !capturing()) event->block(s);
+};
+// The forming of the layers of one call: one event for all that is written.
+class Forming {
+public:
+    explicit Forming(const c10::Device& device) : stream(current_stream(device)), capture(capturing()) {}
+    Forming(const Forming&) = delete;
+    ~Forming() {
+        if (wrote.empty() || capture) return;
+        const auto event = std::make_shared<c10::Event>(stream.device_type());
+        event->record(stream);
+        for (Written* w : wrote) w->event = event;
     }
-    void after(const c10::Stream& s, bool wrote, std::initializer_list<const Tensor*> forms) {
-        if (last && last != s)
+    void before(const Written& w) const {
+        if (w.event && w.last != stream && !capture) w.event->block(stream);
+    }
+    void after(Written& w, bool wrote_it, std::initializer_list<const Tensor*> forms) {
+        if (w.last && w.last != stream)
             for (const Tensor* t : forms)
-                if (t->defined()) t->record_stream(s);
-        if (capturing()) return;
-        if (wrote) {
-            if (!event || event->device_index() != s.device_index()) event.emplace(s.device_type());
-            event->record(s);
-        }
-        last = s;
+                if (t->defined()) t->record_stream(stream);
+        if (capture) return;
+        w.last = stream;
+        if (wrote_it) wrote.push_back(&w);
     }
+    const c10::Stream stream;
+    const bool capture;
+
+private:
+    std::vector<Written*> wrote;
 };
 
 struct LayerSizes {
@@ -262,6 +276,13 @@ struct Weights : LayerSizes {
     }
 };
 
+// (no two handles are ever at the same one)
+inline uint64_t next_epoch() {
+    static uint64_t last = 0;
+    return ++last;
+}
+
+struct NormHandle;
 struct MixerHandle : LayerSizes {
     bool decode_ok = false;   // the shapes are such as mpa_decode_layer_step takes
     bool forward_ok = false;  // ... as stack_forward and block_train take
@@ -272,7 +293,7 @@ struct MixerHandle : LayerSizes {
     // Forms kept for calls without gradients, and the epoch they are of.  Version counters do not show every change
     // of a parameter (writes through .data), and a training loop makes one after each of its calls: a call with
     // gradients forms its own and begins an epoch.
-    uint64_t epoch = 1, formed = 0, padded = 0;  // padded: that of xp .. dtp_t
+    uint64_t epoch = next_epoch(), formed = 0, padded = 0;  // padded: that of xp .. dtp_t
     Written written;
     F32 conv_w, conv_b, dt_b, D;
     Tensor A, xp, dtp;  // (xp and dtp: where the layer's own shapes are padded)
@@ -299,7 +320,7 @@ struct MixerHandle : LayerSizes {
         const bool there = both(in, kInW, kInB, changed) && both(conv, kConvW, kConvB, changed) && both(xp, kXW, kXB, changed) &&
                            both(dtp, kDtW, kDtB, changed) && both(out, kOutW, kOutB, changed) && p[kALog].look(params, k.A_log, changed) &&
                            p[kD].look(params, k.D, changed);
-        if (changed) ++epoch;
+        if (changed) epoch = next_epoch();
         if (changed && !there) forget();
         decode_ok = forward_ok = false;
         if (there) look_over();
@@ -334,7 +355,7 @@ struct MixerHandle : LayerSizes {
         return PyObject_IsTrue(sizes[5].o) == 0;
     }
 
-    void expire() { ++epoch; }
+    void expire() { epoch = next_epoch(); }
 
     void look_over() {
         const Tensor& w = p[kInW].t;
@@ -372,44 +393,9 @@ struct MixerHandle : LayerSizes {
         return w;
     }
 
-    // The kept forms, up to date, xp .. dtp_t among them for a sequence; after ready().  Within a capture nothing
-    // runs yet: the next call still finds them old.
-    std::shared_ptr<const Weights> form(bool sequence) {
-        const c10::Stream s = current_stream(device);
-        written.before(s);
-        const bool small = formed != epoch, wide = sequence && padded != epoch;
-        if (small || wide) {
-            auto w = std::make_shared<Weights>(parameters());
-            std::vector<mpa_cast_job> jobs;
-            auto f32 = [&](F32& form, int i) {
-                if (small) form.take(p[i].t, jobs);
-                return form.t;
-            };
-            w->conv_w = f32(conv_w, kConvW);
-            w->conv_b = f32(conv_b, kConvB);
-            w->dt_b = f32(dt_b, kDtB);
-            w->D = f32(D, kD);
-            w->A = derived(A, {ED, N}, at::kFloat, w->p[kInW]);
-            if (small) jobs.push_back(cast_job(p[kALog].t, A, ED, N, 0, 0, MPA_CAST_NEG_EXP));
-            w->in_wt = w->p[kInW].detach().t();
-            w->out_wt = w->p[kOutW].detach().t();
-            if (sequence) {
-                const Tensor &xw = w->p[kXW], &dw = w->p[kDtW];
-                w->xp = Rp == R ? xw.detach() : derived(xp, {padded_rows(), ED}, dt, xw);
-                w->dtp = Rp == R ? dw.detach() : derived(dtp, {ED, Rp}, dt, dw);
-                w->xp_t = w->xp.t();
-                w->dtp_t = w->dtp.t();
-                if (wide && Rp != R) w->pad_jobs(jobs);
-            }
-            run_casts(jobs, w->p[kInW]);
-            kept = w;
-            const uint64_t of = capturing() ? 0 : epoch;
-            if (small) formed = of;
-            padded = sequence ? of : 0;  // (xp .. dtp_t are not in `kept` otherwise)
-        }
-        written.after(s, small || wide, {&conv_w.own, &conv_b.own, &dt_b.own, &D.own, &A, &xp, &dtp});
-        return kept;
-    }
+    // The kept forms, up to date, xp .. dtp_t among them for a sequence, and those of the norm in front, if given; after
+    // ready().  Within a capture nothing runs yet: the next call still finds them old.
+    std::shared_ptr<const Weights> form(Forming& f, bool sequence, NormHandle* norm);
 };
 
 // The norm in front of a mixer.
@@ -419,8 +405,7 @@ struct NormHandle {
     Param p;
     double eps = 0;
     F32 w;
-    uint64_t formed = 0;  // epoch of the mixer's handle that w is of
-    Written written;
+    uint64_t formed = 0;  // epoch of the mixer's handle that w is of (the mixer's `written` covers it)
 
     explicit NormHandle(PyObject* dict) : modules(get(dict, keys().modules)) {}
     bool belongs_to(PyObject* dict) const { return get(dict, keys().modules) == modules.o; }
@@ -443,21 +428,51 @@ struct NormHandle {
         const Tensor& t = p.t;
         return !t.defined() || (t.numel() == m.d && MixerHandle::small_ok(t, m.device) && reinterpret_cast<uintptr_t>(p.data) % 16 == 0);
     }
-    Tensor form(const MixerHandle& m) {
-        const c10::Stream s = current_stream(m.device);
-        written.before(s);
-        const bool old = changed || formed != m.epoch;
-        if (old) {
-            std::vector<mpa_cast_job> jobs;
-            w.take(p.t, jobs);
-            run_casts(jobs, m.p[kInW].t);
-            changed = false;
-            formed = capturing() ? 0 : m.epoch;
-        }
-        written.after(s, old, {&w.own});
-        return w.t;
-    }
 };
+
+inline std::shared_ptr<const Weights> MixerHandle::form(Forming& f, bool sequence, NormHandle* norm) {
+    f.before(written);
+    const bool small = formed != epoch, wide = sequence && padded != epoch, gain = norm && (norm->changed || norm->formed != epoch);
+    std::vector<mpa_cast_job> jobs;
+    const uint64_t of = f.capture ? 0 : epoch;
+    if (gain) norm->w.take(norm->p.t, jobs);
+    std::shared_ptr<Weights> w;
+    if (small || wide) {
+        w = std::make_shared<Weights>(parameters());
+        auto f32 = [&](F32& form, int i) {
+            if (small) form.take(p[i].t, jobs);
+            return form.t;
+        };
+        w->conv_w = f32(conv_w, kConvW);
+        w->conv_b = f32(conv_b, kConvB);
+        w->dt_b = f32(dt_b, kDtB);
+        w->D = f32(D, kD);
+        w->A = derived(A, {ED, N}, at::kFloat, w->p[kInW]);
+        if (small) jobs.push_back(cast_job(p[kALog].t, A, ED, N, 0, 0, MPA_CAST_NEG_EXP));
+        w->in_wt = w->p[kInW].detach().t();
+        w->out_wt = w->p[kOutW].detach().t();
+        if (sequence) {
+            const Tensor &xw = w->p[kXW], &dw = w->p[kDtW];
+            w->xp = Rp == R ? xw.detach() : derived(xp, {padded_rows(), ED}, dt, xw);
+            w->dtp = Rp == R ? dw.detach() : derived(dtp, {ED, Rp}, dt, dw);
+            w->xp_t = w->xp.t();
+            w->dtp_t = w->dtp.t();
+            if (wide && Rp != R) w->pad_jobs(jobs);
+        }
+    }
+    if (!jobs.empty()) run_casts(jobs, p[kInW].t);
+    if (gain) {
+        norm->changed = f.capture;
+        norm->formed = of;
+    }
+    if (w) {
+        kept = w;
+        if (small) formed = of;
+        padded = sequence ? of : 0;  // (xp .. dtp_t are not in `kept` otherwise)
+    }
+    f.after(written, !jobs.empty(), {&conv_w.own, &conv_b.own, &dt_b.own, &D.own, &A, &xp, &dtp, norm ? &norm->w.own : &A});
+    return kept;
+}
 
 // The products of a layer run on mpa_linear_run while they are small: it costs the host a quarter of a library call
 // (18 us) and takes norms and residual adds along: a bfloat16 stack of width 768 without gradients, 512 steps, 1.4 ms

@@ -34,6 +34,17 @@ struct LayerWeights {
     double eps = 0;
 };
 
+std::vector<LayerWeights> form_layers(const std::vector<Layer>& layers, bool sequence) {
+    Forming f(layers[0].m->device);
+    std::vector<LayerWeights> w;
+    w.reserve(layers.size());
+    for (const Layer& l : layers) {
+        auto m = l.m->form(f, sequence, l.n);
+        w.push_back({std::move(m), l.n->w.t, l.n->eps});
+    }
+    return w;
+}
+
 py::object pair(const Tensor& h, const Tensor& w) { return py::make_tuple(h, w); }
 
 // ---- decode -------------------------------------------------------------------------------------
@@ -106,8 +117,7 @@ py::object stack_step(const py::list& layers, const Tensor& x_in, const py::list
     }
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
-    std::vector<LayerWeights> ws(n);
-    for (size_t i = 0; i < n; ++i) ws[i] = {hs[i].m->form(false), hs[i].n->form(*hs[i].m), hs[i].n->eps};
+    const std::vector<LayerWeights> ws = form_layers(hs, false);
     Tensor y;
     {
         const py::gil_scoped_release nogil;
@@ -130,7 +140,11 @@ py::object block_step(const py::object& block, const Tensor& x_in, const Opt& h_
     if (!l || !l->decode_ok || !cache_fits(in, *l, batch, inplace)) return py::none();
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
-    const std::shared_ptr<const Weights> w = l->form(false);
+    std::shared_ptr<const Weights> w;
+    {
+        Forming f(l->device);
+        w = l->form(f, false, nullptr);
+    }
     py::gil_scoped_release nogil;
     Cache out = in;
     if (!inplace) {
@@ -281,8 +295,7 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
     }
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
-    std::vector<LayerWeights> ws(n);
-    for (size_t i = 0; i < n; ++i) ws[i] = {hs[i].m->form(true), hs[i].n->form(*hs[i].m), hs[i].n->eps};
+    const std::vector<LayerWeights> ws = form_layers(hs, true);
     Tensor y;
     {
         const py::gil_scoped_release nogil;
