@@ -365,9 +365,14 @@ int mpa_decode_layer_step(const mpa_decode_layer* s, const void* x, const void* 
  *     without norm_weight and y_ssq.
  *   residual  optional: (T x M), added to the rounded product or, with `accumulate`, before it is rounded; may be y.
  *   y_ssq  optional: ceil(M / 32) rows of T partial sums of squares of y.
+ *   io_dtype | MPA_LINEAR_X_F32 (with x_ssq), _Y_F32, _RESIDUAL_F32: x, y or residual are float32 in a bfloat16
+ *     call (nothing is rounded on its way into a float32 y).
  * Rows of x are x_pitch apart, those of y and residual y_pitch.  K and x_pitch are multiples of 4 (float32) / 8
  * (bfloat16), M and y_pitch of 4; x, weight and norm_weight 16-byte aligned, the rest four elements.
  */
+#define MPA_LINEAR_X_F32 256
+#define MPA_LINEAR_Y_F32 512
+#define MPA_LINEAR_RESIDUAL_F32 1024
 typedef struct mpa_linear {
     int64_t T, M, K, x_pitch, y_pitch;
     const void *x, *weight, *bias;

@@ -177,12 +177,15 @@ Tensor run_sequence(const std::vector<LayerWeights>& hs, const Tensor& x, std::v
     void* stream = stream_of(x);
     const Tensor normed = empty({T, d}, dt, x), xz = empty({T, 2 * ED}, dt, x), xs = empty({Bs, L, ED}, dt, x),
                  dbc = empty({T, P}, dt, x), delta = empty({T, ED}, dt, x), y = empty({T, ED}, dt, x), hidden = empty({T, d}, dt, x);
-    Tensor sum[2];
-    if (n > 1) { sum[0] = empty({T, d}, dt, x); sum[1] = empty({T, d}, dt, x); }
     bool own = use_linear(dt, T, d, ED, P, {&x});
     for (const LayerWeights& h : hs)
         own &= h.norm_w.defined() &&
                use_linear(dt, T, d, ED, P, {&h.m->p[kInW], &h.m->p[kOutW], &h.m->xp, &h.m->dtp, &h.norm_w, &h.m->p[kInB], &h.m->p[kOutB]});
+    // The residual stream between the layers.  The own products keep it in float32: at bfloat16, its roundings were
+    // the larger part of a deep stack's error (24 layers of width 768: see tests/test_deep_stack_gpu.py).
+    Tensor sum[2];
+    const auto sum_dt = own ? at::kFloat : dt;
+    if (n > 1) { sum[0] = empty({T, d}, sum_dt, x); sum[1] = empty({T, d}, sum_dt, x); }
     const int64_t parts = (d + 31) / 32;
     const Tensor ssq = own ? empty({parts, T}, at::kFloat, x) : Tensor();
     auto linear = [&](const void* in, int64_t pitch, int64_t K, const Tensor& weight, const Tensor& bias, const Tensor& out) {
@@ -226,7 +229,10 @@ Tensor run_sequence(const std::vector<LayerWeights>& hs, const Tensor& x, std::v
         Tensor out = xz;
         if (own) {
             mpa_linear q = linear(i == 0 ? ptr(normed) : ptr(sum[(i - 1) % 2]), d, d, l.p[kInW], l.p[kInB], xz);
-            if (i > 0) { q.norm_weight = norm_w; q.x_ssq = fptr(ssq); q.ssq_parts = parts; q.eps = eps; }
+            if (i > 0) {
+                q.io_dtype |= MPA_LINEAR_X_F32;
+                q.norm_weight = norm_w; q.x_ssq = fptr(ssq); q.ssq_parts = parts; q.eps = eps;
+            }
             run(q);
         } else if (l.p[kInB].defined()) {
             at::addmm_out(out, l.p[kInB].detach(), normed, l.in_wt);
@@ -259,7 +265,12 @@ Tensor run_sequence(const std::vector<LayerWeights>& hs, const Tensor& x, std::v
             const bool last = i + 1 == n;
             mpa_linear q = linear(ptr(y), ED, ED, l.p[kOutW], l.p[kOutB], last ? result : s);
             q.residual = i == 0 ? ptr(x) : ptr(sum[(i - 1) % 2]);
-            if (!last) q.y_ssq = fptr(ssq);
+            q.accumulate = 1;
+            if (i > 0) q.io_dtype |= MPA_LINEAR_RESIDUAL_F32;
+            if (!last) {
+                q.io_dtype |= MPA_LINEAR_Y_F32;
+                q.y_ssq = fptr(ssq);
+            }
             run(q);
         } else if (l.p[kOutB].defined()) {
             at::addmm_out(out, l.p[kOutB].detach(), y, l.out_wt);

@@ -6,6 +6,7 @@
 // the product: with `residual` the sum y + residual is stored, with `ssq_out` the partial sums of squares of its rows;
 // with `ssq`, those of x, the rows of x are normalised on their way into LDS (x * rstd * weight, rounded, as
 // the norm kernel rounds: a factor of the finished product would be cheaper, but rounds elsewhere).
+// The residual stream between bfloat16 layers can be float32: x (with `ssq`), y and residual each have a flag.
 //
 // Tile: BT steps x BM rows of W per workgroup, each wave 32 x 32 of it (2 x 2 MFMA tiles of 16 x 16, W as the left
 // operand, so that a lane's four results are neighbours in y) over its share of K.  K runs in stages of 128 bytes per
@@ -44,6 +45,12 @@ struct LinearOps<bf16_t> {
         for (int e = 0; e < 8; ++e) x[e] = static_cast<__bf16>(static_cast<float>(x[e]) * rs * w[e >> 2][e & 3]);
         return __builtin_bit_cast(u32x4, x);
     }
+    static __device__ __forceinline__ u32x4 scale_f32(const u32x4& lo, const u32x4& hi, float rs, const f32x4 (&w)[2]) {
+        bf16x8 x;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = static_cast<__bf16>(__uint_as_float(e < 4 ? lo[e] : hi[e - 4]) * rs * w[e >> 2][e & 3]);
+        return __builtin_bit_cast(u32x4, x);
+    }
 };
 template <>
 struct LinearOps<float> {
@@ -76,12 +83,19 @@ struct LinearParams {
     const float* norm_w;  // [K], with ssq
     const void* residual;
     int accumulate;
+    int y_f32, residual_f32;  // float32 whatever IO is
     float* ssq_out;  // [M/32 rounded up][T]
 };
 
-template <typename IO, int BT, int BM, int KS, int D, bool NORM, bool NN>
+// How x comes: as it is, to be normalised, or float32 (IO is bfloat16) and to be normalised.
+enum LinearX { kPlainX = 0, kNormX = 1, kNormXF32 = 2 };
+
+template <typename IO, int BT, int BM, int KS, int D, int XMODE, bool NN>
 __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kernel(const LinearParams p) {
     typedef LinearOps<IO> Ops;
+    constexpr bool NORM = XMODE != kPlainX, XF32 = XMODE == kNormXF32;
+    static_assert(!XF32 || sizeof(IO) == 2, "float32 x of a bfloat16 product");
+    constexpr uint32_t kXES = XF32 ? 4 : sizeof(IO);  // bytes of an element of x
     constexpr int kVec = Ops::kVec, kStep = 8 * kVec;  // k of a stage and share
     constexpr uint32_t kES = sizeof(IO);
     constexpr int kThreads = BT / 32 * (BM / 32) * KS * kWave;
@@ -100,7 +114,7 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
     // (buffer loads: a part beyond K gets an offset beyond the window and reads as zero without a branch, which
     // would make every wait one for all loads in flight)
     const rsrc_t rw = make_rsrc(p.w, (uint32_t)p.M * (uint32_t)p.K * kES);  // (both forms of W are dense)
-    const rsrc_t rx = make_rsrc(p.x, ((uint32_t)(p.T - 1) * (uint32_t)p.x_pitch + (uint32_t)p.K) * kES);
+    const rsrc_t rx = make_rsrc(p.x, ((uint32_t)(p.T - 1) * (uint32_t)p.x_pitch + (uint32_t)p.K) * kXES);
     constexpr int kWLoads = BM * kParts / kThreads;  // the loads of W; those of x follow
     constexpr int kRowsPer = sizeof(IO) == 2 ? 2 : 1;  // rows of W that make a word in LDS
     uint32_t off[kLoads];
@@ -117,13 +131,14 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
             continue;
         }
         koff[i] = part * kVec;
-        off[i] = kES * (koff[i] + (row < BM ? (uint32_t)min(m0 + row, p.M - 1) * (uint32_t)p.K
-                                           : (uint32_t)min(t0 + row - BM, p.T - 1) * (uint32_t)p.x_pitch));
+        off[i] = row < BM ? kES * (koff[i] + (uint32_t)min(m0 + row, p.M - 1) * (uint32_t)p.K)
+                          : kXES * (koff[i] + (uint32_t)min(t0 + row - BM, p.T - 1) * (uint32_t)p.x_pitch);
         at[i] = (part >> 3) * (kRows * 8) + row * 8 + ((part & 7) ^ (row & 7));
     }
     const int steps = (p.K + kStep * KS - 1) / (kStep * KS);
     struct Stage {
         u32x4 v[kLoads];
+        u32x4 hi[XF32 ? kLoads - kWLoads : 1];  // float32 x: the second half of a part
         f32x4 w[kVec / 4];  // NORM: norm weight of the thread's k (the same in all its parts)
     };
     const rsrc_t rn = make_rsrc(p.norm_w, (uint32_t)p.K * 4u);
@@ -134,8 +149,12 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
             const int k = s * kStep * KS;
-            const uint32_t at_k = kES * (uint32_t)k * (NN && i < kWLoads ? (uint32_t)p.M : 1u);
-            v[i] = __builtin_amdgcn_raw_buffer_load_b128(i < kWLoads ? rw : rx, k + koff[i] < p.K ? off[i] + at_k : 0xffffffffu, 0, 0);
+            const uint32_t at_k = (i < kWLoads ? kES : kXES) * (uint32_t)k * (NN && i < kWLoads ? (uint32_t)p.M : 1u);
+            const uint32_t at = k + koff[i] < p.K ? off[i] + at_k : 0xffffffe0u;
+            v[i] = __builtin_amdgcn_raw_buffer_load_b128(i < kWLoads ? rw : rx, at, 0, 0);
+            if constexpr (XF32) {
+                if (i >= kWLoads) st.hi[i - kWLoads] = __builtin_amdgcn_raw_buffer_load_b128(rx, at + 16, 0, 0);
+            }
         }
         if constexpr (NORM) {
 #pragma unroll
@@ -168,7 +187,11 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
                 if (i % kRowsPer == 0) store_transposed(st, i, buf);
                 continue;
             }
-            if (NORM && i >= kWLoads) v = Ops::scale(v, rs[i - kWLoads], st.w);
+            if constexpr (XF32) {
+                if (i >= kWLoads) v = Ops::scale_f32(v, st.hi[i - kWLoads], rs[i - kWLoads], st.w);
+            } else if constexpr (NORM) {
+                if (i >= kWLoads) v = Ops::scale(v, rs[i - kWLoads], st.w);
+            }
             lds[buf][at[i]] = v;
         }
     };
@@ -255,18 +278,34 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
             const int t = t0 + wt * 32 + j * 16 + fr;
             if (t >= p.T) continue;
             const int64_t o = (int64_t)t * p.y_pitch + m;
-            typename Ops::Out v, res = {};
-            if (p.residual) res = *reinterpret_cast<const typename Ops::Out*>(static_cast<const IO*>(p.residual) + o);
+            f32x4 res = {};
+            if (p.residual_f32) {
+                res = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p.residual) + o);
+            } else if (p.residual) {
+                const typename Ops::Out r = *reinterpret_cast<const typename Ops::Out*>(static_cast<const IO*>(p.residual) + o);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float f = acc[i][j][e] + Ops::get(bias, e);
-                Ops::set(v, e, p.accumulate ? f + Ops::get(res, e) : f);
-                if (p.residual && !p.accumulate) Ops::set(v, e, Ops::get(v, e) + Ops::get(res, e));
+                for (int e = 0; e < 4; ++e) res[e] = Ops::get(r, e);
             }
-            *reinterpret_cast<typename Ops::Out*>(static_cast<IO*>(p.y) + o) = v;
+            f32x4 f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f[e] = acc[i][j][e] + Ops::get(bias, e);
+            if (p.accumulate) f += res;
+            if (p.y_f32) {
+                if (p.residual && !p.accumulate) f += res;
+                *reinterpret_cast<f32x4*>(static_cast<float*>(p.y) + o) = f;
+            } else {
+                typename Ops::Out v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    Ops::set(v, e, f[e]);
+                    if (p.residual && !p.accumulate) Ops::set(v, e, Ops::get(v, e) + res[e]);
+                    f[e] = Ops::get(v, e);
+                }
+                *reinterpret_cast<typename Ops::Out*>(static_cast<IO*>(p.y) + o) = v;
+            }
             if (p.ssq_out) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) ss[j] = __builtin_fmaf(Ops::get(v, e), Ops::get(v, e), ss[j]);
+                for (int e = 0; e < 4; ++e) ss[j] = __builtin_fmaf(f[e], f[e], ss[j]);
             }
         }
     }
@@ -283,12 +322,13 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
 }
 
 template <typename IO, int BT, int BM, int KS>
-static int launch_linear(const LinearParams& p, bool nn, hipStream_t st) {
+static int launch_linear(const LinearParams& p, bool nn, bool x_f32, hipStream_t st) {
     const int nt = (p.T + BT - 1) / BT, nm = (p.M + BM - 1) / BM, per = (nt * nm + 7) / 8;
     const dim3 grid((unsigned)per * 8), block(BT / 32 * (BM / 32) * KS * kWave);
-    if (nn) hipLaunchKernelGGL((linear_kernel<IO, BT, BM, KS, 2, false, true>), grid, block, 0, st, p);
-    else if (p.ssq) hipLaunchKernelGGL((linear_kernel<IO, BT, BM, KS, 2, true, false>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((linear_kernel<IO, BT, BM, KS, 2, false, false>), grid, block, 0, st, p);
+    if (nn) hipLaunchKernelGGL((linear_kernel<IO, BT, BM, KS, 2, kPlainX, true>), grid, block, 0, st, p);
+    else if (!p.ssq) hipLaunchKernelGGL((linear_kernel<IO, BT, BM, KS, 2, kPlainX, false>), grid, block, 0, st, p);
+    else if (sizeof(IO) == 2 && x_f32) hipLaunchKernelGGL((linear_kernel<IO, BT, BM, KS, 2, sizeof(IO) == 2 ? kNormXF32 : kNormX, false>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((linear_kernel<IO, BT, BM, KS, 2, kNormX, false>), grid, block, 0, st, p);
     return check_launch();
 }
 
@@ -296,14 +336,14 @@ static int launch_linear(const LinearParams& p, bool nn, hipStream_t st) {
 // with K split over more waves (512 steps of a layer of width 768: in_proj 9.0 us with 64 x 128, 9.9 with 64 x
 // 64, 15 with 32 x 32; out_proj 7.9 us with 64 x 32 on eight waves, 10.8 with 64 x 64; x_proj 6.7 and 10.2 us).
 template <typename IO>
-static int dispatch_linear(const LinearParams& p, bool nn, hipStream_t st) {
+static int dispatch_linear(const LinearParams& p, bool nn, bool x_f32, hipStream_t st) {
     auto tiles = [&](int bt, int bm) { return (int64_t)((p.T + bt - 1) / bt) * ((p.M + bm - 1) / bm); };
     constexpr int kFull = 160;
-    if (tiles(64, 128) >= kFull) return launch_linear<IO, 64, 128, 1>(p, nn, st);
-    if (p.K <= 128) return launch_linear<IO, 64, 64, 1>(p, nn, st);  // (one or two stages: nothing to split)
-    if (tiles(64, 64) >= kFull) return p.K >= 1024 ? launch_linear<IO, 64, 64, 2>(p, nn, st) : launch_linear<IO, 64, 64, 1>(p, nn, st);
-    if (tiles(64, 32) >= kFull) return p.K >= 1024 ? launch_linear<IO, 64, 32, 4>(p, nn, st) : launch_linear<IO, 64, 32, 2>(p, nn, st);
-    return launch_linear<IO, 32, 32, 4>(p, nn, st);
+    if (tiles(64, 128) >= kFull) return launch_linear<IO, 64, 128, 1>(p, nn, x_f32, st);
+    if (p.K <= 128) return launch_linear<IO, 64, 64, 1>(p, nn, x_f32, st);  // (one or two stages: nothing to split)
+    if (tiles(64, 64) >= kFull) return p.K >= 1024 ? launch_linear<IO, 64, 64, 2>(p, nn, x_f32, st) : launch_linear<IO, 64, 64, 1>(p, nn, x_f32, st);
+    if (tiles(64, 32) >= kFull) return p.K >= 1024 ? launch_linear<IO, 64, 32, 4>(p, nn, x_f32, st) : launch_linear<IO, 64, 32, 2>(p, nn, x_f32, st);
+    return launch_linear<IO, 32, 32, 4>(p, nn, x_f32, st);
 }
 
 }  // namespace mpa
@@ -313,8 +353,12 @@ using namespace mpa;
 extern "C" int mpa_linear_run(const mpa_linear* s, void* stream) {
     if (!s || !s->x || !s->weight || !s->y) return MPA_ERR_NULL_POINTER;
     if (s->x_ssq && !s->norm_weight) return MPA_ERR_NULL_POINTER;
-    if (s->io_dtype != MPA_F32 && s->io_dtype != MPA_BF16) return MPA_ERR_BAD_DTYPE;
-    const bool f32 = s->io_dtype == MPA_F32;
+    const int wide = MPA_LINEAR_X_F32 | MPA_LINEAR_Y_F32 | MPA_LINEAR_RESIDUAL_F32, io = s->io_dtype & ~wide;
+    if (io != MPA_F32 && io != MPA_BF16) return MPA_ERR_BAD_DTYPE;
+    const bool f32 = io == MPA_F32;
+    const bool x_f32 = !f32 && (s->io_dtype & MPA_LINEAR_X_F32), y_f32 = f32 || (s->io_dtype & MPA_LINEAR_Y_F32);
+    const bool residual_f32 = f32 || (s->io_dtype & MPA_LINEAR_RESIDUAL_F32);
+    if (x_f32 && !s->x_ssq) return MPA_ERR_BAD_DTYPE;
     const int vec = f32 ? 4 : 8;
     if (s->weight_kxm && (s->x_ssq || s->y_ssq || s->M % vec)) return MPA_ERR_BAD_SHAPE;
     // (x and the weight are addressed with 32-bit byte offsets)
@@ -322,8 +366,8 @@ extern "C" int mpa_linear_run(const mpa_linear* s, void* stream) {
         s->y_pitch < s->M || s->T > 1 << 24 || s->M > 1 << 24 || s->K > 1 << 24 || s->T * s->x_pitch >= (int64_t)1 << 29 ||
         s->M * s->K >= (int64_t)1 << 29 || (s->x_ssq && (s->ssq_parts <= 0 || s->ssq_parts > 1 << 20)))
         return MPA_ERR_BAD_SHAPE;
-    if (!aligned_to(s->x, 16) || !aligned_to(s->weight, 16) || !aligned_to(s->bias, f32 ? 16 : 8) || !aligned_to(s->y, f32 ? 16 : 8) ||
-        !aligned_to(s->residual, f32 ? 16 : 8) || !aligned_to(s->norm_weight, 16) || !aligned_to(s->x_ssq, 4) || !aligned_to(s->y_ssq, 4))
+    if (!aligned_to(s->x, 16) || !aligned_to(s->weight, 16) || !aligned_to(s->bias, f32 ? 16 : 8) || !aligned_to(s->y, y_f32 ? 16 : 8) ||
+        !aligned_to(s->residual, residual_f32 ? 16 : 8) || !aligned_to(s->norm_weight, 16) || !aligned_to(s->x_ssq, 4) || !aligned_to(s->y_ssq, 4))
         return MPA_ERR_MISALIGNED;
     LinearParams p{};
     p.x = s->x; p.w = s->weight; p.bias = s->bias;
@@ -333,7 +377,8 @@ extern "C" int mpa_linear_run(const mpa_linear* s, void* stream) {
     p.ssq = s->x_ssq; p.in_parts = (int)s->ssq_parts;
     p.inv_d = 1.0f / (float)s->K; p.eps = s->eps; p.norm_w = s->norm_weight;
     p.residual = s->residual;
+    p.y_f32 = y_f32; p.residual_f32 = residual_f32 && s->residual;
     p.accumulate = s->accumulate; p.ssq_out = s->y_ssq;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    return f32 ? dispatch_linear<float>(p, s->weight_kxm != 0, st) : dispatch_linear<bf16_t>(p, s->weight_kxm != 0, st);
+    return f32 ? dispatch_linear<float>(p, s->weight_kxm != 0, x_f32, st) : dispatch_linear<bf16_t>(p, s->weight_kxm != 0, x_f32, st);
 }

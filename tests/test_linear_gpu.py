@@ -79,3 +79,46 @@ def test_stack_of_any_width(pkg, dev, width, dtype):
     assert rel_err(y.float(), want) <= 2 * TOL[dtype]
     a, b = (t.layers[0].mixer.in_proj.weight.grad.float() for t in (m, ref))
     assert rel_err(a, b) <= 5 * TOL[dtype]
+
+
+# float32 x, y and residual around a bfloat16 product, over the tiles of the dispatch and their remainders
+@pytest.mark.parametrize("T,M,K,pitch", [(1, 4, 8, 8), (33, 100, 72, 80), (65, 520, 1032, 1032), (500, 1540, 264, 264), (700, 1000, 1096, 1096),
+                                         (1000, 1288, 64, 128), (2047, 900, 136, 144)])
+@pytest.mark.parametrize("accumulate", [0, 1])
+def test_linear_with_a_float32_residual_stream(pkg, dev, T, M, K, pitch, accumulate):
+    L, lib = pkg._lib, pkg._lib.load()
+    g = torch.Generator().manual_seed(T)
+    rand = lambda *s: torch.randn(*s, generator=g).to(dev)
+    x, w, bias, res, nw = rand(T, pitch), rand(M, K).bfloat16(), rand(M).bfloat16(), rand(T, M), rand(K)
+    ssq, eps = rand(5, T).square() * K / 5, 1e-5
+    normed = (x[:, :K].double() * (ssq.double().sum(0) / K + eps).rsqrt()[:, None] * nw.double()).bfloat16().double()
+    want = normed @ w.double().t() + bias.double()
+    X, Y, R = 256, 512, 1024
+
+    def run(flags, x, y, res, y_ssq=None, norm=True):
+        q = Linear(io_dtype=1 | flags, T=T, M=M, K=K, x_pitch=x.stride(0), y_pitch=M, x=x.data_ptr(), weight=w.data_ptr(), bias=bias.data_ptr(),
+                   y=y.data_ptr(), residual=res.data_ptr() if res is not None else None, accumulate=accumulate)
+        if norm:
+            q.norm_weight, q.x_ssq, q.ssq_parts, q.eps = nw.data_ptr(), ssq.data_ptr(), 5, eps
+        if y_ssq is not None:
+            q.y_ssq = y_ssq.data_ptr()
+        L.check(lib.mpa_linear_run(ctypes.byref(q), pkg.scan._stream(dev)), "mpa_linear_run")
+        return y
+
+    wide = lambda: torch.full((T, M), float("nan"), device=dev)
+    narrow = lambda: wide().bfloat16()
+    out_ssq = torch.empty((M + 31) // 32, T, device=dev)
+    # float32 all round: only the sums are rounded (and a normalised element here and there the other way than `normed`:
+    # a difference of 2^-8 in one of K factors)
+    y = run(X | Y | R, x, wide(), res, out_ssq)
+    assert rel_err(y, want + res.double()) <= 1e-3
+    assert rel_err(out_ssq.sum(0), y.double().square().sum(1)) <= 1e-5
+    # one flag at a time gives the same within the rounding of what is bfloat16 then
+    assert rel_err(run(X | Y, x, wide(), res.bfloat16()), want + res.bfloat16().double()) <= 1e-3
+    assert rel_err(run(X | R, x, narrow(), res), want + res.double()) <= TOL[torch.bfloat16]
+    assert rel_err(run(X | Y, x, wide(), None), want) <= 1e-3
+    x16 = x.bfloat16()
+    plain = x16[:, :K].double() @ w.double().t() + bias.double()
+    assert rel_err(run(Y | R, x16, wide(), res, norm=False), plain + res.double()) <= 1e-5
+    q = Linear(io_dtype=1 | X, T=T, M=M, K=K, x_pitch=pitch, y_pitch=M, x=x.data_ptr(), weight=w.data_ptr(), y=y.data_ptr())
+    assert lib.mpa_linear_run(ctypes.byref(q), pkg.scan._stream(dev)) == 3     # float32 x only to be normalised
