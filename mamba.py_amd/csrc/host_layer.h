@@ -475,18 +475,27 @@ inline std::shared_ptr<const Weights> MixerHandle::form(Forming& f, bool sequenc
 }
 
 // The products of a layer run on mpa_linear_run while they are small: it costs the host a quarter of a library call
-// (18 us) and takes norms and residual adds along: a bfloat16 stack of width 768 without gradients, 512 steps, 1.4 ms
-// for 24 layers, 2.1 with library calls.  The line is steps x width^2, which the products' arithmetic goes with.  Over
-// 50 shapes of widths 64 to 968 bfloat16 stacks below it are 1.0 to 1.6 times faster than with library calls, float32
-// ones too; at twice the float32 line (1342 steps of width 896, a quarter of the bfloat16 rate) the library's
-// large tiles win 1.1 times.  kLinearSteps bounds what was measured.
+// (18 us) and takes norms and residual adds along.  The line is steps x width^2, which the products' arithmetic goes with.
+// Measured against library calls at 173 shapes of widths 64 to 2560 and 16 to 73728 steps (profiles/linear_dispatch.md:
+// a layer of a stack without gradients; a mixer, forward and backward), times as fast:
+//   bfloat16  below the line 0.96 to 2.0 and 0.99 to 1.7 (0.96 to 1.1 at the line itself), at twice the line 0.84 to 1.1
+//   float32   a quarter of the rate, and every stage of a long K a latency.  Without gradients the line is that of width
+//             704 up to width 512 and falls as its square from there (0.98 to 2.1; on the other side of it 0.72 to 1.2).  A mixer
+//             with gradients makes three times the calls: 0.85 of the line up to width 1536 (1.00 to 1.9; on the other side 0.83 to 1.1).
+// kLinearSteps bounds what was measured.
 constexpr int64_t kLinearWorkBf16 = 2048LL * 768 * 768, kLinearWorkF32 = 1024LL * 704 * 704, kLinearSteps = 3072 * 768;
 inline bool aligned(const void* p, size_t a) { return reinterpret_cast<uintptr_t>(p) % a == 0; }
-inline bool use_linear(at::ScalarType dt, int64_t T, int64_t d, int64_t ED, int64_t P, std::initializer_list<const Tensor*> operands) {
+inline bool below_line(bool bf16, bool training, int64_t T, int64_t d) {
+    const int64_t work = T * d * d;
+    if (bf16) return work <= kLinearWorkBf16;
+    if (training) return work <= kLinearWorkF32 * 17 / 20 && d <= 1536;
+    return work <= kLinearWorkF32 && (d <= 512 || work <= kLinearWorkF32 * 512 / d * 512 / d);
+}
+inline bool use_linear(at::ScalarType dt, bool training, int64_t T, int64_t d, int64_t ED, int64_t P, std::initializer_list<const Tensor*> operands) {
     const bool bf16 = dt == at::kBFloat16;
     if (!bf16 && dt != at::kFloat) return false;
     const int64_t vec = bf16 ? 8 : 4, span = (int64_t)1 << 28;  // (32-bit byte offsets in the kernel)
-    bool ok = T * d <= kLinearSteps && T * d * d <= (bf16 ? kLinearWorkBf16 : kLinearWorkF32) && d % vec == 0 && ED % vec == 0 && P % vec == 0 &&
+    bool ok = T * d <= kLinearSteps && below_line(bf16, training, T, d) && d % vec == 0 && ED % vec == 0 && P % vec == 0 &&
               ED * d < span && ED * P < span && T * std::max(ED, P) < span;
     for (const Tensor* t : operands) ok &= !t->defined() || aligned(t->const_data_ptr(), 16);
     return ok;

@@ -177,10 +177,10 @@ Tensor run_sequence(const std::vector<LayerWeights>& hs, const Tensor& x, std::v
     void* stream = stream_of(x);
     const Tensor normed = empty({T, d}, dt, x), xz = empty({T, 2 * ED}, dt, x), xs = empty({Bs, L, ED}, dt, x),
                  dbc = empty({T, P}, dt, x), delta = empty({T, ED}, dt, x), y = empty({T, ED}, dt, x), hidden = empty({T, d}, dt, x);
-    bool own = use_linear(dt, T, d, ED, P, {&x});
+    bool own = use_linear(dt, false, T, d, ED, P, {&x});
     for (const LayerWeights& h : hs)
         own &= h.norm_w.defined() &&
-               use_linear(dt, T, d, ED, P, {&h.m->p[kInW], &h.m->p[kOutW], &h.m->xp, &h.m->dtp, &h.norm_w, &h.m->p[kInB], &h.m->p[kOutB]});
+               use_linear(dt, false, T, d, ED, P, {&h.m->p[kInW], &h.m->p[kOutW], &h.m->xp, &h.m->dtp, &h.norm_w, &h.m->p[kInB], &h.m->p[kOutB]});
     // The residual stream between the layers.  The own products keep it in float32: at bfloat16, its roundings were
     // the larger part of a deep stack's error (24 layers of width 768: see tests/test_deep_stack_gpu.py).
     Tensor sum[2];

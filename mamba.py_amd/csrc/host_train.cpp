@@ -83,7 +83,7 @@ std::tuple<Tensor, Tensor, Tensor> mixer_forward(Weights& l, const std::array<co
         const int64_t T = m.Bs * m.L, ED = m.ED, N = m.N, P = m.P;
         const Tensor x2 = x.view({T, m.d});
         void* stream = stream_of(x);
-        const bool own = use_linear(dt, T, m.d, ED, P, {&x, &l.p[kInW], &l.p[kOutW], &l.xp, &l.dtp, &l.p[kInB], &l.p[kOutB]});
+        const bool own = use_linear(dt, true, T, m.d, ED, P, {&x, &l.p[kInW], &l.p[kOutW], &l.xp, &l.dtp, &l.p[kInB], &l.p[kOutB]});
         auto product = [&](const Tensor& in, int64_t K, const Tensor& weight, const Tensor& bias) {
             const int64_t M = weight.size(0);
             const Tensor y = empty({T, M}, dt, x);
@@ -198,7 +198,7 @@ variable_list MixerBackward::apply(variable_list&& grads) {
     auto at_col = [&](const Tensor& t, int64_t col) { return static_cast<char*>(ptr(t)) + col * es; };
     const Tensor x2 = x_.view({T, d}), dout = cast(grads[0], dt).contiguous().view({T, d});
 
-    const bool own = use_linear(dt, T, d, ED, P, {&dout, &w[kIOutW], &w[kIInW], &xp, &dtp});
+    const bool own = use_linear(dt, true, T, d, ED, P, {&dout, &w[kIOutW], &w[kIInW], &xp, &dtp});
     // out (T x M) = in (T x K) . weight (K x M), or added to out
     auto product = [&](const void* in, int64_t in_pitch, int64_t K, const Tensor& weight, void* out, int64_t out_pitch, bool add) {
         mpa_linear q = linear_of(io, T, in, in_pitch, K, ptr(weight), weight.size(1), out, out_pitch);
