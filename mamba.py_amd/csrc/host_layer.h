@@ -514,12 +514,13 @@ inline void run_linear(const mpa_linear& q, void* stream) { check(mpa_linear_run
 template <typename H>
 inline H* handle_in(PyObject* dict) {
     PyObject* o = get(dict, keys().handle);
-    if (!o || o == Py_None || !py::cast<H*>(py::handle(o))->belongs_to(dict)) {
-        const py::object h = py::cast(new H(dict), py::return_value_policy::take_ownership);
-        PyDict_SetItem(dict, keys().handle, h.ptr());
-        o = h.ptr();
+    if (o && o != Py_None) {
+        H* h = py::cast<H*>(py::handle(o));
+        if (h->belongs_to(dict)) return h;
     }
-    return py::cast<H*>(py::handle(o));
+    const py::object h = py::cast(new H(dict), py::return_value_policy::take_ownership);
+    PyDict_SetItem(dict, keys().handle, h.ptr());
+    return py::cast<H*>(h);
 }
 
 // The handle of a mixer that can run here, or null.

@@ -84,6 +84,7 @@ struct LinearParams {
     const void* residual;
     int accumulate;
     int y_f32, residual_f32;  // float32 whatever IO is
+    int x_larger;             // x has more bytes than W
     float* ssq_out;  // [M/32 rounded up][T]
 };
 
@@ -103,11 +104,15 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
     constexpr int kRows = BT + BM, kParts = 8 * KS, kLoads = kRows * kParts / kThreads, kStage = kRows * kParts;  // 16-byte parts
     static_assert(D % 2 == 0, "a set of registers always goes to the same buffer");
     __shared__ u32x4 lds[2][kStage];
-    // blocks of one XCD (every eighth) share rows of W: they walk the steps of a tile of W first
+    // Blocks of one XCD (every eighth) take neighbouring tiles and share one operand's rows in its L2: those of W, whose
+    // tiles' steps they walk first, or of x where that is the larger one (each XCD reads the other operand whole) and tiles
+    // are many (17 layers of width 528, 4038 steps: 2.27 -> 2.17 ms; below two rounds of tiles it made no difference).
     const int nt = (p.T + BT - 1) / BT, nm = (p.M + BM - 1) / BM, per = (nt * nm + 7) / 8;
     const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per || tile >= nt * nm) return;  // uniform over the block
-    const int m0 = tile / nt * BM, t0 = tile % nt * BT;
+    const bool by_steps = p.x_larger && nt * nm >= 512;
+    const int inner = by_steps ? nm : nt, major = tile / inner, minor = tile - major * inner;
+    const int m0 = (by_steps ? minor : major) * BM, t0 = (by_steps ? major : minor) * BT;
     const int lane = threadIdx.x & (kWave - 1), wave = wave_id();
     const int ks = wave % KS, wm = wave / KS % (BM / 32), wt = wave / KS / (BM / 32);
 
@@ -135,6 +140,11 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
                           : kXES * (koff[i] + (uint32_t)min(t0 + row - BM, p.T - 1) * (uint32_t)p.x_pitch);
         at[i] = (part >> 3) * (kRows * 8) + row * 8 + ((part & 7) ^ (row & 7));
     }
+    // first of the four columns of the result that a lane holds of tile i
+    auto column = [&](int i) {
+        const int u = wm * 32 + i * 16 + (lane >> 4) * 4;
+        return m0 + (NN && kVec == 8 ? u % (BM / 2) * 2 + u / (BM / 2) * 4 : u);
+    };
     const int steps = (p.K + kStep * KS - 1) / (kStep * KS);
     struct Stage {
         u32x4 v[kLoads];
@@ -251,6 +261,26 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
         compute(i & 1);
         __syncthreads();
     }
+    // The lane's part of the residual, all of it requested at once and before the shares of K are added (one memory latency and
+    // not four; what lies beyond T or M is read from within and not used).
+    f32x4 res[2][2] = {};
+    if (p.residual && ks == 0) {
+        typename Ops::Out narrow[2][2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int64_t o = (int64_t)min(t0 + wt * 32 + j * 16 + fr, p.T - 1) * p.y_pitch + min(column(i), p.M - 4);
+                if (p.residual_f32) res[i][j] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p.residual) + o);
+                else narrow[i][j] = *reinterpret_cast<const typename Ops::Out*>(static_cast<const IO*>(p.residual) + o);
+            }
+        if (!p.residual_f32) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) res[i >> 1][i & 1][e] = Ops::get(narrow[i >> 1][i & 1], e);
+        }
+    }
     if constexpr (KS > 1) {
         // (the stages are done with: the last barrier)
         f32x4* part = reinterpret_cast<f32x4*>(&lds[0][0]);
@@ -268,8 +298,7 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
     float ss[2] = {0.0f, 0.0f};
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const int u = wm * 32 + i * 16 + fq * 4;
-        const int m = m0 + (NN && kVec == 8 ? u % (BM / 2) * 2 + u / (BM / 2) * 4 : u);
+        const int m = column(i);
         if (m >= p.M) continue;
         typename Ops::Out bias = {};
         if (p.bias) bias = *reinterpret_cast<const typename Ops::Out*>(static_cast<const IO*>(p.bias) + m);
@@ -278,27 +307,19 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
             const int t = t0 + wt * 32 + j * 16 + fr;
             if (t >= p.T) continue;
             const int64_t o = (int64_t)t * p.y_pitch + m;
-            f32x4 res = {};
-            if (p.residual_f32) {
-                res = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p.residual) + o);
-            } else if (p.residual) {
-                const typename Ops::Out r = *reinterpret_cast<const typename Ops::Out*>(static_cast<const IO*>(p.residual) + o);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) res[e] = Ops::get(r, e);
-            }
             f32x4 f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) f[e] = acc[i][j][e] + Ops::get(bias, e);
-            if (p.accumulate) f += res;
-            if (p.y_f32) {
-                if (p.residual && !p.accumulate) f += res;
+            if (p.accumulate) f += res[i][j];
+            if (sizeof(IO) == 4 || p.y_f32) {
+                if (p.residual && !p.accumulate) f += res[i][j];
                 *reinterpret_cast<f32x4*>(static_cast<float*>(p.y) + o) = f;
             } else {
                 typename Ops::Out v;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     Ops::set(v, e, f[e]);
-                    if (p.residual && !p.accumulate) Ops::set(v, e, Ops::get(v, e) + res[e]);
+                    if (p.residual && !p.accumulate) Ops::set(v, e, Ops::get(v, e) + res[i][j][e]);
                     f[e] = Ops::get(v, e);
                 }
                 *reinterpret_cast<typename Ops::Out*>(static_cast<IO*>(p.y) + o) = v;
@@ -377,6 +398,7 @@ extern "C" int mpa_linear_run(const mpa_linear* s, void* stream) {
     p.ssq = s->x_ssq; p.in_parts = (int)s->ssq_parts;
     p.inv_d = 1.0f / (float)s->K; p.eps = s->eps; p.norm_w = s->norm_weight;
     p.residual = s->residual;
+    p.x_larger = s->T * (x_f32 || f32 ? 4 : 2) > s->M * (f32 ? 4 : 2);
     p.y_f32 = y_f32; p.residual_f32 = residual_f32 && s->residual;
     p.accumulate = s->accumulate; p.ssq_out = s->y_ssq;
     hipStream_t st = static_cast<hipStream_t>(stream);
