@@ -321,7 +321,7 @@ int mpa_ssm_step(const void* x, const void* delta, const float* A, const void* B
  * Replaces, for one token of each of up to MPA_DECODE_MAX_BATCH sequences, the chain that
  * ResidualBlock.step / MambaBlock.step run (mambapy/mamba.py:114-125, 351-414): RMSNorm, in_proj, the
  * convolution over the rolling window with silu, x_proj, dt_proj, the state update with softplus, the
- * gate, out_proj, residual add; four launches.
+ * gate, out_proj, residual add; three or four launches.
  *   x, y : (batch, d_model) io_dtype contiguous.  norm = 1: y = x + block(rmsnorm(x)), the residual block;
  *     norm = 0: y = block(x), the mixer alone.  y may not alias x.
  *   x_scaled, x_ssq  optional (norm = 1): x times norm_weight in io_dtype, in the order in which the matrix

@@ -39,12 +39,12 @@ def _hipcc() -> str:
 
 
 def source_hash() -> str:
-    """sha256 over the kernel sources (csrc/*.hip, csrc/*.h and the public header, by name) and the
-    compiler flags.  The
+    """sha256 over the kernel sources (csrc/*.hip, the csrc/*.h they include and the public header, by name) and
+    the compiler flags; csrc/host* is the other extension's.  The
     library is built with this string inside (mpa_source_hash()); a profile summary that quotes
     counters of a kernel names the hash of the sources it was measured on."""
     h = hashlib.sha256()
-    files = sorted(f for f in os.listdir(CSRC) if f.endswith((".hip", ".h")))
+    files = sorted(f for f in os.listdir(CSRC) if f.endswith((".hip", ".h")) and not f.startswith("host"))
     for path in [os.path.join(CSRC, f) for f in files] + [os.path.join(_HERE, "..", "include", "mambapy_amd.h")]:
         h.update(os.path.basename(path).encode() + b"\0")
         h.update(open(path, "rb").read())

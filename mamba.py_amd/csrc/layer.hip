@@ -2,8 +2,8 @@
 //
 //   wgrad      weight gradients out = P^T . Q of several projections in one launch (P (T, M) the
 //              gradient of a projection's output, Q (T, N) its input, T = batch * length rows)
-//   prepare    the float32 and padded forms of a layer's parameters, in one launch
-//   finish     the float32 gradients of its small parameters in the parameters' own types, in one launch
+//   cast       up to a dozen conversions of small matrices in one launch: the float32 and padded forms of a layer's
+//              parameters before a pass, the float32 gradients of its small parameters in their own types after it
 //
 // wgrad.  The sum runs over thousands of rows and gives a matrix of a few hundred rows and columns, so
 // a kernel that parallelises over the output alone leaves most of the chip idle: as library GEMMs

@@ -13,9 +13,10 @@
 // share: a stage is staged in LDS in 16-byte parts, rotated by the row (part ^ (row & 7)) so that the operand reads, one row
 // per lane, fall on different banks; D stages are in registers on their way in, two in LDS.
 //
-// At 512 steps the kernels are as fast as the library's in a queue that never runs dry (9.0 / 6.7 / 3.7 / 7.9 us for
-// in_proj, x_proj, dt_proj and out_proj of width 768, the library 9.3 / 5.1 / 5.2 / 8.2 us); what they save is
-// the norm between the layers (6 us) and three quarters of the host time (24 layers: 2.1 ms, all of it host).
+// At 512 steps of width 768, recorded in a graph with the weights of 24 layers: in_proj with the norm in it 12.8 us (11.9 with
+// bfloat16 rows, 9.7 without the norm), x_proj 7.3, dt_proj 3.8, out_proj with the residual stream 8.8 (8.6 without); the
+// library's products alone 9.3, 7.1, 3.9 and 8.0.  What the kernels save is the norm between the layers (6 us) and three
+// quarters of the host time (24 layers of library calls: 2.1 ms, all of it host).
 // float32 runs the same tiles with sixteen times less of the matrix unit's rate (16x16x4, 150 TFLOP/s): the same host
 // time is saved, until the product itself is longer than a library call (a training layer of 1614 steps and width 424
 // 0.69 ms, 0.81 with library calls; 168 steps of ten layers of width 640 without gradients 0.63 and 0.85 ms).

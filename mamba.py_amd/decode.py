@@ -1,8 +1,7 @@
 """Decode loop captured in a HIP graph.
 
-One decode step of a Mamba stack is a few dozen small kernels per layer (projections at batch
-size B, the conv window, the state-update kernel, norms): at decode batch sizes the time goes
-into launching them, not into running them.  `GraphedDecoder` records one step of
+One decode step of a Mamba stack is three or four small kernels per layer (a dozen where a layer
+is not of the plain kind): at decode batch sizes much of the time goes into launching them.  `GraphedDecoder` records one step of
 `LM.step` (or of a bare `Mamba` stack) into a graph once and replays it per token; the
 recurrent state and the conv windows live in fixed buffers that the step updates in place, so a
 replay allocates nothing and launches everything with one call.
@@ -28,8 +27,9 @@ class GraphedDecoder:
     The returned tensor is the decoder's output buffer: it is overwritten by the next call.
     Weights are read from the model's own tensors at replay time, except the float32 forms of
     the small parameters (A, D, biases, conv and norm weights), which live in per-module buffers
-    that an eager forward/step refreshes in place after a weight update; build a new decoder
-    (or run one eager step) after changing those.
+    that an eager forward/step refreshes in place after a weight update (one that moves the parameter's version
+    counter, or any that follows a call with gradients); run one eager step after changing those, or build a new
+    decoder.
     """
 
     def __init__(self, model, caches, warmup: int = 2):

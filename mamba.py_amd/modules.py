@@ -4,9 +4,13 @@ These classes mirror the reference's public surface (constructor arguments, meth
 tensor shapes and `state_dict` keys) so that a model built or trained with mambapy loads
 here and the other way round:
     MambaConfig, MambaBlock, ResidualBlock, Mamba, RMSNorm      mambapy/mamba.py:31-433
-They are the harness around the kernels, not the product: projections, the depthwise
-convolution and the norms stay on PyTorch-ROCm library calls; the scan, its backward and the
-decode-step state update run in libmambapy_amd.so.
+Every class runs module by module in Python, on the package's operators (scan, convolution, norms) and
+torch's projections, and in one native call where it is of the plain kind (csrc/host_model.cpp, host_train.cpp): a
+block with gradients as one graph node, a stack without them, a decode step; small projections, weight gradients
+and the decode step's products are the package's own kernels there.  Both ways give the same results up to
+rounding (a bfloat16 stack over a short sequence is nearer to float64 natively: its residual stream is float32).
+Calls without gradients keep float32 and padded forms of the weights: they see changes that move a version counter or
+a pointer, those made through .data once a call with gradients has run in between.
 """
 import math
 from dataclasses import dataclass
