@@ -13,8 +13,8 @@
 // share: a stage is staged in LDS in 16-byte parts, rotated by the row (part ^ (row & 7)) so that the operand reads, one row
 // per lane, fall on different banks; D stages are in registers on their way in, two in LDS.
 //
-// At 512 steps of width 768, recorded in a graph with the weights of 24 layers: in_proj with the norm in it 12.8 us (11.9 with
-// bfloat16 rows, 9.7 without the norm), x_proj 7.3, dt_proj 3.8, out_proj with the residual stream 8.8 (8.6 without); the
+// At 512 steps of width 768, recorded in a graph with the weights of 24 layers: in_proj with the norm in it 12.7 us (11.9 with
+// bfloat16 rows, 9.3 without the norm), x_proj 7.1, dt_proj 3.7, out_proj with the residual stream 8.8 (8.5 without); the
 // library's products alone 9.3, 7.1, 3.9 and 8.0.  What the kernels save is the norm between the layers (6 us) and three
 // quarters of the host time (24 layers of library calls: 2.1 ms, all of it host).
 // float32 runs the same tiles with sixteen times less of the matrix unit's rate (16x16x4, 150 TFLOP/s): the same host
@@ -73,19 +73,24 @@ struct LinearOps<float> {
     }
 };
 
+// (one word next to the sizes, in registers from the start: a scalar load at the end of the kernel is a latency by itself)
+enum LinearFlags {
+    kAccumulate = 1,   // the residual is added before the result is rounded
+    kYF32 = 2,         // y is float32 whatever IO is
+    kResidualF32 = 4,  // so is the residual
+    kXLarger = 8,      // x has more bytes than W
+};
 struct LinearParams {
     const void *x, *w, *bias;
     int64_t x_pitch, y_pitch;
     int T, M, K;
+    int flags;  // LinearFlags
     void* y;
     const float* ssq;  // [in_parts][T]
     int in_parts;
     float inv_d, eps;
     const float* norm_w;  // [K], with ssq
     const void* residual;
-    int accumulate;
-    int y_f32, residual_f32;  // float32 whatever IO is
-    int x_larger;             // x has more bytes than W
     float* ssq_out;  // [M/32 rounded up][T]
 };
 
@@ -108,10 +113,11 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
     // Blocks of one XCD (every eighth) take neighbouring tiles and share one operand's rows in its L2: those of W, whose
     // tiles' steps they walk first, or of x where that is the larger one (each XCD reads the other operand whole) and tiles
     // are many (17 layers of width 528, 4038 steps: 2.27 -> 2.17 ms; below two rounds of tiles it made no difference).
+    const int flags = p.flags;
     const int nt = (p.T + BT - 1) / BT, nm = (p.M + BM - 1) / BM, per = (nt * nm + 7) / 8;
     const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per || tile >= nt * nm) return;  // uniform over the block
-    const bool by_steps = p.x_larger && nt * nm >= 512;
+    const bool by_steps = (flags & kXLarger) && nt * nm >= 512;
     const int inner = by_steps ? nm : nt, major = tile / inner, minor = tile - major * inner;
     const int m0 = (by_steps ? minor : major) * BM, t0 = (by_steps ? major : minor) * BT;
     const int lane = threadIdx.x & (kWave - 1), wave = wave_id();
@@ -272,10 +278,10 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int64_t o = (int64_t)min(t0 + wt * 32 + j * 16 + fr, p.T - 1) * p.y_pitch + min(column(i), p.M - 4);
-                if (p.residual_f32) res[i][j] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p.residual) + o);
+                if (flags & kResidualF32) res[i][j] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p.residual) + o);
                 else narrow[i][j] = *reinterpret_cast<const typename Ops::Out*>(static_cast<const IO*>(p.residual) + o);
             }
-        if (!p.residual_f32) {
+        if (!(flags & kResidualF32)) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -311,16 +317,16 @@ __global__ void __launch_bounds__(BT / 32 * (BM / 32) * KS * kWave) linear_kerne
             f32x4 f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) f[e] = acc[i][j][e] + Ops::get(bias, e);
-            if (p.accumulate) f += res[i][j];
-            if (sizeof(IO) == 4 || p.y_f32) {
-                if (p.residual && !p.accumulate) f += res[i][j];
+            if (flags & kAccumulate) f += res[i][j];
+            if (sizeof(IO) == 4 || (flags & kYF32)) {
+                if (p.residual && !(flags & kAccumulate)) f += res[i][j];
                 *reinterpret_cast<f32x4*>(static_cast<float*>(p.y) + o) = f;
             } else {
                 typename Ops::Out v;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     Ops::set(v, e, f[e]);
-                    if (p.residual && !p.accumulate) Ops::set(v, e, Ops::get(v, e) + res[i][j][e]);
+                    if (p.residual && !(flags & kAccumulate)) Ops::set(v, e, Ops::get(v, e) + res[i][j][e]);
                     f[e] = Ops::get(v, e);
                 }
                 *reinterpret_cast<typename Ops::Out*>(static_cast<IO*>(p.y) + o) = v;
@@ -399,9 +405,9 @@ extern "C" int mpa_linear_run(const mpa_linear* s, void* stream) {
     p.ssq = s->x_ssq; p.in_parts = (int)s->ssq_parts;
     p.inv_d = 1.0f / (float)s->K; p.eps = s->eps; p.norm_w = s->norm_weight;
     p.residual = s->residual;
-    p.x_larger = s->T * (x_f32 || f32 ? 4 : 2) > s->M * (f32 ? 4 : 2);
-    p.y_f32 = y_f32; p.residual_f32 = residual_f32 && s->residual;
-    p.accumulate = s->accumulate; p.ssq_out = s->y_ssq;
+    p.ssq_out = s->y_ssq;
+    p.flags = (s->accumulate ? kAccumulate : 0) | (y_f32 ? kYF32 : 0) | (residual_f32 ? kResidualF32 : 0) |
+              (s->T * (x_f32 || f32 ? 4 : 2) > s->M * (f32 ? 4 : 2) ? kXLarger : 0);
     hipStream_t st = static_cast<hipStream_t>(stream);
     return f32 ? dispatch_linear<float>(p, s->weight_kxm != 0, x_f32, st) : dispatch_linear<bf16_t>(p, s->weight_kxm != 0, x_f32, st);
 }
