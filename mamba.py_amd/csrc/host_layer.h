@@ -47,6 +47,15 @@ inline PyObject* dict_of(PyObject* module) {
     return d ? *d : nullptr;
 }
 inline PyObject* get(PyObject* dict, PyObject* k) { return dict ? PyDict_GetItem(dict, k) : nullptr; }
+// A number that no two states of any dictionaries share (PEP 509); where Python has none, never the same twice.
+inline uint64_t state_of(PyObject* dict) {
+#if PY_VERSION_HEX < 0x030C0000
+    return reinterpret_cast<PyDictObject*>(dict)->ma_version_tag;
+#else
+    static uint64_t n = 0;
+    return ++n;
+#endif
+}
 
 inline bool empty_dict(PyObject* o) { return o && PyDict_Check(o) && PyDict_Size(o) == 0; }
 
@@ -70,22 +79,41 @@ struct Types {
 };
 inline Types* types = nullptr;  // set by register_types, kept for the interpreter's lifetime
 
-// nothing on the module itself changes or watches its calls
-inline bool plain_instance(PyObject* dict, const std::vector<Ref>& names) {
-    if (!dict) return false;
-    for (const Ref& n : names)
-        if (get(dict, n.o)) return false;
-    for (PyObject* k : keys().hooks)
-        if (!empty_dict(get(dict, k))) return false;
-    return true;
-}
-// the instance dictionary of the plain submodule under `name`, or null
-inline PyObject* plain_sub(PyObject* modules, PyObject* name, const py::object& type, const std::vector<Ref>& names) {
-    PyObject* m = get(modules, name);
-    if (!m || (PyObject*)Py_TYPE(m) != type.ptr()) return nullptr;
-    PyObject* d = dict_of(m);
-    return plain_instance(d, names) ? d : nullptr;
-}
+// A module's instance dictionary, looked through again when it has changed (fifteen look-ups; a layer has seven).
+struct Instance {
+    uint64_t state = 0, params_state = 0;
+    PyObject *params = nullptr, *hooks[4] = {};
+    PyObject* pair[2] = {};  // what its _parameters hold under two names, in params_state
+    // nothing on the module itself changes or watches its calls
+    bool plain(PyObject* dict, const std::vector<Ref>& names) {
+        if (!dict) return false;
+        if (state_of(dict) != state) {
+            state = 0;
+            for (const Ref& n : names)
+                if (get(dict, n.o)) return false;
+            for (int i = 0; i < 4; ++i) hooks[i] = get(dict, keys().hooks[i]);
+            params = get(dict, keys().params);
+            if (!params || !PyDict_Check(params)) return false;
+            state = state_of(dict);
+        }
+        for (PyObject* h : hooks)
+            if (!empty_dict(h)) return false;
+        return true;
+    }
+    void find(PyObject* first, PyObject* second) {  // (always the same two)
+        if (state_of(params) == params_state) return;
+        pair[0] = get(params, first);
+        pair[1] = get(params, second);
+        params_state = state_of(params);
+    }
+    // the instance dictionary of the plain submodule under `name`, or null
+    PyObject* sub(PyObject* modules, PyObject* name, const py::object& type, const std::vector<Ref>& names) {
+        PyObject* m = get(modules, name);
+        if (!m || (PyObject*)Py_TYPE(m) != type.ptr()) return nullptr;
+        PyObject* d = dict_of(m);
+        return plain(d, names) ? d : nullptr;
+    }
+};
 
 // A parameter and the state it was last seen in.
 struct Param {
@@ -93,11 +121,10 @@ struct Param {
     const void* impl = nullptr;
     const void* data = nullptr;
     uint32_t version = 0;
-    // Takes over what `params` holds under `name`, None for no parameter; false if it holds neither that nor a plain tensor
-    // (pruning and parametrisation take the name away).  An inference tensor has no version counter and may
+    // Takes over what a module's _parameters hold under the name, None for no parameter; false if it is neither that nor a
+    // plain tensor (pruning and parametrisation take the name away).  An inference tensor has no version counter and may
     // always have changed.
-    bool look(PyObject* params, PyObject* name, bool& changed) {
-        PyObject* o = get(params, name);
+    bool take(PyObject* o, bool& changed) {
         if (o == Py_None) {
             if (impl) {
                 changed = true;
@@ -236,7 +263,7 @@ struct Weights : LayerSizes {
         const Tensor& w = p[kInW];
         std::vector<mpa_cast_job> jobs;
         auto f32 = [&](const Tensor& q) {
-            if (!q.defined() || q.scalar_type() == at::kFloat) return q.defined() ? q.detach() : q;
+            if (!q.defined() || q.scalar_type() == at::kFloat) return q;
             const Tensor t = empty(q.sizes(), at::kFloat, q);
             jobs.push_back(row_job(q, t));
             return t;
@@ -287,7 +314,9 @@ struct MixerHandle : LayerSizes {
     bool decode_ok = false;   // the shapes are such as mpa_decode_layer_step takes
     bool forward_ok = false;  // ... as stack_forward and block_train take
     Ref modules;
+    Instance self, in_proj, conv1d, x_proj, dt_proj, out_proj;
     Ref sizes[7];  // values of the config, by Keys::sizes
+    uint64_t config_state = 0;
     Param p[kParams];
     bool fused_softplus = true;
     // Forms kept for calls without gradients, and the epoch they are of.  Version counters do not show every change
@@ -306,29 +335,26 @@ struct MixerHandle : LayerSizes {
     // Whether the block with this __dict__ can run here with activations like x.
     bool ready(PyObject* dict, const Tensor& x) {
         const Keys& k = keys();
-        if (!plain_instance(dict, types->block_names) || get(dict, k.dt_layernorm) != Py_None) return false;
+        if (!self.plain(dict, types->block_names) || get(dict, k.dt_layernorm) != Py_None) return false;
         PyObject* mm = modules.o;
-        PyObject* const in = plain_sub(mm, k.in_proj, types->linear, types->linear_names);
-        PyObject* const conv = plain_sub(mm, k.conv1d, types->conv, types->linear_names);
-        PyObject* const xp = plain_sub(mm, k.x_proj, types->linear, types->linear_names);
-        PyObject* const dtp = plain_sub(mm, k.dt_proj, types->linear, types->linear_names);
-        PyObject* const out = plain_sub(mm, k.out_proj, types->linear, types->linear_names);
-        if (!in || !conv || !xp || !dtp || !out) return false;
+        if (!in_proj.sub(mm, k.in_proj, types->linear, types->linear_names) || !conv1d.sub(mm, k.conv1d, types->conv, types->linear_names) ||
+            !x_proj.sub(mm, k.x_proj, types->linear, types->linear_names) || !dt_proj.sub(mm, k.dt_proj, types->linear, types->linear_names) ||
+            !out_proj.sub(mm, k.out_proj, types->linear, types->linear_names))
+            return false;
         bool changed = false;
         if (!read_config(get(dict, k.config), changed)) return false;
-        PyObject* const params = get(dict, k.params);
-        const bool there = both(in, kInW, kInB, changed) && both(conv, kConvW, kConvB, changed) && both(xp, kXW, kXB, changed) &&
-                           both(dtp, kDtW, kDtB, changed) && both(out, kOutW, kOutB, changed) && p[kALog].look(params, k.A_log, changed) &&
-                           p[kD].look(params, k.D, changed);
+        const bool there = look(in_proj, kInW, k.weight, kInB, k.bias, changed) && look(conv1d, kConvW, k.weight, kConvB, k.bias, changed) &&
+                           look(x_proj, kXW, k.weight, kXB, k.bias, changed) && look(dt_proj, kDtW, k.weight, kDtB, k.bias, changed) &&
+                           look(out_proj, kOutW, k.weight, kOutB, k.bias, changed) && look(self, kALog, k.A_log, kD, k.D, changed);
         if (changed) epoch = next_epoch();
         if (changed && !there) forget();
         decode_ok = forward_ok = false;
         if (there) look_over();
         return (decode_ok || forward_ok) && x.scalar_type() == dt && x.device() == device && x.size(-1) == d;
     }
-    bool both(PyObject* dict, int weight, int bias, bool& changed) {
-        PyObject* params = get(dict, keys().params);
-        return p[weight].look(params, keys().weight, changed) && p[bias].look(params, keys().bias, changed);
+    bool look(Instance& m, int i, PyObject* name_i, int j, PyObject* name_j, bool& changed) {
+        m.find(name_i, name_j);
+        return p[i].take(m.pair[0], changed) && p[j].take(m.pair[1], changed);
     }
     // (what has been taken over before a parameter was found missing is looked over again once it is back)
     void forget() {
@@ -336,6 +362,10 @@ struct MixerHandle : LayerSizes {
     }
     bool read_config(PyObject* config, bool& changed) {
         PyObject* dict = config ? dict_of(config) : nullptr;
+        if (!dict) return false;
+        const uint64_t state = state_of(dict);
+        if (state == config_state) return PyObject_IsTrue(sizes[5].o) == 0;
+        config_state = 0;
         PyObject* v[7];
         bool same = true;
         for (int i = 0; i < 7; ++i) {
@@ -352,6 +382,7 @@ struct MixerHandle : LayerSizes {
             fused_softplus = PyObject_IsTrue(sizes[6].o) == 1;
             xp = dtp = Tensor();  // (their zeros are elsewhere)
         }
+        config_state = state;
         return PyObject_IsTrue(sizes[5].o) == 0;
     }
 
@@ -401,6 +432,7 @@ struct MixerHandle : LayerSizes {
 // The norm in front of a mixer.
 struct NormHandle {
     bool changed = false;
+    Instance norm;
     Ref modules, eps_seen;
     Param p;
     double eps = 0;
@@ -411,7 +443,7 @@ struct NormHandle {
     bool belongs_to(PyObject* dict) const { return get(dict, keys().modules) == modules.o; }
     bool ready(const MixerHandle& m) {
         const Keys& k = keys();
-        PyObject* const d = plain_sub(modules.o, k.norm, types->norm, types->norm_names);
+        PyObject* const d = norm.sub(modules.o, k.norm, types->norm, types->norm_names);
         if (!d) return false;
         PyObject *const e = get(d, k.eps), *const gainless = get(d, k.use_mup);
         if (!e || !gainless) return false;
@@ -422,7 +454,7 @@ struct NormHandle {
         if (PyObject_IsTrue(gainless) == 1) {
             changed |= p.impl != nullptr;
             p = Param{};
-        } else if (!p.look(get(d, k.params), k.weight, changed)) {
+        } else if (norm.find(k.weight, k.bias); !p.take(norm.pair[0], changed)) {
             return false;
         }
         const Tensor& t = p.t;
