@@ -917,8 +917,8 @@ __global__ void __launch_bounds__(256) seg_carry_kernel(const float* __restrict_
 // Segments per batch row.  The scan is serial in time, so a launch has only batch * dim/64
 // workgroups; when those cover a fraction of the chip's 256 CUs the sequence is cut into
 // segments that run side by side: up to twice the arithmetic, nseg times the parallelism.
-// `thin` is the coverage below which the cut pays: a third of the CUs for the forward (its first
-// pass costs 0.8 of the second), half of them for the backward (its first pass costs a quarter).
+// `thin` is the coverage below which the cut pays: half of the CUs for the backward (its first pass costs a quarter of
+// the second), a third for a forward whose plan the caller pins (0.8 of it; otherwise fwd_plan decides by an estimate).
 SegPlan seg_layout(const mpa_sscan_shape* s, int64_t want) {
     SegPlan sp{1, 0, 0, 0, 0, 0};
     const int64_t ntiles = (s->seqlen + kTile - 1) / kTile;
