@@ -115,33 +115,34 @@ struct Instance {
     }
 };
 
-// A parameter and the state it was last seen in.
+// The state a parameter was last seen in.  The tensor is not held beyond a call, not even weakly: a model that moves away
+// takes its memory along, and its tensors can be swapped.  What tells another tensor at the same addresses from the old
+// one is the old one's version counter, which is held: a tensor that is gone leaves it to us alone.
 struct Param {
-    Tensor t;
     const void* impl = nullptr;
     const void* data = nullptr;
+    std::optional<c10::VariableVersion> counter;
     uint32_t version = 0;
     // Takes over what a module's _parameters hold under the name, None for no parameter; false if it is neither that nor a
     // plain tensor (pruning and parametrisation take the name away).  An inference tensor has no version counter and may
     // always have changed.
-    bool take(PyObject* o, bool& changed) {
+    bool take(PyObject* o, Tensor& now, bool& changed) {
         if (o == Py_None) {
-            if (impl) {
-                changed = true;
-                *this = Param{};
-            }
+            changed |= impl != nullptr;
+            *this = Param{};
             return true;
         }
         if (!o || !THPVariable_CheckExact(o)) return false;
-        const Tensor& now = THPVariable_Unpack(o);
+        now = THPVariable_Unpack(o);
         if (wrapped(now)) return false;
-        const void* im = now.unsafeGetTensorImpl();
+        const c10::TensorImpl* im = now.unsafeGetTensorImpl();
         const bool counted = !now.is_inference();
-        if (counted && im == impl && now.const_data_ptr() == data && now._version() == version) return true;
+        if (counted && im == impl && counter && !counter->unique() && now.const_data_ptr() == data && now._version() == version) return true;
         changed = true;
-        t = now;
         impl = im;
         data = now.const_data_ptr();
+        counter.reset();
+        if (counted) counter.emplace(im->version_counter());
         version = counted ? now._version() : 0;
         return true;
     }
@@ -183,13 +184,12 @@ inline mpa_cast_job zero_job(const Tensor& dst, int64_t rows, int64_t cols, int6
 }
 // float32 form of a small parameter: the parameter itself when it is that already, else a buffer
 struct F32 {
-    Tensor t, own;
-    void take(const Tensor& p, std::vector<mpa_cast_job>& jobs) {
-        t = Tensor();
-        if (!p.defined()) return;
-        if (p.scalar_type() == at::kFloat) { t = p.detach(); return; }
-        t = derived(own, p.sizes(), at::kFloat, p);
-        jobs.push_back(row_job(p, own));
+    Tensor own;
+    Tensor form(const Tensor& p, bool old, std::vector<mpa_cast_job>& jobs) {
+        if (!p.defined() || p.scalar_type() == at::kFloat) return p;
+        derived(own, p.sizes(), at::kFloat, p);
+        if (old) jobs.push_back(row_job(p, own));
+        return own;
     }
 };
 
@@ -243,8 +243,8 @@ struct LayerSizes {
 struct Weights : LayerSizes {
     Tensor p[kParams];
     Tensor conv_w, conv_b, dt_b, D;              // float32
-    Tensor A;                                    // -exp(A_log), float32
-    Tensor in_wt, out_wt, xp, dtp, xp_t, dtp_t;  // (transposed views of) the GEMM weights
+    Tensor A;                        // -exp(A_log), float32
+    Tensor xp, dtp;                  // x_proj and dt_proj, padded
 
     // x_proj and dt_proj in the shape the GEMM library serves best: the low-rank width R is the K of
     // dt_proj and R + 2N the rows of x_proj, both odd for its tiles (48 and 80 at width 768).  With R
@@ -322,18 +322,17 @@ struct MixerHandle : LayerSizes {
     // Forms kept for calls without gradients, and the epoch they are of.  Version counters do not show every change
     // of a parameter (writes through .data), and a training loop makes one after each of its calls: a call with
     // gradients forms its own and begins an epoch.
-    uint64_t epoch = next_epoch(), formed = 0, padded = 0;  // padded: that of xp .. dtp_t
+    uint64_t epoch = next_epoch(), formed = 0, padded = 0;  // padded: that of xp and dtp
     Written written;
     F32 conv_w, conv_b, dt_b, D;
     Tensor A, xp, dtp;  // (xp and dtp: where the layer's own shapes are padded)
-    std::shared_ptr<const Weights> kept;
 
     explicit MixerHandle(PyObject* dict) : modules(get(dict, keys().modules)) {}
     // the dictionaries are those of this block (a shallow copy brings the handle of its original along)
     bool belongs_to(PyObject* dict) const { return get(dict, keys().modules) == modules.o; }
 
-    // Whether the block with this __dict__ can run here with activations like x.
-    bool ready(PyObject* dict, const Tensor& x) {
+    // Whether the block with this __dict__ can run here with activations like x; its sizes and parameters.
+    bool ready(PyObject* dict, const Tensor& x, Weights& w) {
         const Keys& k = keys();
         if (!self.plain(dict, types->block_names) || get(dict, k.dt_layernorm) != Py_None) return false;
         PyObject* mm = modules.o;
@@ -343,18 +342,19 @@ struct MixerHandle : LayerSizes {
             return false;
         bool changed = false;
         if (!read_config(get(dict, k.config), changed)) return false;
-        const bool there = look(in_proj, kInW, k.weight, kInB, k.bias, changed) && look(conv1d, kConvW, k.weight, kConvB, k.bias, changed) &&
-                           look(x_proj, kXW, k.weight, kXB, k.bias, changed) && look(dt_proj, kDtW, k.weight, kDtB, k.bias, changed) &&
-                           look(out_proj, kOutW, k.weight, kOutB, k.bias, changed) && look(self, kALog, k.A_log, kD, k.D, changed);
+        auto take = [&](Instance& m, int i, PyObject* name_i, int j, PyObject* name_j) {
+            m.find(name_i, name_j);
+            return p[i].take(m.pair[0], w.p[i], changed) && p[j].take(m.pair[1], w.p[j], changed);
+        };
+        const bool there = take(in_proj, kInW, k.weight, kInB, k.bias) && take(conv1d, kConvW, k.weight, kConvB, k.bias) &&
+                           take(x_proj, kXW, k.weight, kXB, k.bias) && take(dt_proj, kDtW, k.weight, kDtB, k.bias) &&
+                           take(out_proj, kOutW, k.weight, kOutB, k.bias) && take(self, kALog, k.A_log, kD, k.D);
         if (changed) epoch = next_epoch();
         if (changed && !there) forget();
         decode_ok = forward_ok = false;
-        if (there) look_over();
+        if (there) look_over(w);
+        static_cast<LayerSizes&>(w) = *this;
         return (decode_ok || forward_ok) && x.scalar_type() == dt && x.device() == device && x.size(-1) == d;
-    }
-    bool look(Instance& m, int i, PyObject* name_i, int j, PyObject* name_j, bool& changed) {
-        m.find(name_i, name_j);
-        return p[i].take(m.pair[0], changed) && p[j].take(m.pair[1], changed);
     }
     // (what has been taken over before a parameter was found missing is looked over again once it is back)
     void forget() {
@@ -388,45 +388,39 @@ struct MixerHandle : LayerSizes {
 
     void expire() { epoch = next_epoch(); }
 
-    void look_over() {
-        const Tensor& w = p[kInW].t;
+    void look_over(const Weights& all) {
+        const Tensor* const t = all.p;
+        const Tensor& w = t[kInW];
         if (d <= 0 || R <= 0 || N <= 0 || !w.defined() || !w.is_cuda() || (w.scalar_type() != at::kFloat && w.scalar_type() != at::kBFloat16)) return;
         dt = w.scalar_type();
         device = w.device();
         for (int i : {kInW, kXW, kDtW, kOutW, kInB, kOutB}) {
-            const Tensor& t = p[i].t;
+            const Tensor& v = t[i];
             const bool optional = i == kInB || i == kOutB;
-            if (!t.defined() && optional) continue;
-            if (!t.defined() || t.scalar_type() != dt || t.device() != device || !t.is_contiguous()) return;
+            if (!v.defined() && optional) continue;
+            if (!v.defined() || v.scalar_type() != dt || v.device() != device || !v.is_contiguous()) return;
         }
         for (int i : {kConvW, kConvB, kDtB, kALog, kD})
-            if (p[i].t.defined() && !small_ok(p[i].t, device)) return;
-        if (!p[kConvW].t.defined() || !p[kALog].t.defined() || !p[kD].t.defined() || p[kXB].t.defined()) return;
-        if (p[kInW].t.sizes() != at::IntArrayRef({2 * ED, d}) || p[kXW].t.sizes() != at::IntArrayRef({R + 2 * N, ED}) ||
-            p[kDtW].t.sizes() != at::IntArrayRef({ED, R}) || p[kOutW].t.sizes() != at::IntArrayRef({d, ED}) ||
-            p[kConvW].t.numel() != ED * K || p[kALog].t.sizes() != at::IntArrayRef({ED, N}) || p[kD].t.numel() != ED)
+            if (t[i].defined() && !small_ok(t[i], device)) return;
+        if (!t[kConvW].defined() || !t[kALog].defined() || !t[kD].defined() || t[kXB].defined()) return;
+        if (t[kInW].sizes() != at::IntArrayRef({2 * ED, d}) || t[kXW].sizes() != at::IntArrayRef({R + 2 * N, ED}) ||
+            t[kDtW].sizes() != at::IntArrayRef({ED, R}) || t[kOutW].sizes() != at::IntArrayRef({d, ED}) ||
+            t[kConvW].numel() != ED * K || t[kALog].sizes() != at::IntArrayRef({ED, N}) || t[kD].numel() != ED)
             return;
         for (const auto& [i, n] : {std::pair<int, int64_t>{kInB, 2 * ED}, {kConvB, ED}, {kDtB, ED}, {kOutB, d}})
-            if (p[i].t.defined() && p[i].t.numel() != n) return;
+            if (t[i].defined() && t[i].numel() != n) return;
         const int64_t vec = dt == at::kFloat ? 4 : 8;
         decode_ok = K >= 2 && K <= 4 && d % vec == 0 && ED % vec == 0 && N % 4 == 0 && N <= MPA_MAX_DSTATE && R <= 2048;
         for (int i : {kInW, kXW, kOutW}) decode_ok &= reinterpret_cast<uintptr_t>(p[i].data) % 16 == 0;
-        forward_ok = K >= 2 && K <= 4 && N <= MPA_MAX_DSTATE && fused_softplus && d % vec == 0 && d <= 512 * vec && p[kDtB].t.defined();
+        forward_ok = K >= 2 && K <= 4 && N <= MPA_MAX_DSTATE && fused_softplus && d % vec == 0 && d <= 512 * vec && t[kDtB].defined();
     }
     static bool small_ok(const Tensor& t, const c10::Device& device) {
         return t.device() == device && t.is_contiguous() && (t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16);
     }
 
-    Weights parameters() const {
-        Weights w;
-        static_cast<LayerSizes&>(w) = *this;
-        for (int i = 0; i < kParams; ++i) w.p[i] = p[i].t;
-        return w;
-    }
-
-    // The kept forms, up to date, xp .. dtp_t among them for a sequence, and those of the norm in front, if given; after
-    // ready().  Within a capture nothing runs yet: the next call still finds them old.
-    std::shared_ptr<const Weights> form(Forming& f, bool sequence, NormHandle* norm);
+    // Fills w, as ready() left it, with the kept forms, up to date: xp and dtp among them for a sequence; and norm_w, as the norm
+    // in front left it, if there is one.  Within a capture nothing runs yet: the next call still finds them old.
+    void form(Forming& f, bool sequence, Weights& w, NormHandle* norm, Tensor* norm_w);
 };
 
 // The norm in front of a mixer.
@@ -441,7 +435,7 @@ struct NormHandle {
 
     explicit NormHandle(PyObject* dict) : modules(get(dict, keys().modules)) {}
     bool belongs_to(PyObject* dict) const { return get(dict, keys().modules) == modules.o; }
-    bool ready(const MixerHandle& m) {
+    bool ready(const MixerHandle& m, Tensor& t) {  // t: the norm's weight
         const Keys& k = keys();
         PyObject* const d = norm.sub(modules.o, k.norm, types->norm, types->norm_names);
         if (!d) return false;
@@ -454,62 +448,45 @@ struct NormHandle {
         if (PyObject_IsTrue(gainless) == 1) {
             changed |= p.impl != nullptr;
             p = Param{};
-        } else if (norm.find(k.weight, k.bias); !p.take(norm.pair[0], changed)) {
+        } else if (norm.find(k.weight, k.bias); !p.take(norm.pair[0], t, changed)) {
             return false;
         }
-        const Tensor& t = p.t;
         return !t.defined() || (t.numel() == m.d && MixerHandle::small_ok(t, m.device) && reinterpret_cast<uintptr_t>(p.data) % 16 == 0);
     }
 };
 
-inline std::shared_ptr<const Weights> MixerHandle::form(Forming& f, bool sequence, NormHandle* norm) {
+inline void MixerHandle::form(Forming& f, bool sequence, Weights& w, NormHandle* norm, Tensor* norm_w) {
     f.before(written);
     const bool small = formed != epoch, wide = sequence && padded != epoch, gain = norm && (norm->changed || norm->formed != epoch);
     std::vector<mpa_cast_job> jobs;
-    const uint64_t of = f.capture ? 0 : epoch;
-    if (gain) norm->w.take(norm->p.t, jobs);
-    std::shared_ptr<Weights> w;
-    if (small || wide) {
-        w = std::make_shared<Weights>(parameters());
-        auto f32 = [&](F32& form, int i) {
-            if (small) form.take(p[i].t, jobs);
-            return form.t;
-        };
-        w->conv_w = f32(conv_w, kConvW);
-        w->conv_b = f32(conv_b, kConvB);
-        w->dt_b = f32(dt_b, kDtB);
-        w->D = f32(D, kD);
-        w->A = derived(A, {ED, N}, at::kFloat, w->p[kInW]);
-        if (small) jobs.push_back(cast_job(p[kALog].t, A, ED, N, 0, 0, MPA_CAST_NEG_EXP));
-        w->in_wt = w->p[kInW].detach().t();
-        w->out_wt = w->p[kOutW].detach().t();
-        if (sequence) {
-            const Tensor &xw = w->p[kXW], &dw = w->p[kDtW];
-            w->xp = Rp == R ? xw.detach() : derived(xp, {padded_rows(), ED}, dt, xw);
-            w->dtp = Rp == R ? dw.detach() : derived(dtp, {ED, Rp}, dt, dw);
-            w->xp_t = w->xp.t();
-            w->dtp_t = w->dtp.t();
-            if (wide && Rp != R) w->pad_jobs(jobs);
-        }
+    if (norm) *norm_w = norm->w.form(*norm_w, gain, jobs);
+    w.conv_w = conv_w.form(w.p[kConvW], small, jobs);
+    w.conv_b = conv_b.form(w.p[kConvB], small, jobs);
+    w.dt_b = dt_b.form(w.p[kDtB], small, jobs);
+    w.D = D.form(w.p[kD], small, jobs);
+    w.A = derived(A, {ED, N}, at::kFloat, w.p[kInW]);
+    if (small) jobs.push_back(cast_job(w.p[kALog], A, ED, N, 0, 0, MPA_CAST_NEG_EXP));
+    if (sequence) {
+        const Tensor &xw = w.p[kXW], &dw = w.p[kDtW];
+        w.xp = Rp == R ? xw : derived(xp, {padded_rows(), ED}, dt, xw);
+        w.dtp = Rp == R ? dw : derived(dtp, {ED, Rp}, dt, dw);
+        if (wide && Rp != R) w.pad_jobs(jobs);
     }
-    if (!jobs.empty()) run_casts(jobs, p[kInW].t);
+    run_casts(jobs, w.p[kInW]);
+    const uint64_t of = f.capture ? 0 : epoch;
     if (gain) {
         norm->changed = f.capture;
         norm->formed = of;
     }
-    if (w) {
-        kept = w;
-        if (small) formed = of;
-        padded = sequence ? of : 0;  // (xp .. dtp_t are not in `kept` otherwise)
-    }
+    if (small) formed = of;
+    if (wide) padded = of;
     f.after(written, !jobs.empty(), {&conv_w.own, &conv_b.own, &dt_b.own, &D.own, &A, &xp, &dtp, norm ? &norm->w.own : &A});
-    return kept;
 }
 
 // The products of a layer run on mpa_linear_run while they are small: it costs the host a quarter of a library call
 // (18 us) and takes norms and residual adds along.  The line is steps x width^2, which the products' arithmetic goes with.
-// Measured against library calls at 173 shapes of widths 64 to 2560 and 16 to 73728 steps (profiles/linear_dispatch.md:
-// a layer of a stack without gradients; a mixer, forward and backward), times as fast:
+// Measured against library calls at 173 shapes of widths 64 to 2560 and 16 to 73728 steps (a layer of a stack without
+// gradients; a mixer, forward and backward), times as fast:
 //   bfloat16  below the line 0.96 to 2.0 and 0.99 to 1.7 (0.96 to 1.1 at the line itself), at twice the line 0.84 to 1.1
 //   float32   a quarter of the rate, and every stage of a long K a latency.  Without gradients the line is that of width
 //             704 up to width 512 and falls as its square from there (0.98 to 2.1; on the other side of it 0.72 to 1.2).  A mixer
@@ -555,25 +532,30 @@ inline H* handle_in(PyObject* dict) {
     return py::cast<H*>(h);
 }
 
-// The handle of a mixer that can run here, or null.
-inline MixerHandle* ready_mixer(PyObject* mixer, const Tensor& x) {
+// The handle of a mixer that can run here and what it has of parameters, or null.
+inline MixerHandle* ready_mixer(PyObject* mixer, const Tensor& x, Weights& w) {
     if (!mixer || (PyObject*)Py_TYPE(mixer) != types->block.ptr()) return nullptr;
     PyObject* dict = dict_of(mixer);
     MixerHandle* m = dict ? handle_in<MixerHandle>(dict) : nullptr;
-    return m && m->ready(dict, x) ? m : nullptr;
+    return m && m->ready(dict, x, w) ? m : nullptr;
 }
 
-// A residual block: its norm and its mixer.
+// A residual block: its norm and its mixer, and what a call takes along of them.
 struct Layer {
     NormHandle* n = nullptr;
     MixerHandle* m = nullptr;
+    Weights w;
+    Tensor norm_w;
+    double eps = 0;
 };
 inline bool find_layer(PyObject* block, const Tensor& x, Layer& l) {
     PyObject* dict = dict_of(block);
-    l.m = ready_mixer(get(get(dict, keys().modules), keys().mixer), x);
+    l.m = ready_mixer(get(get(dict, keys().modules), keys().mixer), x, l.w);
     if (!l.m) return false;
     l.n = handle_in<NormHandle>(dict);
-    return l.n->ready(*l.m);
+    if (!l.n->ready(*l.m, l.norm_w)) return false;
+    l.eps = l.n->eps;
+    return true;
 }
 
 // Whether a native call may run at all: nothing replaces or rewrites the calls it stands in for (autocast does), and x is

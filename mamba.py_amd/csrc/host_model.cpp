@@ -27,22 +27,9 @@ bool cache_fits(const Cache& c, const LayerSizes& l, int64_t batch, bool need_h)
            c.window.sizes() == at::IntArrayRef({batch, l.ED, l.K - 1});
 }
 
-// What a layer's kernels read.
-struct LayerWeights {
-    std::shared_ptr<const Weights> m;
-    Tensor norm_w;
-    double eps = 0;
-};
-
-std::vector<LayerWeights> form_layers(const std::vector<Layer>& layers, bool sequence) {
+void form_layers(std::vector<Layer>& layers, bool sequence) {
     Forming f(layers[0].m->device);
-    std::vector<LayerWeights> w;
-    w.reserve(layers.size());
-    for (const Layer& l : layers) {
-        auto m = l.m->form(f, sequence, l.n);
-        w.push_back({std::move(m), l.n->w.t, l.n->eps});
-    }
-    return w;
+    for (Layer& l : layers) l.m->form(f, sequence, l.w, l.n, &l.norm_w);
 }
 
 py::object pair(const Tensor& h, const Tensor& w) { return py::make_tuple(h, w); }
@@ -50,12 +37,12 @@ py::object pair(const Tensor& h, const Tensor& w) { return py::make_tuple(h, w);
 // ---- decode -------------------------------------------------------------------------------------
 
 // The launches of a step, without the interpreter's lock; `cs` becomes the caches after it.
-Tensor run_steps(const std::vector<LayerWeights>& layers, const Tensor& x, std::vector<Cache>& cs, bool inplace) {
+Tensor run_steps(const std::vector<Layer>& layers, const Tensor& x, std::vector<Cache>& cs, bool inplace) {
     const size_t n = layers.size();
     const int64_t batch = x.size(0);
     std::vector<mpa_decode_layer> desc(n);
     for (size_t i = 0; i < n; ++i) {
-        desc[i] = layers[i].m->desc(batch);
+        desc[i] = layers[i].w.desc(batch);
         desc[i].norm = 1;
         desc[i].eps = (float)layers[i].eps;
         desc[i].norm_weight = fptr(layers[i].norm_w);
@@ -77,7 +64,7 @@ Tensor run_steps(const std::vector<LayerWeights>& layers, const Tensor& x, std::
     const void* scaled = nullptr;
     const float* sums = nullptr;
     for (size_t i = 0; i < n; ++i) {
-        const Weights& l = *layers[i].m;
+        const Weights& l = layers[i].w;
         Cache out = cs[i];
         if (!inplace) {
             out.h = empty({batch, l.ED, l.N}, at::kFloat, x);
@@ -117,11 +104,11 @@ py::object stack_step(const py::list& layers, const Tensor& x_in, const py::list
     }
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
-    const std::vector<LayerWeights> ws = form_layers(hs, false);
+    form_layers(hs, false);
     Tensor y;
     {
         const py::gil_scoped_release nogil;
-        y = run_steps(ws, x, cs, inplace);
+        y = run_steps(hs, x, cs, inplace);
     }
     if (!inplace)
         for (size_t i = 0; i < n; ++i) caches[i] = pair(cs[i].h, cs[i].window);
@@ -134,25 +121,25 @@ py::object block_step(const py::object& block, const Tensor& x_in, const Opt& h_
         return py::none();
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard guard(x_in.device());
-    MixerHandle* l = ready_mixer(block.ptr(), x_in);
+    Weights w;
+    MixerHandle* l = ready_mixer(block.ptr(), x_in, w);
     const int64_t batch = x_in.size(0);
     const Cache in{val(h_in), window};
     if (!l || !l->decode_ok || !cache_fits(in, *l, batch, inplace)) return py::none();
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
-    std::shared_ptr<const Weights> w;
     {
         Forming f(l->device);
-        w = l->form(f, false, nullptr);
+        l->form(f, false, w, nullptr, nullptr);
     }
     py::gil_scoped_release nogil;
     Cache out = in;
     if (!inplace) {
-        out.h = empty({batch, w->ED, w->N}, at::kFloat, x);
-        out.window = empty({batch, w->ED, w->K - 1}, x.scalar_type(), x);
+        out.h = empty({batch, w.ED, w.N}, at::kFloat, x);
+        out.window = empty({batch, w.ED, w.K - 1}, x.scalar_type(), x);
     }
-    const Tensor y = empty({batch, w->d}, x.scalar_type(), x);
-    const mpa_decode_layer s = w->desc(batch);
+    const Tensor y = empty({batch, w.d}, x.scalar_type(), x);
+    const mpa_decode_layer s = w.desc(batch);
     const size_t nbytes = mpa_decode_layer_workspace_bytes(&s);
     const Tensor ws = scratch(nbytes, x);
     check(mpa_decode_layer_step(&s, ptr(x), nullptr, nullptr, ptr(y), nullptr, nullptr, nullptr, fptr(in.h), fptr(out.h), ptr(in.window),
@@ -166,10 +153,10 @@ py::object block_step(const py::object& block, const Tensor& x_in, const Opt& h_
 
 // The launches of a sequence, without the interpreter's lock; with `keep`, `cs` becomes the caches after it.
 // The activations of a layer live in buffers that every layer uses again.
-Tensor run_sequence(const std::vector<LayerWeights>& hs, const Tensor& x, std::vector<Cache>& cs, bool keep, const Plan& plan) {
+Tensor run_sequence(const std::vector<Layer>& hs, const Tensor& x, std::vector<Cache>& cs, bool keep, const Plan& plan) {
     const size_t n = hs.size();
     const int64_t Bs = x.size(0), L = x.size(1), T = Bs * L;
-    const Weights& a = *hs[0].m;
+    const Weights& a = hs[0].w;
     const auto dt = x.scalar_type();
     const int io = io_dtype(dt);
     const int64_t d = a.d, ED = a.ED, N = a.N, P = a.xp.size(0);
@@ -178,9 +165,9 @@ Tensor run_sequence(const std::vector<LayerWeights>& hs, const Tensor& x, std::v
     const Tensor normed = empty({T, d}, dt, x), xz = empty({T, 2 * ED}, dt, x), xs = empty({Bs, L, ED}, dt, x),
                  dbc = empty({T, P}, dt, x), delta = empty({T, ED}, dt, x), y = empty({T, ED}, dt, x), hidden = empty({T, d}, dt, x);
     bool own = use_linear(dt, false, T, d, ED, P, {&x});
-    for (const LayerWeights& h : hs)
+    for (const Layer& h : hs)
         own &= h.norm_w.defined() &&
-               use_linear(dt, false, T, d, ED, P, {&h.m->p[kInW], &h.m->p[kOutW], &h.m->xp, &h.m->dtp, &h.norm_w, &h.m->p[kInB], &h.m->p[kOutB]});
+               use_linear(dt, false, T, d, ED, P, {&h.w.p[kInW], &h.w.p[kOutW], &h.w.xp, &h.w.dtp, &h.norm_w, &h.w.p[kInB], &h.w.p[kOutB]});
     // The residual stream between the layers.  The own products keep it in float32: at bfloat16, its roundings were
     // the larger part of a deep stack's error (24 layers of width 768: see tests/test_deep_stack_gpu.py).
     Tensor sum[2];
@@ -218,7 +205,7 @@ Tensor run_sequence(const std::vector<LayerWeights>& hs, const Tensor& x, std::v
     const void* in = ptr(x);
     const void* residual = nullptr;
     for (size_t i = 0; i < n; ++i) {
-        const Weights& l = *hs[i].m;
+        const Weights& l = hs[i].w;
         const float* norm_w = fptr(hs[i].norm_w);
         const float eps = (float)hs[i].eps;
         const Tensor& s = sum[i % 2];
@@ -235,9 +222,9 @@ Tensor run_sequence(const std::vector<LayerWeights>& hs, const Tensor& x, std::v
             }
             run(q);
         } else if (l.p[kInB].defined()) {
-            at::addmm_out(out, l.p[kInB].detach(), normed, l.in_wt);
+            at::addmm_out(out, l.p[kInB], normed, l.p[kInW].t());
         } else {
-            at::mm_out(out, normed, l.in_wt);
+            at::mm_out(out, normed, l.p[kInW].t());
         }
         Tensor window, h_last;
         if (keep) {
@@ -252,9 +239,9 @@ Tensor run_sequence(const std::vector<LayerWeights>& hs, const Tensor& x, std::v
             run(linear(ptr(dbc), P, l.Rp, l.dtp, Tensor(), delta));
         } else {
             out = dbc;
-            at::mm_out(out, xs2, l.xp_t);
+            at::mm_out(out, xs2, l.xp.t());
             out = delta;
-            at::mm_out(out, dlow, l.dtp_t);
+            at::mm_out(out, dlow, l.dtp.t());
         }
         const char* bc = static_cast<const char*>(ptr(dbc)) + l.Rp * es;
         check(mpa_sscan_fwd(&sc, ptr(xs), ptr(delta), fptr(l.A), bc, bc + N * es, fptr(l.D), static_cast<const char*>(ptr(xz)) + ED * es,
@@ -273,9 +260,9 @@ Tensor run_sequence(const std::vector<LayerWeights>& hs, const Tensor& x, std::v
             }
             run(q);
         } else if (l.p[kOutB].defined()) {
-            at::addmm_out(out, l.p[kOutB].detach(), y, l.out_wt);
+            at::addmm_out(out, l.p[kOutB], y, l.p[kOutW].t());
         } else {
-            at::mm_out(out, y, l.out_wt);
+            at::mm_out(out, y, l.p[kOutW].t());
         }
         in = ptr(hidden);
         if (keep) cs[i] = {h_last, window};
@@ -306,11 +293,11 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
     }
     const Tensor x = x_in.contiguous();
     if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16) return py::none();
-    const std::vector<LayerWeights> ws = form_layers(hs, true);
+    form_layers(hs, true);
     Tensor y;
     {
         const py::gil_scoped_release nogil;
-        y = run_sequence(ws, x, cs, return_caches, unpack(packed));
+        y = run_sequence(hs, x, cs, return_caches, unpack(packed));
     }
     if (!return_caches) return py::make_tuple(y, py::none());
     py::list after;

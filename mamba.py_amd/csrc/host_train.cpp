@@ -135,10 +135,9 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::DeviceGuard guard(x_in.device());
-        MixerHandle* handle = ready_mixer(block.ptr(), x_in);
+        MixerHandle* handle = ready_mixer(block.ptr(), x_in, l);
         if (!handle || !handle->forward_ok || handle->N % 4) return py::none();
         if (unpack(packed).flags & MPA_PLAN_BWD_GENERAL) return py::none();
-        l = handle->parameters();
         const int64_t Bs = x_in.size(0);
         if (hc.defined() && !fits(hc, {Bs, l.ED, l.N}, at::kFloat, l.device)) return py::none();
         if (wc.defined() && !fits(wc, {Bs, l.ED, l.K - 1}, l.dt, l.device)) return py::none();

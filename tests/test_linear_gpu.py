@@ -122,3 +122,20 @@ def test_linear_with_a_float32_residual_stream(pkg, dev, T, M, K, pitch, accumul
     assert rel_err(run(Y | R, x16, wide(), res, norm=False), plain + res.double()) <= 1e-5
     q = Linear(io_dtype=1 | X, T=T, M=M, K=K, x_pitch=pitch, y_pitch=M, x=x.data_ptr(), weight=w.data_ptr(), y=y.data_ptr())
     assert lib.mpa_linear_run(ctypes.byref(q), pkg.scan._stream(dev)) == 3     # float32 x only to be normalised
+
+
+# so many tiles that an XCD takes those of its own steps, and as many where W is the larger operand
+@pytest.mark.parametrize("T,M", [(4111, 1288), (1288, 4112)])
+@pytest.mark.parametrize("kxm", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_linear_of_many_tiles(pkg, dev, T, M, kxm, dtype):
+    L, lib, K = pkg._lib, pkg._lib.load(), 72
+    g = torch.Generator().manual_seed(T)
+    rand = lambda *s: torch.randn(*s, generator=g).to(dev).to(dtype)
+    x, w = rand(T, K), rand(K, M) if kxm else rand(M, K)
+    y = torch.full((T, M), float("nan"), device=dev, dtype=dtype)
+    q = Linear(io_dtype=pkg.scan._DTYPES[dtype], T=T, M=M, K=K, x_pitch=K, y_pitch=M, x=x.data_ptr(), weight=w.data_ptr(), y=y.data_ptr(),
+               weight_kxm=kxm)
+    L.check(lib.mpa_linear_run(ctypes.byref(q), pkg.scan._stream(dev)), "mpa_linear_run")
+    want = x.double() @ (w.double() if kxm else w.double().t())
+    assert rel_err(y, want) <= (1e-5 if dtype == torch.float32 else 2.0 ** -8)      # 72 products in float32; rounded once

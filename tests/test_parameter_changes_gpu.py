@@ -170,3 +170,33 @@ def test_a_capture_does_not_pass_for_a_run(pkg, dev):
         assert same(out, want)
         forward_and_step(warm, x)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("dt_rank", [16, 64])
+def test_nothing_holds_the_parameters_between_calls(pkg, dev, dtype, dt_rank):
+    """A model that moves to the host takes its memory along, but for the small forms; its tensors can be swapped."""
+    torch.manual_seed(8)
+    m = pkg.Mamba(pkg.MambaConfig(d_model=256, n_layers=3, dt_rank=dt_rank)).to(dev).to(dtype)
+    x = torch.randn(2, 30, 256, device=dev).to(dtype)
+    forward_and_step(m, x)
+    train_pass(m, x.clone().requires_grad_(), torch.ones_like(x))
+    forward_and_step(m, x)
+    for layer in m.layers:
+        for name in ("D", "A_log"):
+            p = getattr(layer.mixer, name)
+            torch.utils.swap_tensors(p, torch.nn.Parameter(p.detach() * 0.5))
+        w = layer.mixer.in_proj.weight
+        torch.utils.swap_tensors(w, torch.nn.Parameter(w.detach() * 2))
+        torch.utils.swap_tensors(layer.norm.weight, torch.nn.Parameter(layer.norm.weight.detach() * 3))
+    assert same(forward_and_step(m, x), forward_and_step(copy.deepcopy(m), x))
+    for i in range(10):        # twice between two calls: the second new one may lie where the old one was
+        for k in range(2):
+            m.layers[0].mixer.A_log = torch.nn.Parameter(m.layers[0].mixer.A_log.detach() + 0.05 * (i + 3 * k))
+            m.layers[0].norm.weight = torch.nn.Parameter(m.layers[0].norm.weight.detach() + 0.05 * (i + 3 * k))
+        assert same(forward_and_step(m, x), forward_and_step(copy.deepcopy(m), x))
+    torch.cuda.synchronize()
+    weights = sum(p.numel() * p.element_size() for p in m.parameters())
+    before = torch.cuda.memory_allocated(dev)
+    m.to("cpu")
+    assert before - torch.cuda.memory_allocated(dev) >= 0.95 * weights
