@@ -96,6 +96,8 @@ std::tuple<Tensor, Opt> scan_fwd(const Tensor& x, const Tensor& delta_in, const 
                 " D", D_in.sizes());
     TORCH_CHECK(!zc.defined() || zc.sizes() == x.sizes(), "z must have the shape of x");
     TORCH_CHECK(!bc.defined() || softplus, "delta_bias needs delta_softplus=True");
+    TORCH_CHECK(!bc.defined() || bc.numel() == ED, "delta_bias must have ", ED, " elements, got ", bc.sizes());
+    TORCH_CHECK(!hc.defined() || hc.numel() == Bs * ED * N, "h0 must be (B, ED, N), got ", hc.sizes());
     // whether a backward can follow decides what is kept: checkpoints (and the pre-gate output)
     // are written only then; without them the library may also cut a sequence more finely
     const bool need_grad = tracked({&x, &delta_in, &A_in, &B_in, &C_in, &D_in, &zc, &bc});
@@ -275,6 +277,7 @@ std::tuple<Tensor, Opt> conv(const Tensor& x, const Tensor& w_in, const Opt& b_i
     const int64_t Bs = x.size(0), L = x.size(1), ED = x.size(2), K = w_in.size(-1);
     TORCH_CHECK(w_in.numel() == ED * K, "weight must be (ED, 1, K) or (ED, K), got ", w_in.sizes());
     TORCH_CHECK(!wc.defined() || wc.sizes() == at::IntArrayRef({Bs, ED, K - 1}), "window must be (B, ED, K-1)");
+    TORCH_CHECK(!bc.defined() || bc.numel() == ED, "bias must have ", ED, " elements, got ", bc.sizes());
     const auto dt = x.scalar_type();
     io_dtype(dt);
     std::shared_ptr<ConvBackward> node;
@@ -306,7 +309,10 @@ std::tuple<Tensor, Opt> conv(const Tensor& x, const Tensor& w_in, const Opt& b_i
 Tensor conv_update(const Tensor& x, const Tensor& window, const Tensor& w_in, const Opt& b_in, bool silu) {
     const Tensor bc = val(b_in);
     require_gpu({&x, &window, &w_in, &bc});
+    TORCH_CHECK(x.dim() == 2, "x must be (B, ED)");
     const int64_t Bs = x.size(0), ED = x.size(1), K = w_in.size(-1);
+    TORCH_CHECK(w_in.numel() == ED * K && (!bc.defined() || bc.numel() == ED), "weight must be (ED, 1, K) or (ED, K) and bias (ED), got ",
+                w_in.sizes(), bc.defined() ? bc.sizes() : at::IntArrayRef());
     TORCH_CHECK(window.sizes() == at::IntArrayRef({Bs, ED, K - 1}) && window.scalar_type() == x.scalar_type() && window.is_contiguous(),
                 "window must be a contiguous (B, ED, K-1) tensor of x's dtype");
     at::AutoDispatchBelowADInplaceOrView below;
@@ -365,7 +371,10 @@ std::tuple<Tensor, Opt> rmsnorm(const Tensor& x_in, const Opt& res_in, const Opt
     TORCH_CHECK(!rc.defined() || (rc.sizes() == x_in.sizes() && rc.scalar_type() == x_in.scalar_type()),
                 "residual must have the shape and dtype of x");
     const int io = io_dtype(x_in.scalar_type());
-    const int64_t d = x_in.size(-1), rows = x_in.numel() / d;
+    const int64_t d = x_in.size(-1);
+    TORCH_CHECK(d > 0 && (!wc.defined() || wc.numel() == d), "the last dimension of x must not be empty, and weight as long, got x", x_in.sizes(),
+                " weight", wc.defined() ? wc.sizes() : at::IntArrayRef());
+    const int64_t rows = x_in.numel() / d;
     std::shared_ptr<NormBackward> node;
     if (tracked({&x_in, &rc, &wc})) node = make_node<NormBackward>({&x_in, &rc, &wc});
     Tensor y, sum, x, w;
@@ -406,11 +415,18 @@ std::tuple<Tensor, Tensor> step(const Tensor& x_in, const Tensor& delta_in, cons
     const int io = io_dtype(dt);
     TORCH_CHECK(x_in.dim() == 2 && A_in.dim() == 2, "x must be (B, ED) and A (ED, N)");
     const int64_t Bs = x_in.size(0), ED = x_in.size(1), N = A_in.size(1);
+    auto rows_of = [&](const Tensor& t) { return t.dim() >= 2 && t.size(0) == Bs && t.numel() == Bs * N; };
+    TORCH_CHECK(delta_in.numel() == Bs * ED && A_in.size(0) == ED && rows_of(B_in) && rows_of(C_in) && D_in.numel() == ED &&
+                    (!zc.defined() || (zc.size(0) == Bs && zc.numel() == Bs * ED)) && (!bc.defined() || bc.numel() == ED) &&
+                    (!hc.defined() || hc.numel() == Bs * ED * N),
+                "shape mismatch: x", x_in.sizes(), " delta", delta_in.sizes(), " A", A_in.sizes(), " B", B_in.sizes(), " C", C_in.sizes(),
+                " D", D_in.sizes());
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard guard(x_in.device());
     const Tensor x = x_in.contiguous(), delta = cast(delta_in, dt).contiguous();
-    const Tensor z = zc.defined() ? unit_rows(cast(zc, dt)) : zc;
-    Tensor B = unit_rows(cast(B_in, dt)), C = unit_rows(cast(C_in, dt));
+    auto rows = [&](const Tensor& t, int64_t n) { return unit_rows(cast(t.dim() == 2 ? t : t.reshape({Bs, n}), dt)); };
+    const Tensor z = zc.defined() ? rows(zc, ED) : zc;
+    Tensor B = rows(B_in, N), C = rows(C_in, N);
     if (B.stride(0) != C.stride(0)) { B = B.contiguous(); C = C.contiguous(); }
     const Tensor A = f32c(A_in), D = f32c(D_in), bias = f32c(bc);
     Tensor h = hc;
