@@ -201,17 +201,22 @@ inline bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx(
 struct Written {
     std::shared_ptr<c10::Event> event;
     std::optional<c10::Stream> last;  // the stream that wrote, or one that has waited since
+    bool unordered = false;           // written by a call that failed before its event
 };
-// The forming of the layers of one call: one event for all that is written.
+// The forming of the layers of one call: one event for all that is written, recorded by done().
 class Forming {
 public:
     explicit Forming(const c10::Device& device) : stream(current_stream(device)), capture(capturing()) {}
     Forming(const Forming&) = delete;
     ~Forming() {
-        if (wrote.empty() || capture) return;
+        for (Written* w : wrote) w->unordered = true;
+    }
+    void done() {
+        if (wrote.empty()) return;
         const auto event = std::make_shared<c10::Event>(stream.device_type());
         event->record(stream);
         for (Written* w : wrote) w->event = event;
+        wrote.clear();
     }
     void before(const Written& w) const {
         if (w.event && w.last != stream && !capture) w.event->block(stream);
@@ -457,6 +462,8 @@ struct NormHandle {
 
 inline void MixerHandle::form(Forming& f, bool sequence, Weights& w, NormHandle* norm, Tensor* norm_w) {
     f.before(written);
+    if (written.unordered) expire();
+    written.unordered = false;
     const bool small = formed != epoch, wide = sequence && padded != epoch, gain = norm && (norm->changed || norm->formed != epoch);
     std::vector<mpa_cast_job> jobs;
     if (norm) *norm_w = norm->w.form(*norm_w, gain, jobs);

@@ -30,6 +30,7 @@ bool cache_fits(const Cache& c, const LayerSizes& l, int64_t batch, bool need_h)
 void form_layers(std::vector<Layer>& layers, bool sequence) {
     Forming f(layers[0].m->device);
     for (Layer& l : layers) l.m->form(f, sequence, l.w, l.n, &l.norm_w);
+    f.done();
 }
 
 py::object pair(const Tensor& h, const Tensor& w) { return py::make_tuple(h, w); }
@@ -131,6 +132,7 @@ py::object block_step(const py::object& block, const Tensor& x_in, const Opt& h_
     {
         Forming f(l->device);
         l->form(f, false, w, nullptr, nullptr);
+        f.done();
     }
     py::gil_scoped_release nogil;
     Cache out = in;

@@ -200,3 +200,24 @@ def test_nothing_holds_the_parameters_between_calls(pkg, dev, dtype, dt_rank):
     before = torch.cuda.memory_allocated(dev)
     m.to("cpu")
     assert before - torch.cuda.memory_allocated(dev) >= 0.95 * weights
+
+
+def test_a_call_that_runs_out_of_memory(pkg, dev):
+    """It fails with an exception, while forming the weights or after it; the next call, on another stream, is right."""
+    torch.manual_seed(9)
+    m = pkg.Mamba(pkg.MambaConfig(d_model=512, n_layers=4)).to(dev).to(torch.bfloat16)
+    x = torch.randn(2, 4000, 512, device=dev).to(torch.bfloat16)
+    want = forward_and_step(copy.deepcopy(m), x)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    try:
+        torch.cuda.set_per_process_memory_fraction(0.0, dev)
+        with pytest.raises(RuntimeError, match="out of memory"), torch.no_grad():
+            m(x)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    stream = torch.cuda.Stream(device=dev)
+    with torch.cuda.stream(stream):
+        got = forward_and_step(m, x)
+    torch.cuda.synchronize()
+    assert same(got, want)
