@@ -136,7 +136,8 @@ py::object block_train(const py::object& block, const Tensor& x_in, const Opt& h
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::DeviceGuard guard(x_in.device());
         MixerHandle* handle = ready_mixer(block.ptr(), x_in, l);
-        if (!handle || !handle->forward_ok || handle->N % 4) return py::none();
+        // (mpa_wgrad takes whole 16-byte parts of a row)
+        if (!handle || !handle->forward_ok || handle->N % 4 || handle->ED % (16 / (int64_t)x_in.element_size())) return py::none();
         if (unpack(packed).flags & MPA_PLAN_BWD_GENERAL) return py::none();
         const int64_t Bs = x_in.size(0);
         if (hc.defined() && !fits(hc, {Bs, l.ED, l.N}, at::kFloat, l.device)) return py::none();

@@ -79,6 +79,25 @@ def test_mixer_gradients_match_float64_layer(pkg, dev, dtype, tol, shape, width,
         y.backward(g.to(dev))
 
 
+# not whole 16-byte parts in either type; in bfloat16
+@pytest.mark.parametrize("inner,dtype,tol", [(102, torch.float32, 2e-4), (102, torch.bfloat16, 5e-2), (100, torch.bfloat16, 5e-2)])
+def test_mixer_of_any_inner_width(pkg, dev, inner, dtype, tol):
+    torch.manual_seed(inner)
+    cfg = pkg.MambaConfig(d_model=64, n_layers=1)
+    cfg.d_inner = inner
+    blk = pkg.MambaBlock(cfg).to(dev).to(dtype)
+    x, g = torch.randn(2, 75, 64).to(dtype), torch.randn(2, 75, 64).to(dtype)
+    xr = x.double().requires_grad_()
+    yr, pr = block_forward_ref(blk, xr)
+    yr.backward(g.double())
+    xg = x.to(dev).requires_grad_()
+    y = blk(xg)
+    y.backward(g.to(dev))
+    assert rel_err(y, yr) <= tol and rel_err(xg.grad, xr.grad) <= tol
+    for k, v in blk.named_parameters():
+        assert rel_err(v.grad, pr[k].grad) <= 3 * tol, k
+
+
 def test_mixer_leaves_autocast_and_backward_hooks_to_the_composed_path(pkg, dev):
     torch.manual_seed(9)
     blk = pkg.MambaBlock(pkg.MambaConfig(d_model=64, n_layers=1)).to(dev)
