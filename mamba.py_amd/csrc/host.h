@@ -59,6 +59,10 @@ inline void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t
 inline Tensor cast(const Tensor& t, at::ScalarType dt) { return t.defined() && t.scalar_type() != dt ? t.to(dt) : t; }
 inline Tensor f32c(const Tensor& t) { return t.defined() ? cast(t, at::kFloat).contiguous() : t; }
 inline Tensor dense(const Tensor& t) { return t.defined() ? t.contiguous() : t; }  // (a saved tensor may come back with other strides)
+inline Tensor dense16(const Tensor& t) {  // ... and may start anywhere, as a view of a flat buffer does; for kernels with 16-byte loads
+    const Tensor c = dense(t);
+    return c.defined() && reinterpret_cast<uintptr_t>(c.const_data_ptr()) % 16 ? c.clone() : c;
+}
 inline Tensor unit_rows(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
 inline Tensor empty(at::IntArrayRef shape, at::ScalarType dt, const Tensor& like) {
     return at::empty(shape, at::TensorOptions().dtype(dt).device(like.device()));

@@ -72,7 +72,7 @@ std::tuple<Tensor, Tensor, Tensor> mixer_forward(Weights& l, const std::array<co
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::DeviceGuard guard(x_in.device());
         MixerBackward& m = *node;
-        x = x_in.contiguous();
+        x = dense16(x_in);
         const auto dt = x.scalar_type();
         const int io = io_dtype(dt);
         const size_t es = x.element_size();
@@ -176,7 +176,7 @@ variable_list MixerBackward::apply(variable_list&& grads) {
         if (!v.defined()) return;
         TORCH_CHECK(v.sizes() == shape && v.scalar_type() == type && v.device() == w[kIX].device(), "a saved tensor of a MambaBlock came back as ",
                     v.scalar_type(), v.sizes(), " on ", v.device(), ", was ", type, shape);
-        v = v.contiguous();
+        v = dense16(v);
     };
     given(w[kIX], {Bs, L, d}, dt); given(w[kIInW], {2 * ED, d}, dt); given(w[kIOutW], {d, ED}, dt);
     given(t[kSWin], {Bs, ED, K - 1}, dt); given(t[kSH0], {Bs, ED, N}, f32);
@@ -196,7 +196,7 @@ variable_list MixerBackward::apply(variable_list&& grads) {
     const size_t es = x_.element_size();
     void* stream = stream_of(x_);
     auto at_col = [&](const Tensor& t, int64_t col) { return static_cast<char*>(ptr(t)) + col * es; };
-    const Tensor x2 = x_.view({T, d}), dout = cast(grads[0], dt).contiguous().view({T, d});
+    const Tensor x2 = x_.view({T, d}), dout = dense16(cast(grads[0], dt)).view({T, d});
 
     const bool own = use_linear(dt, true, T, d, ED, P, {&dout, &w[kIOutW], &w[kIInW], &xp, &dtp});
     // out (T x M) = in (T x K) . weight (K x M), or added to out

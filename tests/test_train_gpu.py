@@ -98,6 +98,27 @@ def test_mixer_of_any_inner_width(pkg, dev, inner, dtype, tol):
         assert rel_err(v.grad, pr[k].grad) <= 3 * tol, k
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_mixer_takes_operands_that_start_anywhere(pkg, dev, dtype):
+    """Input and output gradient as views of flat buffers, one element off: the same results bit for bit."""
+    torch.manual_seed(11)
+    blk = pkg.MambaBlock(pkg.MambaConfig(d_model=64, n_layers=1)).to(dev).to(dtype)
+    x, g = (torch.randn(2, 75, 64, device=dev).to(dtype) for _ in range(2))
+
+    def off(t):
+        v = torch.empty(t.numel() + 1, dtype=dtype, device=dev)[1:].view(t.shape)
+        assert v.data_ptr() % 16
+        return v.copy_(t)
+
+    def run(x, g):
+        x = x.detach().requires_grad_()
+        y = blk(x)
+        return [y.detach()] + list(torch.autograd.grad(y, [x] + list(blk.parameters()), g))
+    want = run(x, g)
+    for got in (run(off(x), g), run(x, off(g)), run(off(x), off(g))):
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def test_mixer_leaves_autocast_and_backward_hooks_to_the_composed_path(pkg, dev):
     torch.manual_seed(9)
     blk = pkg.MambaBlock(pkg.MambaConfig(d_model=64, n_layers=1)).to(dev)
