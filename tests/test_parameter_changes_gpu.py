@@ -210,12 +210,19 @@ def test_a_call_that_runs_out_of_memory(pkg, dev):
     want = forward_and_step(copy.deepcopy(m), x)
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
+    held, size = [], 256 << 20
     try:
         torch.cuda.set_per_process_memory_fraction(0.0, dev)
+        while size >= 1 << 20:           # what is left free between the tensors of other tests
+            try:
+                held.append(torch.empty(size, dtype=torch.uint8, device=dev))
+            except torch.cuda.OutOfMemoryError:
+                size //= 2
         with pytest.raises(RuntimeError, match="out of memory"), torch.no_grad():
             m(x)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0, dev)
+        held.clear()
     stream = torch.cuda.Stream(device=dev)
     with torch.cuda.stream(stream):
         got = forward_and_step(m, x)
