@@ -361,7 +361,7 @@ __device__ __forceinline__ void decode_tile(int row_tiles, int groups, int& rt, 
 }
 
 // XP: also the workgroup's share of x_proj, its 16 channels' product with all rows of x_proj's weight, as one
-// more partial sum of dbc; a thread owns one row and every so many sequences.
+// more partial sum of dbc; a thread owns one row and every so many sequences (there are as many threads as rows, or more).
 template <typename IO, int MT, int NT, int NW, int U, int MODE, bool XP = false>
 __global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams p, int row_tiles, int groups) {
     constexpr int kThreads = NW * kWave, kRows = MT * 16, kAll = NT * 16 * kRows, kOuts = (kAll + kThreads - 1) / kThreads;
@@ -808,10 +808,12 @@ template <typename IO, int MODE>
 static int launch_in(const DecodeParams& p, hipStream_t st) {
     const int rt = (2 * p.ED + 15) / 16, bt = (p.batch + 15) / 16;
     if (xproj_fused(p.ED, p.R + 2 * p.N, p.batch)) {
-        // (float32 rows have twice the pieces: from three a wave on, fewer waves with more of them in flight, 1 x 768 20.2 -> 19.0 us a
-        // layer, but 1 x 424 6.1 us for in_proj and 5.5 on eight; with two, the second is better requested as the first is used: 6 layers of
-        // 1 x 512 118.7 us with both in flight, 116.0)
-        if (sizeof(IO) == 4 && p.d >= 704) hipLaunchKernelGGL((decode_in_kernel<IO, 1, 1, 4, 4, MODE, true>), decode_grid(rt, bt, 1), dim3(256), 0, st, p, rt, bt);
+        // (float32 rows have twice the pieces.  From 704 columns on fewer waves with more pieces in flight, a measured line: 1 x 768 20.2 ->
+        // 19.0 us a layer, but below it eight waves are 1 to 3 % faster at every width tried, 12 layers of 1 x 700 210 us and 215, of
+        // 16 x 576 229 and 235.  Up to 512 columns a wave has two pieces at most, and the second is better requested as the first is
+        // used: 6 layers of 1 x 512 118.7 us with both in flight, 116.0.  Four waves have a thread for 256 rows of x_proj; more of them
+        // take eight at any width.)
+        if (sizeof(IO) == 4 && p.d >= 704 && p.R + 2 * p.N <= 256) hipLaunchKernelGGL((decode_in_kernel<IO, 1, 1, 4, 4, MODE, true>), decode_grid(rt, bt, 1), dim3(256), 0, st, p, rt, bt);
         else if (sizeof(IO) == 4 && p.d > 256 && p.d <= 512) hipLaunchKernelGGL((decode_in_kernel<IO, 1, 1, 8, 1, MODE, true>), decode_grid(rt, bt, 1), dim3(512), 0, st, p, rt, bt);
         else hipLaunchKernelGGL((decode_in_kernel<IO, 1, 1, 8, 2, MODE, true>), decode_grid(rt, bt, 1), dim3(512), 0, st, p, rt, bt);
     } else if (rt * bt < kManyTiles) {

@@ -48,6 +48,14 @@ def test_float32_step_at_the_lines_of_in_proj(pkg, dev, batch, width):
     test_float32_step_matches_float64(pkg, dev, batch, width, {})
 
 
+# x_proj inside in_proj takes a thread for each of its dt_rank + 2 * d_state rows: more of them than four waves have, as many,
+# and the most that are taken at this width.
+@pytest.mark.parametrize("batch,width,kw", [(1, 704, dict(d_state=128)), (16, 704, dict(d_state=128)), (5, 768, dict(d_state=112, dt_rank=33)),
+                                            (5, 768, dict(d_state=112, dt_rank=32)), (2, 704, dict(d_state=128, dt_rank=116))])
+def test_float32_step_with_many_rows_of_x_proj(pkg, dev, batch, width, kw):
+    test_float32_step_matches_float64(pkg, dev, batch, width, dict(kw, expand_factor=1))
+
+
 # bfloat16, two batch tiles a workgroup: up to 1024 columns on four waves, then on eight.
 @pytest.mark.parametrize("batch,width", [(97, 1024), (128, 1000), (97, 1032)])
 def test_bfloat16_step_at_the_line_of_in_proj(pkg, dev, batch, width):
