@@ -635,7 +635,7 @@ struct DtVec<float, 4> {
 // A thread owns a quarter of the states and of the dt_rank of one channel, for BT sequences: the
 // quarter sums of dt_proj meet in a quad (two exchanges), after which every lane of the quad has
 // delta and goes on with its own states.  State loads are issued before the dt_proj sum.
-// MANY: dbc comes as many partial sums (see xproj_fused).
+// MANY: dbc comes as many partial sums (see xproj_fused); otherwise as eight at most (see decode_splits).
 template <typename IO, int BT, bool N16, int DTV, bool MANY>
 __global__ void __launch_bounds__(256) decode_ssm_kernel(const DecodeParams p) {
     extern __shared__ float dbc[];  // [BT][R + 2N], as many times as threads allow while it is summed
@@ -667,7 +667,7 @@ __global__ void __launch_bounds__(256) decode_ssm_kernel(const DecodeParams p) {
         const rsrc_t parts = window(p.dbc, (int64_t)p.splits * p.batch * P, 4);
         for (int i = threadIdx.x; i < BT * P; i += 256) {
             const int t = i / P, b = b0 + t;
-            float v[8], s = 0.0f;  // (requested together: splits <= 8)
+            float v[8], s = 0.0f;  // (requested together)
 #pragma unroll
             for (int q = 0; q < 8; ++q)
                 v[q] = ld_f32(parts, (uint32_t)((q * p.batch + b) * P + (i - t * P)) * 4u, b < p.batch && q < p.splits);
@@ -846,19 +846,14 @@ static int launch_out(const DecodeParams& p, hipStream_t st) {
     return check_launch();
 }
 
-template <typename IO, int BT>
+template <typename IO, int BT, bool MANY = false>
 static int launch_ssm(const DecodeParams& p, hipStream_t st) {
     const dim3 grid((p.ED + 63) / 64, (p.batch + BT - 1) / BT);
     const int outs = BT * (p.R + 2 * p.N);
     const size_t lds = (size_t)(outs < 256 ? 256 : outs) * sizeof(float);
     if (lds > 48 * 1024) return MPA_ERR_BAD_SHAPE;
     const bool v4 = p.R % 4 == 0 && aligned_to(p.dt_w, 4 * sizeof(IO));
-    const bool many = BT == 1 && xproj_fused(p.ED, p.R + 2 * p.N, p.batch);
-#define MPA_SSM(N16_, V_)                                                                                              \
-    do {                                                                                                               \
-        if (many) hipLaunchKernelGGL((decode_ssm_kernel<IO, 1, N16_, V_, true>), grid, dim3(256), lds, st, p);         \
-        else hipLaunchKernelGGL((decode_ssm_kernel<IO, BT, N16_, V_, false>), grid, dim3(256), lds, st, p);            \
-    } while (0)
+#define MPA_SSM(N16_, V_) hipLaunchKernelGGL((decode_ssm_kernel<IO, BT, N16_, V_, MANY>), grid, dim3(256), lds, st, p)
     if (p.N == 16) { if (v4) MPA_SSM(true, 4); else MPA_SSM(true, 1); }
     else { if (v4) MPA_SSM(false, 4); else MPA_SSM(false, 1); }
 #undef MPA_SSM
@@ -879,12 +874,14 @@ static int decode_launch(DecodeParams p, bool norm, void* xw, float* ssq, hipStr
     }
     int rc = !norm ? launch_in<IO, kInPlain>(p, st) : p.xw ? launch_in<IO, kInReady>(p, st) : launch_in<IO, kInNorm>(p, st);
     if (rc != MPA_OK) return rc;
-    if (!xproj_fused(p.ED, p.R + 2 * p.N, p.batch)) rc = launch_xproj<IO>(p, st);
+    const bool fused = xproj_fused(p.ED, p.R + 2 * p.N, p.batch);
+    if (!fused) rc = launch_xproj<IO>(p, st);
     if (rc != MPA_OK) return rc;
     // sequences per workgroup: four (weights and A read once for them) while that leaves two
-    // workgroups per CU
+    // workgroups per CU; one where dbc is many partial sums, whose summing takes all threads
     const int64_t cols = (p.ED + 63) / 64;
-    rc = cols * ((p.batch + 3) / 4) >= 512 ? launch_ssm<IO, 4>(p, st)
+    rc = fused ? launch_ssm<IO, 1, true>(p, st)
+         : cols * ((p.batch + 3) / 4) >= 512 ? launch_ssm<IO, 4>(p, st)
          : cols * ((p.batch + 1) / 2) >= 512 ? launch_ssm<IO, 2>(p, st) : launch_ssm<IO, 1>(p, st);
     if (rc != MPA_OK) return rc;
     return norm ? launch_out<IO, true>(p, st) : launch_out<IO, false>(p, st);

@@ -56,6 +56,14 @@ def test_float32_step_with_many_rows_of_x_proj(pkg, dev, batch, width, kw):
     test_float32_step_matches_float64(pkg, dev, batch, width, dict(kw, expand_factor=1))
 
 
+# Few rows of x_proj over many channels: its partial sums, one per 16 channels, are 256 and 512, and the batch is large enough that
+# the state kernel would take two and four sequences a workgroup.
+@pytest.mark.parametrize("batch,width,kw", [(16, 512, dict(d_state=16, dt_rank=32)), (13, 1024, dict(d_state=8, dt_rank=8))])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_step_of_many_channels_matches_float64(pkg, dev, dtype, batch, width, kw):
+    test_decode_gpu.test_stack_step_matches_float64_layers(pkg, dev, dtype, batch, width, dict(kw, expand_factor=8))
+
+
 # bfloat16, two batch tiles a workgroup: up to 1024 columns on four waves, then on eight.
 @pytest.mark.parametrize("batch,width", [(97, 1024), (128, 1000), (97, 1032)])
 def test_bfloat16_step_at_the_line_of_in_proj(pkg, dev, batch, width):
