@@ -453,13 +453,14 @@ int mpa_cast(const mpa_cast_job* jobs, int32_t n, void* stream);
 
 /* ---- wide float32 products ---------------------------------------------------------------------------
  * y (T x M) = x (T x K) . w (M x K)^T [+ bias] in float32 on the 16-bit matrix cores: each operand is cut into two
- * float16 parts per value with one power of two per row (split.hip says what that keeps), mpa_split_run, and up to
- * MPA_SPLIT_MAX_PRODUCTS products of cut operands run in one launch, mpa_split_product.
+ * float16 parts per value with one power of two per row, mpa_split_run, and up to MPA_SPLIT_MAX_PRODUCTS products of cut operands
+ * run in one launch, mpa_split_product.  A value keeps 2^-23 of itself, 2^-20 where it is below 2^-28 of its row's largest; a row with
+ * values more than 2^31 apart (zeros aside) or with an infinity is multiplied as it is, in float32 (split.hip).
  *
  * An operand has `rows` rows of length k: element (row, i) is src[row * pitch + i], or with by_cols
  * src[i * pitch + row].  The fast dimension's size and the pitch are multiples of 4, src is 16-byte aligned.  `split`
- * (256-byte aligned, mpa_split_bytes bytes) receives the parts.  A product takes w with M rows, a multiple of 4, and
- * x with T rows; src must still hold what was cut (rows with an infinity or a value of 2^64 or more are summed from it).  y and bias are 16-byte
+ * (256-byte aligned, mpa_split_bytes bytes: 4 bytes a value of rows rounded up to 32, k to 32, and a little) receives the parts.  A
+ * product takes w with M rows, a multiple of 4, and x with T rows, and reads their parts only.  y and bias are 16-byte
  * aligned, y_pitch a multiple of 4.  The workspace (16-byte aligned) may be NULL where its query says 0.
  */
 #define MPA_SPLIT_MAX_OPERANDS 8
