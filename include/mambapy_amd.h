@@ -386,7 +386,7 @@ int mpa_decode_layer_step(const mpa_decode_layer* s, const void* x, const void* 
  *   weight_kxm  the weight is (K x M), M a multiple of 4 (float32) / 8: y = x . weight, the product of a projection's backward;
  *     without norm_weight and y_ssq.
  *   residual  optional: (T x M), added to the rounded product or, with `accumulate`, before it is rounded; may be y.
- *   y_ssq  optional: ceil(M / 32) rows of T partial sums of squares of y.
+ *   y_ssq  optional: ceil(M / 32) rows of T partial sums of squares of y (NaN with an infinity among them).
  *   io_dtype | MPA_LINEAR_X_F32 (with x_ssq), _Y_F32, _RESIDUAL_F32: x, y or residual are float32 in a bfloat16
  *     call (nothing is rounded on its way into a float32 y).
  * Rows of x are x_pitch apart, those of y and residual y_pitch.  K and x_pitch are multiples of 4 (float32) / 8
@@ -411,7 +411,8 @@ int mpa_linear_run(const mpa_linear* s, void* stream);
  * 1 / rms to the product of them:
  *   y_weight, y_scaled  optional: y * y_weight (M, float32), rounded to io_dtype, in rows of M.
  *   x_ssq without norm_weight: x holds such rows, and the product is multiplied by 1 / sqrt(sum / K + eps) of its row
- *     before bias and residual.  Not with weight_kxm or a float32 x in a bfloat16 call.
+ *     before bias and residual; where the sum is an infinity (squares beyond float32) it is zero, whatever the product is.  Not
+ *     with weight_kxm or a float32 x in a bfloat16 call.
  * y_weight is 16-byte aligned, y_scaled four elements.
  */
 int mpa_linear_run_scaled(const mpa_linear* s, const float* y_weight, void* y_scaled, void* stream);

@@ -389,7 +389,8 @@ __global__ void __launch_bounds__(linear_threads(BT, BM, KS, RT)) linear_kernel(
             const int t = step(j);
             if (t >= p.T) continue;
             const int64_t o = (int64_t)t * p.y_pitch + m;
-            if constexpr (XMODE == kFactor) acc[i][j] *= factor[j];
+            // (a factor of zero: squares beyond float32, and the sum may be an infinity; a normalised row is zeros)
+            if constexpr (XMODE == kFactor) acc[i][j] = factor[j] == 0.0f ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : acc[i][j] * factor[j];
             f32x4 f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) f[e] = acc[i][j][e] + Ops::get(bias, e);
@@ -415,7 +416,7 @@ __global__ void __launch_bounds__(linear_threads(BT, BM, KS, RT)) linear_kernel(
             }
             if (p.ssq_out) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) ss[j] = __builtin_fmaf(f[e], f[e], ss[j]);
+                for (int e = 0; e < 4; ++e) ss[j] = __builtin_fmaf(f[e], f[e], ss[j]) + (f[e] - f[e]);  // (NaN with an infinity)
             }
         }
     }

@@ -41,3 +41,21 @@ def test_linear_between_layers(pkg, dev, T, M, K, parts, dtype):
     assert rel_err(y, want - res.double()) <= 1e-5
     q.weight_kxm = 1
     assert lib.mpa_linear_run_scaled(ctypes.byref(q), None, None, pkg.scan._stream(dev)) == 2
+
+
+# A residual stream whose squares are beyond float32: 1 / rms is zero, and so is the normalised row (as x * rsqrt(mean(x^2) + eps) has it),
+# whatever the product of the row itself is.  An infinity makes a NaN of its row, and of that row alone.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_stack_of_huge_rows(pkg, dev, dtype):
+    torch.manual_seed(0)
+    m = pkg.Mamba(pkg.MambaConfig(d_model=64, n_layers=3)).to(dev).to(dtype)
+    with torch.no_grad():
+        for layer in m.layers:
+            layer.mixer.in_proj.weight.fill_(4.0)          # (a sum of the row's values is beyond float32 as well)
+        x = torch.randn(1, 40, 64, device=dev).to(dtype)
+        x[0, 20], x[0, 30] = 3e38, 1e25
+        x[0, 35, 3] = float("inf")
+        y, plain = m(x), m(x[:, :20])
+    assert torch.equal(y[0, 20], x[0, 20]) and torch.equal(y[0, 30], x[0, 30])
+    assert y[0, 35].isnan().all() and y[0, :35].isfinite().all()
+    assert torch.equal(y[0, :20], plain[0])
