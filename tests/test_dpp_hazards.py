@@ -1,10 +1,11 @@
-"""Static check of the generated gfx950 code of the scan kernels (CPU only; needs hipcc).
+"""Static check of the generated gfx950 code of the kernels with inline DPP (CPU only; needs hipcc).
 
-The kernels use DPP instructions written as inline assembly (common.h: fmac_bcast,
-mul_bcast).  On gfx9-family hardware a DPP instruction that reads a vector register written
-by a VALU instruction less than two wait states earlier reads the old value; the compiler
-inserts the wait states for its own DPP instructions but cannot see into inline assembly.
-This test compiles the two scan kernels to assembly and checks that no DPP instruction reads,
+The scan kernels and the convolution with x_proj use DPP instructions written as inline
+assembly (common.h: fmac_bcast, mul_bcast; conv_proj.hip: mov_bcast).  On gfx9-family
+hardware a DPP instruction that reads a vector register written by a VALU instruction less
+than two wait states earlier reads the old value; the compiler inserts the wait states for
+its own DPP instructions but cannot see into inline assembly.
+This test compiles those sources to assembly and checks that no DPP instruction reads,
 as its DPP operand, a register that one of the two preceding instructions wrote on the VALU.
 """
 import os
@@ -74,7 +75,7 @@ def test_checker_sees_a_hazard_and_accepts_wait_states():
     assert find_dpp_hazards(bad)[1] and not find_dpp_hazards(ok)[1] and not find_dpp_hazards(far)[1]
 
 
-@pytest.mark.parametrize("src", ["sscan_fwd.hip", "sscan_bwd_fast.hip"])
+@pytest.mark.parametrize("src", ["sscan_fwd.hip", "sscan_bwd_fast.hip", "conv_proj.hip"])
 def test_no_dpp_operand_is_read_too_early(src, tmp_path):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
