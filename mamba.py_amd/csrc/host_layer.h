@@ -542,16 +542,26 @@ inline mpa_linear linear_of(int io, int64_t T, const void* in, int64_t x_pitch, 
 inline void run_linear(const mpa_linear& q, void* stream) { check(mpa_linear_run(&q, stream), "mpa_linear_run"); }
 
 // The wide float32 products of a layer on cut operands (mpa_split_run, mpa_split_product), where a product is long enough to pay
-// for cutting its operands.  Measured against library products at 28 shapes, widths 256 to 2048 and 128 to 16384 steps, each
-// with the cutting of both operands: one product is 0.5 to 1.0 times as fast below 2.4 * 2^30 multiplications (0.95 to 1.3 just
-// above), 1.8 at 8 and 2.1 at 16 times 2^30; the input gradient and both weight gradients together, one cutting for three
-// products of which the library's weight gradients are its slowest, 1.1 to 1.5 from 2^31 for the input gradient on, 1.4 to 2.1
-// at twice that.
-constexpr int64_t kSplitOne = 5LL << 29, kSplitThree = 1LL << 31;
-inline bool use_split(at::ScalarType dt, int64_t line, int64_t T, int64_t M, int64_t K, std::initializer_list<const Tensor*> operands) {
-    bool ok = dt == at::kFloat && T < 1 << 24 && M % 4 == 0 && K % 4 == 0 && T * M * K >= line;
+// for cutting its operands.  Measured against library products, widths 256 to 2560 and 128 to 32768 steps, each
+// with the cutting of both operands: one product is 0.6 to 1.4 times as fast below 2.5 * 2^30 multiplications, 1.0 to 2.0 just
+// above, 1.2 to 2.4 at 8 and 1.9 to 2.5 at 16 times 2^30.  A value is cut once and multiplied as often as the other operand has rows:
+// with few steps against a wide weight cutting it is what costs, and below 300 (half the harmonic mean of T and M) one product of 2.5 to
+// 5 * 2^30 is 0.6 to 1.0 times as fast (160 / 256 / 288 steps of width 2048 0.60 / 0.91 / 0.98, 352 1.22; 284 of 1536 0.86, 352 1.4; a
+// stack of two layers, 160 / 284 steps of width 2048, without gradients 318 / 386 us with it and 237 / 348, at 320 steps 393 and 376, with
+// gradients 1199 and 1230).
+// The input gradient and both weight gradients together, one cutting for three products of which the library's weight
+// gradients are its slowest: 1.04 to 2.1 from 2^31 for the input gradient on, 1.2 to 2.2 at four times that.
+constexpr int64_t kSplitOne = 5LL << 29, kSplitThree = 1LL << 31, kSplitRows = 300;
+inline bool split_ok(at::ScalarType dt, int64_t T, int64_t M, int64_t K, std::initializer_list<const Tensor*> operands) {
+    bool ok = dt == at::kFloat && T < 1 << 24 && M % 4 == 0 && K % 4 == 0;
     for (const Tensor* t : operands) ok &= !t->defined() || aligned(t->const_data_ptr(), 16);
     return ok;
+}
+inline bool use_split(at::ScalarType dt, int64_t T, int64_t M, int64_t K, std::initializer_list<const Tensor*> operands) {
+    return T * M * K >= kSplitOne && T * M >= kSplitRows * (T + M) && split_ok(dt, T, M, K, operands);
+}
+inline bool use_split_three(at::ScalarType dt, int64_t T, int64_t M, int64_t K, std::initializer_list<const Tensor*> operands) {
+    return T * M * K >= kSplitThree && split_ok(dt, T, M, K, operands);
 }
 // Operands of one launch; `hold` keeps their cut forms until the launches that read them are enqueued.
 class Split {
@@ -596,7 +606,7 @@ private:
 // y = x . weight^T (+ bias) on cut operands; false: not a product for them
 inline bool split_product(const Tensor& x, const Tensor& weight, const Tensor& bias, const Tensor& y, void* stream) {
     const int64_t M = weight.size(0), K = weight.size(1), T = x.numel() / K;
-    if (!use_split(x.scalar_type(), kSplitOne, T, M, K, {&x, &weight, &bias})) return false;
+    if (!use_split(x.scalar_type(), T, M, K, {&x, &weight, &bias})) return false;
     Split s(x, stream);
     const int w = s.rows(ptr(weight), M, K, K), r = s.rows(ptr(x), T, K, K);
     s.run();

@@ -219,7 +219,7 @@ variable_list MixerBackward::apply(variable_list&& grads) {
     if (own) {
         dy = empty({T, ED}, dt, x_);
         product(ptr(dout), d, d, w[kIOutW], ptr(dy), ED, false);
-    } else if (use_split(dt, kSplitOne, T, ED, d, {&dout, &w[kIOutW]})) {
+    } else if (use_split(dt, T, ED, d, {&dout, &w[kIOutW]})) {
         dy = empty({T, ED}, dt, x_);
         Split s(x_, stream);
         const int weight = s.cols(ptr(w[kIOutW]), ED, d, ED), in = s.rows(ptr(dout), T, d, d);
@@ -259,7 +259,7 @@ variable_list MixerBackward::apply(variable_list&& grads) {
               "mpa_conv1d_bwd");
     }
     const bool want_x = task_should_compute_output(kIX), want_in = task_should_compute_output(kIInW), want_out = task_should_compute_output(kIOutW);
-    const bool cut = !own && use_split(dt, kSplitThree, T, d, 2 * ED, {&dout, &x_, &y, &w[kIInW]});
+    const bool cut = !own && use_split_three(dt, T, d, 2 * ED, {&dout, &x_, &y, &w[kIInW]});
     if (cut && (want_x || want_in || want_out)) {
         // the input's gradient and those of the wide weights, in one launch
         Split s(x_, stream);
