@@ -382,7 +382,8 @@ int mpa_decode_layer_step(const mpa_decode_layer* s, const void* x, const void* 
  * y (T x M) = x (T x K) . weight (M x K)^T + bias, io_dtype with float32 sums, around it the norm and the
  * residual add of a pre-norm stack (mambapy/mamba.py:114-125):
  *   norm_weight, x_ssq  optional: `ssq_parts` rows of T partial sums of squares of the rows of x, which are
- *     multiplied by 1 / sqrt(sum / K + eps) and by norm_weight (K, float32) and rounded before the product.
+ *     multiplied by 1 / sqrt(sum / K + eps) and by norm_weight (K, float32) and rounded before the product.  (For callers with rows
+ *     that are not yet scaled; this package's own stacks use mpa_linear_run_scaled, which is faster.)
  *   weight_kxm  the weight is (K x M), M a multiple of 4 (float32) / 8: y = x . weight, the product of a projection's backward;
  *     without norm_weight and y_ssq.
  *   residual  optional: (T x M), added to the rounded product or, with `accumulate`, before it is rounded; may be y.
@@ -455,8 +456,9 @@ int mpa_cast(const mpa_cast_job* jobs, int32_t n, void* stream);
 /* ---- wide float32 products ---------------------------------------------------------------------------
  * y (T x M) = x (T x K) . w (M x K)^T [+ bias] in float32 on the 16-bit matrix cores: each operand is cut into two
  * float16 parts per value with one power of two per row, mpa_split_run, and up to MPA_SPLIT_MAX_PRODUCTS products of cut operands
- * run in one launch, mpa_split_product.  A value keeps 2^-23 of itself, 2^-20 where it is below 2^-28 of its row's largest; a row with
- * values more than 2^31 apart (zeros aside) or with an infinity is multiplied as it is, in float32 (split.hip).
+ * run in one launch, mpa_split_product.  A value keeps 2^-23 of itself, 2^-20 (from K = 2048 on K / 64 * 2^-24) where it is below 2^-28 of
+ * its row's largest; a row with values more than 2^31 (K / 1024 * 2^31) apart, zeros aside, or with an infinity is multiplied as it is,
+ * in float32 (split.hip).
  *
  * An operand has `rows` rows of length k: element (row, i) is src[row * pitch + i], or with by_cols
  * src[i * pitch + row].  The fast dimension's size and the pitch are multiples of 4, src is 16-byte aligned.  `split`
