@@ -5,9 +5,9 @@
 // run one tile per workgroup, as many workgroups as the shape offers, and take over the element-wise work around
 // the product: with `residual` the sum y + residual is stored, with `ssq_out` the partial sums of squares of its rows;
 // with `ssq`, those of x, the rows of x are normalised on their way into LDS (x * rstd * weight, rounded, as the norm
-// kernel rounds).  Between the layers of a stack the norm is in two places instead: out_proj stores the rows of the stream times the next
-// norm's weight as well, rounded once as a normalised row is, and in_proj multiplies its product with their rstd.
-// The residual stream between bfloat16 layers can be float32: x (with `ssq`), y and residual each have a flag.
+// kernel rounds; a form for callers of the C interface).  Between the layers of a stack the norm is in two places instead: out_proj
+// stores the rows of the stream times the next norm's weight as well, rounded once as a normalised row is, and in_proj multiplies its
+// product with their rstd.  The residual stream between bfloat16 layers can be float32: x (with `ssq`), y and residual each have a flag.
 //
 // Tile: BT steps x BM rows of W per workgroup, each wave 32 * RT x 32 of it (2 * RT x 2 MFMA tiles of 16 x 16, W as the left
 // operand, so that a lane's four results are neighbours in y) over its share of K.  K runs in stages of 128 bytes per
@@ -17,8 +17,9 @@
 // At 512 steps of width 768, recorded in a graph with the weights of 24 layers: in_proj with the rows' factor 9.7 us (11.8 with rows
 // of the float32 stream normalised on their way, twice the bytes and their conversion between load and LDS; 32 steps 6.3 for 8.1,
 // 2048 steps 20.8 for 26.3), x_proj 7.1, dt_proj 3.7, out_proj with the residual stream 8.8 (8.5 without); the library's products
-// alone 9.3, 7.1, 3.9 and 8.0.  Four stages in registers instead of two change nothing: it is the way of a stage through LDS and the barrier.  What the kernels save is the norm between the layers (6 us) and three
-// quarters of the host time (24 layers of library calls: 2.1 ms, all of it host).
+// alone 9.3, 7.1, 3.9 and 8.0.  Four stages in registers instead of two change nothing: it is the way of a stage through LDS and the
+// barrier.  What the kernels save is the norm between the layers (6 us) and three quarters of the host time (24 layers of library
+// calls: 2.1 ms, all of it host).
 // float32 runs the same tiles with sixteen times less of the matrix unit's rate (16x16x4, 150 TFLOP/s): the same host
 // time is saved, until the product itself is longer than a library call (a training layer of 1614 steps and width 424
 // 0.69 ms, 0.81 with library calls; 168 steps of ten layers of width 640 without gradients 0.63 and 0.85 ms).
@@ -454,7 +455,8 @@ static int launch_linear(const LinearParams& p, const LinearForm& f, hipStream_t
 // 64, 15 with 32 x 32; out_proj 7.9 us with 64 x 32 on eight waves, 10.8 with 64 x 64; x_proj 6.7 and 10.2 us).
 // Where those are more than one round and tiles twice as long are not, these (bfloat16, in_proj: 1024 steps of width 768
 // 12.8 us for 14.4, 1400 of 512 10.7 for 11.7, 2048 of 400 11.0 for 12.1; in one round the small ones: 700 of 640 9.1 for 11.4; with
-// more than one round of either there is no difference).
+// more than one round of either there is no difference).  Of the plain products in training it makes no difference (four layers of
+// 1400 steps of width 512, forward and backward, 862 us of kernels and 863), and they take them by the same rule.
 template <typename IO>
 static int dispatch_linear(const LinearParams& p, const LinearForm& f, hipStream_t st) {
     auto tiles = [&](int bt, int bm) { return (int64_t)((p.T + bt - 1) / bt) * ((p.M + bm - 1) / bm); };

@@ -288,7 +288,7 @@ __device__ __forceinline__ void chain_segments(const float* hend, const float* d
 // instructions of the idle matrix pipe a tile and wave stand in for a product of its own over the whole sequence and for
 // delta's way through memory.  Rounded to bfloat16, as that product's output is, it is the same delta.  (With lanes on 64
 // channels and sixteen v_mfma_f32_4x4x4_16b the loaders fell behind: 8 x 3000 x 1536 17 us slower.)  24 layers of width 768:
-// 8 x 3000 steps 12.87 -> 12.22 ms, 1 x 512 steps 1433 -> 1342 us.
+// 8 x 3000 steps 13.31 -> 12.86 ms (the scan is 13 us of 176 longer, the product that went took 25), 1 x 512 steps 1269 -> 1187 us.
 constexpr int kProjRank = MPA_PROJ_RANK;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
