@@ -356,7 +356,8 @@ __global__ void __launch_bounds__((NW + kSvc) * kWave) sscan_bwd_fast_kernel(con
                 wd = left(p.d_sb, p.d_sl, p.d_sd, p.ED, kESd);
                 wy = left(p.y_sb, p.y_sl, p.y_sd, p.ED);
                 wz = left(p.z_sb, p.z_sl, p.z_sd, p.ED);
-                wbc = window_bytes((p.batch - 1) * p.bc_sb + (p.L - 1) * p.bc_sl + p.N, b * p.bc_sb + tb * p.bc_sl, kES);
+                // (of B and C to the end of this row: padded steps multiply them by zero, and what follows may be a NaN)
+                wbc = ((uint32_t)(p.L - 1 - pc * kTile) * (uint32_t)p.bc_sl + (uint32_t)p.N) * kES;
             }
             const Steps sx = steps_of(rowx), sy = steps_of(rowy), sd = steps_of(rowd);
             const Steps sz = steps_of(rowz);
@@ -440,7 +441,7 @@ __global__ void __launch_bounds__((NW + kSvc) * kWave) sscan_bwd_fast_kernel(con
             tile_st(sX + s4, ci, qi, xv[0], xv[1], xv[2], xv[3]);
 #pragma unroll
             for (int r = 0; r < kBcPer; ++r) {
-                // states beyond d_state: B = C = 0 (padded steps need no care: u = dy = 0)
+                // states beyond d_state: B = C = 0 (padded steps read zeros, see load_tile: u = dy = 0 as well)
                 const bool ok = bcn[r] < p.N;
                 float* dst = sBC + (k & 1) * kBcF + bcn[r] * kTile + bct[r];
                 dst[0] = ok ? to_float(raw.b[r]) : 0.0f;

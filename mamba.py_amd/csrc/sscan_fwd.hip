@@ -464,7 +464,8 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
                     else
                         wd = left(p.d_sb, p.d_sl, p.d_sd, p.ED, kESd);
                     wz = left(p.z_sb, p.z_sl, p.z_sd, p.ED);
-                    wbc = window_bytes((p.batch - 1) * p.bc_sb + (p.L - 1) * p.bc_sl + p.N, b * p.bc_sb + tb * p.bc_sl, kES);
+                    // (of B and C to the end of this row: padded steps multiply them by zero, and what follows may be a NaN)
+                    wbc = ((uint32_t)(p.L - 1 - pc * kTile) * (uint32_t)p.bc_sl + (uint32_t)p.N) * kES;
                 }
 #pragma unroll
                 for (int j = 0; j < S; ++j) {
@@ -493,8 +494,8 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
                 if (!kBcast) asm volatile("" ::"v"(raw.warm.x), "v"(raw.warm.w));  // keeps the touch alive
 #pragma unroll
                 for (int r = 0; r < kBcPer; ++r) {
-                    // states beyond d_state: B = C = 0 (padded steps need no care: u = 0 there
-                    // and their y is never stored)
+                    // states beyond d_state: B = C = 0 (padded steps read zeros, see load_tile, or what
+                    // stands in this row: u = 0 there and their y is never stored)
                     const bool ok = bcn[r] < p.N;
                     if (NP * kTile % kSvcThreads != 0 && bcn[r] >= NP) continue;
                     float* dst = sBC + (k & 1) * (2 * NP * kTile) + bcn[r] * kTile + bct[r];
@@ -519,6 +520,21 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
 #pragma unroll
                     for (int j = 0; j < S; ++j) dv[j] = softplus_f(dv[j] + bias);
                 }
+                auto gate = [&] {
+#pragma unroll
+                    for (int j = 0; j < S; ++j) {
+                        const float zv = to_float(raw.z[j]);
+                        gg[j] = zv * sigmoid_f(zv);
+                    }
+                };
+                if constexpr (MODE == kGCarry) {
+                    // `x` is the upstream gradient dy here; the recurrence sees dy * silu(z) (z of a padded step may be a NaN)
+                    if (has_z) {
+                        gate();
+#pragma unroll
+                        for (int j = 0; j < S; ++j) xv[j] *= gg[j];
+                    }
+                }
                 const int pc = phys_chunk(k);
                 if (!group_full || (ragged_seq && pc == last_chunk)) {
                     // ragged edge: delta = 0, u = 0 keeps the state of padded steps/channels
@@ -536,19 +552,10 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
                 }
                 const int q4 = S * qi;
                 put_steps<S>(&sDl[k & 1][ci][q4], dv);
-                if (has_z) {
-#pragma unroll
-                    for (int j = 0; j < S; ++j) {
-                        const float zv = to_float(raw.z[j]);
-                        gg[j] = zv * sigmoid_f(zv);
-                    }
+                if constexpr (MODE != kGCarry) {
+                    if (has_z) gate();
                 }
                 if constexpr (MODE == kGCarry) {
-                    // `x` is the upstream gradient dy here; the recurrence sees dy * silu(z)
-                    if (has_z) {
-#pragma unroll
-                        for (int j = 0; j < S; ++j) xv[j] *= gg[j];
-                    }
                     put_steps<S>(&sU[k & 1][ci][q4], xv);
                 } else {
                     float uv[S];
