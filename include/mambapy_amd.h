@@ -457,7 +457,7 @@ int mpa_cast(const mpa_cast_job* jobs, int32_t n, void* stream);
  * y (T x M) = x (T x K) . w (M x K)^T [+ bias] in float32 on the 16-bit matrix cores: each operand is cut into two
  * float16 parts per value with one power of two per row, mpa_split_run, and up to MPA_SPLIT_MAX_PRODUCTS products of cut operands
  * run in one launch, mpa_split_product.  A value keeps 2^-23 of itself, 2^-20 (from K = 2048 on K / 64 * 2^-24) where it is below 2^-28 of
- * its row's largest; a row with values more than 2^31 (K / 1024 * 2^31) apart, zeros aside, or with an infinity is multiplied as it is,
+ * its row's largest; a row with values more than 2^31 (K / 1024 * 2^31) apart, zeros aside, or with an infinity is multiplied
  * in float32 (split.hip).
  *
  * An operand has `rows` rows of length k: element (row, i) is src[row * pitch + i], or with by_cols
