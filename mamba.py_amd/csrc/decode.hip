@@ -100,19 +100,14 @@ __device__ __forceinline__ u32x4 ld16(const void* p) { return *static_cast<const
 // Loads that may not be wanted are buffer loads at an offset beyond the window, which read zero: a load within a branch makes the
 // compiler wait for all loads in flight at the next use of any (the product loop then had one memory latency for every
 // piece of a wave; 64 sequences through in_proj at width 2560, float32, 56 us).
-__device__ __forceinline__ uint32_t wanted(uint32_t at, bool ok) {
-    asm("" : "+v"(at));  // (formed either way: or the choice becomes a branch around its arithmetic, and around the load)
-    return ok ? at : 0xffffffe0u;
-}
-__device__ __forceinline__ u32x4 ld16(rsrc_t r, uint32_t at, bool ok) { return __builtin_amdgcn_raw_buffer_load_b128(r, wanted(at, ok), 0, 0); }
-__device__ __forceinline__ float ld_f32(rsrc_t r, uint32_t at, bool ok) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, wanted(at, ok), 0, 0));
-}
 template <typename IO>
-__device__ __forceinline__ IO ld_io(rsrc_t r, uint32_t i, bool ok) {
-    const uint32_t at = wanted(i * (uint32_t)sizeof(IO), ok);
-    if constexpr (sizeof(IO) == 4) return __builtin_bit_cast(IO, __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0));
-    else return __builtin_bit_cast(IO, __builtin_amdgcn_raw_buffer_load_b16(r, at, 0, 0));
+__device__ __forceinline__ auto ld_bits(rsrc_t r, uint32_t at) {
+    if constexpr (sizeof(IO) == 4) return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0);
+    else return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, at, 0, 0);
+}
+__device__ __forceinline__ float ld_f32(rsrc_t r, uint32_t at, bool ok) {
+    asm("" : "+v"(at));  // (formed either way: or the choice becomes a branch around its arithmetic, and around the load)
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, ok ? at : 0xffffffe0u, 0, 0));
 }
 // window of n elements, none without a pointer
 __device__ __forceinline__ rsrc_t window(const void* p, int64_t n, int es) { return make_rsrc(p, p ? (uint32_t)(n * es) : 0u); }
@@ -126,20 +121,15 @@ __device__ __forceinline__ int64_t frag_at(int b, int k, int K) {
     return (tile * (8 / kVec) + k % 8 / kVec) * (64 * kVec) + ((b & 15) + 16 * (k % 32 / 8)) * kVec + k % kVec;
 }
 __host__ __device__ inline int64_t frag_bytes(int64_t batch, int64_t K, int es) { return (batch + 15) / 16 * ((K + 31) / 32) * 512 * es; }
-// One value of an activation; the last four of a float32 row whose eight are not whole bring the zeros after them.
-template <typename IO>
-__device__ __forceinline__ void frag_store(void* base, int b, int k, int K, IO v) {
-    IO* const to = static_cast<IO*>(base) + frag_at<IO>(b, k, K);
-    *to = v;
-    if constexpr (sizeof(IO) == 4) {
-        if (k % 8 < 4 && k + 4 >= K) to[256] = 0.0f;
-    }
-}
 template <typename IO>
 __device__ __forceinline__ float frag_load(const void* base, int b, int k, int K) {
     return load_as_float<IO>(base, frag_at<IO>(b, k, K));
 }
-// Activations in operand order.
+// An offset beyond any window here (they are below 2 GB): the load reads zero, with a scalar offset on top as well.
+constexpr uint32_t kNowhere = 0x80000000u;
+
+// Activations in operand order; request() takes a chunk of 32 k, of which `left` are wanted (any number, also below zero).  Offsets
+// within a chunk are formed once, the chunk is a scalar offset.
 template <typename IO, int NT>
 struct FragAct {
     static constexpr int kLoads = 8 / Frag<IO>::kVec;
@@ -148,18 +138,19 @@ struct FragAct {
     };
     rsrc_t r;
     uint32_t at[NT];
-    bool live[NT];
+    int kl;
     __device__ __forceinline__ void setup(const void* base, int b0, int batch, int K, int lane) {
-        r = make_rsrc(base, (uint32_t)frag_bytes(batch, K, sizeof(IO)));
+        const uint32_t tile = (uint32_t)((K + 31) / 32) * (512u * sizeof(IO));
+        r = make_rsrc(static_cast<const char*>(base) + (int64_t)(b0 >> 4) * tile, (uint32_t)(((batch - b0 + 15) >> 4) * tile));
+        kl = 8 * (lane >> 4);
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            at[t] = (uint32_t)(sizeof(IO) * frag_at<IO>(b0 + t * 16, 0, K)) + lane * 16;
-            live[t] = b0 + t * 16 + (lane & 15) < batch;  // (one sequence then reads a sixteenth of its tile)
-        }
+        for (int t = 0; t < NT; ++t)  // (one sequence then reads a sixteenth of its tile)
+            at[t] = b0 + t * 16 + (lane & 15) < batch ? t * tile + lane * 16u : kNowhere;
     }
-    __device__ __forceinline__ void request(Raw& v, int t, int chunk, int, int, bool ok) {
+    __device__ __forceinline__ void request(Raw& v, int t, int chunk, int left) {
+        const uint32_t from = kl < left ? at[t] : kNowhere;
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i) v.x[i] = ld16(r, at[t] + (uint32_t)(chunk * kLoads + i) * 1024u, ok && live[t]);
+        for (int i = 0; i < kLoads; ++i) v.x[i] = __builtin_amdgcn_raw_buffer_load_b128(r, from + i * 1024u, (uint32_t)(chunk * kLoads) * 1024u, 0);
     }
     __device__ __forceinline__ typename Frag<IO>::Op operand(const Raw& v, int) { return Frag<IO>::from(v.x); }
 };
@@ -175,26 +166,29 @@ struct RowAct {
     };
     rsrc_t r, rw;
     uint32_t at[NT];
-    bool live[NT], gain;
+    int kl;
+    bool gain;
     float ss[NT];
     __device__ __forceinline__ void setup(const void* base, const float* w, int b0, int batch, int K, int lane) {
         r = window(base, (int64_t)batch * K, sizeof(IO));
         rw = window(w, K, 4);
         gain = w != nullptr;
+        kl = 8 * (lane >> 4);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             const int b = b0 + t * 16 + (lane & 15);
-            live[t] = b < batch;
-            at[t] = (uint32_t)b * (uint32_t)K * (uint32_t)sizeof(IO);
+            at[t] = b < batch ? ((uint32_t)b * (uint32_t)K + kl) * (uint32_t)sizeof(IO) : kNowhere;
             ss[t] = 0.0f;
         }
     }
-    __device__ __forceinline__ void request(Raw& v, int t, int, int k, int K, bool ok) {
+    __device__ __forceinline__ void request(Raw& v, int t, int chunk, int left) {
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i) v.x[i] = ld16(r, at[t] + (uint32_t)(k + i * kVec) * (uint32_t)sizeof(IO), ok && live[t] && k + i * kVec < K);
+        for (int i = 0; i < kLoads; ++i)
+            v.x[i] = __builtin_amdgcn_raw_buffer_load_b128(r, (kl + i * kVec < left ? at[t] : kNowhere) + i * 16u, (uint32_t)chunk * 32u * (uint32_t)sizeof(IO), 0);
         if constexpr (NORM) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) v.w[i] = __builtin_bit_cast(f32x4, ld16(rw, (uint32_t)(k + 4 * i) * 4u, k + 4 * i < K));
+            for (int i = 0; i < 2; ++i)
+                v.w[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, kl + 4 * i < left ? (uint32_t)(kl + 4 * i) * 4u : kNowhere, (uint32_t)chunk * 128u, 0));
         }
     }
     __device__ __forceinline__ typename Frag<IO>::Op operand(const Raw& v, int t) {
@@ -226,37 +220,45 @@ struct alignas(16) WaveLds {
 template <int NW, typename L>
 __device__ __forceinline__ float tile_sum(const L (&lds)[NW], int row, int b) {
     const int at = ((b >> 4) * L::kMT + (row >> 4)) * 256 + ((row % 16 >> 2) * 16 + (b & 15)) * 4 + (row & 3);
-    float s = lds[0].v[at];
+    float s[NW];
 #pragma unroll
-    for (int w = 1; w < NW; ++w) s += lds[w].v[at];
-    return s;
+    for (int w = 0; w < NW; ++w) s[w] = lds[w].v[at];
+#pragma unroll
+    for (int o = 1; o < NW; o *= 2)  // (pairs: additions in a row are 9 clocks each)
+#pragma unroll
+        for (int w = 0; w + o < NW; w += 2 * o) s[w] += s[w + o];
+    return s[0];
+}
+// sum over the 16 lanes of a row, in all of them
+__device__ __forceinline__ float row_sum(float v) {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x128, 0xf, 0xf, true));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x124, 0xf, 0xf, true));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x122, 0xf, 0xf, true));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x121, 0xf, 0xf, true));
+    return v;
 }
 
 // Rows n0 .. n0+16*MT-1 of `W . x^T` for NT batch tiles, over the 128-byte pieces first + wave, + NW, ...
 // below `last` of the rows of W; the wave leaves its partial tiles in its LDS.  U pieces are in flight (`more` issues the caller's own
 // loads behind them), each with its activations: loads return in the order they were issued, so
 // activations requested later than weights of pieces further on would wait for those as well.
-template <typename IO, int NW, int U, int MT, int NT, typename ACT, typename MORE>
+// ONCE: no wave has more than U pieces, and there is no loop.
+// What a wave does before its first load and between the last one's arrival and its result is time that nothing hides (a wave
+// issues an instruction every five clocks at best, and a step of one sequence is a chain of such kernels): offsets of lanes are formed
+// once, pieces are scalar offsets, what lies beyond the rows or beyond K reads zero.
+template <typename IO, int NW, int U, bool ONCE, int MT, int NT, typename ACT, typename MORE>
 __device__ __forceinline__ void decode_product(WaveLds<MT, NT>& lds, const void* W, int rows, int K, int n0, int first, int last, int wave,
                                                int lane, ACT& act, MORE&& more) {
     constexpr int kVec = Frag<IO>::kVec, kES = sizeof(IO);
     char* const slot = reinterpret_cast<char*>(lds.v);
     // lane -> 16 bytes of row 8*i + lane/8: the piece's eight 16-byte parts are stored rotated by the row
     // (part ^ (row & 7)), so that the operand reads, one row per lane, fall on different banks
-    const uint32_t part = ((lane & 7) ^ (lane >> 3)) * 16u;
-    const int left = rows - n0;
-    const rsrc_t rw = make_rsrc(static_cast<const IO*>(W) + (int64_t)n0 * K, (uint32_t)min(left, 16 * MT) * (uint32_t)K * kES);
+    const int part = ((lane & 7) ^ (lane >> 3)) * 16;
+    const rsrc_t rw = make_rsrc(static_cast<const IO*>(W) + (int64_t)n0 * K, (uint32_t)max(min(rows - n0, 16 * MT), 0) * (uint32_t)K * kES);
     uint32_t row[2 * MT];
 #pragma unroll
-    for (int i = 0; i < 2 * MT; ++i) row[i] = (uint32_t)min(8 * i + (lane >> 3), left - 1) * (uint32_t)K * kES + part;
+    for (int i = 0; i < 2 * MT; ++i) row[i] = (uint32_t)(lane >> 3) * (uint32_t)K * kES + part + (uint32_t)(8 * i * K) * kES;
     constexpr int kOps = Frag<IO>::kOps, kReads = 2 / kOps;  // operands of a piece; 16-byte parts of one
-    const int kl = 8 * (lane >> 4);
-    int frag[kOps][kReads];
-#pragma unroll
-    for (int h = 0; h < kOps; ++h)
-#pragma unroll
-        for (int i = 0; i < kReads; ++i) frag[h][i] = (lane & 15) * 128 + ((((lane >> 4) * kReads + i + 4 * h) ^ (lane & 7)) << 4);
-    const int count = first + wave < last ? (last - first - wave + NW - 1) / NW : 0;  // pieces of this wave
     const int k_end = min(last * 8 * kVec, K);
 
     struct Piece {
@@ -266,16 +268,22 @@ __device__ __forceinline__ void decode_product(WaveLds<MT, NT>& lds, const void*
     Piece r[U];
     auto request = [&](Piece& v, int s) {
         const int piece = first + wave + s * NW;
+        const bool ok = part < k_end * kES - piece * 128;
 #pragma unroll
-        for (int i = 0; i < 2 * MT; ++i) v.w[i] = ld16(rw, row[i] + (uint32_t)piece * 128u, (uint32_t)piece * 128u + part < (uint32_t)k_end * kES);
+        for (int i = 0; i < 2 * MT; ++i) v.w[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, ok ? row[i] : kNowhere, (uint32_t)piece * 128u, 0);
 #pragma unroll
         for (int h = 0; h < kOps; ++h) {
-            const int chunk = kOps * piece + h, k = chunk * 32 + kl;
+            const int chunk = kOps * piece + h;
 #pragma unroll
-            for (int t = 0; t < NT; ++t) act.request(v.a[t][h], t, chunk, k, K, k < k_end);
+            for (int t = 0; t < NT; ++t) act.request(v.a[t][h], t, chunk, k_end - chunk * 32);
         }
     };
     f32x4 acc[MT][NT] = {};
+    int frag[kOps][kReads];
+#pragma unroll
+    for (int h = 0; h < kOps; ++h)
+#pragma unroll
+        for (int i = 0; i < kReads; ++i) frag[h][i] = (lane & 15) * 128 + ((((lane >> 4) * kReads + i + 4 * h) ^ (lane & 7)) << 4);
     auto multiply = [&](const Piece& v, int u) {
         char* const at = slot + (u & 1) * (2048 * MT);
 #pragma unroll
@@ -297,19 +305,26 @@ __device__ __forceinline__ void decode_product(WaveLds<MT, NT>& lds, const void*
 #pragma unroll
     for (int u = 0; u < U; ++u) request(r[u], u);
     more();
-    // (whole groups without a branch; what is requested beyond the last piece are zeros)
-    int s = 0;
-    for (; s + U <= count; s += U) {
+    if constexpr (ONCE) {
+        // (all pieces; what lies beyond the last are zeros)
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            multiply(r[u], u);
-            request(r[u], s + u + U);
+        for (int u = 0; u < U; ++u) multiply(r[u], u);
+    } else {
+        const int count = first + wave < last ? (last - first - wave + NW - 1) / NW : 0;  // pieces of this wave
+        // (whole groups without a branch; what is requested beyond the last piece are zeros)
+        int s = 0;
+        for (; s + U <= count; s += U) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                multiply(r[u], u);
+                request(r[u], s + u + U);
+            }
         }
-    }
 #pragma unroll
-    for (int u = 0; u < U - 1; ++u) {
-        if (s + u >= count) break;  // uniform over the wave
-        multiply(r[u], u);
+        for (int u = 0; u < U - 1; ++u) {
+            if (s + u >= count) break;  // uniform over the wave
+            multiply(r[u], u);
+        }
     }
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -319,7 +334,10 @@ __device__ __forceinline__ void decode_product(WaveLds<MT, NT>& lds, const void*
 
 struct DecodeParams {
     int batch, d, ED, N, R, K;  // K: convolution taps
-    float eps;
+    int P4;         // dt_rank + 2 d_state to a multiple of four: pitch of dbc
+    uint32_t span_inv;  // of a launch's tiles, see decode_tile
+    int groups;
+    float eps, inv_d;
     int splits, ssq_tiles;  // partial sums of x_proj; row tiles of d (partial sums of squares)
     const void* x;
     const void* xw;        // x times the norm weight in operand order, or null: formed from x
@@ -335,7 +353,7 @@ struct DecodeParams {
     const void* win_in;
     void* win_out;
     void *xs, *z, *g;  // in the workspace: convolved x, gate (batch, ED), gated readout; xs and g in operand order
-    float* dbc;        // [splits][batch][R + 2N]
+    float* dbc;        // [splits][batch][P4]
     void* y;
     const float* next_w;  // norm weight of the next layer, with y_w and ssq_out
     void* y_w;
@@ -346,92 +364,121 @@ struct DecodeParams {
 enum { kInPlain, kInNorm, kInReady };
 
 // grid: (row tiles) x (batch tile groups), batch groups of one row tile eight blocks apart: the
-// blocks of an XCD (every eighth) then meet the same rows of W again in their own L2.
+// blocks of an XCD (every eighth) then meet the same rows of W again in their own L2.  (id / (8 * groups) as a product with
+// span_inv = 2^32 / (8 * groups) rounded up, exact below 2^25 blocks.)  A tile beyond the last has no rows: it reads zeros and stores nothing.
 template <int NT>
-__device__ __forceinline__ void decode_tile(int row_tiles, int groups, int& rt, int& bt) {
-    const int id = blockIdx.x;
-    if (groups == 1) {
-        rt = id;
-        bt = 0;
-        return;
-    }
-    const int span = 8 * groups, g = id / span, in = id - g * span;
-    rt = g * 8 + (in & 7);
-    bt = (in >> 3) * NT;
+__device__ __forceinline__ void decode_tile(const DecodeParams& p, int& rt, int& bt) {
+    const uint32_t id = blockIdx.x, g = __umulhi(id, p.span_inv), in = id - g * 8u * (uint32_t)p.groups;
+    rt = (int)(g * 8 + (in & 7));
+    bt = (int)(in >> 3) * NT;
 }
+
+template <typename IO>
+__device__ __forceinline__ void st_io(rsrc_t r, uint32_t at, IO v) {
+    if constexpr (sizeof(IO) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, at, 0, 0);
+    else __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, at, 0, 0);
+}
+// byte offset of an activation in operand order, and its store (with the zeros after the last four of a float32 row whose eight are not whole)
+template <typename IO>
+__device__ __forceinline__ uint32_t frag_offset(int b, int k, int K) {
+    constexpr uint32_t kVec = Frag<IO>::kVec;
+    const uint32_t tile = (uint32_t)(b >> 4) * (uint32_t)((K + 31) / 32) + ((uint32_t)k >> 5);
+    return (uint32_t)sizeof(IO) * (tile * 512u + ((uint32_t)k % 8 / kVec) * (64 * kVec) + ((b & 15) + 16 * ((uint32_t)k % 32 / 8)) * kVec + (uint32_t)k % kVec);
+}
+template <typename IO>
+__device__ __forceinline__ void frag_store_at(rsrc_t r, uint32_t at, int k, int K, IO v) {
+    st_io<IO>(r, at, v);
+    if constexpr (sizeof(IO) == 4) st_io<float>(r, k % 8 < 4 && k + 4 >= K ? at + 1024u : kNowhere, 0.0f);
+}
+// n / d for n < 2^20: (n + 1/2) / d is at least 1 / 2d from a whole number, and off by n / d * 2^-22 at most
+__device__ __forceinline__ int div_small(int n, int d) { return (int)(((float)n + 0.5f) * __builtin_amdgcn_rcpf((float)d)); }
 
 // XP: also the workgroup's share of x_proj, its 16 channels' product with all rows of x_proj's weight, as one
 // more partial sum of dbc; a thread owns one row and every so many sequences (there are as many threads as rows, or more).
-template <typename IO, int MT, int NT, int NW, int U, int MODE, bool XP = false>
-__global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams p, int row_tiles, int groups) {
+template <typename IO, int MT, int NT, int NW, int U, bool ONCE, int MODE, bool XP = false>
+__global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams p) {
     constexpr int kThreads = NW * kWave, kRows = MT * 16, kAll = NT * 16 * kRows, kOuts = (kAll + kThreads - 1) / kThreads;
     static_assert(!XP || MT == 1, "x_proj by 16 channels");
     __shared__ WaveLds<MT, NT> tile[NW];
     __shared__ float ssq[NW][NT][16];
-    __shared__ float xl[XP ? NT * 16 : 1][16];  // convolved x of the tile
+    __shared__ alignas(16) float xl[XP ? NT * 16 : 1][16];  // convolved x of the tile
     int rt, bt;
-    decode_tile<NT>(row_tiles, groups, rt, bt);
-    if (rt >= row_tiles) return;  // uniform over the block
+    decode_tile<NT>(p, rt, bt);
     const int lane = threadIdx.x & (kWave - 1), wave = wave_id();
     const int n0 = rt * kRows, b0 = bt * 16, rows = 2 * p.ED;
     const int pieces = (p.d + 8 * Frag<IO>::kVec - 1) / (8 * Frag<IO>::kVec);
-    // the epilogue's operands: thread -> outputs (row o % kRows, sequence o / kRows)
-    IO win[kOuts][3];
-    float cw[kOuts][4], cb[kOuts], ib[kOuts];
+    // the epilogue's operands: thread -> outputs (row o % kRows, sequence o / kRows), and where its results go
+    IO win[kOuts][3], ib[kOuts];
+    float cw[kOuts][4], cb[kOuts];
+    uint32_t to_win[kOuts], to_z[kOuts], to_xs[kOuts];
     float ss[NT] = {};
     const int P = p.R + 2 * p.N;
+    int xrow = 0, xgroup = 0;
     u32x4 xw[XP ? 16 / Frag<IO>::kVec : 1];
-    // wave w, lane group q: partial sums of squares 4w + q, 4w + q + 4*NW, ... of column lane % 16, four requested together and the
-    // first four ahead of the product
+    // wave w, lane group q: partial sums of squares 4w + q, 4w + q + 4*NW, ... of column lane % 16, up to a width of 1024 requested together
+    // and ahead of the product
+    constexpr int kSums = NW >= 16 ? 1 : 16 / NW;
     const rsrc_t rs = window(p.ssq, (int64_t)p.ssq_tiles * p.batch, 4);
-    float sq[NT][4];
+    float sq[NT][kSums];
     auto request_sums = [&](int q0) {
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < kSums; ++i) {
                 const int b = b0 + t * 16 + (lane & 15), q = q0 + 4 * (wave + NW * i) + (lane >> 4);
-                sq[t][i] = ld_f32(rs, (uint32_t)(q * p.batch + b) * 4u, b < p.batch && q < p.ssq_tiles);
+                // (beyond the last row of sums is beyond the window)
+                sq[t][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, b < p.batch ? (uint32_t)(q * p.batch + b) * 4u : kNowhere, 0, 0));
             }
     };
+    const rsrc_t rwo = window(p.win_out, (int64_t)p.batch * p.ED * (p.K - 1), sizeof(IO)), rz = window(p.z, (int64_t)p.batch * p.ED, sizeof(IO)),
+                 rxs = make_rsrc(p.xs, (uint32_t)frag_bytes(p.batch, p.ED, sizeof(IO)));
     auto more = [&] {
-        if constexpr (XP) {
-            // (a part beyond the last channel is read at the row's start and meets zeros)
-            const IO* row = static_cast<const IO*>(p.xp_w) + (int64_t)(threadIdx.x % P) * p.ED;
-#pragma unroll
-            for (int i = 0; i < 16 / Frag<IO>::kVec; ++i) {
-                const int k = n0 + i * Frag<IO>::kVec;
-                xw[i] = ld16(row + (k < p.ED ? k : 0));
-            }
-        }
+        if constexpr (MODE == kInReady) request_sums(0);
         const rsrc_t rb = window(p.in_b, rows, sizeof(IO)), rwin = window(p.win_in, (int64_t)p.batch * p.ED * (p.K - 1), sizeof(IO)),
                      rcw = window(p.conv_w, (int64_t)p.ED * p.K, 4), rcb = window(p.conv_b, p.ED, 4);
 #pragma unroll
         for (int i = 0; i < kOuts; ++i) {
             const int o = threadIdx.x + i * kThreads, n = n0 + o % kRows, b = b0 + o / kRows;
-            const bool some = o < kAll && n < rows && b < p.batch, conv = some && n < p.ED;
-            ib[i] = to_float(ld_io<IO>(rb, n, some));
+            const bool some = (kOuts * kThreads == kAll || o < kAll) && n < rows && b < p.batch, conv = some && n < p.ED;
+            const uint32_t at = (uint32_t)b * (uint32_t)p.ED + (uint32_t)n;
+            to_win[i] = conv ? at * (uint32_t)(p.K - 1) * (uint32_t)sizeof(IO) : kNowhere;
+            to_z[i] = some && n >= p.ED ? (at - (uint32_t)p.ED) * (uint32_t)sizeof(IO) : kNowhere;
+            to_xs[i] = conv ? frag_offset<IO>(b, n, p.ED) : kNowhere;
+            ib[i] = __builtin_bit_cast(IO, ld_bits<IO>(rb, (uint32_t)n * (uint32_t)sizeof(IO)));
+            // (taps that the layer does not have are read from what follows, and not used)
 #pragma unroll
-            for (int j = 0; j < 3; ++j) win[i][j] = ld_io<IO>(rwin, (uint32_t)(b * p.ED + n) * (uint32_t)(p.K - 1) + j, conv && j < p.K - 1);
+            for (int j = 0; j < 3; ++j) win[i][j] = __builtin_bit_cast(IO, ld_bits<IO>(rwin, to_win[i] + j * (uint32_t)sizeof(IO)));
+            const uint32_t cat = conv ? (uint32_t)(n * p.K) * 4u : kNowhere;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) cw[i][j] = ld_f32(rcw, (uint32_t)(n * p.K + j) * 4u, conv && j < p.K);
-            cb[i] = ld_f32(rcb, (uint32_t)n * 4u, conv);
+            for (int j = 0; j < 4; ++j) cw[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rcw, cat + 4u * j, 0, 0));
+            cb[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rcb, (uint32_t)n * 4u, 0, 0));
         }
-        if constexpr (MODE == kInReady) request_sums(0);
+        if constexpr (XP) {
+            xgroup = div_small(threadIdx.x, P);
+            xrow = (int)threadIdx.x - xgroup * P;
+            const rsrc_t rx = window(p.xp_w, (int64_t)P * p.ED, sizeof(IO));
+#pragma unroll
+            for (int i = 0; i < 16 / Frag<IO>::kVec; ++i) {  // (zeros beyond the last channel)
+                const int k = n0 + i * Frag<IO>::kVec;
+                xw[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, k < p.ED ? (uint32_t)(xrow * p.ED + k) * (uint32_t)sizeof(IO) : kNowhere, 0, 0);
+            }
+        }
     };
     if constexpr (MODE == kInReady) {
         FragAct<IO, NT> act;
         act.setup(p.xw, b0, p.batch, p.d, lane);
-        decode_product<IO, NW, U>(tile[wave], p.in_w, rows, p.d, n0, 0, pieces, wave, lane, act, more);
+        decode_product<IO, NW, U, ONCE>(tile[wave], p.in_w, rows, p.d, n0, 0, pieces, wave, lane, act, more);
         for (int q0 = 0;; request_sums(q0)) {
 #pragma unroll
-            for (int t = 0; t < NT; ++t) ss[t] += (sq[t][0] + sq[t][1]) + (sq[t][2] + sq[t][3]);
-            if ((q0 += 16 * NW) >= p.ssq_tiles) break;
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int i = 0; i < kSums; ++i) ss[t] += sq[t][i];
+            if ((q0 += 4 * NW * kSums) >= p.ssq_tiles) break;
         }
     } else {
         RowAct<IO, NT, MODE == kInNorm> act;
         act.setup(p.x, p.norm_w, b0, p.batch, p.d, lane);
-        decode_product<IO, NW, U>(tile[wave], p.in_w, rows, p.d, n0, 0, pieces, wave, lane, act, more);
+        decode_product<IO, NW, U, ONCE>(tile[wave], p.in_w, rows, p.d, n0, 0, pieces, wave, lane, act, more);
 #pragma unroll
         for (int t = 0; t < NT; ++t) ss[t] = act.ss[t];
     }
@@ -447,54 +494,66 @@ __global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kOuts; ++i) {
-        const int o = threadIdx.x + i * kThreads, row = o % kRows, bl = o / kRows, n = n0 + row, b = b0 + bl;
-        if (o >= kAll || n >= rows || b >= p.batch) continue;
+        const int o = threadIdx.x + i * kThreads, row = o % kRows, bl = o / kRows, n = n0 + row;
+        if (kOuts * kThreads != kAll && o >= kAll) break;  // uniform over a wave
         float v = tile_sum(tile, row, bl);
         if constexpr (MODE != kInPlain) {
             float s = ssq[0][bl >> 4][bl & 15];
 #pragma unroll
             for (int w = 1; w < NW; ++w) s += ssq[w][bl >> 4][bl & 15];
-            v *= __builtin_amdgcn_rsqf(s / (float)p.d + p.eps);
+            v *= __builtin_amdgcn_rsqf(s * p.inv_d + p.eps);
         }
-        const IO vr = from_float<IO>(v + ib[i]);
-        if (n >= p.ED) {
-            static_cast<IO*>(p.z)[(int64_t)b * p.ED + n - p.ED] = vr;
+        const IO vr = from_float<IO>(v + to_float(ib[i]));
+        if (n0 >= p.ED) {  // uniform over the block
+            st_io<IO>(rz, to_z[i], vr);
             continue;
         }
         // newest tap first, then the window from its newest input backwards
-        const int last = p.K - 2;
-        IO* wo = static_cast<IO*>(p.win_out) + ((int64_t)b * p.ED + n) * (p.K - 1);
         float c = cb[i];
+        IO keep[3] = {win[i][1], win[i][2], vr};  // the window after this step
+        if (p.K == 4) {
+            c = __builtin_fmaf(cw[i][3], to_float(vr), c);
 #pragma unroll
-        for (int j = 3; j >= 0; --j)
-            if (j == p.K - 1) c = __builtin_fmaf(cw[i][j], to_float(vr), c);
-            else if (j < p.K - 1) c = __builtin_fmaf(cw[i][j], to_float(win[i][j < 3 ? j : 2]), c);
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            if (j <= last) wo[j] = j < last ? win[i][j < 2 ? j + 1 : 2] : vr;
+            for (int j = 2; j >= 0; --j) c = __builtin_fmaf(cw[i][j], to_float(win[i][j]), c);
+        } else if (p.K == 3) {
+            c = __builtin_fmaf(cw[i][2], to_float(vr), c);
+            c = __builtin_fmaf(cw[i][1], to_float(win[i][1]), c);
+            c = __builtin_fmaf(cw[i][0], to_float(win[i][0]), c);
+            keep[1] = vr;
+        } else {
+            c = __builtin_fmaf(cw[i][1], to_float(vr), c);
+            c = __builtin_fmaf(cw[i][0], to_float(win[i][0]), c);
+            keep[0] = vr;
+        }
         c *= sigmoid_f(c);
         const IO cr = from_float<IO>(c);
-        frag_store<IO>(p.xs, b, n, p.ED, cr);
-        if constexpr (XP) xl[bl][row] = to_float(cr);
+        if constexpr (XP) xl[bl][row] = n < p.ED ? to_float(cr) : 0.0f;
+        frag_store_at<IO>(rxs, to_xs[i], n, p.ED, cr);
+        st_io<IO>(rz, to_z[i], vr);  // (of a tile with the last channels of x and the first of z)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            if (j < p.K - 1) st_io<IO>(rwo, to_win[i] + j * (uint32_t)sizeof(IO), keep[j]);
     }
     if constexpr (XP) {
         if (n0 >= p.ED) return;  // uniform over the block
-        if (n0 + 16 > p.ED)
-            for (int o = threadIdx.x; o < kAll; o += kThreads)
-                if (n0 + o % 16 >= p.ED) xl[o / 16][o % 16] = 0.0f;
         __syncthreads();
-        const int G = kThreads / P, g = threadIdx.x / P, nb = min(p.batch - b0, NT * 16);
-        if (g >= G) return;
-        for (int b = g; b < nb; b += G) {
-            float s = 0.0f;
+        const int G = div_small(kThreads, P), nb = min(p.batch - b0, NT * 16);
+        if (xgroup >= G) return;
+        float w[16];
 #pragma unroll
-            for (int i = 0; i < 16 / Frag<IO>::kVec; ++i) {
-                float w[Frag<IO>::kVec];
-                Frag<IO>::unpack(xw[i], w);
+        for (int i = 0; i < 16 / Frag<IO>::kVec; ++i) {
+            float part[Frag<IO>::kVec];
+            Frag<IO>::unpack(xw[i], part);
 #pragma unroll
-                for (int e = 0; e < Frag<IO>::kVec; ++e) s = __builtin_fmaf(w[e], xl[b][i * Frag<IO>::kVec + e], s);
-            }
-            p.dbc[((int64_t)rt * p.batch + b0 + b) * P + threadIdx.x % P] = s;
+            for (int e = 0; e < Frag<IO>::kVec; ++e) w[i * Frag<IO>::kVec + e] = part[e];
+        }
+        for (int b = xgroup; b < nb; b += G) {
+            float s[4] = {};  // (four chains of four)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[i] = __builtin_fmaf(w[4 * i + e], xl[b][4 * i + e], s[i]);
+            p.dbc[((int64_t)rt * p.batch + b0 + b) * p.P4 + xrow] = (s[0] + s[1]) + (s[2] + s[3]);
         }
     }
 }
@@ -535,72 +594,74 @@ __global__ void __launch_bounds__(256) decode_scale_kernel(const DecodeParams p,
     if (threadIdx.x == 0) ssq[b] = (part[0] + part[1]) + (part[2] + part[3]);
 }
 
-template <typename IO, int NW>
-__global__ void __launch_bounds__(NW* kWave) decode_xproj_kernel(const DecodeParams p, int row_tiles, int groups) {
+template <typename IO, int NW, int U, bool ONCE>
+__global__ void __launch_bounds__(NW* kWave) decode_xproj_kernel(const DecodeParams p) {
     __shared__ WaveLds<1, 1> tile[NW];
     int rt, bt;
-    decode_tile<1>(row_tiles, groups, rt, bt);
-    if (rt >= row_tiles) return;
+    decode_tile<1>(p, rt, bt);
     const int lane = threadIdx.x & (kWave - 1), wave = wave_id(), rows = p.R + 2 * p.N;
     const int pieces = (p.ED + 8 * Frag<IO>::kVec - 1) / (8 * Frag<IO>::kVec);
     const int per = (pieces + gridDim.y - 1) / gridDim.y, first = (int)blockIdx.y * per;
+    const int o = threadIdx.x, n = rt * 16 + (o & 15), b = bt * 16 + (o >> 4);
+    const rsrc_t rd = make_rsrc(p.dbc + (int64_t)blockIdx.y * p.batch * p.P4, (uint32_t)(p.batch * p.P4) * 4u);
+    const uint32_t to = o < 256 && n < rows && b < p.batch ? (uint32_t)(b * p.P4 + n) * 4u : kNowhere;
     FragAct<IO, 1> act;
     act.setup(p.xs, bt * 16, p.batch, p.ED, lane);
-    decode_product<IO, NW, 2>(tile[wave], p.xp_w, rows, p.ED, rt * 16, first, min(pieces, first + per), wave, lane, act, [] {});
+    decode_product<IO, NW, U, ONCE>(tile[wave], p.xp_w, rows, p.ED, rt * 16, first, min(pieces, first + per), wave, lane, act, [] {});
     __syncthreads();
-    const int o = threadIdx.x, n = rt * 16 + (o & 15), b = bt * 16 + (o >> 4);
-    if (o < 256 && n < rows && b < p.batch) p.dbc[((int64_t)blockIdx.y * p.batch + b) * rows + n] = tile_sum(tile, o & 15, o >> 4);
+    if (wave >= 4) return;
+    st_io<float>(rd, to, tile_sum(tile, o & 15, o >> 4));
 }
 
 // y = out_proj(g) [+ x]; with next_w also y * next_w and the sums of squares of 16 columns each
-template <typename IO, int MT, int NT, int NW, int U, bool RES>
-__global__ void __launch_bounds__(NW* kWave) decode_out_kernel(const DecodeParams p, int row_tiles, int groups) {
+template <typename IO, int MT, int NT, int NW, int U, bool ONCE, bool RES>
+__global__ void __launch_bounds__(NW* kWave) decode_out_kernel(const DecodeParams p) {
     constexpr int kThreads = NW * kWave, kRows = MT * 16, kAll = NT * 16 * kRows, kOuts = (kAll + kThreads - 1) / kThreads;
     __shared__ WaveLds<MT, NT> tile[NW];
     int rt, bt;
-    decode_tile<NT>(row_tiles, groups, rt, bt);
-    if (rt >= row_tiles) return;
+    decode_tile<NT>(p, rt, bt);
     const int lane = threadIdx.x & (kWave - 1), wave = wave_id();
     const int n0 = rt * kRows, b0 = bt * 16;
-    float bias[kOuts], xv[kOuts], nw[kOuts];
+    IO bias[kOuts], xv[kOuts];
+    float nw[kOuts];
+    uint32_t to[kOuts], to_yw[kOuts], to_ssq[kOuts];  // of y, y_w and ssq_out
+    const bool next = RES && p.next_w;
+    const rsrc_t ry = window(p.y, (int64_t)p.batch * p.d, sizeof(IO)), ryw = make_rsrc(p.y_w, next ? (uint32_t)frag_bytes(p.batch, p.d, sizeof(IO)) : 0u),
+                 rso = window(next ? p.ssq_out : nullptr, (int64_t)((p.d + 15) / 16) * p.batch, 4);
     auto more = [&] {
         const rsrc_t rb = window(p.out_b, p.d, sizeof(IO)), rx = window(RES ? p.x : nullptr, (int64_t)p.batch * p.d, sizeof(IO)),
                      rn = window(RES ? p.next_w : nullptr, p.d, 4);
 #pragma unroll
         for (int i = 0; i < kOuts; ++i) {
             const int o = threadIdx.x + i * kThreads, n = n0 + o % kRows, b = b0 + o / kRows;
-            const bool ok = o < kAll && n < p.d && b < p.batch;
-            bias[i] = to_float(ld_io<IO>(rb, n, ok));
-            xv[i] = to_float(ld_io<IO>(rx, (uint32_t)(b * p.d + n), ok));
-            nw[i] = ld_f32(rn, (uint32_t)n * 4u, ok);
+            const bool ok = (kOuts * kThreads == kAll || o < kAll) && n < p.d && b < p.batch;
+            to[i] = ok ? (uint32_t)(b * p.d + n) * (uint32_t)sizeof(IO) : kNowhere;
+            to_yw[i] = ok ? frag_offset<IO>(b, n, p.d) : kNowhere;
+            to_ssq[i] = ok && n % 16 == 0 ? (uint32_t)((n >> 4) * p.batch + b) * 4u : kNowhere;
+            bias[i] = __builtin_bit_cast(IO, ld_bits<IO>(rb, (uint32_t)n * (uint32_t)sizeof(IO)));
+            xv[i] = __builtin_bit_cast(IO, ld_bits<IO>(rx, to[i]));
+            nw[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rn, (uint32_t)n * 4u, 0, 0));
         }
     };
     FragAct<IO, NT> act;
     act.setup(p.g, b0, p.batch, p.ED, lane);
-    decode_product<IO, NW, U>(tile[wave], p.out_w, p.d, p.ED, n0, 0, (p.ED + 8 * Frag<IO>::kVec - 1) / (8 * Frag<IO>::kVec), wave,
-                                      lane, act, more);
+    decode_product<IO, NW, U, ONCE>(tile[wave], p.out_w, p.d, p.ED, n0, 0, (p.ED + 8 * Frag<IO>::kVec - 1) / (8 * Frag<IO>::kVec), wave,
+                                    lane, act, more);
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kOuts; ++i) {
-        const int o = threadIdx.x + i * kThreads, row = o % kRows, bl = o / kRows, n = n0 + row, b = b0 + bl;
-        if (o >= kAll) break;  // uniform over a wave
-        const bool ok = n < p.d && b < p.batch;
-        const int64_t at = (int64_t)b * p.d + n;
-        IO v = from_float<IO>(tile_sum(tile, row, bl) + bias[i]);
+        const int o = threadIdx.x + i * kThreads, row = o % kRows, bl = o / kRows, n = n0 + row;
+        if (kOuts * kThreads != kAll && o >= kAll) break;  // uniform over a wave
+        IO v = from_float<IO>(tile_sum(tile, row, bl) + to_float(bias[i]));
         if constexpr (RES) {
-            v = from_float<IO>(to_float(v) + xv[i]);
-            if (p.next_w) {
-                const float f = ok ? to_float(v) : 0.0f;
-                float s = f * f;
-                s += __shfl_xor(s, 1);
-                s += __shfl_xor(s, 2);
-                s += __shfl_xor(s, 4);
-                s += __shfl_xor(s, 8);
-                if (ok) frag_store<IO>(p.y_w, b, n, p.d, from_float<IO>(f * nw[i]));
-                if (ok && row % 16 == 0) p.ssq_out[(int64_t)(n / 16) * p.batch + b] = s;
+            v = from_float<IO>(to_float(v) + to_float(xv[i]));
+            if (next) {
+                const float f = n < p.d ? to_float(v) : 0.0f;
+                frag_store_at<IO>(ryw, to_yw[i], n, p.d, from_float<IO>(f * nw[i]));
+                st_io<float>(rso, to_ssq[i], row_sum(f * f));
             }
         }
-        if (ok) static_cast<IO*>(p.y)[at] = v;
+        st_io<IO>(ry, to[i], v);
     }
 }
 
@@ -664,13 +725,13 @@ __global__ void __launch_bounds__(256) decode_ssm_kernel(const DecodeParams p) {
 #pragma unroll
     for (int i = 0; i < kPre; ++i) pre[i] = Dt::load(wr + min(DTV * (part + 4 * i), p.R - DTV));
     if constexpr (!MANY) {
-        const rsrc_t parts = window(p.dbc, (int64_t)p.splits * p.batch * P, 4);
+        const rsrc_t parts = window(p.dbc, (int64_t)p.splits * p.batch * p.P4, 4);
         for (int i = threadIdx.x; i < BT * P; i += 256) {
-            const int t = i / P, b = b0 + t;
+            const int t = div_small(i, P), b = b0 + t;
             float v[8], s = 0.0f;  // (requested together)
 #pragma unroll
             for (int q = 0; q < 8; ++q)
-                v[q] = ld_f32(parts, (uint32_t)((q * p.batch + b) * P + (i - t * P)) * 4u, b < p.batch && q < p.splits);
+                v[q] = ld_f32(parts, (uint32_t)((q * p.batch + b) * p.P4 + (i - t * P)) * 4u, b < p.batch && q < p.splits);
 #pragma unroll
             for (int q = 0; q < 8; ++q) s += v[q];
             dbc[i] = s;
@@ -683,7 +744,7 @@ __global__ void __launch_bounds__(256) decode_ssm_kernel(const DecodeParams p) {
         const int G = max(256 / P, 1), g = G > 1 ? threadIdx.x / P : 0;
         const auto sum = [&](const float* src, auto some) {
             constexpr int kSome = decltype(some)::value;
-            const int64_t pitch = (int64_t)p.batch * P;
+            const int64_t pitch = (int64_t)p.batch * p.P4;
             float s = 0.0f;
             for (int q0 = g; q0 < p.splits; q0 += kSome * G) {
                 float v[kSome];
@@ -696,7 +757,7 @@ __global__ void __launch_bounds__(256) decode_ssm_kernel(const DecodeParams p) {
             return s;
         };
         for (int i = G > 1 ? threadIdx.x % P : threadIdx.x; i < P && g < G; i += 256) {
-            const float* src = p.dbc + (int64_t)b0 * P + i;
+            const float* src = p.dbc + (int64_t)b0 * p.P4 + i;
             const float s = p.splits <= 8 * G    ? sum(src, std::integral_constant<int, 8>())
                             : p.splits <= 16 * G ? sum(src, std::integral_constant<int, 16>())
                                                  : sum(src, std::integral_constant<int, 32>());
@@ -756,7 +817,92 @@ __global__ void __launch_bounds__(256) decode_ssm_kernel(const DecodeParams p) {
         acc += __shfl_xor(acc, 1);
         acc += __shfl_xor(acc, 2);
         if (mine && part == 0)
-            frag_store<IO>(p.g, b, d, p.ED, from_float<IO>(__builtin_fmaf(Dv, xv[t], acc) * zv[t] * sigmoid_f(zv[t])));
+            frag_store_at<IO>(make_rsrc(p.g, (uint32_t)frag_bytes(p.batch, p.ED, sizeof(IO))), frag_offset<IO>(b, d, p.ED), d, p.ED,
+                              from_float<IO>(__builtin_fmaf(Dv, xv[t], acc) * zv[t] * sigmoid_f(zv[t])));
+    }
+}
+
+// The same where dbc comes as many partial sums, 16 states: a row of 16 lanes owns CH channels of one sequence, a lane one of their states and
+// a sixteenth of dt_rank.  For one sequence it is a chain of latencies, and short: the partial sums in 16-byte parts,
+// eight or fewer to a thread, three products, one exponential and two sums over a row of lanes (four states a lane, a thread
+// for every output and 32 partial sums each: 3.4 us from the first instruction to the last, 1400 instructions).
+template <typename IO, int CH>
+__global__ void __launch_bounds__(256) decode_ssm_row_kernel(const DecodeParams p) {
+    extern __shared__ float lds[];  // [groups][P4] partial sums; then their sums in front
+    const int b = blockIdx.y, n = threadIdx.x & 15, parts4 = p.P4 >> 2;
+    const int G = div_small(256, parts4), g = div_small(threadIdx.x, parts4), quad = (int)threadIdx.x - g * parts4;
+    const rsrc_t rp = make_rsrc(p.dbc + (int64_t)b * p.P4, (uint32_t)(((p.splits - 1) * p.batch + 1) * p.P4) * 4u);
+    const uint32_t pitch = (uint32_t)(p.batch * p.P4) * 4u;
+    const uint32_t at = g < G ? (uint32_t)g * pitch + (uint32_t)quad * 16u : kNowhere;
+    constexpr int kSome = 8, kPre = 4;
+    u32x4 v[kSome];
+    auto request = [&](int q0) {  // (beyond the last partial sum is beyond the window)
+#pragma unroll
+        for (int i = 0; i < kSome; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(rp, at == kNowhere ? kNowhere : at + (uint32_t)(q0 + i * G) * pitch, 0, 0);
+    };
+    request(0);
+    IO xv[CH], zv[CH], w[CH][kPre];
+    float h[CH], a[CH], Dv[CH], bias[CH];
+    const rsrc_t rx = make_rsrc(p.xs, (uint32_t)frag_bytes(p.batch, p.ED, sizeof(IO))), rz = window(p.z, (int64_t)p.batch * p.ED, sizeof(IO)),
+                 rw = window(p.dt_w, (int64_t)p.ED * p.R, sizeof(IO)), rA = window(p.A, (int64_t)p.ED * 16, 4), rD = window(p.D, p.ED, 4),
+                 rb = window(p.dt_b, p.ED, 4), rg = make_rsrc(p.g, (uint32_t)frag_bytes(p.batch, p.ED, sizeof(IO)));
+    const int64_t row0 = (int64_t)b * p.ED;
+    const rsrc_t rh = window(p.h_in ? p.h_in + row0 * 16 : nullptr, (int64_t)p.ED * 16, 4), ro = make_rsrc(p.h_out + row0 * 16, (uint32_t)p.ED * 64u);
+    int ch[CH];
+    uint32_t frag[CH];
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {  // (a channel beyond the last is beyond the windows of its rows)
+        const int d = ch[j] = (blockIdx.x * CH + j) * 16 + (threadIdx.x >> 4);
+        frag[j] = d < p.ED ? frag_offset<IO>(b, d, p.ED) : kNowhere;
+        xv[j] = __builtin_bit_cast(IO, ld_bits<IO>(rx, frag[j]));
+        zv[j] = __builtin_bit_cast(IO, ld_bits<IO>(rz, d < p.ED ? (uint32_t)(row0 + d) * (uint32_t)sizeof(IO) : kNowhere));
+        h[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rh, (uint32_t)(d * 16 + n) * 4u, 0, 0));
+        a[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rA, (uint32_t)(d * 16 + n) * 4u, 0, 0));
+        Dv[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rD, (uint32_t)d * 4u, 0, 0));
+        bias[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, (uint32_t)d * 4u, 0, 0));
+#pragma unroll
+        for (int i = 0; i < kPre; ++i)
+            w[j][i] = __builtin_bit_cast(IO, ld_bits<IO>(rw, n + 16 * i < p.R ? (uint32_t)(d * p.R + n + 16 * i) * (uint32_t)sizeof(IO) : kNowhere));
+    }
+    f32x4 s = {};
+    for (int q0 = 0;; request(q0)) {
+        f32x4 t[kSome];
+#pragma unroll
+        for (int i = 0; i < kSome; ++i) t[i] = __builtin_bit_cast(f32x4, v[i]);
+#pragma unroll
+        for (int o = 1; o < kSome; o *= 2)
+#pragma unroll
+            for (int i = 0; i < kSome; i += 2 * o) t[i] += t[i + o];
+        s += t[0];
+        if ((q0 += kSome * G) >= p.splits) break;
+    }
+    float* const sums = lds + G * p.P4;
+    if (g < G) *reinterpret_cast<f32x4*>(lds + g * p.P4 + quad * 4) = s;
+    __syncthreads();
+    for (int i = threadIdx.x; i < p.P4; i += 256) {
+        float t[4] = {};
+        for (int q = 0; q < G; q += 4)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) t[e] += q + e < G ? lds[(q + e) * p.P4 + i] : 0.0f;
+        sums[i] = (t[0] + t[1]) + (t[2] + t[3]);
+    }
+    __syncthreads();
+    const float Bn = sums[p.R + n], Cn = sums[p.R + 16 + n];
+    float low[kPre];
+#pragma unroll
+    for (int i = 0; i < kPre; ++i) low[i] = n + 16 * i < p.R ? sums[n + 16 * i] : 0.0f;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        float dl = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kPre; ++i) dl = __builtin_fmaf(to_float(w[j][i]), low[i], dl);
+        for (int r = n + 16 * kPre; r < p.R; r += 16)
+            dl = __builtin_fmaf(to_float(__builtin_bit_cast(IO, ld_bits<IO>(rw, (uint32_t)(ch[j] * p.R + r) * (uint32_t)sizeof(IO)))), sums[r], dl);
+        const float delta = softplus_f(row_sum(dl) + bias[j]), x = to_float(xv[j]), z = to_float(zv[j]);
+        const float hn = __builtin_fmaf(delta * x, Bn, fast_exp2(delta * kLog2e * a[j]) * h[j]);
+        st_io<float>(ro, (uint32_t)(ch[j] * 16 + n) * 4u, hn);
+        const float y = row_sum(Cn * hn);
+        frag_store_at<IO>(rg, n == 0 ? frag[j] : kNowhere, ch[j], p.ED, from_float<IO>(__builtin_fmaf(Dv[j], x, y) * z * sigmoid_f(z)));
     }
 }
 
@@ -788,10 +934,6 @@ static int decode_splits(const mpa_decode_layer* s) {
 
 static size_t round256(size_t v) { return (v + 255) / 256 * 256; }
 
-static dim3 decode_grid(int64_t row_tiles, int64_t groups, int splits) {
-    return dim3((unsigned)((row_tiles + 7) / 8 * 8 * groups), (unsigned)splits);
-}
-
 // Workgroup tiles (row tiles x batch tiles, waves, pieces in flight of each), from sweeps over fourteen of them at widths 768 to
 // 2560 and batches 1 to 128.  in_proj: one 16 x 16 tile on eight waves, two pieces, is best or within 3 % while its tiles are
 // fewer than 1536; from there two batch tiles (64 x 2560: float32 128 -> 115 us a layer, bfloat16 80 -> 75).  Larger tiles read less
@@ -804,58 +946,96 @@ constexpr int kManyTiles = 1536;
 // sums, 56 -> 72).
 static bool xproj_fused(int ED, int P, int batch) { return batch <= 16 && P <= 512 && (int64_t)((ED + 15) / 16) * P <= 16384; }
 
+// grid of a product: sets what decode_tile reads
+static dim3 decode_grid(DecodeParams& p, int row_tiles, int groups, int splits = 1) {
+    p.groups = groups;
+    p.span_inv = (uint32_t)((((uint64_t)1 << 32) + 8 * groups - 1) / (8 * groups));
+    return dim3((unsigned)(groups == 1 ? row_tiles : (row_tiles + 7) / 8 * 8 * groups), (unsigned)splits);
+}
+// 128-byte pieces of a row of K elements
+template <typename IO>
+static int pieces_of(int K) { return (K + 128 / (int)sizeof(IO) - 1) / (128 / (int)sizeof(IO)); }
+
+// One tile of rows and sequences: all pieces of a wave are in flight at once and nothing loops while four waves have three pieces each at
+// most, then eight (layers of 1 x 768: bfloat16 13.8 us on eight looping waves -> 10.8, float32 17.0 -> 13.9; 64 x 768 20.8 -> 17.9;
+// 1 x 256 10.8 -> 9.7, all with the other changes of the same kernels).  Above, as measured before: float32 four waves with more pieces in flight.
 template <typename IO, int MODE>
-static int launch_in(const DecodeParams& p, hipStream_t st) {
-    const int rt = (2 * p.ED + 15) / 16, bt = (p.batch + 15) / 16;
-    if (xproj_fused(p.ED, p.R + 2 * p.N, p.batch)) {
-        // (float32 rows have twice the pieces.  From 704 columns on fewer waves with more pieces in flight, a measured line: 1 x 768 20.2 ->
-        // 19.0 us a layer, but below it eight waves are 1 to 3 % faster at every width tried, 12 layers of 1 x 700 210 us and 215, of
-        // 16 x 576 229 and 235.  Up to 512 columns a wave has two pieces at most, and the second is better requested as the first is
-        // used: 6 layers of 1 x 512 118.7 us with both in flight, 116.0.  Four waves have a thread for 256 rows of x_proj; more of them
-        // take eight at any width.)
-        if (sizeof(IO) == 4 && p.d >= 704 && p.R + 2 * p.N <= 256) hipLaunchKernelGGL((decode_in_kernel<IO, 1, 1, 4, 4, MODE, true>), decode_grid(rt, bt, 1), dim3(256), 0, st, p, rt, bt);
-        else if (sizeof(IO) == 4 && p.d > 256 && p.d <= 512) hipLaunchKernelGGL((decode_in_kernel<IO, 1, 1, 8, 1, MODE, true>), decode_grid(rt, bt, 1), dim3(512), 0, st, p, rt, bt);
-        else hipLaunchKernelGGL((decode_in_kernel<IO, 1, 1, 8, 2, MODE, true>), decode_grid(rt, bt, 1), dim3(512), 0, st, p, rt, bt);
+static int launch_in(DecodeParams p, hipStream_t st) {
+    const int rt = (2 * p.ED + 15) / 16, bt = (p.batch + 15) / 16, P = p.R + 2 * p.N, pieces = pieces_of<IO>(p.d);
+    const bool fused = xproj_fused(p.ED, P, p.batch);
+#define MPA_IN(MT_, NT_, NW_, U_, ONCE_, XP_, GROUPS_) \
+    hipLaunchKernelGGL((decode_in_kernel<IO, MT_, NT_, NW_, U_, ONCE_, MODE, XP_>), decode_grid(p, rt, GROUPS_), dim3(NW_ * kWave), 0, st, p)
+    if (fused) {
+        // (Four waves have a thread for 256 rows of x_proj; more of them take eight at any width.)
+        if (pieces <= 12 && P <= 256) MPA_IN(1, 1, 4, 3, true, true, bt);
+        else if (pieces <= 24) MPA_IN(1, 1, 8, 3, true, true, bt);
+        else if (sizeof(IO) == 4 && P <= 256) MPA_IN(1, 1, 4, 4, false, true, bt);
+        else MPA_IN(1, 1, 8, 2, false, true, bt);
     } else if (rt * bt < kManyTiles) {
-        hipLaunchKernelGGL((decode_in_kernel<IO, 1, 1, 8, 2, MODE>), decode_grid(rt, bt, 1), dim3(512), 0, st, p, rt, bt);
+        if (pieces <= 12) MPA_IN(1, 1, 4, 3, true, false, bt);
+        else if (pieces <= 24) MPA_IN(1, 1, 8, 3, true, false, bt);
+        else MPA_IN(1, 1, 8, 2, false, false, bt);
     } else {
         const int groups = (bt + 1) / 2;
         // (four waves where eight would have two pieces each or fewer: 128 x 1000 in bfloat16 14.2 us on eight, 11.2 on four)
-        if (p.d * (int)sizeof(IO) <= 2048) hipLaunchKernelGGL((decode_in_kernel<IO, 1, 2, 4, 2, MODE>), decode_grid(rt, groups, 1), dim3(256), 0, st, p, rt, groups);
-        else hipLaunchKernelGGL((decode_in_kernel<IO, 1, 2, 8, 2, MODE>), decode_grid(rt, groups, 1), dim3(512), 0, st, p, rt, groups);
+        if (p.d * (int)sizeof(IO) <= 2048) MPA_IN(1, 2, 4, 2, false, false, groups);
+        else MPA_IN(1, 2, 8, 2, false, false, groups);
     }
+#undef MPA_IN
     return check_launch();
 }
 
 template <typename IO>
-static int launch_xproj(const DecodeParams& p, hipStream_t st) {
-    const int rt = (p.R + 2 * p.N + 15) / 16, bt = (p.batch + 15) / 16;
-    hipLaunchKernelGGL((decode_xproj_kernel<IO, kXprojWaves>), decode_grid(rt, bt, p.splits), dim3(kXprojWaves * kWave), 0, st, p, rt, bt);
+static int launch_xproj(DecodeParams p, hipStream_t st) {
+    const int rt = (p.R + 2 * p.N + 15) / 16, bt = (p.batch + 15) / 16, per = (pieces_of<IO>(p.ED) + p.splits - 1) / p.splits;
+    const dim3 grid = decode_grid(p, rt, bt, p.splits);
+    if (per <= kXprojWaves) hipLaunchKernelGGL((decode_xproj_kernel<IO, kXprojWaves, 1, true>), grid, dim3(kXprojWaves * kWave), 0, st, p);
+    else hipLaunchKernelGGL((decode_xproj_kernel<IO, kXprojWaves, 2, false>), grid, dim3(kXprojWaves * kWave), 0, st, p);
     return check_launch();
 }
 
-// out_proj has half the rows and twice the K: sixteen waves while one workgroup per CU is all there is (1 x 2560 float32: 56 us a
-// layer, 58 on eight), then two batch tiles on eight waves, and from 512 tiles two row tiles as well (64 x 1536: float32 61 -> 58 us a
+// out_proj has half the rows and twice the K: while one workgroup per CU is all there is, as many waves as have three pieces each
+// (see launch_in), or sixteen (1 x 2560 float32: 56 us a layer, 58 on eight), then two batch tiles on eight waves, and from 512 tiles two row tiles as well (64 x 1536: float32 61 -> 58 us a
 // layer, 64 x 2560 123 -> 120; bfloat16 42 -> 40 and 80 -> 75).
 template <typename IO, bool RES>
-static int launch_out(const DecodeParams& p, hipStream_t st) {
-    const int rt = (p.d + 15) / 16, bt = (p.batch + 15) / 16, groups = (bt + 1) / 2, pairs = (rt + 1) / 2;
-    if (rt * bt <= 256) hipLaunchKernelGGL((decode_out_kernel<IO, 1, 1, 16, 2, RES>), decode_grid(rt, bt, 1), dim3(1024), 0, st, p, rt, bt);
-    else if (rt * bt < 512) hipLaunchKernelGGL((decode_out_kernel<IO, 1, 2, 8, 2, RES>), decode_grid(rt, groups, 1), dim3(512), 0, st, p, rt, groups);
-    else hipLaunchKernelGGL((decode_out_kernel<IO, 2, 2, 8, 2, RES>), decode_grid(pairs, groups, 1), dim3(512), 0, st, p, pairs, groups);
+static int launch_out(DecodeParams p, hipStream_t st) {
+    const int rt = (p.d + 15) / 16, bt = (p.batch + 15) / 16, groups = (bt + 1) / 2, pairs = (rt + 1) / 2, pieces = pieces_of<IO>(p.ED);
+#define MPA_OUT(MT_, NT_, NW_, U_, ONCE_, TILES_, GROUPS_) \
+    hipLaunchKernelGGL((decode_out_kernel<IO, MT_, NT_, NW_, U_, ONCE_, RES>), decode_grid(p, TILES_, GROUPS_), dim3(NW_ * kWave), 0, st, p)
+    if (rt * bt <= 256) {
+        if (pieces <= 12) MPA_OUT(1, 1, 4, 3, true, rt, bt);
+        else if (pieces <= 24) MPA_OUT(1, 1, 8, 3, true, rt, bt);
+        else if (pieces <= 48) MPA_OUT(1, 1, 16, 3, true, rt, bt);
+        else MPA_OUT(1, 1, 16, 2, false, rt, bt);
+    } else if (rt * bt < 512) MPA_OUT(1, 2, 8, 2, false, rt, groups);
+    else MPA_OUT(2, 2, 8, 2, false, pairs, groups);
+#undef MPA_OUT
     return check_launch();
 }
 
 template <typename IO, int BT, bool MANY = false>
 static int launch_ssm(const DecodeParams& p, hipStream_t st) {
+    if constexpr (MANY) {
+        if (p.N == 16) {
+            const int G = 256 / (p.P4 / 4);
+            const size_t lds = (size_t)(G + 1) * p.P4 * sizeof(float);
+            const int tiles = (p.ED + 15) / 16;
+            // (four channels a lane from two workgroups per CU on: the sums of dbc are then formed a quarter as often)
+            if (tiles * p.batch <= 512) hipLaunchKernelGGL((decode_ssm_row_kernel<IO, 1>), dim3(tiles, p.batch), dim3(256), lds, st, p);
+            else hipLaunchKernelGGL((decode_ssm_row_kernel<IO, 4>), dim3((tiles + 3) / 4, p.batch), dim3(256), lds, st, p);
+            return check_launch();
+        }
+    }
     const dim3 grid((p.ED + 63) / 64, (p.batch + BT - 1) / BT);
     const int outs = BT * (p.R + 2 * p.N);
     const size_t lds = (size_t)(outs < 256 ? 256 : outs) * sizeof(float);
     if (lds > 48 * 1024) return MPA_ERR_BAD_SHAPE;
     const bool v4 = p.R % 4 == 0 && aligned_to(p.dt_w, 4 * sizeof(IO));
 #define MPA_SSM(N16_, V_) hipLaunchKernelGGL((decode_ssm_kernel<IO, BT, N16_, V_, MANY>), grid, dim3(256), lds, st, p)
-    if (p.N == 16) { if (v4) MPA_SSM(true, 4); else MPA_SSM(true, 1); }
-    else { if (v4) MPA_SSM(false, 4); else MPA_SSM(false, 1); }
+    if constexpr (!MANY) {
+        if (p.N == 16) { if (v4) MPA_SSM(true, 4); else MPA_SSM(true, 1); return check_launch(); }
+    }
+    if (v4) MPA_SSM(false, 4); else MPA_SSM(false, 1);
 #undef MPA_SSM
     return check_launch();
 }
@@ -903,7 +1083,7 @@ static size_t decode_scaled_ws(const mpa_decode_layer* s) {
 extern "C" size_t mpa_decode_layer_workspace_bytes(const mpa_decode_layer* s) {
     if (decode_validate(s) != MPA_OK) return 0;
     const size_t act = (size_t)frag_bytes(s->batch, s->dim, (int)dtype_size(s->io_dtype));
-    return 3 * act + round256((size_t)decode_splits(s) * s->batch * (s->dt_rank + 2 * s->dstate) * sizeof(float)) + decode_scaled_ws(s);
+    return 3 * act + round256((size_t)decode_splits(s) * s->batch * ((s->dt_rank + 2 * s->dstate + 3) / 4 * 4) * sizeof(float)) + decode_scaled_ws(s);
 }
 
 extern "C" int mpa_decode_layer_step(const mpa_decode_layer* s, const void* x, const void* x_scaled, const float* x_ssq, void* y,
@@ -929,7 +1109,8 @@ extern "C" int mpa_decode_layer_step(const mpa_decode_layer* s, const void* x, c
     if (workspace_bytes < mpa_decode_layer_workspace_bytes(s)) return MPA_ERR_WORKSPACE;
     DecodeParams p{};
     p.batch = (int)s->batch; p.d = (int)s->d_model; p.ED = (int)s->dim; p.N = (int)s->dstate; p.R = (int)s->dt_rank;
-    p.K = s->d_conv; p.eps = s->eps; p.splits = decode_splits(s); p.ssq_tiles = (p.d + 15) / 16;
+    p.P4 = (p.R + 2 * p.N + 3) / 4 * 4;
+    p.K = s->d_conv; p.eps = s->eps; p.inv_d = 1.0f / (float)p.d; p.splits = decode_splits(s); p.ssq_tiles = (p.d + 15) / 16;
     p.x = x; p.xw = x_scaled; p.ssq = x_ssq; p.norm_w = s->norm_weight;
     p.in_w = s->in_weight; p.in_b = s->in_bias; p.conv_w = s->conv_weight; p.conv_b = s->conv_bias;
     p.xp_w = s->x_weight; p.dt_w = s->dt_weight; p.dt_b = s->dt_bias; p.A = s->A; p.D = s->D;
