@@ -127,6 +127,11 @@ __device__ __forceinline__ float frag_load(const void* base, int b, int k, int K
 }
 // An offset beyond any window here (they are below 2 GB): the load reads zero, with a scalar offset on top as well.
 constexpr uint32_t kNowhere = 0x80000000u;
+// (formed either way: or the choice becomes a branch around its arithmetic, and around the load)
+__device__ __forceinline__ uint32_t where(bool ok, uint32_t at) {
+    asm("" : "+v"(at));
+    return ok ? at : kNowhere;
+}
 
 // Activations in operand order; request() takes a chunk of 32 k, of which `left` are wanted (any number, also below zero).  Offsets
 // within a chunk are formed once, the chunk is a scalar offset.
@@ -254,7 +259,9 @@ __device__ __forceinline__ void decode_product(WaveLds<MT, NT>& lds, const void*
     // lane -> 16 bytes of row 8*i + lane/8: the piece's eight 16-byte parts are stored rotated by the row
     // (part ^ (row & 7)), so that the operand reads, one row per lane, fall on different banks
     const int part = ((lane & 7) ^ (lane >> 3)) * 16;
-    const rsrc_t rw = make_rsrc(static_cast<const IO*>(W) + (int64_t)n0 * K, (uint32_t)max(min(rows - n0, 16 * MT), 0) * (uint32_t)K * kES);
+    // (a scalar, which the compiler's v_med3 is not: every load would be a loop over the lanes' descriptors)
+    const uint32_t rows_left = (uint32_t)__builtin_amdgcn_readfirstlane(max(min(rows - n0, 16 * MT), 0));
+    const rsrc_t rw = make_rsrc(static_cast<const IO*>(W) + (int64_t)n0 * K, rows_left * (uint32_t)K * kES);
     uint32_t row[2 * MT];
 #pragma unroll
     for (int i = 0; i < 2 * MT; ++i) row[i] = (uint32_t)(lane >> 3) * (uint32_t)K * kES + part + (uint32_t)(8 * i * K) * kES;
@@ -402,6 +409,10 @@ __global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams
     __shared__ WaveLds<MT, NT> tile[NW];
     __shared__ float ssq[NW][NT][16];
     __shared__ alignas(16) float xl[XP ? NT * 16 : 1][16];  // convolved x of the tile
+    // (all arguments requested at once: the compiler otherwise loads some where they are used, each a round trip in a step's chain)
+    asm volatile("" ::"s"(p.batch), "s"(p.d), "s"(p.ED), "s"(p.N), "s"(p.R), "s"(p.K), "s"(p.P4), "s"(p.span_inv), "s"(p.groups), "s"(p.eps), "s"(p.inv_d),
+                 "s"(p.ssq_tiles), "s"(p.x), "s"(p.xw), "s"(p.ssq), "s"(p.norm_w), "s"(p.in_w), "s"(p.in_b), "s"(p.conv_w), "s"(p.conv_b), "s"(p.xp_w),
+                 "s"(p.win_in), "s"(p.win_out), "s"(p.xs), "s"(p.z), "s"(p.dbc));
     int rt, bt;
     decode_tile<NT>(p, rt, bt);
     const int lane = threadIdx.x & (kWave - 1), wave = wave_id();
@@ -422,13 +433,13 @@ __global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams
     float sq[NT][kSums];
     auto request_sums = [&](int q0) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+        for (int t = 0; t < NT; ++t) {
+            const int b = b0 + t * 16 + (lane & 15);
+            const uint32_t at = ((uint32_t)(q0 + 4 * wave + (lane >> 4)) * (uint32_t)p.batch + (uint32_t)b) * 4u, step = 16u * NW * (uint32_t)p.batch;
 #pragma unroll
-            for (int i = 0; i < kSums; ++i) {
-                const int b = b0 + t * 16 + (lane & 15), q = q0 + 4 * (wave + NW * i) + (lane >> 4);
-                // (beyond the last row of sums is beyond the window)
-                sq[t][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, b < p.batch ? (uint32_t)(q * p.batch + b) * 4u : kNowhere, 0, 0));
-            }
+            for (int i = 0; i < kSums; ++i)  // (beyond the last row of sums is beyond the window)
+                sq[t][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, where(b < p.batch, at + i * step), 0, 0));
+        }
     };
     const rsrc_t rwo = window(p.win_out, (int64_t)p.batch * p.ED * (p.K - 1), sizeof(IO)), rz = window(p.z, (int64_t)p.batch * p.ED, sizeof(IO)),
                  rxs = make_rsrc(p.xs, (uint32_t)frag_bytes(p.batch, p.ED, sizeof(IO)));
@@ -441,14 +452,14 @@ __global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams
             const int o = threadIdx.x + i * kThreads, n = n0 + o % kRows, b = b0 + o / kRows;
             const bool some = (kOuts * kThreads == kAll || o < kAll) && n < rows && b < p.batch, conv = some && n < p.ED;
             const uint32_t at = (uint32_t)b * (uint32_t)p.ED + (uint32_t)n;
-            to_win[i] = conv ? at * (uint32_t)(p.K - 1) * (uint32_t)sizeof(IO) : kNowhere;
-            to_z[i] = some && n >= p.ED ? (at - (uint32_t)p.ED) * (uint32_t)sizeof(IO) : kNowhere;
-            to_xs[i] = conv ? frag_offset<IO>(b, n, p.ED) : kNowhere;
+            to_win[i] = where(conv, at * (uint32_t)(p.K - 1) * (uint32_t)sizeof(IO));
+            to_z[i] = where(some && n >= p.ED, (at - (uint32_t)p.ED) * (uint32_t)sizeof(IO));
+            to_xs[i] = where(conv, frag_offset<IO>(b, n, p.ED));
             ib[i] = __builtin_bit_cast(IO, ld_bits<IO>(rb, (uint32_t)n * (uint32_t)sizeof(IO)));
             // (taps that the layer does not have are read from what follows, and not used)
 #pragma unroll
             for (int j = 0; j < 3; ++j) win[i][j] = __builtin_bit_cast(IO, ld_bits<IO>(rwin, to_win[i] + j * (uint32_t)sizeof(IO)));
-            const uint32_t cat = conv ? (uint32_t)(n * p.K) * 4u : kNowhere;
+            const uint32_t cat = where(conv, (uint32_t)(n * p.K) * 4u);
 #pragma unroll
             for (int j = 0; j < 4; ++j) cw[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rcw, cat + 4u * j, 0, 0));
             cb[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rcb, (uint32_t)n * 4u, 0, 0));
@@ -460,7 +471,7 @@ __global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams
 #pragma unroll
             for (int i = 0; i < 16 / Frag<IO>::kVec; ++i) {  // (zeros beyond the last channel)
                 const int k = n0 + i * Frag<IO>::kVec;
-                xw[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, k < p.ED ? (uint32_t)(xrow * p.ED + k) * (uint32_t)sizeof(IO) : kNowhere, 0, 0);
+                xw[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, where(k < p.ED, (uint32_t)(xrow * p.ED + k) * (uint32_t)sizeof(IO)), 0, 0);
             }
         }
     };
@@ -597,14 +608,16 @@ __global__ void __launch_bounds__(256) decode_scale_kernel(const DecodeParams p,
 template <typename IO, int NW, int U, bool ONCE>
 __global__ void __launch_bounds__(NW* kWave) decode_xproj_kernel(const DecodeParams p) {
     __shared__ WaveLds<1, 1> tile[NW];
+    // (all arguments requested at once: the compiler otherwise loads some where they are used, each a round trip in a step's chain)
+    asm volatile("" ::"s"(p.batch), "s"(p.ED), "s"(p.N), "s"(p.R), "s"(p.P4), "s"(p.span_inv), "s"(p.groups), "s"(p.splits), "s"(p.xp_w), "s"(p.xs), "s"(p.dbc));
     int rt, bt;
     decode_tile<1>(p, rt, bt);
     const int lane = threadIdx.x & (kWave - 1), wave = wave_id(), rows = p.R + 2 * p.N;
     const int pieces = (p.ED + 8 * Frag<IO>::kVec - 1) / (8 * Frag<IO>::kVec);
-    const int per = (pieces + gridDim.y - 1) / gridDim.y, first = (int)blockIdx.y * per;
+    const int per = (pieces + p.splits - 1) / p.splits, first = (int)blockIdx.y * per;
     const int o = threadIdx.x, n = rt * 16 + (o & 15), b = bt * 16 + (o >> 4);
     const rsrc_t rd = make_rsrc(p.dbc + (int64_t)blockIdx.y * p.batch * p.P4, (uint32_t)(p.batch * p.P4) * 4u);
-    const uint32_t to = o < 256 && n < rows && b < p.batch ? (uint32_t)(b * p.P4 + n) * 4u : kNowhere;
+    const uint32_t to = where(o < 256 && n < rows && b < p.batch, (uint32_t)(b * p.P4 + n) * 4u);
     FragAct<IO, 1> act;
     act.setup(p.xs, bt * 16, p.batch, p.ED, lane);
     decode_product<IO, NW, U, ONCE>(tile[wave], p.xp_w, rows, p.ED, rt * 16, first, min(pieces, first + per), wave, lane, act, [] {});
@@ -618,6 +631,9 @@ template <typename IO, int MT, int NT, int NW, int U, bool ONCE, bool RES>
 __global__ void __launch_bounds__(NW* kWave) decode_out_kernel(const DecodeParams p) {
     constexpr int kThreads = NW * kWave, kRows = MT * 16, kAll = NT * 16 * kRows, kOuts = (kAll + kThreads - 1) / kThreads;
     __shared__ WaveLds<MT, NT> tile[NW];
+    // (all arguments requested at once: the compiler otherwise loads some where they are used, each a round trip in a step's chain)
+    asm volatile("" ::"s"(p.batch), "s"(p.d), "s"(p.ED), "s"(p.span_inv), "s"(p.groups), "s"(p.x), "s"(p.out_w), "s"(p.out_b), "s"(p.g), "s"(p.y), "s"(p.next_w),
+                 "s"(p.y_w), "s"(p.ssq_out));
     int rt, bt;
     decode_tile<NT>(p, rt, bt);
     const int lane = threadIdx.x & (kWave - 1), wave = wave_id();
@@ -635,9 +651,9 @@ __global__ void __launch_bounds__(NW* kWave) decode_out_kernel(const DecodeParam
         for (int i = 0; i < kOuts; ++i) {
             const int o = threadIdx.x + i * kThreads, n = n0 + o % kRows, b = b0 + o / kRows;
             const bool ok = (kOuts * kThreads == kAll || o < kAll) && n < p.d && b < p.batch;
-            to[i] = ok ? (uint32_t)(b * p.d + n) * (uint32_t)sizeof(IO) : kNowhere;
-            to_yw[i] = ok ? frag_offset<IO>(b, n, p.d) : kNowhere;
-            to_ssq[i] = ok && n % 16 == 0 ? (uint32_t)((n >> 4) * p.batch + b) * 4u : kNowhere;
+            to[i] = where(ok, (uint32_t)(b * p.d + n) * (uint32_t)sizeof(IO));
+            to_yw[i] = where(ok, frag_offset<IO>(b, n, p.d));
+            to_ssq[i] = where(ok && n % 16 == 0, (uint32_t)((n >> 4) * p.batch + b) * 4u);
             bias[i] = __builtin_bit_cast(IO, ld_bits<IO>(rb, (uint32_t)n * (uint32_t)sizeof(IO)));
             xv[i] = __builtin_bit_cast(IO, ld_bits<IO>(rx, to[i]));
             nw[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rn, (uint32_t)n * 4u, 0, 0));
@@ -700,6 +716,9 @@ struct DtVec<float, 4> {
 template <typename IO, int BT, bool N16, int DTV, bool MANY>
 __global__ void __launch_bounds__(256) decode_ssm_kernel(const DecodeParams p) {
     extern __shared__ float dbc[];  // [BT][R + 2N], as many times as threads allow while it is summed
+    // (all arguments requested at once: the compiler otherwise loads some where they are used, each a round trip in a step's chain)
+    asm volatile("" ::"s"(p.batch), "s"(p.ED), "s"(p.N), "s"(p.R), "s"(p.P4), "s"(p.splits), "s"(p.dt_w), "s"(p.dt_b), "s"(p.A), "s"(p.D), "s"(p.h_in), "s"(p.h_out),
+                 "s"(p.xs), "s"(p.z), "s"(p.g), "s"(p.dbc));
     const int P = p.R + 2 * p.N;
     const int b0 = blockIdx.y * BT;
     const int part = threadIdx.x & 3, ch = blockIdx.x * 64 + (threadIdx.x >> 2);
@@ -829,6 +848,9 @@ __global__ void __launch_bounds__(256) decode_ssm_kernel(const DecodeParams p) {
 template <typename IO, int CH>
 __global__ void __launch_bounds__(256) decode_ssm_row_kernel(const DecodeParams p) {
     extern __shared__ float lds[];  // [groups][P4] partial sums; then their sums in front
+    // (all arguments requested at once: the compiler otherwise loads some where they are used, each a round trip in a step's chain)
+    asm volatile("" ::"s"(p.batch), "s"(p.ED), "s"(p.R), "s"(p.P4), "s"(p.splits), "s"(p.dt_w), "s"(p.dt_b), "s"(p.A), "s"(p.D), "s"(p.h_in), "s"(p.h_out), "s"(p.xs),
+                 "s"(p.z), "s"(p.g), "s"(p.dbc));
     const int b = blockIdx.y, n = threadIdx.x & 15, parts4 = p.P4 >> 2;
     const int G = div_small(256, parts4), g = div_small(threadIdx.x, parts4), quad = (int)threadIdx.x - g * parts4;
     const rsrc_t rp = make_rsrc(p.dbc + (int64_t)b * p.P4, (uint32_t)(((p.splits - 1) * p.batch + 1) * p.P4) * 4u);
@@ -957,8 +979,8 @@ template <typename IO>
 static int pieces_of(int K) { return (K + 128 / (int)sizeof(IO) - 1) / (128 / (int)sizeof(IO)); }
 
 // One tile of rows and sequences: all pieces of a wave are in flight at once and nothing loops while four waves have three pieces each at
-// most, then eight (layers of 1 x 768: bfloat16 13.8 us on eight looping waves -> 10.8, float32 17.0 -> 13.9; 64 x 768 20.8 -> 17.9;
-// 1 x 256 10.8 -> 9.7, all with the other changes of the same kernels).  Above, as measured before: float32 four waves with more pieces in flight.
+// most, then eight (layers of 1 x 768: bfloat16 13.8 us on eight looping waves -> 10.8, float32 17.0 -> 13.6; 64 x 768 20.8 -> 17.2;
+// 1 x 256 10.8 -> 9.5, all with the other changes of the same kernels).  Above, as measured before: float32 four waves with more pieces in flight.
 template <typename IO, int MODE>
 static int launch_in(DecodeParams p, hipStream_t st) {
     const int rt = (2 * p.ED + 15) / 16, bt = (p.batch + 15) / 16, P = p.R + 2 * p.N, pieces = pieces_of<IO>(p.d);
