@@ -82,12 +82,15 @@ enum LinearFlags {
     kYF32 = 2,         // y is float32 whatever IO is
     kResidualF32 = 4,  // so is the residual
     kXLarger = 8,      // x has more bytes than W
+    kBySteps = 16,     // tiles walk W first: set by the launch
 };
 struct LinearParams {
     const void *x, *w, *bias;
     int64_t x_pitch, y_pitch;
     int T, M, K;
     int flags;  // LinearFlags
+    int tiles, tiles_per_xcd, inner;  // of the launch: all, an XCD's share, those of the dimension that is walked first
+    uint32_t inner_inv;
     void* y;
     const float* ssq;  // [in_parts][T]
     int in_parts;
@@ -103,6 +106,15 @@ struct LinearParams {
 // factor of the product.
 enum LinearX { kPlainX = 0, kNormX = 1, kNormXF32 = 2, kFactor = 3 };
 
+// 16 bytes a lane from memory into LDS, lane l's to lds + 16 * l (lds: a byte address, the same for the wave).
+__device__ __forceinline__ void load_to_lds(const u32x4& window, uint32_t at, uint32_t scalar, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(at), "s"(window), "s"(scalar) : "memory");
+}
+__device__ __forceinline__ u32x4 lds_window(const void* base, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, bytes, 0x00020000u};
+}
+
 constexpr int linear_threads(int BT, int BM, int KS, int RT) { return BT / (32 * RT) * (BM / 32) * KS * kWave; }
 
 template <typename IO, int BT, int BM, int KS, int RT, int D, int XMODE, bool NN>
@@ -117,16 +129,21 @@ __global__ void __launch_bounds__(linear_threads(BT, BM, KS, RT)) linear_kernel(
     static_assert(BM * 8 * KS % kThreads == 0, "a load instruction reads W or x");
     constexpr int kRows = BT + BM, kParts = 8 * KS, kLoads = kRows * kParts / kThreads, kStage = kRows * kParts;  // 16-byte parts
     static_assert(D % 2 == 0, "a set of registers always goes to the same buffer");
-    __shared__ u32x4 lds[2][kStage];
+    // Rows as they are in memory go to LDS directly, kBuffers - 1 stages ahead; W by columns and rows to be scaled pass through registers.
+    constexpr bool kDirect = !NN && !NORM;
+    constexpr int kBuffers = kDirect ? 3 : 2;
+    __shared__ u32x4 lds[kBuffers][kStage];
+    asm volatile("" ::"s"(p.x), "s"(p.w), "s"(p.bias), "s"(p.x_pitch), "s"(p.y_pitch), "s"(p.T), "s"(p.M), "s"(p.K), "s"(p.flags), "s"(p.y), "s"(p.ssq),
+                 "s"(p.in_parts), "s"(p.tiles), "s"(p.tiles_per_xcd), "s"(p.inner), "s"(p.inner_inv), "s"(p.inv_d), "s"(p.eps), "s"(p.residual), "s"(p.ssq_out), "s"(p.y_weight), "s"(p.y_scaled));
     // Blocks of one XCD (every eighth) take neighbouring tiles and share one operand's rows in its L2: those of W, whose
     // tiles' steps they walk first, or of x where that is the larger one (each XCD reads the other operand whole) and tiles
     // are many (17 layers of width 528, 4038 steps: 2.27 -> 2.17 ms; below two rounds of tiles it made no difference).
+    // (the division by tiles of the inner dimension as a product with its reciprocal, rounded up: exact below 2^16 tiles)
     const int flags = p.flags;
-    const int nt = (p.T + BT - 1) / BT, nm = (p.M + BM - 1) / BM, per = (nt * nm + 7) / 8;
-    const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per || tile >= nt * nm) return;  // uniform over the block
-    const bool by_steps = (flags & kXLarger) && nt * nm >= 512;
-    const int inner = by_steps ? nm : nt, major = tile / inner, minor = tile - major * inner;
+    const int tile = (int)(blockIdx.x & 7) * p.tiles_per_xcd + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= p.tiles_per_xcd || tile >= p.tiles) return;  // uniform over the block
+    const int major = p.inner_inv ? (int)__umulhi((uint32_t)tile, p.inner_inv) : tile / p.inner, minor = tile - major * p.inner;
+    const bool by_steps = flags & kBySteps;
     const int m0 = (by_steps ? minor : major) * BM, t0 = (by_steps ? major : minor) * BT;
     const int lane = threadIdx.x & (kWave - 1), wave = wave_id();
     const int ks = wave % KS, wm = wave / KS % kWavesM, wt = wave / KS / kWavesM;
@@ -139,8 +156,22 @@ __global__ void __launch_bounds__(linear_threads(BT, BM, KS, RT)) linear_kernel(
     constexpr int kRowsPer = sizeof(IO) == 2 ? 2 : 1;  // rows of W that make a word in LDS
     uint32_t off[kLoads];
     int koff[kLoads], at[kLoads];
+    // Direct loads: a wave fetches for its own share of K, 64 places of LDS (eight rows) at a time, W's rows first; a lane's part of K is the
+    // same in all of them.  (Rows beyond the last are read from anywhere in the window, or as zeros; their results are not stored.)
+    constexpr int kShareWaves = kThreads / kWave / KS, kRowStep = 8 * kShareWaves;
+    static_assert(!kDirect || (BM % kRowStep == 0 && kRows % kRowStep == 0), "a load instruction reads W or x");
+    const int share_wave = wave / KS, part_of = (lane & 7) ^ (lane >> 3);
+    const int kl = (ks * 8 + part_of) * kVec;
+    const u32x4 win_w = lds_window(p.w, (uint32_t)p.M * (uint32_t)p.K * kES), win_x = lds_window(p.x, ((uint32_t)(p.T - 1) * (uint32_t)p.x_pitch + (uint32_t)p.K) * kES);
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
+    for (int i = 0; kDirect && i < kLoads; ++i) {
+        const bool isw = i * kRowStep < BM;
+        const uint32_t pitch = isw ? (uint32_t)p.K : (uint32_t)p.x_pitch;
+        if (i == 0 || i * kRowStep == BM) off[i] = kES * (kl + (uint32_t)((isw ? m0 : t0) + share_wave * 8 + (lane >> 3)) * pitch);
+        else off[i] = off[i - 1] + kES * kRowStep * pitch;
+    }
+#pragma unroll
+    for (int i = 0; !kDirect && i < kLoads; ++i) {
         const int c = threadIdx.x + i * kThreads, row = c / kParts, part = c % kParts;
         if (NN && i < kWLoads) {
             // eight columns of two neighbouring rows of W (K x M), or four of one: see store_transposed
@@ -169,6 +200,15 @@ __global__ void __launch_bounds__(linear_threads(BT, BM, KS, RT)) linear_kernel(
     const rsrc_t rn = make_rsrc(p.norm_w, (uint32_t)p.K * 4u);
     float rs[kLoads - kWLoads];  // rstd of the rows of x the thread stages
     Stage r[D];
+    // (a stage beyond the last, and what lies beyond K: zeros)
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)&lds[0][0]) + (uint32_t)(ks * (kRows * 8) + share_wave * kWave) * 16u;
+    auto fetch = [&](int s, int buf) {
+        const int k = s * kStep * KS;
+        const bool some = k + kl < p.K;
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i)
+            load_to_lds(i * kRowStep < BM ? win_w : win_x, some ? off[i] : 0x80000000u, (uint32_t)k * kES, lds0 + (uint32_t)(buf * kStage + i * kShareWaves * kWave) * 16u);
+    };
     auto load = [&](Stage& st, int s) {
         u32x4(&v)[kLoads] = st.v;
 #pragma unroll
@@ -270,8 +310,8 @@ __global__ void __launch_bounds__(linear_threads(BT, BM, KS, RT)) linear_kernel(
         };
         float v[2 * RT][kSome];
         request(v);
-#pragma unroll
-        for (int i = 0; i < D; ++i) load(r[i], i);
+        fetch(0, 0);
+        fetch(1, 1);
         sum(v);
         for (q0 = 4 * kSome; q0 < p.in_parts; q0 += 4 * kSome) {
             request(v);
@@ -283,6 +323,9 @@ __global__ void __launch_bounds__(linear_threads(BT, BM, KS, RT)) linear_kernel(
             factor[j] += __shfl_xor(factor[j], 32);
             factor[j] = __builtin_amdgcn_rsqf(factor[j] * p.inv_d + p.eps);
         }
+    } else if constexpr (kDirect) {
+        fetch(0, 0);
+        fetch(1, 1);
     } else {
 #pragma unroll
         for (int i = 0; i < D; ++i) load(r[i], i);
@@ -314,27 +357,50 @@ __global__ void __launch_bounds__(linear_threads(BT, BM, KS, RT)) linear_kernel(
             rs[i] = __builtin_amdgcn_rsqf(s[i] * p.inv_d + p.eps);
         }
     }
-    store(r[0], 0);
-    load(r[0], D);
-    __syncthreads();
-    // (whole groups of D stages without a branch, so that every wait is for the one stage it needs; loads and
-    // stores beyond the last stage are of zeros)
-    int s0 = 0;
-    for (; s0 + D <= steps; s0 += D) {
+    if constexpr (kDirect) {
+        // A stage's loads are in flight while the two before it are multiplied.  Its wave waits for its own, the barrier for all waves', and
+        // for the reads of the buffer that is filled next.
+        auto ready = [&] { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLoads) : "memory"); };
+        int s0 = 0;
+        for (; s0 + kBuffers <= steps; s0 += kBuffers) {
 #pragma unroll
-        for (int i = 0; i < D; ++i) {
+            for (int i = 0; i < kBuffers; ++i) {
+                ready();
+                fetch(s0 + i + 2, (i + 2) % kBuffers);
+                compute(i);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kBuffers - 1; ++i) {
+            if (s0 + i >= steps) break;
+            ready();
+            fetch(s0 + i + 2, (i + 2) % kBuffers);
+            compute(i);
+        }
+        if constexpr (KS > 1) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    } else {
+        store(r[0], 0);
+        load(r[0], D);
+        __syncthreads();
+        // (whole groups of D stages without a branch, so that every wait is for the one stage it needs; loads and
+        // stores beyond the last stage are of zeros)
+        int s0 = 0;
+        for (; s0 + D <= steps; s0 += D) {
+#pragma unroll
+            for (int i = 0; i < D; ++i) {
+                store(r[(i + 1) % D], (i + 1) & 1);
+                load(r[(i + 1) % D], s0 + i + 1 + D);
+                compute(i & 1);
+                __syncthreads();
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < D - 1; ++i) {
+            if (s0 + i >= steps) break;
             store(r[(i + 1) % D], (i + 1) & 1);
-            load(r[(i + 1) % D], s0 + i + 1 + D);
             compute(i & 1);
             __syncthreads();
         }
-    }
-#pragma unroll
-    for (int i = 0; i < D - 1; ++i) {
-        if (s0 + i >= steps) break;
-        store(r[(i + 1) % D], (i + 1) & 1);
-        compute(i & 1);
-        __syncthreads();
     }
     // The lane's part of the residual and the weights of its scaled rows, requested at once and before the shares of K are added (one memory latency and
     // not four; what lies beyond T or M is read from within and not used).
@@ -364,7 +430,7 @@ __global__ void __launch_bounds__(linear_threads(BT, BM, KS, RT)) linear_kernel(
     }
     constexpr int kTiles = 4 * RT;
     if constexpr (KS > 1) {
-        static_assert(kThreads / kWave * kTiles * kWave <= 2 * kStage, "the shares of K use the stages' memory");
+        static_assert(kThreads / kWave * kTiles * kWave <= kBuffers * kStage, "the shares of K use the stages' memory");
         // (the stages are done with: the last barrier)
         f32x4* part = reinterpret_cast<f32x4*>(&lds[0][0]);
         if (ks > 0) {
@@ -438,8 +504,14 @@ struct LinearForm {
     bool nn, x_f32, factor;
 };
 template <typename IO, int BT, int BM, int KS, int RT = 1>
-static int launch_linear(const LinearParams& p, const LinearForm& f, hipStream_t st) {
+static int launch_linear(LinearParams p, const LinearForm& f, hipStream_t st) {
     const int nt = (p.T + BT - 1) / BT, nm = (p.M + BM - 1) / BM, per = (nt * nm + 7) / 8;
+    const bool by_steps = (p.flags & kXLarger) && nt * nm >= 512;
+    if (by_steps) p.flags |= kBySteps;
+    p.tiles = nt * nm;
+    p.tiles_per_xcd = per;
+    p.inner = by_steps ? nm : nt;
+    p.inner_inv = p.tiles < 1 << 16 && p.inner > 1 ? (uint32_t)((((uint64_t)1 << 32) + p.inner - 1) / p.inner) : 0;
     const dim3 grid((unsigned)per * 8), block(linear_threads(BT, BM, KS, RT));
     auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, st, p); };
     if (f.nn) run(linear_kernel<IO, BT, BM, KS, RT, 2, kPlainX, true>);
@@ -467,8 +539,9 @@ static int dispatch_linear(const LinearParams& p, const LinearForm& f, hipStream
     }
     if (tiles(64, 128) >= kFull) return launch_linear<IO, 64, 128, 1>(p, f, st);
     if (p.K <= 128) return launch_linear<IO, 64, 64, 1>(p, f, st);  // (one or two stages: nothing to split)
-    if (tiles(64, 64) >= kFull) return p.K >= 1024 ? launch_linear<IO, 64, 64, 2>(p, f, st) : launch_linear<IO, 64, 64, 1>(p, f, st);
-    if (tiles(64, 32) >= kFull) return p.K >= 1024 ? launch_linear<IO, 64, 32, 4>(p, f, st) : launch_linear<IO, 64, 32, 2>(p, f, st);
+    const bool one = p.K >= 1024;
+    if (tiles(64, 64) >= kFull) return one && tiles(64, 64) <= 256 ? launch_linear<IO, 64, 64, 2>(p, f, st) : launch_linear<IO, 64, 64, 1>(p, f, st);
+    if (tiles(64, 32) >= kFull) return one && tiles(64, 32) <= 256 ? launch_linear<IO, 64, 32, 4>(p, f, st) : launch_linear<IO, 64, 32, 2>(p, f, st);
     return launch_linear<IO, 32, 32, 4>(p, f, st);
 }
 
