@@ -31,7 +31,8 @@ struct BwdParams {
     // walk (the order in which the backward visits them); ag0 [rows][ED][Nst] = a*g flowing into
     // every segment from the one visited before it (NULL = zeros: not cut)
     const float* ag0;
-    int nseg, seg_tiles;
+    int nseg, seg_tiles;  // (the last takes what is left)
+    int last_first;       // the last segments of all batch rows are launched first, then those before them
     int expire_waits;  // test hook: treat every bounded wait as run out
     int reverse;       // the forward walk ran from the last physical step to the first
     int batch, L, ED, N, nchunks;

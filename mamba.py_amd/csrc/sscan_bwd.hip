@@ -485,6 +485,7 @@ __global__ void __launch_bounds__(256) sscan_bwd_finish_kernel(
 // states per lane of the backward kernels (at most 4) and, for that choice, how a thin launch
 // is cut: half of the CUs or fewer covered (the first pass of a cut costs a quarter of the second)
 static constexpr int kBwdThin = 2;
+static constexpr int64_t kFillTiles = 2, kUnevenTiles = 8;
 static int bwd_states_per_lane(const mpa_sscan_shape* s) {
     const int ns = pick_states_per_lane(s->dstate, 4, s->plan_states_per_lane);
     return ns < 0 ? 4 : ns;
@@ -498,12 +499,32 @@ static mpa_sscan_shape fast_block_shape(const mpa_sscan_shape* s) {
     if (blk.dstate > kFastStates) blk.dstate = kFastStates;
     return blk;
 }
+// More than half of the CUs covered, but not all: a sequence cut into equal parts would be more rounds of shorter workgroups.
+// Cut in two, the short part (the one that the walk visits first, whose carry the other needs) takes what the CUs without a long part do in the
+// time of a long one; the long ones are launched first.  Workgroups go to the 32 shader engines in turn and wait there for one of its eight CUs
+// (at 210 workgroups, sized as if any free CU took the next one, the cut call was 6 to 10 % slower than the uncut one), so k short parts in turn
+// on each of the CUs that are left in an engine have to be done with the long one; each fills its pipeline first.
+// Backward of a call, uncut and cut: 8 x 2048 x 1536 float32 352 -> 332 us, 8 x 1000 x 1536 gated bfloat16 188 -> 176, 5 x 1500 x 1984 224 -> 185,
+// 13 x 2000 x 640 with 24 states 709 -> 566; with seven short parts in turn 7 x 4096 x 1920 676 -> 642, 7 x 2048 x 1920 348 -> 336, and no gain
+// below eight tiles (8 x 700 x 1536, ten: 133 and 134).
+// Returns the tiles of the short part, 0: not cut.
+static int64_t uneven_tiles(const mpa_sscan_shape* s) {
+    constexpr int64_t kCUs = 256, kEngines = 32, kEngineCUs = kCUs / kEngines;
+    const int64_t rows = s->batch * ((s->dim + kWave - 1) / kWave), ntiles = (s->seqlen + kTile - 1) / kTile;
+    if (s->plan_segments > 0 || rows * kBwdThin <= kCUs || s->batch * 2 > 65535) return 0;
+    const int64_t per = (rows + kEngines - 1) / kEngines, left = kEngineCUs - per;
+    if (left < 1) return 0;
+    const int64_t k = (per + left - 1) / left, tiles = (ntiles - kFillTiles * (k - 1)) / (k + 1);
+    return tiles >= kUnevenTiles ? tiles : 0;
+}
 // The cut exists on the fast kernel only.
 static SegPlan bwd_seg_plan(const mpa_sscan_shape* s) {
     const mpa_sscan_shape blk = fast_block_shape(s);
     const int ns = bwd_states_per_lane(&blk);
     if (!bwd_fast_supported(ns, padded_states(blk.dstate) / ns) || (s->plan_flags & MPA_PLAN_BWD_GENERAL))
         return SegPlan{1, 0, 0, 0, 0, 0};
+    const int64_t uneven = uneven_tiles(s);
+    if (uneven > 0) return seg_buffers(s, 2, uneven);
     return seg_layout(s, seg_plan(&blk, ns, kBwdThin).nseg);  // (buffers for all states)
 }
 
@@ -648,6 +669,7 @@ extern "C" int mpa_sscan_bwd(const mpa_sscan_shape* s, const void* x, const void
         const int nblk = (p.N + kFastStates - 1) / kFastStates;
         const size_t es_ = dtype_size(s->io_dtype);
         float* const seg = wsf + ws.offSeg;
+        const float* ag0 = seg + ws.seg.off_h0;
         if (nseg > 1) {
             // Sequence cut into segments that run side by side.  The reverse recurrence
             // ag[t] = a[t] * (ag[t+1] + C[t]*dy[t]) is linear in its state like the forward one,
@@ -659,7 +681,7 @@ extern "C" int mpa_sscan_bwd(const mpa_sscan_shape* s, const void* x, const void
             g.x = dy; g.delta = delta; g.z = z; g.D = D; g.dbias = delta_bias;
             g.bc_sb = s->bc_sb; g.bc_sl = s->bc_sl;
             g.dsum = seg + ws.seg.off_dsum;
-            g.nseg = nseg; g.seg_tiles = ws.seg.seg_tiles;
+            g.nseg = nseg; g.seg_tiles = ws.seg.seg_tiles; g.run_segs = nseg - 1;
             g.batch = p.batch; g.L = p.L; g.ED = p.ED; g.nchunks = p.nchunks;
             g.a_st = g.h_st = g.ck_st = p.N;
             g.softplus = p.softplus; g.delta_f32 = p.delta_f32; g.reverse = p.reverse ? 0 : 1;
@@ -676,11 +698,15 @@ extern "C" int mpa_sscan_bwd(const mpa_sscan_shape* s, const void* x, const void
                 rc = launch_fwd_any(g, s->io_dtype, cns, padded_states(g.N) / cns, kGCarry, st);
                 if (rc != MPA_OK) return rc;
             }
-            // (chained by seg_carry_kernel for any number of segments: in front of the kernel below, which has no
-            // registers to spare, the chain cost the uncut call 6 %)
-            rc = launch_seg_carry(A, nullptr, seg + ws.seg.off_hend, seg + ws.seg.off_dsum, seg + ws.seg.off_h0, nullptr, p.batch,
-                                  nseg, p.ED, p.N, p.N, p.N, st);
-            if (rc != MPA_OK) return rc;
+            // (chained by seg_carry_kernel: in front of the kernel below, which has no registers to spare, the chain cost the uncut
+            // call 6 %.  Of two segments the second's is the first one's end value as it is: a row before its own in the buffer.)
+            if (nseg == 2) {
+                ag0 = seg + ws.seg.off_hend - (int64_t)p.ED * p.N;
+            } else {
+                rc = launch_seg_carry(A, nullptr, seg + ws.seg.off_hend, seg + ws.seg.off_dsum, seg + ws.seg.off_h0, nullptr, p.batch,
+                                      nseg, p.ED, p.N, p.N, p.N, st);
+                if (rc != MPA_OK) return rc;
+            }
         }
         for (int sb = 0; sb < nblk && rc == MPA_OK; ++sb) {
             const int n0 = sb * kFastStates;
@@ -696,7 +722,8 @@ extern "C" int mpa_sscan_bwd(const mpa_sscan_shape* s, const void* x, const void
             q.row0 = sb * p.batch * nseg;
             if (nseg > 1) {
                 q.nseg = nseg; q.seg_tiles = ws.seg.seg_tiles;
-                q.ag0 = seg + ws.seg.off_h0 + n0;
+                q.last_first = uneven_tiles(s) > 0;
+                q.ag0 = ag0 + n0;
             }
             rc = launch_bwd_fast(q, fns, fnw, s->io_dtype, st);
         }

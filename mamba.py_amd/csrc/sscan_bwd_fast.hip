@@ -168,12 +168,15 @@ __global__ void __launch_bounds__((NW + kSvc) * kWave) sscan_bwd_fast_kernel(con
     const int w = wave_id();
     // Row of the launch: a batch row, or one segment of it.  Tiles of the row are counted from
     // the end of the forward walk: tile k of the row is backward-walk tile k0 + k.
-    const int bs = blockIdx.y;
-    int b = bs, k0 = 0, ntiles = p.nchunks;
+    int bs = blockIdx.y;
+    int b = bs, seg = 0, k0 = 0, ntiles = p.nchunks;
     if (p.nseg > 1) {
-        b = bs / p.nseg;
-        k0 = (bs - b * p.nseg) * p.seg_tiles;
-        ntiles = min(p.seg_tiles, p.nchunks - k0);
+        const int per = p.last_first ? p.batch : p.nseg, q = bs / per, r = bs - q * per;
+        b = p.last_first ? r : q;
+        seg = p.last_first ? p.nseg - 1 - q : r;
+        bs = b * p.nseg + seg;
+        k0 = seg * p.seg_tiles;
+        ntiles = seg + 1 == p.nseg ? p.nchunks - k0 : p.seg_tiles;
     }
     const int cg = blockIdx.x;
     const int d0 = cg * kWave;
@@ -676,7 +679,7 @@ __global__ void __launch_bounds__((NW + kSvc) * kWave) sscan_bwd_fast_kernel(con
         const bool ok = dvalid && n < p.N;
         A2[i] = ok ? av * kLog2e : 0.0f;
         // a*g flowing in from the steps after this row's last one (zero at the sequence end)
-        const float ag_in = p.ag0 ? p.ag0[(int64_t)bs * p.ED * p.Nst + dn] : 0.0f;
+        const float ag_in = seg > 0 ? p.ag0[(int64_t)bs * p.ED * p.Nst + dn] : 0.0f;
         ag[i] = ok ? ag_in : 0.0f;
         dAacc[i] = 0.0f;
     }

@@ -26,7 +26,9 @@ struct FwdParams {
     const float* chain_hend;  // segmented mode, second pass: the first pass' end states and sums of delta; the
     const float* chain_dsum;  // workgroup makes its initial state from those of the segments before its own
     int nseg;        // > 1: every batch row is cut into nseg segments of seg_tiles tiles, one
-    int seg_tiles;   // workgroup row (blockIdx.y) per (batch row, segment)
+    int seg_tiles;   // workgroup row (blockIdx.y) per (batch row, segment); the last one takes what is left
+    int run_segs;    // (nseg > 1) segments of a batch row that the launch walks, the first ones: a carry pass leaves out
+                     // the last where no one asks for its end state
     int batch, L, ED, N, nchunks;
     // A wide d_state runs as passes over blocks of states: N = states of this launch, and the
     // arrays indexed by state keep the row stride of the whole call, with their pointers advanced
@@ -58,7 +60,7 @@ struct FwdParams {
 //            decay applied after the addition.
 enum FwdMode { kScan = 0, kCarry = 1, kGCarry = 2 };
 
-// A sequence cut into nseg segments of seg_tiles tiles (the last one may be shorter), and where
+// A sequence cut into nseg segments of seg_tiles tiles (the last one takes what is left, see bwd_seg_plan for one that is longer), and where
 // the per-segment buffers sit in the workspace (offsets in floats): end states from zero
 // [rows][dim][dstate], true initial states (same shape), sums of delta [rows][4][dim];
 // rows = batch * nseg.  nseg = 1: not cut, no buffers.
@@ -68,6 +70,8 @@ struct SegPlan {
 };
 SegPlan seg_plan(const mpa_sscan_shape* s, int ns, int thin);
 SegPlan seg_layout(const mpa_sscan_shape* s, int64_t want);
+// nseg segments of seg_tiles tiles with their buffers
+SegPlan seg_buffers(const mpa_sscan_shape* s, int nseg, int64_t seg_tiles);
 // Launch sscan_fwd_kernel in `mode` (FwdMode) for the (ns, nw) decomposition; the carry modes
 // exist for ns <= 8.
 int launch_fwd_any(const FwdParams& p, int io_dtype, int ns, int nw, int mode, hipStream_t stream);

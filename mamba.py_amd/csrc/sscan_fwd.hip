@@ -320,12 +320,14 @@ __global__ void __launch_bounds__((kFwdWaves<NW, MODE, CH>) * kWave) sscan_fwd_k
     // Row of the launch: a batch row, or one segment of it (segmented mode).  h0 / h_last / dsum
     // are indexed by the launch row, the caller's tensors by (batch row, physical step).
     // Tiles are counted in WALK order: walk tile kk is the kk-th tile the recurrence visits.
-    const int bs = blockIdx.y;
+    int bs = blockIdx.y;
     int b = bs, tile0 = 0, ntiles = p.nchunks;
     if (p.nseg > 1) {
-        b = bs / p.nseg;
-        tile0 = (bs - b * p.nseg) * p.seg_tiles;
-        ntiles = min(p.seg_tiles, p.nchunks - tile0);
+        b = bs / p.run_segs;
+        const int seg = bs - b * p.run_segs;
+        bs = b * p.nseg + seg;
+        tile0 = seg * p.seg_tiles;
+        ntiles = seg + 1 == p.nseg ? p.nchunks - tile0 : p.seg_tiles;
     }
     // walk tile -> physical chunk of kTile steps; inside a tile walk step s is physical step
     // s (forward) or kTile-1-s (reverse).  The ragged chunk is always the physical last one, so a
@@ -978,9 +980,15 @@ SegPlan seg_layout(const mpa_sscan_shape* s, int64_t want) {
     const int64_t ntiles = (s->seqlen + kTile - 1) / kTile;
     if (want > ntiles) want = ntiles;
     if (want < 2 || s->batch * want > 65535) return sp;
-    sp.seg_tiles = (int)((ntiles + want - 1) / want);
-    sp.nseg = (int)((ntiles + sp.seg_tiles - 1) / sp.seg_tiles);
-    if (sp.nseg < 2) return SegPlan{1, 0, 0, 0, 0, 0};
+    const int64_t seg_tiles = (ntiles + want - 1) / want;
+    return seg_buffers(s, (int)((ntiles + seg_tiles - 1) / seg_tiles), seg_tiles);
+}
+
+SegPlan seg_buffers(const mpa_sscan_shape* s, int nseg, int64_t seg_tiles) {
+    SegPlan sp{1, 0, 0, 0, 0, 0};
+    if (nseg < 2) return sp;
+    sp.nseg = nseg;
+    sp.seg_tiles = (int)seg_tiles;
     const size_t rows = (size_t)s->batch * sp.nseg, per = (size_t)s->dim * s->dstate;
     sp.off_hend = 0;
     sp.off_h0 = rows * per;
@@ -1067,7 +1075,7 @@ static FwdPlan fwd_plan(const mpa_sscan_shape* s, int ns) {
 
 template <typename IO, int NS, int NW, bool HAS_Z, int MODE, int CH = 64, bool PROJ = false>
 static int launch_fwd(const FwdParams& p, hipStream_t stream) {
-    dim3 grid((p.ED + CH - 1) / CH, p.batch * (p.nseg > 1 ? p.nseg : 1));
+    dim3 grid((p.ED + CH - 1) / CH, p.batch * (p.nseg > 1 ? p.run_segs : 1));
     dim3 block(kFwdWaves<NW, MODE, CH> * kWave);
     constexpr size_t lds = sizeof(float) * FwdLds<NS, NW, CH>::floats;
     static LdsLimitOnce lds_limit;
@@ -1302,13 +1310,16 @@ static int sscan_fwd_impl(const mpa_sscan_shape* s, const void* x, const void* d
         if (sp.nseg <= 1) return launch_fwd_any(q, s->io_dtype, ns, nw, kScan, st);
         FwdParams p1 = q;
         p1.nseg = sp.nseg; p1.seg_tiles = sp.seg_tiles;
+        // (the last segment's end state: only for an h_last that seg_carry_kernel forms)
+        const bool chained = sp.nseg <= kChainSegments;
+        p1.run_segs = chained || !q.hlast ? sp.nseg - 1 : sp.nseg;
         p1.z = nullptr; p1.y = nullptr; p1.ypre = nullptr; p1.yacc = nullptr; p1.h0 = nullptr; p1.ckpt = nullptr;
         p1.hlast = wsf + sp.off_hend; p1.dsum = wsf + sp.off_dsum; p1.h_st = q.N;
         int r = launch_fwd_any(p1, s->io_dtype, ns, nw, kCarry, st);
         if (r != MPA_OK) return r;
         FwdParams p2 = q;
-        p2.nseg = sp.nseg; p2.seg_tiles = sp.seg_tiles;
-        if (sp.nseg <= kChainSegments) {
+        p2.nseg = p2.run_segs = sp.nseg; p2.seg_tiles = sp.seg_tiles;
+        if (chained) {
             p2.chain_hend = wsf + sp.off_hend; p2.chain_dsum = wsf + sp.off_dsum;
         } else {
             r = launch_seg_carry(q.A, q.h0, wsf + sp.off_hend, wsf + sp.off_dsum, wsf + sp.off_h0, q.hlast, q.batch,
