@@ -76,6 +76,15 @@ typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes = 0xffffffffu) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
 }
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+// 16 bytes a lane from memory into LDS, lane l's to lds + 16 * l (lds: a byte address, the same for the wave).
+__device__ __forceinline__ void load_to_lds(const u32x4& window, uint32_t at, uint32_t scalar, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(at), "s"(window), "s"(scalar) : "memory");
+}
+__device__ __forceinline__ u32x4 lds_window(const void* base, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, bytes, 0x00020000u};
+}
 // bytes from element offset `at` to the end of a tensor of `end` elements, as a buffer window
 __device__ __forceinline__ uint32_t window_bytes(int64_t end, int64_t at, int es) {
     const int64_t left = (end - at) * es;
@@ -105,7 +114,6 @@ __device__ __forceinline__ uint32_t ld_bits16(const void* base, uint32_t voff, u
 }
 __device__ __forceinline__ float bits_to_float(uint32_t bits, uint32_t shift) { return __uint_as_float(bits << shift); }
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void st_off(float2* base, uint32_t voff, float2 v, uint32_t soff = 0) {
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), make_rsrc(base), voff, soff, 0);
 }

@@ -10,7 +10,7 @@
 // the four products of a layer at width 768 and 8000 rows (3072 x 768, 768 x 1536, 80 x 1536,
 // 1536 x 48) took 88 + 80 + 80 + 54 us.  Here the 128 x 128 output tiles of all of them are one grid,
 // cut over T into `splits` parts that a second kernel adds in a fixed order.
-#include "common.h"
+#include "wgrad.h"
 
 namespace mpa {
 
@@ -303,6 +303,19 @@ static int wgrad_params(WgradParams& p, const mpa_wgrad_job* jobs, int n, int64_
     return MPA_OK;
 }
 
+static size_t wgrad_bytes(const WgradParams& p, int io_dtype) {
+    return (size_t)p.splits * p.tiles * wgrad_tile(io_dtype) * wgrad_tile(io_dtype) * sizeof(float);
+}
+
+// Estimated time of the bfloat16 kernels here, against which wgrad_wide.hip measures its tiles: a step of 64 rows takes 0.75 us with one workgroup
+// a CU and 1.27 with two, the sums of the parts come at 4.5 TB/s, and 10 us are launches and latencies.  (Layers of a width and a number of
+// rows, here and there: 768 x 8000 94 and 74 us, 1024 x 16384 319 and 191, 512 x 8192 49 and 47, 640 x 4000 46 and 45; 768 x 2048 35 and 38,
+// 256 x 16000 35 and 41, 128 x 4096 17 and 23.)
+static float wgrad_bf16_us(const WgradParams& p) {
+    const float workgroups = (float)p.tiles * (float)p.splits, steps = (float)((p.T + kWgStep - 1) / kWgStep) / (float)p.splits;
+    return 10.0f + 0.0146f * workgroups + steps * (workgroups <= 256.0f ? 0.75f : 1.27f * (workgroups <= 512.0f ? 1.0f : workgroups / 512.0f));
+}
+
 // ---- small parameters ---------------------------------------------------------------------------
 
 struct CastParams {
@@ -363,7 +376,8 @@ using namespace mpa;
 extern "C" size_t mpa_wgrad_workspace_bytes(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_t io_dtype) {
     WgradParams p{};
     if (wgrad_params(p, jobs, n, T, io_dtype) != MPA_OK) return 0;
-    return (size_t)p.splits * p.tiles * wgrad_tile(io_dtype) * wgrad_tile(io_dtype) * sizeof(float);
+    if (const size_t wide = io_dtype == MPA_BF16 ? wgrad_wide_bytes(jobs, n, T, wgrad_bf16_us(p)) : 0) return wide;
+    return wgrad_bytes(p, io_dtype);
 }
 
 extern "C" int mpa_wgrad(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_t io_dtype, void* workspace, size_t workspace_bytes,
@@ -378,9 +392,13 @@ extern "C" int mpa_wgrad(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_
     }
     if (!workspace) return MPA_ERR_NULL_POINTER;
     if (!aligned_to(workspace, 256)) return MPA_ERR_MISALIGNED;
-    if (workspace_bytes < mpa_wgrad_workspace_bytes(jobs, n, T, io_dtype)) return MPA_ERR_WORKSPACE;
-    p.part = static_cast<float*>(workspace);
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (io_dtype == MPA_BF16) {
+        const int wide = wgrad_wide_run(jobs, n, T, wgrad_bf16_us(p), workspace, workspace_bytes, st);
+        if (wide != kNotWide) return wide;
+    }
+    if (workspace_bytes < wgrad_bytes(p, io_dtype)) return MPA_ERR_WORKSPACE;
+    p.part = static_cast<float*>(workspace);
     const int groups = 8 / p.splits, per = (p.tiles + groups - 1) / groups;
     const dim3 grid((unsigned)(8 * per)), sums((unsigned)(io_dtype == MPA_F32 ? kWgTileF * kWgTileF / 4 / 256 * p.tiles : kWgTile * kWgTile / 8 / 256 * p.tiles));
     if (io_dtype == MPA_F32) {

@@ -106,15 +106,6 @@ struct LinearParams {
 // factor of the product.
 enum LinearX { kPlainX = 0, kNormX = 1, kNormXF32 = 2, kFactor = 3 };
 
-// 16 bytes a lane from memory into LDS, lane l's to lds + 16 * l (lds: a byte address, the same for the wave).
-__device__ __forceinline__ void load_to_lds(const u32x4& window, uint32_t at, uint32_t scalar, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(at), "s"(window), "s"(scalar) : "memory");
-}
-__device__ __forceinline__ u32x4 lds_window(const void* base, uint32_t bytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(base);
-    return u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, bytes, 0x00020000u};
-}
-
 constexpr int linear_threads(int BT, int BM, int KS, int RT) { return BT / (32 * RT) * (BM / 32) * KS * kWave; }
 
 template <typename IO, int BT, int BM, int KS, int RT, int D, int XMODE, bool NN>
