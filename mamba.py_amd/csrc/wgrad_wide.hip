@@ -124,9 +124,10 @@ __device__ __forceinline__ void wide_tile(const Region& g, int ta, int tb, int64
             left[o] -= ahead[o];
         }
     };
-    auto fetch = [&](int i, int buf) {  // load i of the stage that aim() was called for
-        load_to_lds(window[i >> 2], off[i >> 2][i & 3], 0, lds0 + (uint32_t)(buf * kStageBytes + (i >> 2) * kOperand + (i & 3) * 2 * kPitch));
-    };
+    // load i of the stage that aim() was called for, in two parts with a product between them: where to, and the load.  (A lone wave
+    // issues an instruction every five clocks, and a product takes sixteen.)
+    auto aim_load = [&](int i, uint32_t to) { asm volatile("s_add_u32 m0, %0, %1" ::"s"(to), "n"((i >> 2) * kOperand + (i & 3) * 2 * kPitch) : "scc"); };
+    auto load = [&](int i) { asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off[i >> 2][i & 3]), "s"(window[i >> 2]) : "memory"); };
     // reads: lane -> row 4 * (lane / 16) + lane % 16 / 4 of the first sixteen (the other sixteen behind them), four columns from 4 * (lane % 4)
     const int rowl = 4 * (lane >> 4) + ((lane & 15) >> 2), r7 = rowl & 7;
     uint32_t at_a[kA], at_b[kB];
@@ -149,7 +150,11 @@ __device__ __forceinline__ void wide_tile(const Region& g, int ta, int tb, int64
     for (int s = 0; s < kRing; ++s) {
         aim();
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i) fetch(i, s);
+        for (int i = 0; i < kLoads; ++i) {
+            aim_load(i, lds0 + (uint32_t)(s * kStageBytes));
+            asm volatile("s_nop 0");
+            load(i);
+        }
     }
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((kRing - 1) * kLoads) : "memory");
 #pragma unroll
@@ -163,16 +168,22 @@ __device__ __forceinline__ void wide_tile(const Region& g, int ta, int tb, int64
         const int x = buf & 1, y = x ^ 1;
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((kRing - 2) * kLoads) : "memory");
         aim();
+        const uint32_t to = lds0 + (uint32_t)(buf * kStageBytes);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
 #pragma unroll
             for (int j = 0; j < kB; ++j) {
                 multiply(acc[j][i], __builtin_bit_cast(bf16x8, b[x][j]), __builtin_bit_cast(bf16x8, a[x][i]));
-                // (one of the others behind a product each: they issue while it runs)
-                constexpr int kEvery = kB / 4;
-                if (j == 0) fetch(i, buf);
-                if (j % kEvery == kEvery - 1 && j / kEvery < 2) read(a[y][i].half[j / kEvery], at_a[i], (buf + 1) % kRing, j / kEvery);
-                if (j % kEvery == kEvery - 1 && j / kEvery >= 2 && i < kB) read(b[y][i].half[j / kEvery - 2], at_b[i], (buf + 1) % kRing, j / kEvery - 2);
+                // (one of the others behind a product each: it issues while the product runs; the reads done some way before the wait for them)
+                constexpr int kFetches = NARROW ? 4 : 8;
+                const int at = i * kB + j, n = at;
+                if (n < 2 * (kA + kB)) {
+                    const int o = n >> 1, half = n & 1;
+                    if (o < kB) read(b[y][o].half[half], at_b[o], (buf + 1) % kRing, half);
+                    else read(a[y][o - kB].half[half], at_a[o - kB], (buf + 1) % kRing, half);
+                }
+                if (at % kFetches == 0 && at / kFetches < kLoads) aim_load(at / kFetches, to);
+                if (at % kFetches == 1 && at / kFetches < kLoads) load(at / kFetches);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
