@@ -437,6 +437,22 @@ size_t mpa_wgrad_workspace_bytes(const mpa_wgrad_job* jobs, int32_t n, int64_t T
 int mpa_wgrad(const mpa_wgrad_job* jobs, int32_t n, int64_t T, int32_t io_dtype, void* workspace,
               size_t workspace_bytes, void* stream);
 
+/* ---- products of many rows -----------------------------------------------------------------------
+ * y (T x M) = x (T x K) . W^T in bfloat16, sums in float32, rounded once: the projections of a layer over long sequences and their
+ * input gradients (mambapy/mamba.py:210, 232).  weight is (M, K), or (K, M) with weight_kxm; pitches are of rows, in elements.  M, K and
+ * the pitches are multiples of 8, pointers 16-byte aligned; bounds: T, M and K at most 2^24, 256 rows of x, of y and of a weight (M, K)
+ * below 2^31 bytes, and all of a weight (K, M).
+ * mpa_gemm_faster: 1 where it is expected to be faster than the GEMM library, 0 where not and for calls that mpa_gemm_run refuses.
+ */
+typedef struct mpa_gemm {
+    const void *x, *weight;
+    void* y;
+    int64_t T, M, K, x_pitch, weight_pitch, y_pitch;
+    int32_t weight_kxm;
+} mpa_gemm;
+int mpa_gemm_faster(const mpa_gemm* s);
+int mpa_gemm_run(const mpa_gemm* s, void* stream);
+
 /* ---- conversions of small matrices ----------------------------------------------------------------
  * Up to MPA_CAST_MAX_JOBS copies of rows x cols elements between float32 and bfloat16 in one launch, each
  * optionally through -exp(v) (A from A_log, mambapy/mamba.py:239) or v * factor (float32, contiguous);

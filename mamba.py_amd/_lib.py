@@ -36,7 +36,7 @@ EXPORTS = ("mpa_version", "mpa_arch", "mpa_source_hash", "mpa_status_string", "m
            "mpa_conv1d_fwd", "mpa_conv1d_bwd", "mpa_conv1d_bwd_workspace_bytes", "mpa_conv1d_proj_suits", "mpa_conv1d_proj_fwd",
            "mpa_rmsnorm_fwd", "mpa_rmsnorm_bwd", "mpa_rmsnorm_bwd_workspace_bytes",
            "mpa_decode_layer_workspace_bytes", "mpa_decode_scaled_bytes", "mpa_decode_layer_step",
-           "mpa_wgrad_workspace_bytes", "mpa_wgrad", "mpa_cast", "mpa_linear_run", "mpa_linear_run_scaled",
+           "mpa_wgrad_workspace_bytes", "mpa_wgrad", "mpa_gemm_faster", "mpa_gemm_run", "mpa_cast", "mpa_linear_run", "mpa_linear_run_scaled",
            "mpa_split_bytes", "mpa_split_run", "mpa_split_product_workspace_bytes", "mpa_split_product")
 
 
@@ -62,6 +62,11 @@ class DecodeLayer(ctypes.Structure):
                [(n, ctypes.c_void_p) for n in (
                    "norm_weight", "in_weight", "in_bias", "conv_weight", "conv_bias", "x_weight", "dt_weight",
                    "dt_bias", "A", "D", "out_weight", "out_bias")]
+
+
+class Gemm(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in ("x", "weight", "y")] + \
+               [(n, ctypes.c_int64) for n in ("T", "M", "K", "x_pitch", "weight_pitch", "y_pitch")] + [("weight_kxm", ctypes.c_int32)]
 
 
 class WgradJob(ctypes.Structure):
@@ -144,6 +149,9 @@ def load():
     lib.mpa_decode_scaled_bytes.argtypes = [dp]
     lib.mpa_decode_scaled_bytes.restype = sz
     lib.mpa_decode_layer_step.argtypes = [dp] + [vp] * 12 + [sz, vp]
+    gp = ctypes.POINTER(Gemm)
+    lib.mpa_gemm_faster.argtypes = [gp]
+    lib.mpa_gemm_run.argtypes = [gp, vp]
     wp = ctypes.POINTER(WgradJob)
     lib.mpa_wgrad_workspace_bytes.argtypes = [wp, i32, i64, i32]
     lib.mpa_wgrad_workspace_bytes.restype = sz

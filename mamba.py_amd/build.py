@@ -15,7 +15,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(CSRC, "libmambapy_amd.so")
 SOURCES = ["sscan_fwd.hip", "sscan_bwd.hip", "sscan_bwd_fast.hip", "pscan.hip", "step.hip", "conv1d.hip", "conv_proj.hip", "rmsnorm.hip",
-           "decode.hip", "layer.hip", "wgrad_wide.hip", "linear.hip", "split.hip"]
+           "decode.hip", "layer.hip", "wgrad_wide.hip", "gemm_wide.hip", "linear.hip", "split.hip"]
 HOST_SOURCES = ["host.cpp", "host_model.cpp", "host_train.cpp"]
 HOST_PATH = os.path.join(CSRC, "_mpa_host.so")
 ARCH = "gfx950"

@@ -615,6 +615,17 @@ inline bool split_product(const Tensor& x, const Tensor& weight, const Tensor& b
     return true;
 }
 
+// y = x . weight^T, or x . weight (kxm), of matrices with dense rows.
+inline void mm_into(const Tensor& y, const Tensor& x, const Tensor& weight, bool kxm, void* stream) {
+    const mpa_gemm g{ptr(x), ptr(weight), ptr(y), x.size(0), y.size(1), x.size(1), x.stride(0), weight.stride(0), y.stride(0), kxm};
+    if (x.scalar_type() == at::kBFloat16 && x.stride(1) == 1 && weight.stride(1) == 1 && mpa_gemm_faster(&g)) {
+        check(mpa_gemm_run(&g, stream), "mpa_gemm_run");
+    } else {
+        Tensor out = y;
+        at::mm_out(out, x, kxm ? weight : weight.t());
+    }
+}
+
 template <typename H>
 inline H* handle_in(PyObject* dict) {
     PyObject* o = get(dict, keys().handle);

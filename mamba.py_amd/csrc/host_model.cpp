@@ -231,7 +231,7 @@ Tensor run_sequence(const std::vector<Layer>& hs, const Tensor& x, std::vector<C
         } else if (l.p[kInB].defined()) {
             at::addmm_out(out, l.p[kInB], normed, l.p[kInW].t());
         } else {
-            at::mm_out(out, normed, l.p[kInW].t());
+            mm_into(xz, normed, l.p[kInW], false, stream);
         }
         Tensor window, h_last;
         if (keep) {
@@ -276,7 +276,7 @@ Tensor run_sequence(const std::vector<Layer>& hs, const Tensor& x, std::vector<C
         } else if (l.p[kOutB].defined()) {
             at::addmm_out(out, l.p[kOutB], y, l.p[kOutW].t());
         } else {
-            at::mm_out(out, y, l.p[kOutW].t());
+            mm_into(hidden, y, l.p[kOutW], false, stream);
         }
         in = ptr(hidden);
         if (keep) cs[i] = {h_last, window};

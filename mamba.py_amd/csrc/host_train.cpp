@@ -98,7 +98,9 @@ std::tuple<Tensor, Tensor, Tensor> mixer_forward(Weights& l, const std::array<co
             const Tensor y = empty({T, weight.size(0)}, dt, x);
             if (split_product(in, weight, bias, y, stream)) return y;
             Tensor out = y;
-            return bias.defined() ? at::addmm_out(out, bias, in, weight.t()) : at::mm_out(out, in, weight.t());
+            if (bias.defined()) at::addmm_out(out, bias, in, weight.t());
+            else mm_into(y, in, weight, false, stream);
+            return y;
         };
         const Tensor xz = wide(x2, l.p[kInW], l.p[kInB]);
         const Tensor xs = empty({T, ED}, dt, x);
@@ -227,7 +229,8 @@ variable_list MixerBackward::apply(variable_list&& grads) {
         s.product(weight, in, Tensor(), ptr(dy), ED);
         s.run_products();
     } else {
-        dy = at::mm(dout, w[kIOutW]);
+        dy = empty({T, ED}, dt, x_);
+        mm_into(dy, dout, w[kIOutW], true, stream);
     }
     const Tensor dxz = empty({T, 2 * ED}, dt, x_), dxs_ddelta = empty({T, 2 * ED}, dt, x_), ddbc = empty({T, P}, dt, x_);
     const Tensor dA = empty({ED, N}, at::kFloat, x_), dD = empty({ED}, at::kFloat, x_), ddt_b = empty({ED}, at::kFloat, x_);
@@ -295,7 +298,8 @@ variable_list MixerBackward::apply(variable_list&& grads) {
             g[kIX] = empty({Bs, L, d}, dt, x_);
             product(ptr(dxz), 2 * ED, 2 * ED, w[kIInW], ptr(g[kIX]), d, false);
         } else {
-            g[kIX] = at::mm(dxz, w[kIInW]).view({Bs, L, d});
+            g[kIX] = empty({Bs, L, d}, dt, x_);
+            mm_into(g[kIX].view({T, d}), dxz, w[kIInW], true, stream);
         }
     }
 
