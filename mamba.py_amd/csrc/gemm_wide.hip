@@ -322,8 +322,8 @@ float gemm_plan(const mpa_gemm* s, GemmParams& p) {
 // Against the library, at widths 256 to 1024 and 1500 to 24 000 rows, the products of a layer (W as M x K: 4d x d, d x 2d; as K x M: 2d x d, d x 4d) and
 // 50 280 x d; its time over the library's:
 //   K up to 512       0.4 to 0.98
-//   rows of x or W that are not whole 128 bytes (K % 64), or of y (M % 64; a y of 50 280 columns is no matter): 0.4 to 0.9 where tiles fill
-//                     the chip.  The library runs these at 500 to 900 TFLOP/s, 700 is what it is taken for, and 18 us at least (host).
+//   rows of x or W that are not whole 128 bytes (K % 64), or of y (M % 64; of 50 280 columns up to 4000 rows, 0.96 to 1.09 above): 0.4 to 0.9
+//                     where tiles fill the chip.  The library runs these at 500 to 900 TFLOP/s, 700 is what it is taken for, and 18 us at least (host).
 //   others            both take tiles of this size, and whole rounds of them are 0 to 9 % faster there; where this kernel saves a part of a
 //                     round by halves, up to K = 1024 (a longer sum leaves the first loads and the stores a smaller part): 0.61 to 0.98
 extern "C" int mpa_gemm_faster(const mpa_gemm* s) {
@@ -331,7 +331,7 @@ extern "C" int mpa_gemm_faster(const mpa_gemm* s) {
     GemmParams p{};
     const float us = gemm_plan(s, p);
     if (s->K <= 512) return 1;
-    if (s->K % 64 || (s->M % 64 && s->M <= 4096)) return us + 3.0f < std::max(18.0f, 6.0f + 2e-9f * (float)s->T * (float)s->M * (float)s->K / 0.7f);
+    if (s->K % 64 || (s->M % 64 && (s->M <= 4096 || s->T <= 4096))) return us + 3.0f < std::max(18.0f, 6.0f + 2e-9f * (float)s->T * (float)s->M * (float)s->K / 0.7f);
     return s->K <= 1024 && us <= 0.93f * (float)((p.tiles_t * p.tiles_m + kCUs - 1) / kCUs) * tile_us((p.K + kStageK - 1) / kStageK);
 }
 

@@ -319,6 +319,39 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
     return py::make_tuple(y, after);
 }
 
+// A plain nn.Linear without bias over many rows (the head of a model, by which its scores of a sequence are formed), where the kernel of this
+// package is the faster one; else None.
+constexpr int64_t kHeadRows = 64;
+py::object linear_rows(const py::object& module, const Tensor& x_in) {
+    if (at::GradMode::is_enabled() || !native_call(x_in) || (PyObject*)Py_TYPE(module.ptr()) != types->linear.ptr() || x_in.dim() < 2 ||
+        x_in.scalar_type() != at::kBFloat16 || x_in.numel() == 0)
+        return py::none();
+    Instance self;
+    if (!self.plain(dict_of(module.ptr()), types->linear_names)) return py::none();
+    const Keys& k = keys();
+    self.find(k.weight, k.bias);
+    Param weight;
+    Tensor w;
+    bool changed = false;
+    if (self.pair[1] != Py_None || !weight.take(self.pair[0], w, changed) || !w.defined() || w.scalar_type() != at::kBFloat16 || w.dim() != 2 ||
+        w.device() != x_in.device() || w.size(1) != x_in.size(-1) || !w.is_contiguous())
+        return py::none();
+    at::AutoDispatchBelowADInplaceOrView below;
+    const c10::DeviceGuard guard(x_in.device());
+    const int64_t K = w.size(1), M = w.size(0), T = x_in.numel() / K;
+    if (T < kHeadRows || !x_in.is_contiguous()) return py::none();
+    mpa_gemm g{ptr(x_in), ptr(w), ptr(w), T, M, K, K, K, M, 0};  // (y: for the rule)
+    if (!mpa_gemm_faster(&g)) return py::none();
+    std::vector<int64_t> sizes = x_in.sizes().vec();
+    sizes.back() = M;
+    const py::gil_scoped_release nogil;
+    const Tensor y = empty(sizes, at::kBFloat16, x_in);
+    g.y = ptr(y);
+    check(mpa_gemm_run(&g, stream_of(x_in)), "mpa_gemm_run");
+    const py::gil_scoped_acquire gil;
+    return py::cast(y);
+}
+
 }  // namespace
 
 void bind_model(py::module_& m) {
@@ -359,6 +392,7 @@ void bind_model(py::module_& m) {
     m.def("stack_step", &stack_step);
     m.def("block_step", &block_step);
     m.def("stack_forward", &stack_forward);
+    m.def("linear_rows", &linear_rows);
 }
 
 }  // namespace mpa_host

@@ -13,7 +13,7 @@ import math
 import torch
 import torch.nn as nn
 
-from .modules import Mamba, MambaConfig, RMSNorm
+from .modules import Mamba, MambaConfig, RMSNorm, _host
 
 
 class LM(nn.Module):
@@ -48,8 +48,9 @@ class LM(nn.Module):
 
     def forward(self, tokens):
         """tokens : (B, L) int64 -> logits (B, L, vocab)."""
-        x = self.mamba(self.embedding(tokens))
-        return self.lm_head(self.norm_f(x))
+        x = self.norm_f(self.mamba(self.embedding(tokens)))
+        y = None if torch.is_grad_enabled() or not x.is_cuda else _host().linear_rows(self.lm_head, x)
+        return self.lm_head(x) if y is None else y
 
     @torch.no_grad()
     def prefill(self, tokens, caches=None):
