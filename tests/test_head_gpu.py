@@ -26,6 +26,23 @@ def test_logits(pkg, dev, batch, length):
     assert rel_err(got, want) <= TOL[torch.bfloat16] / 4
 
 
+@pytest.mark.parametrize("rows", [(1, 256), (1, 400), (3, 333)])
+def test_logits_float32(pkg, dev, rows):
+    m = _lm(pkg, dev, 1024, 8004, torch.float32)
+    vocab = m.vocab_size
+    h = torch.randn(*rows, 1024, device=dev)
+    with torch.no_grad():
+        got = pkg.modules._host().linear_rows(m.lm_head, h)
+    # (half the harmonic mean of the row counts: from 300 on)
+    T = rows[0] * rows[1]
+    assert (got is not None) == (T * vocab >= 300 * (T + vocab) and T * vocab * 1024 >= 5 << 29)
+    if got is not None:
+        want = h.double() @ m.lm_head.weight.double().t()
+        # sixteen products are added exactly: K / 16 sums of 2^-24 each at most
+        scale = h.abs().double() @ m.lm_head.weight.abs().double().t()
+        assert got.shape == (*rows, vocab) and ((got - want).abs() <= 1024 / 16 * 2.0 ** -24 * scale + 2.0 ** -21 * scale).all()
+
+
 def test_what_it_leaves_to_the_module(pkg, dev):
     m = _lm(pkg, dev)
     host, x = pkg.modules._host(), torch.randn(2, 100, 72, device=dev).bfloat16()
