@@ -34,8 +34,7 @@ def test_logits_float32(pkg, dev, rows):
     with torch.no_grad():
         got = pkg.modules._host().linear_rows(m.lm_head, h)
     # (half the harmonic mean of the row counts: from 300 on)
-    T = rows[0] * rows[1]
-    assert (got is not None) == (T * vocab >= 300 * (T + vocab) and T * vocab * 1024 >= 5 << 29)
+    assert (got is not None) == (rows[0] * rows[1] >= 400)
     if got is not None:
         want = h.double() @ m.lm_head.weight.double().t()
         # sixteen products are added exactly: K / 16 sums of 2^-24 each at most
