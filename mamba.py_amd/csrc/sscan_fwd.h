@@ -68,7 +68,6 @@ struct SegPlan {
     int nseg, seg_tiles;
     size_t off_hend, off_h0, off_dsum, floats;
 };
-SegPlan seg_plan(const mpa_sscan_shape* s, int ns, int thin);
 SegPlan seg_layout(const mpa_sscan_shape* s, int64_t want);
 // nseg segments of seg_tiles tiles with their buffers
 SegPlan seg_buffers(const mpa_sscan_shape* s, int nseg, int64_t seg_tiles);

@@ -25,7 +25,7 @@
 //    launch would cover a fraction of the chip, the sequence is cut into segments that run side
 //    by side: a first pass (kernel mode kCarry: no readout) finds every segment's end state
 //    from zero and its sum of delta, seg_carry_kernel chains them, a second pass is the normal
-//    kernel from the true initial states (see seg_plan).  The backward uses the same first pass
+//    kernel from the true initial states (see fwd_plan).  The backward uses the same first pass
 //    for its own carry (mode kGCarry, see sscan_bwd.hip).
 //  * Time is addressed through one mapping, walk position -> physical step, so that the scan
 //    can run from the last step to the first (MPA_SSCAN_REVERSE) without flipped copies: the
@@ -973,8 +973,6 @@ __global__ void __launch_bounds__(256) seg_carry_kernel(const float* __restrict_
 // Segments per batch row.  The scan is serial in time, so a launch has only batch * dim/64
 // workgroups; when those cover a fraction of the chip's 256 CUs the sequence is cut into
 // segments that run side by side: up to twice the arithmetic, nseg times the parallelism.
-// `thin` is the coverage below which the cut pays: half of the CUs for the backward (its first pass costs a quarter of
-// the second), a third for a forward whose plan the caller pins (0.8 of it; otherwise fwd_plan decides by an estimate).
 SegPlan seg_layout(const mpa_sscan_shape* s, int64_t want) {
     SegPlan sp{1, 0, 0, 0, 0, 0};
     const int64_t ntiles = (s->seqlen + kTile - 1) / kTile;
@@ -997,14 +995,17 @@ SegPlan seg_buffers(const mpa_sscan_shape* s, int nseg, int64_t seg_tiles) {
     return sp;
 }
 
-SegPlan seg_plan(const mpa_sscan_shape* s, int ns, int thin) {
+static constexpr int kFwdThin = 3;
+// A forward whose plan the caller pins in part (otherwise fwd_plan decides by an estimate): its first pass costs 0.8 of the second, so a third
+// of the CUs or fewer covered.
+static SegPlan seg_plan(const mpa_sscan_shape* s, int ns) {
     if (ns > 8) return SegPlan{1, 0, 0, 0, 0, 0};
     const int64_t ntiles = (s->seqlen + kTile - 1) / kTile;
     const int64_t groups = s->batch * ((s->dim + kWave - 1) / kWave);
     int64_t want = 1;
     if (s->plan_segments > 0) {
         want = s->plan_segments;
-    } else if (groups * thin <= 256 && ntiles >= 32) {
+    } else if (groups * kFwdThin <= 256 && ntiles >= 32) {
         want = 256 / groups;
         if (want > ntiles / 8) want = ntiles / 8;  // segments of 128 steps or more
         if (want > 64) want = 64;
@@ -1034,7 +1035,6 @@ struct FwdPlan {
 // 0.9 us per segment before its own, under the loaders' latency); with more seg_carry_kernel, which reads
 // them once and takes about 7 us with its launch.
 static constexpr int kChainSegments = 8;
-static constexpr int kFwdThin = 3;  // (seg_plan) a third of the CUs or fewer covered
 static FwdPlan fwd_plan(const mpa_sscan_shape* s, int ns) {
     const int pins = MPA_PLAN_GROUP_16 | MPA_PLAN_GROUP_32 | MPA_PLAN_GROUP_48 | MPA_PLAN_GROUP_64;
     const bool narrow_ok = ns <= 8 && s->dstate <= 64 && s->plan_states_per_lane == 0;
@@ -1042,7 +1042,7 @@ static FwdPlan fwd_plan(const mpa_sscan_shape* s, int ns) {
         return FwdPlan{(s->plan_flags & MPA_PLAN_GROUP_16) ? 16 : 32, seg_layout(s, s->plan_segments > 0 ? s->plan_segments : 1)};
     const bool form48 = ns == 2 && s->dstate <= 16;  // the 48-channel kernel: not cut
     if (!narrow_ok || s->plan_segments > 0 || (s->plan_flags & pins)) {
-        FwdPlan p{64, seg_plan(s, ns, kFwdThin)};
+        FwdPlan p{64, seg_plan(s, ns)};
         if (form48 && p.seg.nseg == 1 && !(s->plan_flags & MPA_PLAN_GROUP_64) &&
             ((s->plan_flags & MPA_PLAN_GROUP_48) || s->batch * ((s->dim + 47) / 48) <= 256))
             p.group = 48;
