@@ -2,6 +2,10 @@
 // residual blocks in one call from Python.
 #include "host_layer.h"
 
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+
 namespace mpa_host {
 namespace {
 
@@ -327,6 +331,10 @@ constexpr int64_t kHeadRows = 64;
 py::object linear_rows(const py::object& module, const Tensor& x_in) {
     if (at::GradMode::is_enabled() || !native_call(x_in) || (PyObject*)Py_TYPE(module.ptr()) != types->linear.ptr() || x_in.dim() < 2 ||
         (x_in.scalar_type() != at::kBFloat16 && x_in.scalar_type() != at::kFloat) || x_in.numel() == 0)
+        return py::none();
+    // (a trace or a mode sees the calls of torch that this one would stand in for)
+    if (torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::PythonTorchFunctionTLS::stack_len() > 0 ||
+        x_in.key_set().has(c10::DispatchKey::Python))
         return py::none();
     Instance self;
     if (!self.plain(dict_of(module.ptr()), types->linear_names)) return py::none();

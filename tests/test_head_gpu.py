@@ -2,6 +2,7 @@
 import pytest
 import torch
 import torch.nn as nn
+from torch.utils.flop_counter import FlopCounterMode
 
 from util import TOL, rel_err
 
@@ -63,6 +64,11 @@ def test_what_it_leaves_to_the_module(pkg, dev):
         del head.forward
         with torch.autocast("cuda", dtype=torch.bfloat16):
             assert host.linear_rows(head, x) is None
+
+        with FlopCounterMode(display=False) as counted:
+            assert host.linear_rows(head, x) is None
+            m.lm_head(x)
+        assert counted.get_total_flops() == 2 * 200 * 72 * 1000
 
         class Other(nn.Linear):
             pass
