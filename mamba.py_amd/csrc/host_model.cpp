@@ -323,14 +323,13 @@ py::object stack_forward(const py::list& layers, const Tensor& x_in, const py::o
     return py::make_tuple(y, after);
 }
 
-// A plain nn.Linear without bias over many rows (the head of a model, by which its scores of a sequence are formed), where a kernel of this
-// package is the faster one; else None.  float32: on cut operands by the line of a layer's products (use_split), though the weight is cut for
-// one product here.  50 280 columns, widths 256 / 480 / 768, cutting and product over library: 300 steps 0.76 / 0.67 / 0.80, 930
-// 0.59 / 0.59 / 0.57, 4000 0.59 / 0.51 / 0.45 (2335 us -> 1047); against 64 bits 1.9e-7 where the library has 5.0e-7 (width 768).
+// A plain bfloat16 nn.Linear without bias over many rows (the head of a model, by which its scores of a sequence are formed), where a kernel of
+// this package is the faster one; else None.  (Not float32, though a product on cut operands takes half the library's time: it keeps 2^-23 of a
+// value, so that a weight that selects a column does not give that column.)
 constexpr int64_t kHeadRows = 64;
 py::object linear_rows(const py::object& module, const Tensor& x_in) {
     if (at::GradMode::is_enabled() || !native_call(x_in) || (PyObject*)Py_TYPE(module.ptr()) != types->linear.ptr() || x_in.dim() < 2 ||
-        (x_in.scalar_type() != at::kBFloat16 && x_in.scalar_type() != at::kFloat) || x_in.numel() == 0)
+        x_in.scalar_type() != at::kBFloat16 || x_in.numel() == 0)
         return py::none();
     // (a trace or a mode sees the calls of torch that this one would stand in for)
     if (torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::PythonTorchFunctionTLS::stack_len() > 0 ||
@@ -343,23 +342,21 @@ py::object linear_rows(const py::object& module, const Tensor& x_in) {
     Param weight;
     Tensor w;
     bool changed = false;
-    if (self.pair[1] != Py_None || !weight.take(self.pair[0], w, changed) || !w.defined() || w.scalar_type() != x_in.scalar_type() || w.dim() != 2 ||
+    if (self.pair[1] != Py_None || !weight.take(self.pair[0], w, changed) || !w.defined() || w.scalar_type() != at::kBFloat16 || w.dim() != 2 ||
         w.device() != x_in.device() || w.size(1) != x_in.size(-1) || !w.is_contiguous())
         return py::none();
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard guard(x_in.device());
     const int64_t K = w.size(1), M = w.size(0), T = x_in.numel() / K;
     if (T < kHeadRows || !x_in.is_contiguous()) return py::none();
-    const bool bf16 = x_in.scalar_type() == at::kBFloat16;
     mpa_gemm g{ptr(x_in), ptr(w), ptr(w), T, M, K, K, K, M, 0};  // (y: for the rule)
-    if (bf16 ? !mpa_gemm_faster(&g) : !use_split(at::kFloat, T, M, K, {&x_in, &w})) return py::none();
+    if (!mpa_gemm_faster(&g)) return py::none();
     std::vector<int64_t> sizes = x_in.sizes().vec();
     sizes.back() = M;
     const py::gil_scoped_release nogil;
-    const Tensor y = empty(sizes, x_in.scalar_type(), x_in);
+    const Tensor y = empty(sizes, at::kBFloat16, x_in);
     g.y = ptr(y);
-    if (bf16) check(mpa_gemm_run(&g, stream_of(x_in)), "mpa_gemm_run");
-    else split_product(x_in, w, Tensor(), y, stream_of(x_in));
+    check(mpa_gemm_run(&g, stream_of(x_in)), "mpa_gemm_run");
     const py::gil_scoped_acquire gil;
     return py::cast(y);
 }
