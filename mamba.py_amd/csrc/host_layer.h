@@ -542,30 +542,25 @@ inline mpa_linear linear_of(int io, int64_t T, const void* in, int64_t x_pitch, 
 inline void run_linear(const mpa_linear& q, void* stream) { check(mpa_linear_run(&q, stream), "mpa_linear_run"); }
 
 // The wide float32 products of a layer on cut operands (mpa_split_run, mpa_split_product), where a product is long enough to pay
-// for cutting its operands.  Measured against library products, widths 200 to 2560 and 128 to 32768 steps, each
-// with the cutting of both operands.  A value is cut once and multiplied as often as the other operand has rows, so the line goes by
-// those (half the harmonic mean of T and M) as well.  From 700 on one product is 1.15 to 2.7 times as fast from 3 * 2^28 multiplications
-// (1500 / 3000 steps of 1568 x 392 1.7 / 2.0, of 2048 x 512 1.25; 4100 of 800 x 200 2.0; below the line 0.9 to 1.5: 2000 of 1024 x 256
-// 0.97, 1500 of 1312 x 328 0.97).  From 300 rows on 1.06 to 2.0 from 2^31 (3000 steps of 640 x 1280 1.06, of 392 x 784 at 8000 1.8; below
-// 0.65 to 1.3: 3000 of 392 x 784 0.72, 1000 of 1920 x 480 0.88, 3000 of 480 x 960 0.88), 1.2 to 2.4 at 8 and 1.9 to 2.5 at 16
-// times 2^30.  With few steps against a wide weight cutting it is what costs, and below 300 rows one product of 2.5 to 5 * 2^30 is
-// 0.6 to 1.0 times as fast (160 / 256 / 288 steps of width 2048 0.60 / 0.91 / 0.98, 352 1.22; 284 of 1536 0.86, 352 1.4; a
+// for cutting its operands.  Measured against library products, widths 256 to 2560 and 128 to 32768 steps, each
+// with the cutting of both operands: one product is 0.6 to 1.4 times as fast below 2.5 * 2^30 multiplications, 1.0 to 2.0 just
+// above, 1.2 to 2.4 at 8 and 1.9 to 2.5 at 16 times 2^30.  A value is cut once and multiplied as often as the other operand has rows:
+// with few steps against a wide weight cutting it is what costs, and below 300 (half the harmonic mean of T and M) one product of 2.5 to
+// 5 * 2^30 is 0.6 to 1.0 times as fast (160 / 256 / 288 steps of width 2048 0.60 / 0.91 / 0.98, 352 1.22; 284 of 1536 0.86, 352 1.4; a
 // stack of two layers, 160 / 284 steps of width 2048, without gradients 318 / 386 us with it and 237 / 348, at 320 steps 393 and 376, with
 // gradients 1199 and 1230).
 // The input gradient and both weight gradients together, one cutting for three products of which the library's weight
-// gradients are its slowest: 1.04 to 2.1 from 2^31 for the input gradient on, 1.2 to 2.2 at four times that; below 2^31 a layer with
-// gradients is 1.00 to 1.12 times as fast with all of these lines as with 2.5 * 2^30 for one product and 2^31 for three (4158 steps of width
-// 328, three layers, 1621 us -> 1518; 4096 of 392, two, 1265 -> 1134; 2000 of 512 916 -> 850; 1000 of 704 882 -> 819; without
-// gradients 4000 of 400, six layers, 2080 -> 1680).
-constexpr int64_t kSplitOne = 1LL << 31, kSplitMany = 3LL << 28, kSplitThree = 1LL << 30, kSplitRows = 300, kSplitManyRows = 700;
+// gradients are its slowest: 1.04 to 2.1 from 2^31 for the input gradient on, 1.2 to 2.2 at four times that.
+// (Time alone would take lower lines: 3 * 2^28 where both operands have 700 rows or more, 2^30 for three, 1.0 to 2.0 times as fast.  But a cut value is
+// 2^-23 of itself, and operands that a float32 sum keeps whole, as a weight of ones and zeros does, come out 2^-24 off.)
+constexpr int64_t kSplitOne = 5LL << 29, kSplitThree = 1LL << 31, kSplitRows = 300;
 inline bool split_ok(at::ScalarType dt, int64_t T, int64_t M, int64_t K, std::initializer_list<const Tensor*> operands) {
     bool ok = dt == at::kFloat && T < 1 << 24 && M % 4 == 0 && K % 4 == 0;
     for (const Tensor* t : operands) ok &= !t->defined() || aligned(t->const_data_ptr(), 16);
     return ok;
 }
 inline bool use_split(at::ScalarType dt, int64_t T, int64_t M, int64_t K, std::initializer_list<const Tensor*> operands) {
-    const int64_t rows = T * M / (T + M);
-    return (rows >= kSplitManyRows ? T * M * K >= kSplitMany : rows >= kSplitRows && T * M * K >= kSplitOne) && split_ok(dt, T, M, K, operands);
+    return T * M * K >= kSplitOne && T * M >= kSplitRows * (T + M) && split_ok(dt, T, M, K, operands);
 }
 inline bool use_split_three(at::ScalarType dt, int64_t T, int64_t M, int64_t K, std::initializer_list<const Tensor*> operands) {
     return T * M * K >= kSplitThree && split_ok(dt, T, M, K, operands);
