@@ -344,7 +344,7 @@ struct DecodeParams {
     int P4;         // dt_rank + 2 d_state to a multiple of four: pitch of dbc
     uint32_t span_inv;  // of a launch's tiles, see decode_tile
     int groups;
-    float eps, inv_d;
+    float eps;
     int splits, ssq_tiles;  // partial sums of x_proj; row tiles of d (partial sums of squares)
     const void* x;
     const void* xw;        // x times the norm weight in operand order, or null: formed from x
@@ -410,7 +410,7 @@ __global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams
     __shared__ float ssq[NW][NT][16];
     __shared__ alignas(16) float xl[XP ? NT * 16 : 1][16];  // convolved x of the tile
     // (all arguments requested at once: the compiler otherwise loads some where they are used, each a round trip in a step's chain)
-    asm volatile("" ::"s"(p.batch), "s"(p.d), "s"(p.ED), "s"(p.N), "s"(p.R), "s"(p.K), "s"(p.P4), "s"(p.span_inv), "s"(p.groups), "s"(p.eps), "s"(p.inv_d),
+    asm volatile("" ::"s"(p.batch), "s"(p.d), "s"(p.ED), "s"(p.N), "s"(p.R), "s"(p.K), "s"(p.P4), "s"(p.span_inv), "s"(p.groups), "s"(p.eps),
                  "s"(p.ssq_tiles), "s"(p.x), "s"(p.xw), "s"(p.ssq), "s"(p.norm_w), "s"(p.in_w), "s"(p.in_b), "s"(p.conv_w), "s"(p.conv_b), "s"(p.xp_w),
                  "s"(p.win_in), "s"(p.win_out), "s"(p.xs), "s"(p.z), "s"(p.dbc));
     int rt, bt;
@@ -512,7 +512,7 @@ __global__ void __launch_bounds__(NW* kWave) decode_in_kernel(const DecodeParams
             float s = ssq[0][bl >> 4][bl & 15];
 #pragma unroll
             for (int w = 1; w < NW; ++w) s += ssq[w][bl >> 4][bl & 15];
-            v *= __builtin_amdgcn_rsqf(s * p.inv_d + p.eps);
+            v *= __builtin_amdgcn_rsqf(s / (float)p.d + p.eps);
         }
         const IO vr = from_float<IO>(v + to_float(ib[i]));
         if (n0 >= p.ED) {  // uniform over the block
@@ -1132,7 +1132,7 @@ extern "C" int mpa_decode_layer_step(const mpa_decode_layer* s, const void* x, c
     DecodeParams p{};
     p.batch = (int)s->batch; p.d = (int)s->d_model; p.ED = (int)s->dim; p.N = (int)s->dstate; p.R = (int)s->dt_rank;
     p.P4 = (p.R + 2 * p.N + 3) / 4 * 4;
-    p.K = s->d_conv; p.eps = s->eps; p.inv_d = 1.0f / (float)p.d; p.splits = decode_splits(s); p.ssq_tiles = (p.d + 15) / 16;
+    p.K = s->d_conv; p.eps = s->eps; p.splits = decode_splits(s); p.ssq_tiles = (p.d + 15) / 16;
     p.x = x; p.xw = x_scaled; p.ssq = x_ssq; p.norm_w = s->norm_weight;
     p.in_w = s->in_weight; p.in_b = s->in_bias; p.conv_w = s->conv_weight; p.conv_b = s->conv_bias;
     p.xp_w = s->x_weight; p.dt_w = s->dt_weight; p.dt_b = s->dt_bias; p.A = s->A; p.D = s->D;

@@ -60,3 +60,18 @@ def test_an_infinite_sequence_stays_alone(pkg, dev, dtype):
     for (h0, w0), (h1, w1) in zip(c0, c1):
         assert torch.equal(h0[keep], h1[keep]) and torch.equal(w0[keep], w1[keep])
     assert not torch.isfinite(y1[2].float()).any()
+
+
+@pytest.mark.parametrize("width", [328, 376, 488])
+def test_the_mean_of_squares_is_a_quotient(pkg, dev, width):
+    """Rows of one value, whose squares and their sum are exact: their mean does not depend on the width, and neither does what in_proj, a selection
+    of columns, leaves in the convolution's window.  (A product with a rounded 1 / width does.)"""
+    def newest(d):
+        m = pkg.Mamba(pkg.MambaConfig(d_model=d, n_layers=1, rms_norm_eps=1e-30)).to(dev)
+        x = (torch.arange(9, 41, device=dev).float() / 16)[:, None].repeat(1, d)
+        with torch.no_grad():
+            w = m.layers[0].mixer.in_proj.weight
+            w.zero_()
+            w[torch.arange(w.size(0)), torch.arange(w.size(0)) % d] = 1.0
+            return m.step(x, m.empty_caches(32, device=dev))[1][0][1][:, 0, -1]
+    assert torch.equal(newest(width), newest(256))
