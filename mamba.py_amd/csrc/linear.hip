@@ -24,6 +24,7 @@
 // time is saved, until the product itself is longer than a library call (a training layer of 1614 steps and width 424
 // 0.69 ms, 0.81 with library calls; 168 steps of ten layers of width 640 without gradients 0.63 and 0.85 ms).
 #include "common.h"
+#include "row_offset.h"
 
 namespace mpa {
 
@@ -83,6 +84,7 @@ enum LinearFlags {
     kResidualF32 = 4,  // so is the residual
     kXLarger = 8,      // x has more bytes than W
     kBySteps = 16,     // tiles walk W first: set by the launch
+    kRowsWrap = 32,    // rows beyond the last have to be kept outside of the windows: set by the launch
 };
 struct LinearParams {
     const void *x, *w, *bias;
@@ -148,7 +150,8 @@ __global__ void __launch_bounds__(linear_threads(BT, BM, KS, RT)) linear_kernel(
     uint32_t off[kLoads];
     int koff[kLoads], at[kLoads];
     // Direct loads: a wave fetches for its own share of K, 64 places of LDS (eight rows) at a time, W's rows first; a lane's part of K is the
-    // same in all of them.  (Rows beyond the last are read from anywhere in the window, or as zeros; their results are not stored.)
+    // same in all of them.  (Rows beyond the last are read as zeros: they are
+    // beyond the window.  Their results are not stored.)
     constexpr int kShareWaves = kThreads / kWave / KS, kRowStep = 8 * kShareWaves;
     static_assert(!kDirect || (BM % kRowStep == 0 && kRows % kRowStep == 0), "a load instruction reads W or x");
     const int share_wave = wave / KS, part_of = (lane & 7) ^ (lane >> 3);
@@ -160,6 +163,14 @@ __global__ void __launch_bounds__(linear_threads(BT, BM, KS, RT)) linear_kernel(
         const uint32_t pitch = isw ? (uint32_t)p.K : (uint32_t)p.x_pitch;
         if (i == 0 || i * kRowStep == BM) off[i] = kES * (kl + (uint32_t)((isw ? m0 : t0) + share_wave * 8 + (lane >> 3)) * pitch);
         else off[i] = off[i - 1] + kES * kRowStep * pitch;
+    }
+    // (a choice for every row is 24 instructions of a wave at most, 70 ns of every launch)
+    if (kDirect && (flags & kRowsWrap)) {
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const bool isw = i * kRowStep < BM;
+            off[i] = row_offset((isw ? m0 : t0 - BM) + i * kRowStep + share_wave * 8 + (lane >> 3), isw ? p.M : p.T, off[i]);
+        }
     }
 #pragma unroll
     for (int i = 0; !kDirect && i < kLoads; ++i) {
@@ -198,7 +209,7 @@ __global__ void __launch_bounds__(linear_threads(BT, BM, KS, RT)) linear_kernel(
         const bool some = k + kl < p.K;
 #pragma unroll
         for (int i = 0; i < kLoads; ++i)
-            load_to_lds(i * kRowStep < BM ? win_w : win_x, some ? off[i] : 0x80000000u, (uint32_t)k * kES, lds0 + (uint32_t)(buf * kStage + i * kShareWaves * kWave) * 16u);
+            load_to_lds(i * kRowStep < BM ? win_w : win_x, some ? off[i] : kNoRow, (uint32_t)k * kES, lds0 + (uint32_t)(buf * kStage + i * kShareWaves * kWave) * 16u);
     };
     auto load = [&](Stage& st, int s) {
         u32x4(&v)[kLoads] = st.v;
@@ -499,6 +510,7 @@ static int launch_linear(LinearParams p, const LinearForm& f, hipStream_t st) {
     const int nt = (p.T + BT - 1) / BT, nm = (p.M + BM - 1) / BM, per = (nt * nm + 7) / 8;
     const bool by_steps = (p.flags & kXLarger) && nt * nm >= 512;
     if (by_steps) p.flags |= kBySteps;
+    if (rows_wrap(p.T, BT, p.x_pitch, sizeof(IO)) || rows_wrap(p.M, BM, p.K, sizeof(IO))) p.flags |= kRowsWrap;
     p.tiles = nt * nm;
     p.tiles_per_xcd = per;
     p.inner = by_steps ? nm : nt;

@@ -40,3 +40,20 @@ def test_products_against_float64(pkg, dev, dtype, T, M, K, pad):
     q.y = y2.data_ptr()
     L.check(lib.mpa_linear_run_scaled(ctypes.byref(q), None, None, pkg.scan._stream(dev)), "mpa_linear_run_scaled")
     assert ((y2.double().cpu() - ref).abs() <= 2 * bound + 2.0 ** -20 * ref.abs()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,M,K,pitch", [(2, 4, 264, 1 << 27), (3, 36, 64, 89478480), (2, 4, (1 << 24) - 8, (1 << 24) - 8)])
+def test_pitches_of_which_a_tile_has_more_than_32_bits(pkg, dev, dtype, T, M, K, pitch):
+    """Sums of whole numbers up to 2^24, exact in any order."""
+    L = pkg._lib
+    lib = L.load()
+    torch.manual_seed(M)
+    x = torch.empty((T - 1) * pitch + K, dtype=dtype, device=dev).as_strided((T, K), (pitch, 1))
+    x.copy_(torch.randint(-1, 2, (T, K), device=dev))
+    w = torch.randint(-1, 2, (M, K), device=dev).to(dtype)
+    y = torch.zeros(T, M, dtype=dtype, device=dev)
+    q = Linear(io_dtype=pkg.scan._DTYPES[dtype], T=T, M=M, K=K, x_pitch=pitch, y_pitch=M, x=x.data_ptr(), weight=w.data_ptr(), y=y.data_ptr())
+    L.check(lib.mpa_linear_run(ctypes.byref(q), pkg.scan._stream(dev)), "mpa_linear_run")
+    want = torch.stack([torch.stack([(a.float() * b.float()).sum(dtype=torch.float64) for b in w]) for a in x])
+    assert torch.equal(y, want.to(dtype))
