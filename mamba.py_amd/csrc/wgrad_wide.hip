@@ -30,6 +30,7 @@ typedef short i16x4 __attribute__((ext_vector_type(4)));
 namespace {
 
 constexpr int kWide = 256, kNarrow = 128, kSlice = 32, kRing = 4, kMaxSplits = 16;
+constexpr uint32_t kNoColumn = 0x80000000u;  // an offset beyond every window
 constexpr int kFullFloats = kWide * kWide, kNarrowFloats = kNarrow * kWide;
 
 // Tiles of one kind of one job: `a` is the operand that gives the tile's rows (the narrow one of a narrow tile), `b` its columns.
@@ -107,19 +108,20 @@ __device__ __forceinline__ void wide_tile(const Region& g, int ta, int tb, int64
         const int row = 8 * wave + 2 * i + (lane >> 5), part = (lane & 31) ^ (2 * (row & 7));
         const int ca = a_begin + 8 * part, cb = b_begin + 8 * part;
         // (columns beyond the operand's last: of its last eight, into results that are not stored)
-        off[0][i] = NARROW && part >= kNarrow / 8 ? 0x80000000u : ((uint32_t)row * (uint32_t)g.lda + (uint32_t)min(ca, g.a_cols - 8)) * 2u;
+        off[0][i] = NARROW && part >= kNarrow / 8 ? kNoColumn : ((uint32_t)row * (uint32_t)g.lda + (uint32_t)min(ca, g.a_cols - 8)) * 2u;
         off[1][i] = ((uint32_t)row * (uint32_t)g.ldb + (uint32_t)min(cb, g.b_cols - 8)) * 2u;
     }
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)lds) + (uint32_t)wave * (8 * kPitch);
     // the next slice to request; rows from t_end on read as zeros
     const char* src[2] = {static_cast<const char*>(g.a) + t_begin * g.lda * 2, static_cast<const char*>(g.b) + t_begin * g.ldb * 2};
     int64_t left[2] = {(t_end - t_begin) * g.lda * 2, (t_end - t_begin) * g.ldb * 2};
+    // (a window ends at 2^31 bytes, where the columns that a narrow tile does not have are; a slice of 32 rows is shorter, see wide_plan)
     const int64_t ahead[2] = {kSlice * 2 * g.lda, kSlice * 2 * g.ldb};
     u32x4 window[2];
     auto aim = [&] {
 #pragma unroll
         for (int o = 0; o < 2; ++o) {
-            window[o] = lds_window(src[o], window_bytes(left[o], 0, 1));
+            window[o] = lds_window(src[o], left[o] <= 0 ? 0u : left[o] > kNoColumn ? kNoColumn : (uint32_t)left[o]);
             src[o] += ahead[o];
             left[o] -= ahead[o];
         }
@@ -287,6 +289,8 @@ __global__ void __launch_bounds__(256) wgrad_wide_sum_kernel(const WideParams p)
 bool wide_plan(WideParams& p, const mpa_wgrad_job* jobs, int n, int64_t T, float other_us) {
     p.regions = p.full = p.narrow = 0;
     p.T = T;
+    for (int i = 0; i < n; ++i)
+        if (std::max(jobs[i].ldp, jobs[i].ldq) >= (int64_t)kNoColumn / (kSlice * 2)) return false;
     auto add = [&](const mpa_wgrad_job& s, bool swapped, int a0, int a_blocks, int b_blocks, int& tiles) {
         if (a_blocks == 0 || b_blocks == 0) return;
         Region& r = p.region[p.regions++];
