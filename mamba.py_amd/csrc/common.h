@@ -79,7 +79,8 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes = 0
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 // 16 bytes a lane from memory into LDS, lane l's to lds + 16 * l (lds: a byte address, the same for the wave).
 __device__ __forceinline__ void load_to_lds(const u32x4& window, uint32_t at, uint32_t scalar, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(at), "s"(window), "s"(scalar) : "memory");
+    uint32_t spot;  // (m0, in which the load finds its place: named, so that the compiler keeps nothing there)
+    asm volatile("s_mov_b32 %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds" : "=&{m0}"(spot) : "s"(lds), "v"(at), "s"(window), "s"(scalar) : "memory");
 }
 __device__ __forceinline__ u32x4 lds_window(const void* base, uint32_t bytes) {
     const uint64_t a = reinterpret_cast<uint64_t>(base);

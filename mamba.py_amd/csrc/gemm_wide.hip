@@ -122,9 +122,11 @@ __global__ void __launch_bounds__(256, 1) gemm_wide_kernel(const GemmParams p) {
     };
     // Load i of the next chunk of x or W, in two parts with a product between them: where to (in place `to`), and the load (k beyond the last: zeros).
     // (A lone wave issues an instruction every five clocks, and a product takes sixteen: with all of it behind one, loads cost a tenth of the time.)
-    auto aim_load = [&](int i, uint32_t to) { asm volatile("s_add_u32 m0, %0, %1" ::"s"(to), "n"(i * 1024) : "scc"); };
+    // (m0 is where a load finds its place: the value is handed from one to the other in it, so that the compiler leaves it there)
+    uint32_t spot;
+    auto aim_load = [&](int i, uint32_t to) { asm volatile("s_add_u32 %0, %1, %2" : "={m0}"(spot) : "s"(to), "n"(i * 1024) : "scc"); };
     auto load = [&](const u32x4& window, uint32_t off, uint32_t k) {
-        asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(off), "s"(window), "s"(k) : "memory");
+        asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(off), "s"(window), "s"(k), "{m0}"(spot) : "memory");
     };
     auto load_x = [&](int i) { load(window_x, TAIL && next_k + kx >= p.K ? kNowhere : off_x[i], (uint32_t)next_k * 2u); };
     auto load_w = [&](int i) {

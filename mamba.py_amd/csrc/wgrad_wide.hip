@@ -128,8 +128,10 @@ __device__ __forceinline__ void wide_tile(const Region& g, int ta, int tb, int64
     };
     // load i of the stage that aim() was called for, in two parts with a product between them: where to, and the load.  (A lone wave
     // issues an instruction every five clocks, and a product takes sixteen.)
-    auto aim_load = [&](int i, uint32_t to) { asm volatile("s_add_u32 m0, %0, %1" ::"s"(to), "n"((i >> 2) * kOperand + (i & 3) * 2 * kPitch) : "scc"); };
-    auto load = [&](int i) { asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off[i >> 2][i & 3]), "s"(window[i >> 2]) : "memory"); };
+    // (m0 is where a load finds its place: the value is handed from one to the other in it, so that the compiler leaves it there)
+    uint32_t spot;
+    auto aim_load = [&](int i, uint32_t to) { asm volatile("s_add_u32 %0, %1, %2" : "={m0}"(spot) : "s"(to), "n"((i >> 2) * kOperand + (i & 3) * 2 * kPitch) : "scc"); };
+    auto load = [&](int i) { asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off[i >> 2][i & 3]), "s"(window[i >> 2]), "{m0}"(spot) : "memory"); };
     // reads: lane -> row 4 * (lane / 16) + lane % 16 / 4 of the first sixteen (the other sixteen behind them), four columns from 4 * (lane % 4)
     const int rowl = 4 * (lane >> 4) + ((lane & 15) >> 2), r7 = rowl & 7;
     uint32_t at_a[kA], at_b[kB];
