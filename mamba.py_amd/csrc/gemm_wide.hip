@@ -321,19 +321,33 @@ float gemm_plan(const mpa_gemm* s, GemmParams& p) {
 
 }  // namespace
 
-// Against the library, at widths 256 to 1024 and 1500 to 24 000 rows, the products of a layer (W as M x K: 4d x d, d x 2d; as K x M: 2d x d, d x 4d) and
-// 50 280 x d; its time over the library's:
-//   K up to 512       0.4 to 0.98
-//   rows of x or W that are not whole 128 bytes (K % 64), or of y (M % 64; of 50 280 columns up to 4000 rows, 0.96 to 1.09 above): 0.4 to 0.9
-//                     where tiles fill the chip.  The library runs these at 500 to 900 TFLOP/s, 700 is what it is taken for, and 18 us at least (host).
+// Against the library, at 2800 products of 64 to 70 000 rows, 128 to 128 000 columns and a K of 64 to 4096 (W as M x K and, up to 4096 columns, as
+// K x M), among them the products of a layer of widths 64 to 1024 (W as M x K: 4d x d, d x 2d; as K x M: 2d x d, d x 4d) and 50 280 x d; its time
+// over the library's:
+//   K up to 512       0.3 to 1.03 (14 of 1094 up to 1.12, 2048 columns or more by two rounds or three), layers 0.4 to 0.96 (one of 155 1.05).  Not where it is slower: 2048 columns or more in whole tiles over more
+//                     than one round, K 64 to 256 (0.57 to 1.42: y is what takes the time, and the library is as fast there), and more than 51 200
+//                     columns by a K below 128 (up to 1.18).
+//   rows of x or W that are not whole 128 bytes (K % 64), or of y (M % 64; up to 4000 rows or 4096 columns): 0.4 to 1.02
+//                     where tiles fill the chip.  The library runs these at 400 to 900 TFLOP/s, 700 is what it is taken for, and 18 us at least (host).
+//                     With W as M x K in whole tiles it reaches up to 1340 (0.83 to 1.22): taken for 1400, which leaves its parts of rounds.  Of more than
+//                     51 200 columns some are 1.01 to 1.14.
 //   others            both take tiles of this size, and whole rounds of them are 0 to 9 % faster there; where this kernel saves a part of a
 //                     round by halves, up to K = 1024 (a longer sum leaves the first loads and the stores a smaller part): 0.61 to 0.98
 extern "C" int mpa_gemm_faster(const mpa_gemm* s) {
     if (gemm_check(s) != MPA_OK) return 0;
     GemmParams p{};
     const float us = gemm_plan(s, p);
-    if (s->K <= 512) return 1;
-    if (s->K % 64 || (s->M % 64 && (s->M <= 4096 || s->T <= 4096))) return us + 3.0f < std::max(18.0f, 6.0f + 2e-9f * (float)s->T * (float)s->M * (float)s->K / 0.7f);
+    constexpr int64_t kMostM = 51200;
+    const bool whole = s->M % kTileSide == 0;
+    if (s->K <= 512) {
+        const int tiles = p.tiles_t * p.tiles_m, most = tiles <= 2 * kCUs && !s->weight_kxm ? 384 : 256;
+        if (whole && s->M >= 2048 && s->K <= most && s->K % 64 == 0 && tiles > kCUs) return 0;
+        return s->M <= kMostM || s->K >= 128;
+    }
+    if (s->K % 64 || (s->M % 64 && (s->M <= 4096 || s->T <= 4096))) {
+        const float rate = whole && !s->weight_kxm ? 1.4f : 0.7f;
+        return s->M <= kMostM && us + 3.0f < std::max(18.0f, 6.0f + 2e-9f * (float)s->T * (float)s->M * (float)s->K / rate);
+    }
     return s->K <= 1024 && us <= 0.93f * (float)((p.tiles_t * p.tiles_m + kCUs - 1) / kCUs) * tile_us((p.K + kStageK - 1) / kStageK);
 }
 
