@@ -487,7 +487,7 @@ __global__ void __launch_bounds__(256) sscan_bwd_finish_kernel(
 // states per lane of the backward kernels (at most 4) and, for that choice, how a thin launch
 // is cut: half of the CUs or fewer covered (the first pass of a cut costs a quarter of the second)
 static constexpr int kBwdThin = 2;
-static constexpr int64_t kFillTiles = 2, kUnevenTiles = 8, kShortest = 3, kCutTiles = 7, kCutMany = 28, kCutTwo = 24;
+static constexpr int64_t kFillTiles = 2, kUnevenTiles = 8, kShortest = 3, kCutTiles = 7, kCutMany = 32, kCutTwo = 28;
 static int bwd_states_per_lane(const mpa_sscan_shape* s) {
     const int ns = pick_states_per_lane(s->dstate, 4, s->plan_states_per_lane);
     return ns < 0 ? 4 : ns;
@@ -522,12 +522,13 @@ static int64_t uneven_tiles(const mpa_sscan_shape* s) {
 // Segments of equal parts where half of the CUs or fewer are covered: as many as the CUs take in one round, of three tiles (48 steps) at least.
 // A tile is 2 to 2.5 us of the backward and a tile of the carry pass less than half of that; the carry pass and the chaining of its end states are
 // launches of 5 to 10 us, of which two segments need one, and which the passes over a wide d_state share.  Backward of a call, uncut (from 32 tiles on:
-// in segments of eight tiles at least) and now: 4 x 396 x 101 with 24 states 126 -> 50 us, 1 x 400 x 256 with 64 289 -> 91, 2 x 420 x 1000 70 -> 37,
-// 8 x 420 x 1000 72 -> 60, 10 x 580 x 148 gated bfloat16 63 -> 52, 5 x 1205 x 77 49.5 -> 44, 1 x 2000 x 64 with 32 94 -> 69.  Segments of two tiles are
-// within 1 us of three.  Fewer than 28 tiles in all passes (68 us) are left whole, 24 where there are two segments: the launches are 4 us of the host each
-// as well, which is what a shorter call waits for (2 x 390 x 1024, 25 tiles, forward and backward in a loop: 87 us whole; in segments 57 where the host
-// is fast and 91 where it is slow), and below seven the pipeline's fill is what a segment takes (48 states: 2 x 100 x 1000 89 -> 76, 2 x 70 x 1000 71.5
-// and 71.2).
+// in segments of eight tiles at least) and now: 4 x 396 x 101 with 24 states 126 -> 50 us, 1 x 400 x 256 with 64 289 -> 91, 10 x 580 x 148 gated
+// bfloat16 63 -> 52, 5 x 1205 x 77 49.5 -> 44, 1 x 2000 x 64 with 32 94 -> 69.  Segments of two tiles are within 1 us of three.
+// Fewer than 32 tiles in all passes (77 us) are left whole, 28 where there are two segments: the launches are 4 us of the host each as well, which is
+// what a shorter call waits for.  Forward and backward in a loop, whole and in segments, where the host is slow: 25 tiles, 2 x 390 x 1024, 87 us and
+// 91; 29, 2 x 460 x 500, 91 and 98; 30, 1 x 480 x 64, 92 and 98; two segments of 25, 6 x 400 x 1000, 91 and 94, of 28, 8 x 440 x 1000, 103 and 92.
+// (Where it is fast, the first was 57 in segments.)  Below seven tiles a pass the pipeline's fill is what a segment takes (48 states: 2 x 100 x 1000
+// 89 -> 76, 2 x 70 x 1000 71.5 and 71.2).
 static int64_t even_segments(const mpa_sscan_shape* s) {
     const int64_t rows = s->batch * ((s->dim + kWave - 1) / kWave), ntiles = (s->seqlen + kTile - 1) / kTile;
     if (s->plan_segments > 0) return s->plan_segments;

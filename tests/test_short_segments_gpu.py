@@ -10,12 +10,15 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("Bs,L,ED,N,kw", [
-    (1, 432, 64, 16, {}), (1, 433, 64, 16, {}),                        # 27 tiles: whole; 28, the last of one step
-    (3, 450, 70, 16, dict(reverse=True)), (85, 448, 40, 9, {}),        # 29; 85 workgroups: three segments
-    (86, 368, 33, 16, {}), (86, 369, 33, 16, dict(reverse=True)), (128, 393, 64, 16, {}),  # 86 and 128: two, from 24 tiles on
+    (1, 432, 64, 16, {}), (1, 433, 64, 16, {}), (3, 450, 70, 16, dict(reverse=True)), (85, 448, 40, 9, {}),  # 27 to 29 tiles: whole
+    (1, 496, 64, 16, {}), (1, 497, 64, 16, {}),                        # 31 tiles: whole; 32, the last of one step
+    (3, 520, 70, 16, dict(reverse=True)), (85, 500, 40, 9, {}),        # 33; 85 workgroups: three segments
+    (86, 368, 33, 16, {}), (86, 369, 33, 16, dict(reverse=True)), (128, 393, 64, 16, {}),
+    (86, 432, 33, 16, {}), (86, 433, 33, 16, dict(reverse=True)), (128, 450, 64, 16, {}),  # 86 and 128: two, from 28 tiles on
     (129, 393, 20, 16, {}),                                            # 129: not this cut
-    (2, 208, 90, 24, {}), (2, 209, 90, 24, dict(reverse=True)),        # two passes over the states: from fourteen tiles on
-    (2, 96, 65, 64, {}), (2, 97, 65, 64, {}), (1, 250, 10, 130, {}),   # four: from seven; two launches of the carry pass and more
+    (2, 208, 90, 24, {}), (2, 209, 90, 24, dict(reverse=True)), (2, 241, 90, 24, dict(reverse=True)),  # two passes over the states: from sixteen tiles on
+    (2, 96, 65, 64, {}), (2, 97, 65, 64, {}), (2, 113, 65, 64, {}),    # four: from eight
+    (2, 96, 33, 80, {}), (2, 97, 33, 80, {}), (1, 250, 10, 130, {}),   # five: from seven; two launches of the carry pass and more
     (1, 3100, 20, 16, {}), (1, 2999, 64, 40, dict(reverse=True)),      # 64 segments, of four tiles and one that is shorter
 ])
 def test_against_oracle(pkg, dev, Bs, L, ED, N, kw):
@@ -28,7 +31,7 @@ def test_against_oracle(pkg, dev, Bs, L, ED, N, kw):
         assert rel_err(got[k], r) <= TOL[torch.float32], k
 
 
-@pytest.mark.parametrize("Bs,L,ED,N,dtype,reverse", [(2, 460, 100, 16, torch.bfloat16, False), (1, 137, 1500, 48, torch.float32, True),
+@pytest.mark.parametrize("Bs,L,ED,N,dtype,reverse", [(2, 460, 100, 16, torch.bfloat16, False), (2, 560, 100, 16, torch.bfloat16, False), (1, 137, 1500, 48, torch.float32, True),
                                                      (5, 300, 250, 32, torch.bfloat16, True), (60, 400, 100, 16, torch.float32, False)])
 def test_gated_against_uncut(pkg, dev, Bs, L, ED, N, dtype, reverse):
     g = torch.Generator().manual_seed(Bs)
