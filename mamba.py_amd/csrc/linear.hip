@@ -532,6 +532,9 @@ static int launch_linear(LinearParams p, const LinearForm& f, hipStream_t st) {
 // 12.8 us for 14.4, 1400 of 512 10.7 for 11.7, 2048 of 400 11.0 for 12.1; in one round the small ones: 700 of 640 9.1 for 11.4; with
 // more than one round of either there is no difference).  Of the plain products in training it makes no difference (four layers of
 // 1400 steps of width 512, forward and backward, 862 us of kernels and 863), and they take them by the same rule.
+// Tiles of 32 x 32 with K in four shares fill a CU's LDS: where they are more than a round of the CUs, 64 x 32 at any number (out_proj, 400 steps of width
+// 640: 10.3 us in 260 tiles of 32 x 32, 7.5 in 140; 9.3 with two stages in LDS, of which a CU has two.  700 of 392 9.8 and 6.7, x_proj, 4950
+// of 128, 7.2 and 4.7; float32 0.73 to 0.83 of the time, input gradients 0.74 to 0.94).
 template <typename IO>
 static int dispatch_linear(const LinearParams& p, const LinearForm& f, hipStream_t st) {
     auto tiles = [&](int bt, int bm) { return (int64_t)((p.T + bt - 1) / bt) * ((p.M + bm - 1) / bm); };
@@ -544,7 +547,7 @@ static int dispatch_linear(const LinearParams& p, const LinearForm& f, hipStream
     if (p.K <= 128) return launch_linear<IO, 64, 64, 1>(p, f, st);  // (one or two stages: nothing to split)
     const bool one = p.K >= 1024;
     if (tiles(64, 64) >= kFull) return one && tiles(64, 64) <= 256 ? launch_linear<IO, 64, 64, 2>(p, f, st) : launch_linear<IO, 64, 64, 1>(p, f, st);
-    if (tiles(64, 32) >= kFull) return one && tiles(64, 32) <= 256 ? launch_linear<IO, 64, 32, 4>(p, f, st) : launch_linear<IO, 64, 32, 2>(p, f, st);
+    if (tiles(64, 32) >= kFull || tiles(32, 32) > 256) return one && tiles(64, 32) <= 256 ? launch_linear<IO, 64, 32, 4>(p, f, st) : launch_linear<IO, 64, 32, 2>(p, f, st);
     return launch_linear<IO, 32, 32, 4>(p, f, st);
 }
 

@@ -15,6 +15,7 @@ pytestmark = pytest.mark.gpu
     (1, 4, 8, 0), (1, 36, 64, 8), (65, 132, 72, 0), (63, 100, 128, 16), (64, 128, 136, 0), (70, 132, 192, 8), (33, 64, 200, 0), (64, 32, 256, 8),
     (40, 64, 320, 0), (129, 260, 448, 8), (31, 36, 520, 0), (200, 68, 776, 8),    # one to seven stages of a share, one to four shares of K
     (300, 2560, 264, 0), (1400, 772, 1032, 8), (1400, 420, 1032, 0),               # 64 x 128; more than one round of 64 x 64 and of 64 x 32
+    (400, 640, 1280, 0), (700, 392, 784, 8), (3000, 80, 264, 0),                   # 64 x 32, where 32 x 32 are more than a round
     (1100, 1540, 136, 0), (8200, 516, 72, 0),                                      # 128 x 128; W walked first
 ])
 def test_products_against_float64(pkg, dev, dtype, T, M, K, pad):
