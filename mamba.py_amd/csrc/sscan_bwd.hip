@@ -487,7 +487,7 @@ __global__ void __launch_bounds__(256) sscan_bwd_finish_kernel(
 // states per lane of the backward kernels (at most 4) and, for that choice, how a thin launch
 // is cut: half of the CUs or fewer covered (the first pass of a cut costs a quarter of the second)
 static constexpr int kBwdThin = 2;
-static constexpr int64_t kFillTiles = 2, kUnevenTiles = 8, kShortest = 3, kCutTiles = 7, kCutMany = 32, kCutTwo = 28;
+static constexpr int64_t kFillTiles = 2, kUnevenTiles = 8, kShortest = 3, kManySegments = 32, kLongOfMany = 8, kCutTiles = 7, kCutMany = 32, kCutTwo = 28;
 static int bwd_states_per_lane(const mpa_sscan_shape* s) {
     const int ns = pick_states_per_lane(s->dstate, 4, s->plan_states_per_lane);
     return ns < 0 ? 4 : ns;
@@ -524,6 +524,8 @@ static int64_t uneven_tiles(const mpa_sscan_shape* s) {
 // launches of 5 to 10 us, of which two segments need one, and which the passes over a wide d_state share.  Backward of a call, uncut (from 32 tiles on:
 // in segments of eight tiles at least) and now: 4 x 396 x 101 with 24 states 126 -> 50 us, 1 x 400 x 256 with 64 289 -> 91, 10 x 580 x 148 gated
 // bfloat16 63 -> 52, 5 x 1205 x 77 49.5 -> 44, 1 x 2000 x 64 with 32 94 -> 69.  Segments of two tiles are within 1 us of three.
+// More than 32 segments only of eight tiles or more: chaining their end states and adding their parts of dA is time by itself (forward and backward of
+// 4 x 4096 x 40, 64 segments 92 us, 32 84; 3 x 2900 x 64, 61 85, 32 76; 1 x 16384 x 32, 64 126, 32 159).
 // Fewer than 32 tiles in all passes (77 us) are left whole, 28 where there are two segments: the launches are 4 us of the host each as well, which is
 // what a shorter call waits for.  Forward and backward in a loop, whole and in segments, where the host is slow: 25 tiles, 2 x 390 x 1024, 87 us and
 // 91; 29, 2 x 460 x 500, 91 and 98; 30, 1 x 480 x 64, 92 and 98; two segments of 25, 6 x 400 x 1000, 91 and 94, of 28, 8 x 440 x 1000, 103 and 92.
@@ -536,7 +538,7 @@ static int64_t even_segments(const mpa_sscan_shape* s) {
     if (rows * kBwdThin > 256) return 1;
     const int64_t most = std::min<int64_t>(256 / rows, 64);
     if (ntiles < kCutTiles || ntiles * passes < (most > 2 ? kCutMany : kCutTwo)) return 1;
-    return std::min(most, (ntiles + kShortest - 1) / kShortest);
+    return std::min(most, std::max(std::min((ntiles + kShortest - 1) / kShortest, kManySegments), ntiles / kLongOfMany));
 }
 // The cut exists on the fast kernel only.
 static SegPlan bwd_seg_plan(const mpa_sscan_shape* s) {
