@@ -322,7 +322,7 @@ bool wide_plan(WideParams& p, const mpa_wgrad_job* jobs, int n, int64_t T, float
     // loads and the sums' way out; one workgroup a CU, the narrow ones on the CUs that the last round of whole ones leaves; the sums of the parts are
     // read at 4.5 TB/s.
     constexpr int kCUs = 256;
-    constexpr float kOnceUs = 12.0f;  // two launches, what the sums take beyond their bytes, and 4 us for being sure
+    constexpr float kOnceUs = 13.0f;  // two launches, what the sums take beyond their bytes, and 5 us for being sure (4: 6000 rows of width 512 42.2 us -> 44.5)
     const int64_t slices = (T + kSlice - 1) / kSlice;
     float best = 1e30f;
     for (int s = 1; s <= kMaxSplits && (s == 1 || (slices >= 8 * s && p.full * (s - 1) <= 2 * kCUs)); ++s) {
