@@ -11,15 +11,20 @@
 //
 // Tile: BT steps x BM rows of W per workgroup, each wave 32 * RT x 32 of it (2 * RT x 2 MFMA tiles of 16 x 16, W as the left
 // operand, so that a lane's four results are neighbours in y) over its share of K.  K runs in stages of 128 bytes per
-// share: a stage is staged in LDS in 16-byte parts, rotated by the row (part ^ (row & 7)) so that the operand reads, one row
-// per lane, fall on different banks; D stages are in registers on their way in, two in LDS.
+// share: a stage is in LDS in 16-byte parts, rotated by the row (part ^ (row & 7)) so that the operand reads, one row
+// per lane, fall on different banks.  Rows that are multiplied as they stand in memory (with a factor or without) go to LDS directly, three stages:
+// two are on their way while one is multiplied, by one barrier a stage.  What has to be changed between memory and LDS (rows that are
+// normalised, W by columns) passes through D sets of registers, two stages in LDS.
 //
-// At 512 steps of width 768, recorded in a graph with the weights of 24 layers: in_proj with the rows' factor 9.7 us (11.8 with rows
-// of the float32 stream normalised on their way, twice the bytes and their conversion between load and LDS; 32 steps 6.3 for 8.1,
-// 2048 steps 20.8 for 26.3), x_proj 7.1, dt_proj 3.7, out_proj with the residual stream 8.8 (8.5 without); the library's products
-// alone 9.3, 7.1, 3.9 and 8.0.  Four stages in registers instead of two change nothing: it is the way of a stage through LDS and the
-// barrier.  What the kernels save is the norm between the layers (6 us) and three quarters of the host time (24 layers of library
-// calls: 2.1 ms, all of it host).
+// Width 768, recorded in a graph with the operands of 24 layers, through registers / directly / the library's product alone:
+//              in_proj with the rows' factor   out_proj, residual, scaled rows   x_proj         dt_proj
+//   32 steps          6.4 /  5.9 /  7.0 us           7.8 /  6.2 /  7.2            6.9 / 5.4      3.6 / 3.2
+//   512               9.6 /  8.2 /  9.0              9.1 /  8.0 /  7.9            7.3 / 5.7      3.8 / 3.4
+//   2048             23.4 / 24.3 / 17.1             19.4 / 18.5 / 17.0            7.6 / 6.6      6.3 / 5.8
+// (In a whole pass of 512 steps, under the profiler, they are 10.3 and 9.2.  The third stage in LDS leaves two workgroups a CU instead of three of 64 x
+// 128: in_proj in 640 to 768 such tiles is 2 to 6 % slower for it, out_proj of the same steps 5 to 7 % faster.)  What bounds the short
+// ones is latency: the launch, the first rows from memory, a barrier a stage, the way of the results.  Besides, the kernels save the norm between the
+// layers (6 us) and three quarters of the host time (24 layers of library calls: 2.1 ms, all of it host).
 // float32 runs the same tiles with sixteen times less of the matrix unit's rate (16x16x4, 150 TFLOP/s): the same host
 // time is saved, until the product itself is longer than a library call (a training layer of 1614 steps and width 424
 // 0.69 ms, 0.81 with library calls; 168 steps of ten layers of width 640 without gradients 0.63 and 0.85 ms).

@@ -506,9 +506,9 @@ static mpa_sscan_shape fast_block_shape(const mpa_sscan_shape* s) {
 // time of a long one; the long ones are launched first.  Workgroups go to the 32 shader engines in turn and wait there for one of its eight CUs
 // (at 210 workgroups, sized as if any free CU took the next one, the cut call was 6 to 10 % slower than the uncut one), so k short parts in turn
 // on each of the CUs that are left in an engine have to be done with the long one; each fills its pipeline first.
-// Backward of a call, uncut and cut: 8 x 2048 x 1536 float32 352 -> 332 us, 8 x 1000 x 1536 gated bfloat16 188 -> 176, 5 x 1500 x 1984 224 -> 185,
-// 13 x 2000 x 640 with 24 states 709 -> 566; with seven short parts in turn 7 x 4096 x 1920 676 -> 642, 7 x 2048 x 1920 348 -> 336, and no gain
-// below eight tiles (8 x 700 x 1536, ten: 133 and 134).
+// Backward of a call (forward and backward in a loop less the forward), uncut and cut: 8 x 2048 x 1536 float32 291 -> 257 us, 8 x 1000 x 1536 gated
+// bfloat16 178 -> 164, 5 x 1500 x 1984 224 -> 186, 13 x 2000 x 640 with 24 states 580 -> 458; with seven short parts in turn 7 x 4096 x 1920 575 -> 539,
+// 7 x 2048 x 1920 292 -> 282, and little below eight tiles (8 x 700 x 1536, ten: 109 and 103).
 // Returns the tiles of the short part, 0: not cut.
 static int64_t uneven_tiles(const mpa_sscan_shape* s) {
     constexpr int64_t kCUs = 256, kEngines = 32, kEngineCUs = kCUs / kEngines;
